@@ -122,7 +122,9 @@ class _FxLowering:
     # ---- shapes ---------------------------------------------------------------------
     def _propagate_shapes(self):
         torch = self.torch
-        if all("example_value" in n.meta or "tensor_meta" in n.meta for n in self.gm.graph.nodes if n.op not in ("output",)):
+        # only dynamo's annotation is that of these inputs: a "tensor_meta" may be left from a lowering of the same graph for
+        # other shapes, whose kernels would read past the ends of smaller inputs
+        if all("example_value" in n.meta for n in self.gm.graph.nodes if n.op not in ("output",)):
             return
         if any(not isinstance(a, (torch.Tensor, int, float, bool)) for a in self.example_inputs):
             return  # symbolic inputs: dynamo has already annotated the graph

@@ -424,6 +424,19 @@ def test_torch_models_of_one_name_and_shape_get_libraries_of_their_own(tmp_path,
     assert again.lib_path == first.lib_path
 
 
+def test_a_torch_program_is_lowered_for_the_shapes_of_each_call():
+    # the traced graph is kept between calls: what the lowering for 40 rows noted on its nodes must not size the kernels for 3
+    class Lin(torch.nn.Module):
+        def forward(self, x, w):
+            return torch.nn.functional.linear(x, w)
+
+    program = docc_torch.compile_torch(Lin(), None, target="rocm")
+    w = torch.randn(24, 16)
+    for rows in (40, 3):
+        node = program.to_sdfg(torch.randn(rows, 16), w).library_nodes()[0]
+        assert node["code"] == "GEMM" and int(node["m"]) == rows
+
+
 def test_reductions_and_softmax_pieces_used_on_their_own():
     @native
     def stats(x):
