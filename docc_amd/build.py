@@ -46,6 +46,12 @@ KERNEL_FAMILIES = {
     "gemm_bf16_async_big_epilogue": "gemm_bf16_async_big_epilogue.hip",
     "gemm_f32_big": "gemm_f32_big.hip",
     "gemm_f32_big_epilogue": "gemm_f32_big_epilogue.hip",
+    "gemm_finish": "gemm_finish.hip",
+    "gemm_bf16_async_finish": "gemm_bf16_async_finish.hip",
+    "gemm_bf16_async_big_finish": "gemm_bf16_async_big_finish.hip",
+    "gemm_f32_finish": "gemm_f32_finish.hip",
+    "gemm_f32_big_finish": "gemm_f32_big_finish.hip",
+    "layernorm": "layernorm.hip",
     "conv2d": "conv2d.hip",
     "attention": "attention.hip",
     "elementwise": "elementwise.hip",
@@ -67,6 +73,8 @@ FAMILY_FLAGS = {
     "gemm_f64_epilogue": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "gemm_f32_epilogue": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "gemm_bf16_async_epilogue": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+    "gemm_bf16_async_finish": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+    "gemm_f32_finish": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "conv2d": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "attention": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "gemm_skinny": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],

@@ -28,6 +28,13 @@ typedef uint16_t u16x8a __attribute__((ext_vector_type(8)));
 typedef short s16x4a __attribute__((ext_vector_type(4)));
 typedef short s16x8a __attribute__((ext_vector_type(8)));
 
+// what the store of a kernel takes: C and the BLAS scalars (with bias / activation in the "_e" variants), or a GemmFinish
+#ifdef DOCC_GEMM_FINISH
+#define DOCC_STORE_PARAMS(T) float alpha, const GemmFinish& fin
+#else
+#define DOCC_STORE_PARAMS(T) long ldc, T alpha, T beta, const T* bias, int act
+#endif
+
 template <typename T>
 struct AsyncTraits;
 template <>
@@ -182,8 +189,7 @@ struct AsyncGemmKernel {
     static_assert(!SPREAD || STAGES >= 3, "copies dealt over a K-step need a stage that nobody reads meanwhile");
 
     static __device__ __forceinline__ void run(const T* __restrict__ A, const T* __restrict__ B, out_t* __restrict__ C,
-                                               long M, long N, long K, long lda, long ldb, long ldc, out_t alpha,
-                                               out_t beta, const out_t* bias, int act) {
+                                               long M, long N, long K, long lda, long ldb, DOCC_STORE_PARAMS(out_t)) {
         extern __shared__ __attribute__((aligned(16))) unsigned char docc_gemm_lds[];
         T* const lds = reinterpret_cast<T*>(docc_gemm_lds);
 
@@ -488,9 +494,17 @@ struct AsyncGemmKernel {
         kstep(kt, std::integral_constant<int, 2>{});
 
         // ---- epilogue ------------------------------------------------------------------------------
+#ifdef DOCC_GEMM_FINISH
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();   // every wave's reads and copies of the ring are over: it holds the rows on their way out
+        gemm_finish_wave<TM, TN, MT, X::NACC>(fin, alpha, M, N, m0 + wm * WTM, n0 + wn * WTN, lidx, lane,
+                                              reinterpret_cast<float*>(docc_gemm_lds) + wave * FinishShape<TM, TN, MT>::WAVE_FLOATS, acc,
+                                              [&](int r) { return Mfma<float>::acc_row(lane, r); });
+#else
         gemm_store_wave<kGemmEpilogue, TM, TN, MT, X::NACC>(C, ldc, M, N, m0 + wm * WTM, n0 + wn * WTN, lidx, alpha, beta, bias, act, acc, [&](int r) {
             return (sizeof(T) == 8) ? Mfma<double>::acc_row(lane, r) : Mfma<float>::acc_row(lane, r);
         });
+#endif
     }
 };
 
@@ -527,3 +541,14 @@ struct AsyncGemmKernel {
     DOCC_AGEMM_ONE(PREFIX, T, OT, BM, BN, BK, WM, WN, ST, false, true, nt)    \
     DOCC_AGEMM_ONE(PREFIX, T, OT, BM, BN, BK, WM, WN, ST, true, false, tn)    \
     DOCC_AGEMM_ONE(PREFIX, T, OT, BM, BN, BK, WM, WN, ST, true, true, tt)
+
+// with the store of gemm_finish.h (one product a launch): docc_<prefix>a_<BM>x<BN>x<BK>s<STAGES>_<nn|nt>_f, A stored by rows
+#define DOCC_AGEMM_FINISH_ONE(PREFIX, T, OT, BM, BN, BK, WM, WN, ST, TB, TAG)                                       \
+    extern "C" __global__ __launch_bounds__(64 * WM * WN) void DOCC_GEMM_NAME(docc_##PREFIX##a_##BM##x##BN##x##BK##s##ST##_##TAG)(  \
+        const T* A, const T* B, long M, long N, long K, long lda, long ldb, float alpha, docc_k::GemmFinish fin) {  \
+        docc_k::AsyncGemmKernel<T, BM, BN, BK, WM, WN, ST, false, TB>::run(A, B, nullptr, M, N, K, lda, ldb, alpha, fin); \
+    }
+
+#define DOCC_AGEMM_FINISH_CONFIG(PREFIX, T, OT, BM, BN, BK, WM, WN, ST)            \
+    DOCC_AGEMM_FINISH_ONE(PREFIX, T, OT, BM, BN, BK, WM, WN, ST, false, nn)          \
+    DOCC_AGEMM_FINISH_ONE(PREFIX, T, OT, BM, BN, BK, WM, WN, ST, true, nt)

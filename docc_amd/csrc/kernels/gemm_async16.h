@@ -48,7 +48,7 @@ struct AsyncGemm16Kernel {
     static_assert((STAGES - 2) * LOADS + EARLY < 64, "vmcnt holds at most 63 outstanding loads");
 
     static __device__ __forceinline__ void run(const T* __restrict__ A, const T* __restrict__ B, float* __restrict__ C, long M, long N,
-                                               long K, long lda, long ldb, long ldc, float alpha, float beta, const float* bias, int act) {
+                                               long K, long lda, long ldb, DOCC_STORE_PARAMS(float)) {
         extern __shared__ __attribute__((aligned(16))) unsigned char docc_gemm_lds[];
         T* const lds = reinterpret_cast<T*>(docc_gemm_lds);
 
@@ -170,8 +170,15 @@ struct AsyncGemm16Kernel {
         // the copies that nobody waits for
         asm volatile("s_nop 15\n s_nop 15\n s_waitcnt vmcnt(0)" ::: "memory");
         // 16 x 16 fp32 result tile: register r of lane l is row 4 (l / 16) + r, column l % 16
+#ifdef DOCC_GEMM_FINISH
+        __syncthreads();
+        gemm_finish_wave<TM, TN, MT, NACC>(fin, alpha, M, N, m0 + wm * WTM, n0 + wn * WTN, lidx, lane,
+                                           reinterpret_cast<float*>(docc_gemm_lds) + wave * FinishShape<TM, TN, MT>::WAVE_FLOATS, acc,
+                                           [&](int r) { return 4 * lg + r; });
+#else
         gemm_store_wave<kGemmEpilogue, TM, TN, MT, NACC>(C, ldc, M, N, m0 + wm * WTM, n0 + wn * WTN, lidx, alpha, beta, bias, act, acc,
                                                          [&](int r) { return 4 * lg + r; });
+#endif
     }
 };
 
@@ -192,3 +199,10 @@ struct AsyncGemm16Kernel {
     DOCC_AGEMM16_ONE(BM, BN, WM, WN, ST, false, true, nt)  \
     DOCC_AGEMM16_ONE(BM, BN, WM, WN, ST, true, false, tn)  \
     DOCC_AGEMM16_ONE(BM, BN, WM, WN, ST, true, true, tt)
+
+// with the store of gemm_finish.h: docc_bgemma_<BM>x<BN>x32q<STAGES>_<nn|nt>_f
+#define DOCC_AGEMM16_FINISH_ONE(BM, BN, WM, WN, ST, TB, TAG)                                                                    \
+    extern "C" __global__ __launch_bounds__(64 * WM * WN) void DOCC_GEMM_NAME(docc_bgemma_##BM##x##BN##x32q##ST##_##TAG)(       \
+        const uint16_t* A, const uint16_t* B, long M, long N, long K, long lda, long ldb, float alpha, docc_k::GemmFinish fin) { \
+        docc_k::AsyncGemm16Kernel<BM, BN, WM, WN, ST, false, TB>::run(A, B, nullptr, M, N, K, lda, ldb, alpha, fin);            \
+    }

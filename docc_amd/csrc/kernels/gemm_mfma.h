@@ -21,11 +21,17 @@
 #pragma once
 
 #include "elementwise_ops.h"
+#ifdef DOCC_GEMM_FINISH
+#include "gemm_finish.h"
+#endif
 
 // A translation unit compiled with DOCC_GEMM_EPILOGUE holds the epilogue variants of its kernels:
 // same tiles, names with the suffix "_e", C = act(alpha A B + beta C + bias) in the store.
+// Compiled with DOCC_GEMM_FINISH the asynchronous kernels have the store of gemm_finish.h instead (suffix "_f").
 #ifdef DOCC_GEMM_EPILOGUE
 #define DOCC_GEMM_NAME(base) base##_e
+#elif defined(DOCC_GEMM_FINISH)
+#define DOCC_GEMM_NAME(base) base##_f
 #else
 #define DOCC_GEMM_NAME(base) base
 #endif

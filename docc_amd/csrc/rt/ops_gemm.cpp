@@ -30,6 +30,23 @@ size_t gemm_lds_bytes(const TileConfig& c, bool ta, bool tb, size_t elem) {
     return 2 * (a_elems + b_elems) * elem;
 }
 
+// What GemmFinish of csrc/kernels/gemm_finish.h holds: the rest of a layer behind a product.
+struct LinearFinish {
+    const void *bias, *residual;
+    void* out;
+    int flags, act;
+};
+enum { kBiasBf16 = 1, kResidualBf16 = 2, kOutBf16 = 4, kRoundBeforeAct = 8, kRoundAfterAct = 16 };
+
+// the chain on `parts` fp32 products in memory
+int finish_parts(hipStream_t s, const void* P, int64_t m, int64_t n, int parts, float alpha, const LinearFinish& f) {
+    const bool vec = n % 8 == 0 && ((uintptr_t) P | (uintptr_t) f.bias | (uintptr_t) f.residual | (uintptr_t) f.out) % 16 == 0;
+    const int64_t units = m * n / (vec ? 8 : 1);
+    int64_t blocks = (units + 255) / 256;
+    if (blocks > 8192) blocks = 8192;
+    return launch(vec ? "docc_gemm_finish_v8" : "docc_gemm_finish_v1", (uint32_t) blocks, 1, 1, 256, 0, s, P, (long) m, (long) n, parts, alpha, f);
+}
+
 // One output column or one output row: the matrix-vector kernels (csrc/kernels/gemv.hip). Returns 1 when the
 // shape is not one of theirs (the caller goes on to the tiled kernels), 0 or an error code otherwise.
 template <typename T, typename S>
@@ -188,7 +205,8 @@ template <typename T, typename S = T>
 int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int trans_b, int64_t m, int64_t n,
                 int64_t k, S alpha, const T* A, int64_t lda, const T* B, int64_t ldb, S beta, S* C, int64_t ldc,
                 TileConfig (*pick)(int64_t m, int64_t n, int64_t batch, bool aligned, int force), const S* bias = nullptr,
-                int activation = -1, int64_t batch = 1, int64_t batch_a = 0, int64_t batch_b = 0, int64_t batch_c = 0) {
+                int activation = -1, int64_t batch = 1, int64_t batch_a = 0, int64_t batch_b = 0, int64_t batch_c = 0,
+                const LinearFinish* fin = nullptr) {
     if ((trans_a != DOCC_ROCM_NO_TRANS && trans_a != DOCC_ROCM_TRANS) ||
         (trans_b != DOCC_ROCM_NO_TRANS && trans_b != DOCC_ROCM_TRANS))
         return fail(DOCC_ROCM_ERR_INVALID_ARGUMENT, "%s: transpose code must be 111 or 112", prefix);
@@ -206,11 +224,25 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
     if (batch_a < 0 || batch_b < 0 || batch_c < 0) return fail(DOCC_ROCM_ERR_INVALID_ARGUMENT, "%s: negative batch stride", prefix);
     if (m == 0 || n == 0 || batch == 0) return 0;
     if (batch > 1 && batch_c < (m - 1) * ldc + n) return fail(DOCC_ROCM_ERR_INVALID_ARGUMENT, "%s: the C matrices of the batch overlap", prefix);
-    if (!C || (k > 0 && (!A || !B))) return fail(DOCC_ROCM_ERR_INVALID_ARGUMENT, "%s: null pointer", prefix);
+    if ((!C && !fin) || (k > 0 && (!A || !B))) return fail(DOCC_ROCM_ERR_INVALID_ARGUMENT, "%s: null pointer", prefix);
     int rc = ensure_device();
     if (rc) return rc;
     hipStream_t s = (hipStream_t) stream;
     char name[96];
+    // with a finish (docc_rocm_linear): where no kernel has it in its store, the product goes to a block of the device block
+    // cache and the chain runs as one pass over it. `product(C)` returns 1 where it does not take the shape.
+    auto through_memory = [&](auto&& product) -> int {
+        void* wide = nullptr;
+        if (int r = docc_rocm_malloc_async(&wide, (size_t) (m * n) * sizeof(S), stream)) return r;
+        int r = product((S*) wide);
+        if (r == 0) r = finish_parts(s, wide, m, n, 1, 1.0f, *fin);
+        const int r2 = docc_rocm_free_async(wide, stream);
+        return r ? r : r2;
+    };
+    auto plain_product = [&](S* to) {
+        return gemm_launch<T, S>(prefix, stream, trans_a, trans_b, m, n, k, alpha, A, lda, B, ldb, (S) 0, to, n, pick);
+    };
+    if (fin && (k == 0 || alpha == (S) 0)) return through_memory(plain_product);
     if (k == 0 || alpha == (S) 0) {   // an empty product, or one BLAS does not reference ("when ALPHA is zero ...")
         std::snprintf(name, sizeof(name), "docc_%s_scale_c", prefix);
         int64_t blocks = (m * n + 255) / 256;
@@ -233,6 +265,7 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
     // into a block of the device block cache first (k x n elements), and the product runs as A B'^T.
     if (!tb && batch == 1 && n >= 2 && n <= 64 && ldb == n && m >= 1024 && k >= 256 && k % (16 / (int64_t) sizeof(T)) == 0 &&
         (n <= 4 || n % (16 / (int64_t) sizeof(T)) != 0) && !std::getenv("DOCC_ROCM_GEMV_OFF")) {
+        if (fin) return through_memory(plain_product);
         void* bt = nullptr;
         if ((rc = docc_rocm_malloc_async(&bt, (size_t) (n * k) * sizeof(T), stream))) return rc;
         const int64_t shape[2] = {k, n}, perm[2] = {1, 0};
@@ -263,7 +296,10 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
     const bool skinny_f64 = sizeof(T) == 8 && skinny_base && !tb && m >= 5 && m <= 16 && (n * k >= (int64_t(4) << 20) || skinny_any_size) &&
                             lda % 2 == 0 && ldb % 2 == 0 && k % 2 == 0 && n % 2 == 0;
     const bool skinny = skinny_f32 || skinny_bf16 || skinny_f64;
-    if ((m <= 8 || n <= 8) && !skinny && batch == 1 && (!epilogue || ldc == n)) {
+    if (fin && (m <= 8 || n <= 8) && !skinny && batch == 1) {
+        rc = through_memory([&](S* to) { return gemv_launch<T, S>(prefix, s, ta, tb, m, n, k, alpha, A, lda, B, ldb, (S) 0, to, n); });
+        if (rc != 1) return rc;
+    } else if ((m <= 8 || n <= 8) && !skinny && batch == 1 && (!epilogue || ldc == n)) {
         rc = gemv_launch<T, S>(prefix, s, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc);
         if (rc == 0 && epilogue) {
             // the few rows or columns of output are a small tensor: bias and activation as one elementwise pass over it,
@@ -319,7 +355,7 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
             const int64_t kpart = part_length(parts);
             parts = (k + kpart - 1) / kpart;
             const int64_t bytes = parts * m * n * (int64_t) sizeof(S);
-            const bool direct = parts == 1 && (tb || ((uintptr_t) C % 16 == 0 && ldc % (skinny_f64 ? 2 : 4) == 0));
+            const bool direct = !fin && parts == 1 && (tb || ((uintptr_t) C % 16 == 0 && ldc % (skinny_f64 ? 2 : 4) == 0));
             if (direct || bytes <= (int64_t(64) << 20)) {
                 PartialsLease lease;
                 void* buf = nullptr;
@@ -340,7 +376,9 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
                 rc = launch(name, (uint32_t) col_blocks, (uint32_t) parts, 1, 64 * nw, (uint32_t) (nw / 2) * slot_bytes, s, A, (long) lda, B, (long) ldb,
                             direct ? (void*) C : buf, (long) (direct ? ldc : n), (long) m, (long) n, (long) k, (long) kpart, alpha, beta,
                             direct ? 1 : 0);
-                if (!rc && !direct) {
+                if (!rc && fin) {
+                    rc = finish_parts(s, buf, m, n, (int) parts, (float) alpha, *fin);
+                } else if (!rc && !direct) {
                     int64_t blocks = (m * n + 255) / 256;
                     if (blocks > 4096) blocks = 4096;
                     rc = launch(sizeof(S) == 8 ? "docc_splitk_combine_f64" : "docc_splitk_combine_f32", (uint32_t) blocks, 1, 1, 256, 0, s, (const S*) buf, C,
@@ -441,7 +479,9 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
             const int64_t part = k / splits;
             rc = gemm_launch<T, S>(prefix, stream, trans_a, trans_b, m, n, part, (S) 1, A, lda, B, ldb, (S) 0, (S*) parts, n, pick, nullptr, -1, splits,
                                    ta ? part * lda : part, tb ? part : part * ldb, m * n);
-            if (!rc) {
+            if (!rc && fin) {
+                rc = finish_parts(s, parts, m, n, (int) splits, (float) alpha, *fin);
+            } else if (!rc) {
                 int64_t blocks = (m * n + 255) / 256;
                 if (blocks > 4096) blocks = 4096;
                 rc = launch(sizeof(S) == 8 ? "docc_splitk_combine_f64" : "docc_splitk_combine_f32", (uint32_t) blocks, 1, 1, 256, 0, s, (const S*) parts, C,
@@ -460,6 +500,18 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
         }
     }
     size_t lds;
+    if (fin) {
+        // kernels with the chain in their store: the asynchronous ones the picker chooses from, A stored by rows
+        const bool built = cfg.stages > 0 && !ta && sizeof(T) <= 4 && (sizeof(T) == 4 || cfg.bm == 128 || cfg.small) && n % 8 == 0 &&
+                           ((uintptr_t) fin->bias | (uintptr_t) fin->residual | (uintptr_t) fin->out) % 16 == 0;
+        if (!built) return through_memory(plain_product);
+        std::snprintf(name, sizeof(name), "docc_%sa_%dx%dx%d%c%d_n%c_f", prefix, cfg.bm, cfg.bn, cfg.bk, cfg.small ? 'q' : 's', cfg.stages, tb ? 't' : 'n');
+        const size_t ring = (size_t) cfg.stages * ((size_t) cfg.bm * cfg.bk + (size_t) cfg.bk * cfg.bn) * sizeof(T);
+        // a wave's (of 2 x 2) rows on their way out, up to 64 of them, padded by four floats (FinishShape)
+        const size_t turned = (size_t) cfg.waves * (cfg.bm / 2 < 64 ? cfg.bm / 2 : 64) * (cfg.bn / 2 + 4) * sizeof(float);
+        return launch(name, (uint32_t) tiles, 1, 1, 64 * cfg.waves, (uint32_t) (ring > turned ? ring : turned), s, A, B, (long) m, (long) n, (long) k,
+                      (long) lda, (long) ldb, (float) alpha, *fin);
+    }
     if (cfg.stages > 0) {
         std::snprintf(name, sizeof(name), "docc_%sa_%dx%dx%d%c%d_%c%c", prefix, cfg.bm, cfg.bn, cfg.bk, cfg.small ? 'q' : cfg.spread ? 'p' : 's', cfg.stages,
                       ta ? 't' : 'n', tb ? 't' : 'n');
@@ -581,6 +633,31 @@ int docc_rocm_bf16gemm_f32_epilogue(docc_rocm_stream_t stream, int trans_a, int 
                                     float* C, int64_t ldc, const float* bias, int activation) {
     return gemm_launch<uint16_t, float>("bgemm", stream, trans_a, trans_b, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc,
                                         pick_bgemm, bias, activation);
+}
+
+int docc_rocm_linear(docc_rocm_stream_t stream, int type, int trans_a, int trans_b, int64_t m, int64_t n, int64_t k, float alpha, const void* A,
+                     int64_t lda, const void* B, int64_t ldb, const void* bias, int bias_type, int activation, const void* residual,
+                     int residual_type, int rounding, void* Y, int y_type) {
+    auto is = [](int t, int a, int b) { return t == a || t == b; };
+    if (!is(type, DOCC_ROCM_TYPE_F32, DOCC_ROCM_TYPE_BF16) || !is(y_type, DOCC_ROCM_TYPE_F32, DOCC_ROCM_TYPE_BF16) ||
+        (bias && !is(bias_type, DOCC_ROCM_TYPE_F32, DOCC_ROCM_TYPE_BF16)) || (residual && !is(residual_type, DOCC_ROCM_TYPE_F32, DOCC_ROCM_TYPE_BF16)))
+        return fail(DOCC_ROCM_ERR_INVALID_ARGUMENT, "linear: operands are float32 or bf16");
+    if (activation != -1 && activation != DOCC_ROCM_UNARY_ABS && activation != DOCC_ROCM_UNARY_RELU && activation != DOCC_ROCM_UNARY_SIGMOID &&
+        activation != DOCC_ROCM_UNARY_TANH && !(activation >= DOCC_ROCM_ACT_GELU && activation <= DOCC_ROCM_ACT_SILU))
+        return fail(DOCC_ROCM_ERR_INVALID_ARGUMENT, "linear: unknown activation %d", activation);
+    if (rounding & ~(DOCC_ROCM_ROUND_BEFORE_ACT | DOCC_ROCM_ROUND_AFTER_ACT)) return fail(DOCC_ROCM_ERR_INVALID_ARGUMENT, "linear: unknown rounding %d", rounding);
+    if (m > 0 && n > 0 && !Y) return fail(DOCC_ROCM_ERR_INVALID_ARGUMENT, "linear: null pointer");
+    LinearFinish f{bias, residual, Y, 0, activation};
+    if (bias && bias_type == DOCC_ROCM_TYPE_BF16) f.flags |= kBiasBf16;
+    if (residual && residual_type == DOCC_ROCM_TYPE_BF16) f.flags |= kResidualBf16;
+    if (y_type == DOCC_ROCM_TYPE_BF16) f.flags |= kOutBf16;
+    if (rounding & DOCC_ROCM_ROUND_BEFORE_ACT) f.flags |= kRoundBeforeAct;
+    if (rounding & DOCC_ROCM_ROUND_AFTER_ACT) f.flags |= kRoundAfterAct;
+    if (type == DOCC_ROCM_TYPE_F32)
+        return gemm_launch<float>("sgemm", stream, trans_a, trans_b, m, n, k, alpha, (const float*) A, lda, (const float*) B, ldb, 0.0f, (float*) nullptr, n,
+                                  pick_sgemm, (const float*) nullptr, -1, 1, 0, 0, 0, &f);
+    return gemm_launch<uint16_t, float>("bgemm", stream, trans_a, trans_b, m, n, k, alpha, (const uint16_t*) A, lda, (const uint16_t*) B, ldb, 0.0f,
+                                        (float*) nullptr, n, pick_bgemm, (const float*) nullptr, -1, 1, 0, 0, 0, &f);
 }
 
 int docc_rocm_sgemm_batched(docc_rocm_stream_t stream, int trans_a, int trans_b, int64_t m, int64_t n, int64_t k, float alpha,

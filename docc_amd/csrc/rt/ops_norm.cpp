@@ -1,0 +1,39 @@
+// Launcher of the layer normalisation kernels (see include/docc_rocm_ops.h, csrc/kernels/layernorm.hip).
+#include <cstdio>
+
+#include "docc_rocm_ops.h"
+#include "rt_state.h"
+
+using namespace docc::rt::rocm;
+
+extern "C" int docc_rocm_layer_norm(docc_rocm_stream_t stream, int type, int64_t rows, int64_t cols, float eps, const void* X, const void* weight,
+                                    const void* bias, void* Y) {
+    if (type != DOCC_ROCM_TYPE_F32 && type != DOCC_ROCM_TYPE_BF16) return fail(DOCC_ROCM_ERR_INVALID_ARGUMENT, "layer_norm: float32 or bf16 tensors");
+    if (rows < 0 || cols < 0) return fail(DOCC_ROCM_ERR_INVALID_ARGUMENT, "layer_norm: negative dimension");
+    if (rows == 0 || cols == 0) return 0;
+    if (!X || !Y) return fail(DOCC_ROCM_ERR_INVALID_ARGUMENT, "layer_norm: null pointer");
+    if (rows > 0x7fffffffLL) return fail(DOCC_ROCM_ERR_UNSUPPORTED, "layer_norm: too many rows");
+    if (int rc = ensure_device()) return rc;
+    int cus = compute_units();
+    if (cus <= 0) cus = 256;
+    const bool bf16 = type == DOCC_ROCM_TYPE_BF16;
+    const int full = bf16 ? 8 : 4;
+    const bool vec = cols % full == 0 && ((uintptr_t) X | (uintptr_t) weight | (uintptr_t) bias | (uintptr_t) Y) % 16 == 0;
+    const int64_t lane = vec ? full : 1;   // elements of a lane's access
+    // vectors a lane holds with `lanes` of them on a row: the smallest built count that covers the row, 0 if none does
+    auto held = [&](int64_t lanes) -> int {
+        const int64_t n = (cols + lanes * lane - 1) / (lanes * lane);
+        if (!vec) return n <= 4 ? 4 : lanes == 256 && n <= 16 ? 16 : 0;
+        return n <= 1 ? 1 : n <= 2 ? 2 : n <= 4 ? 4 : !bf16 && lanes == 256 && n <= 8 ? 8 : 0;
+    };
+    // a wavefront a row where that gives every CU its four rows, or where a row is one access of 64 lanes
+    const int w = held(64), b = held(256);
+    const bool wave = w != 0 && (rows >= 4 * (int64_t) cus || cols <= 64 * lane);
+    char name[64];
+    if (!wave && !b) {
+        std::snprintf(name, sizeof(name), "docc_layernorm_%s_long", bf16 ? "bf16" : "f32");
+        return launch(name, (uint32_t) rows, 1, 1, 1024, 0, (hipStream_t) stream, (long) rows, (long) cols, eps, X, weight, bias, Y);
+    }
+    std::snprintf(name, sizeof(name), "docc_layernorm_%s_%c_%c%d", bf16 ? "bf16" : "f32", vec ? 'v' : 's', wave ? 'w' : 'b', wave ? w : b);
+    return launch(name, (uint32_t) (wave ? (rows + 3) / 4 : rows), 1, 1, 256, 0, (hipStream_t) stream, (long) rows, (long) cols, eps, X, weight, bias, Y);
+}

@@ -41,6 +41,12 @@ const char* const kKernelImages[] = {
     "docc_rocm_gemm_bf16_async_big_epilogue.hsaco",
     "docc_rocm_gemm_f32_big.hsaco",
     "docc_rocm_gemm_f32_big_epilogue.hsaco",
+    "docc_rocm_gemm_finish.hsaco",
+    "docc_rocm_gemm_bf16_async_finish.hsaco",
+    "docc_rocm_gemm_bf16_async_big_finish.hsaco",
+    "docc_rocm_gemm_f32_finish.hsaco",
+    "docc_rocm_gemm_f32_big_finish.hsaco",
+    "docc_rocm_layernorm.hsaco",
     "docc_rocm_conv2d.hsaco",
     "docc_rocm_attention.hsaco",
     "docc_rocm_elementwise.hsaco",

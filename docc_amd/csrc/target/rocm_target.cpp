@@ -19,6 +19,18 @@ using structured_control_flow::Block;
 namespace blas = math::blas;
 namespace tensor = math::tensor;
 
+void emit_runtime_preamble(PrettyPrinter& globals, const Function& function) {
+    if (globals.str().find("#define DOCC_ROCM_CHECK") != std::string::npos) return;  // once per file
+    globals << "#include \"docc_rocm_rt.h\"" << std::endl;
+    globals << "#include \"docc_rocm_ops.h\"" << std::endl;
+    globals << "#ifndef DOCC_ROCM_CHECK" << std::endl;
+    globals << "#define DOCC_ROCM_ON_FAILURE " << (function.return_container().empty() ? "return" : "return nullptr") << std::endl;
+    globals << "#define DOCC_ROCM_CHECK(call) do { int __docc_rc = (call); if (__docc_rc != 0) { "
+               "docc_rocm_report_failure(__func__, #call, __docc_rc); DOCC_ROCM_ON_FAILURE; } } while (0)"
+            << std::endl;
+    globals << "#endif" << std::endl;
+}
+
 namespace {
 
 bool is_rocm_impl(const std::string& impl) {
@@ -41,19 +53,6 @@ bool is_math_node(const LibraryNode& node) {
            c == blas::LibraryNodeType_DOT || c == LibraryNodeType_ROCM_Map ||
            std::find(tensor::ActivationNodeCodes.begin(), tensor::ActivationNodeCodes.end(), c) != tensor::ActivationNodeCodes.end() ||
            is_elementwise_code(c) || std::find(tensor::ReduceNodeCodes.begin(), tensor::ReduceNodeCodes.end(), c) != tensor::ReduceNodeCodes.end();
-}
-
-// Preamble every rocm dispatcher puts into the globals stream (duplicates are folded by the generator).
-void emit_runtime_preamble(PrettyPrinter& globals, const Function& function) {
-    if (globals.str().find("#define DOCC_ROCM_CHECK") != std::string::npos) return;  // once per file
-    globals << "#include \"docc_rocm_rt.h\"" << std::endl;
-    globals << "#include \"docc_rocm_ops.h\"" << std::endl;
-    globals << "#ifndef DOCC_ROCM_CHECK" << std::endl;
-    globals << "#define DOCC_ROCM_ON_FAILURE " << (function.return_container().empty() ? "return" : "return nullptr") << std::endl;
-    globals << "#define DOCC_ROCM_CHECK(call) do { int __docc_rc = (call); if (__docc_rc != 0) { "
-               "docc_rocm_report_failure(__func__, #call, __docc_rc); DOCC_ROCM_ON_FAILURE; } } while (0)"
-            << std::endl;
-    globals << "#endif" << std::endl;
 }
 
 // ---- with-transfers scaffolding ---------------------------------------------------------
@@ -924,6 +923,7 @@ void register_plugin(plugins::Context& context) {
     for (auto& code : tensor::ReduceNodeCodes) register_math<ReduceNodeDispatcher_ROCM>(reg, code);
     register_math<FusedElementWiseDispatcher_ROCM>(reg, LibraryNodeType_ROCM_FusedElementWise);
     register_math<ROCMMapDispatcher>(reg, LibraryNodeType_ROCM_Map);
+    register_launch_dispatchers(reg);
     reg.register_library_node_dispatcher(
         LibraryNodeType_ROCM_Offloading + "::" + ImplementationType_NONE,
         [](LanguageExtension& le, const Function& f, const DataFlowGraph& b, const LibraryNode& n) {
@@ -1705,6 +1705,8 @@ void rocm_scheduling_passes(builder::StructuredSDFGBuilder& builder, analysis::A
         RocmElementwiseFusionPass fusion;
         fusion.run_pass(builder, analysis_manager);
     }
+    // the code generator reads this (RocmLaunchFusionPass)
+    if (options.fuse_elementwise) builder.subject().add_metadata(Metadata_FuseLaunches, "1");
     if (options.fuse_elementwise && options.fuse_maps) {
         RocmMapFusionPass maps;
         maps.run_pass(builder, analysis_manager);

@@ -94,6 +94,22 @@ public:
     bool run_pass(builder::StructuredSDFGBuilder& builder, analysis::AnalysisManager& analysis_manager);
 };
 
+// Merges launches when host code is generated (launch_fusion.cpp): a GEMM with the elementwise block behind it, the blocks a layer
+// norm is spelled with. Runs on the copy of the SDFG that the generator works on, if the program was scheduled with fusion (which
+// the scheduler notes in the metadata); not for an instrumented program, whose nodes are regions of their own.
+inline const std::string Metadata_FuseLaunches = "rocm_fuse_launches";
+class RocmLaunchFusionPass {
+public:
+    std::string name() { return "RocmLaunchFusion"; }
+    bool run_pass(builder::StructuredSDFGBuilder& builder, analysis::AnalysisManager& analysis_manager);
+};
+inline const std::string LibraryNodeType_ROCM_Linear = "ROCMLinear";
+inline const std::string LibraryNodeType_ROCM_LayerNorm = "ROCMLayerNorm";
+void register_launch_dispatchers(codegen::LibraryNodeDispatcherRegistry& reg);
+
+// Preamble every rocm dispatcher puts into the globals stream (duplicates are folded by the generator).
+void emit_runtime_preamble(codegen::PrettyPrinter& globals, const Function& function);
+
 // Recognises softmax written out in its pieces - the form numpy code takes, and what the reference's SoftmaxNode
 // expands to (softmax_node.cpp:142-252): m = Max(X, axes, keepdims); e = Exp(X - broadcast(m)); Y = e / broadcast(Sum(e,
 // axes, keepdims)) - and replaces the seven nodes by one ml::Softmax when every value in between is a transient that
@@ -135,7 +151,7 @@ struct ScheduleOptions {
     std::string offload = "function";
     // refuse to leave a math node unmapped (there is no CPU lowering in this target)
     bool require_all_mapped = true;
-    // run RocmElementwiseFusionPass after the mapping
+    // run RocmElementwiseFusionPass after the mapping, and let the code generator merge launches (RocmLaunchFusionPass)
     bool fuse_elementwise = true;
     // run RocmSoftmaxPatternPass before the mapping
     bool match_softmax = true;

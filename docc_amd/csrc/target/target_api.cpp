@@ -65,6 +65,12 @@ Generated generate(StructuredSDFG& sdfg, const char* output_dir, const char* ins
     auto snippets = std::make_shared<codegen::CodeSnippetFactory>(dir);
     auto plan = codegen::InstrumentationPlan::from_mode(sdfg, instrumentation_mode ? instrumentation_mode : "");
     if (instrumented) *instrumented = !plan->empty();
+    if (plan->empty() && sdfg.metadata().count(rocm::Metadata_FuseLaunches)) {
+        builder::StructuredSDFGBuilder builder(sdfg);
+        analysis::AnalysisManager analysis_manager(sdfg);
+        rocm::RocmLaunchFusionPass launches;
+        launches.run_pass(builder, analysis_manager);
+    }
     codegen::CPPCodeGenerator gen(sdfg, snippets, "", plan.get());
     gen.generate();
     Generated g;

@@ -89,6 +89,33 @@ int docc_rocm_bf16gemm_f32_epilogue(docc_rocm_stream_t stream, int trans_a, int 
                                     float beta, float* C, int64_t ldc, const float* bias, int activation);
 
 /*
+ * A product with the rest of a layer behind it, the sums in fp32:
+ *     Y = act(round1(alpha * op(A) op(B) + bias[column]));   with a residual:  Y = round2(act(...)) + residual
+ * A and B both float32 or both bf16 (`type`, DOCC_ROCM_TYPE_*), `bias` (n values) and `residual` (dense [m, n]) float32 or bf16 or
+ * NULL, Y dense [m, n] in either type. `activation`: -1, DOCC_ROCM_UNARY_ABS / RELU / SIGMOID / TANH or DOCC_ROCM_ACT_*.
+ * `rounding`: DOCC_ROCM_ROUND_* bits, where a chain of bf16 nodes rounds in between (round1: before the activation, round2: before
+ * the residual). Y may be the residual itself. What the code generator emits for a GEMM node and the elementwise node that alone
+ * reads its result; the reference expands the latter to a Map of its own (python/bindings/py_structured_sdfg.cpp:258-260).
+ */
+#define DOCC_ROCM_ACT_GELU 16      /* x Phi(x) */
+#define DOCC_ROCM_ACT_GELU_TANH 17 /* 0.5 x (1 + tanh(sqrt(2 / pi) (x + 0.044715 x^3))) */
+#define DOCC_ROCM_ACT_SILU 18      /* x / (1 + exp(-x)) */
+#define DOCC_ROCM_ROUND_BEFORE_ACT 1
+#define DOCC_ROCM_ROUND_AFTER_ACT 2
+int docc_rocm_linear(docc_rocm_stream_t stream, int type, int trans_a, int trans_b, int64_t m, int64_t n, int64_t k, float alpha, const void* A,
+                     int64_t lda, const void* B, int64_t ldb, const void* bias, int bias_type, int activation, const void* residual,
+                     int residual_type, int rounding, void* Y, int y_type);
+
+/*
+ * The normalisation of a layer over the last axis:
+ *     Y[r, :] = (X[r, :] - mean) / sqrt(var + eps) * weight + bias,   mean and var (mean of the squared differences) in fp32,
+ * X, Y and the optional weight and bias (cols values) all float32 or all bf16 (`type`). X == Y is allowed. What the code generator
+ * emits for the reduction and elementwise nodes a layer norm is spelled with.
+ */
+int docc_rocm_layer_norm(docc_rocm_stream_t stream, int type, int64_t rows, int64_t cols, float eps, const void* X, const void* weight,
+                         const void* bias, void* Y);
+
+/*
  * A batch of `batch` equally shaped products in one launch: entry z uses
  * A + z*stride_a, B + z*stride_b, C + z*stride_c (strides in elements; 0
  * shares an input across the batch, the C matrices must not overlap).

@@ -1,0 +1,126 @@
+"""docc_rocm_linear (a product with bias, activation, roundings and residual behind it) and docc_rocm_layer_norm, and the programs
+the code generator emits them for. Against float64 on the CPU, with the roundings to bf16 that the chain asks for."""
+import ctypes
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+from docc_amd import runtime as rt
+
+pytestmark = pytest.mark.gpu
+
+ACTS = {None: -1, "relu": 2, "sigmoid": 3, "tanh": 5, "gelu": 16, "gelu_tanh": 17, "silu": 18}
+REF = {None: lambda x: x, "relu": torch.relu, "sigmoid": torch.sigmoid, "tanh": torch.tanh, "gelu": F.gelu,
+       "gelu_tanh": lambda x: F.gelu(x, approximate="tanh"), "silu": F.silu}
+TYPE = {torch.bfloat16: 1, torch.float32: 2}
+
+
+def ptr(t):
+    return ctypes.c_void_p(t.data_ptr() if t is not None else None)
+
+
+def linear(a, w, trans_b, bias, act, residual, rounding, out_dtype):
+    m, k = a.shape
+    n = w.shape[0] if trans_b else w.shape[1]
+    y = torch.full((m, n), float("nan"), device="cuda", dtype=out_dtype)
+    rt.call("docc_rocm_linear", 0, TYPE[a.dtype], rt.NO_TRANS, rt.TRANS if trans_b else rt.NO_TRANS, m, n, k, 1.0, ptr(a), k, ptr(w), w.shape[1],
+            ptr(bias), TYPE[bias.dtype] if bias is not None else 2, ACTS[act], ptr(residual), TYPE[residual.dtype] if residual is not None else 2,
+            rounding, ptr(y), TYPE[out_dtype])
+    torch.cuda.synchronize()
+    return y
+
+
+def reference(a, w, trans_b, bias, act, residual, rounding):
+    v = a.double().cpu() @ (w.double().cpu().T.contiguous() if trans_b else w.double().cpu())
+    if bias is not None:
+        v = v + bias.double().cpu()
+    if rounding & 1:
+        v = v.float().bfloat16().double()
+    v = REF[act](v)
+    if residual is not None:
+        if rounding & 2:
+            v = v.float().bfloat16().double()
+        v = v + residual.double().cpu()
+    return v
+
+
+# rows: matrix-vector, few-row kernels, tiles of 64 / 128 / 256 with ragged edges, K in parts; columns off a vector of eight too
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("m,n,k", [(1, 512, 512), (2, 1024, 2048), (8, 4096, 2048), (17, 8192, 1024), (64, 256, 1024), (100, 72, 96), (129, 200, 64),
+                                   (130, 77, 33), (384, 1032, 512), (1000, 136, 4096), (2050, 1160, 128), (4100, 4104, 128)])
+def test_linear_over_the_launchers_forms(dtype, m, n, k):
+    gen = torch.Generator().manual_seed(m * 31 + n)
+    a = torch.randn(m, k, generator=gen).to(dtype).cuda()
+    w = (torch.randn(n, k, generator=gen) * k ** -0.5).to(dtype).cuda()
+    bias = torch.randn(n, generator=gen).to(dtype).cuda()
+    res = torch.randn(m, n, generator=gen).to(dtype).cuda()
+    for act, b, r, rounding in (("gelu", bias, None, 1), (None, bias, res, 2), ("relu", None, res, 3)):
+        rounding = rounding if dtype == torch.bfloat16 else 0
+        ref = reference(a, w, True, b, act, r, rounding)
+        got = linear(a, w, True, b, act, r, rounding, dtype)
+        # the fp32 sums: k products of size 1 / sqrt(k), each rounded at 2^-24, the error growing with sqrt(k): 2^-24 * sqrt(4096) * a few
+        # at most, whatever the size of the result. bf16 on top of that: a last
+        # bit (at most 2^-7 of the value) of the result, and one of the value that is rounded in between where the fp32 sum and the exact
+        # one lie on different sides of a boundary - before the activation, whose slope is at most 1.13, or behind it, where it is smaller
+        err = (got.double().cpu() - ref).abs()
+        between = reference(a, w, True, b, None, None, 0).abs()
+        bound = 2e-5 * (1 + ref.abs()) + (0 if dtype == torch.float32 else 2.0 ** -7 * (1.13 * between + ref.abs()))
+        assert bool((err <= bound).all()), (act, float((err / bound).max()))
+
+
+@pytest.mark.parametrize("act", list(ACTS))
+@pytest.mark.parametrize("trans_b", [True, False])
+def test_linear_activations(act, trans_b):
+    gen = torch.Generator().manual_seed(5)
+    a = torch.randn(192, 64, generator=gen).cuda()
+    w = (torch.randn(136, 64, generator=gen) * 0.4).cuda()
+    w = w if trans_b else w.T.contiguous()
+    bias = torch.randn(136, generator=gen).cuda()
+    got = linear(a, w, trans_b, bias, act, None, 0, torch.float32).double().cpu()
+    ref = reference(a, w, trans_b, bias, act, None, 0)
+    # |x| up to about 15; sums of 64 terms in fp32 (2e-6) through slopes of at most 1.13
+    assert float((got - ref).abs().max()) <= 1e-5
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows,cols", [(1, 8), (3, 250), (5, 1000), (1025, 256), (2000, 1024), (8, 2048), (1030, 2048), (7, 4096), (5, 4097), (3, 8192),
+                                       (2, 16384), (2, 9001)])
+def test_layer_norm_over_row_lengths(dtype, rows, cols):
+    gen = torch.Generator().manual_seed(cols)
+    x = (torch.randn(rows, cols, generator=gen) * 3 + 1).to(dtype).cuda()
+    w, b = torch.randn(cols, generator=gen).to(dtype).cuda(), torch.randn(cols, generator=gen).to(dtype).cuda()
+    for weight, bias in ((w, b), (None, None), (w, None)):
+        y = torch.full_like(x, float("nan"))
+        rt.call("docc_rocm_layer_norm", 0, TYPE[dtype], rows, cols, 1e-5, ptr(x), ptr(weight), ptr(bias), ptr(y))
+        torch.cuda.synchronize()
+        up = lambda t: None if t is None else t.double().cpu()
+        ref = F.layer_norm(up(x), (cols,), up(weight), up(bias), 1e-5)
+        err = (y.double().cpu() - ref).abs()
+        bound = 1e-5 * (1 + ref.abs()) if dtype == torch.float32 else 2.0 ** -8 * (1e-3 + ref.abs())
+        assert bool((err <= bound).all()), float((err / bound).max())
+
+
+class Block(torch.nn.Module):
+    def __init__(self, width, approximate):
+        super().__init__()
+        self.width, self.approximate = width, approximate
+
+    def forward(self, x, g, b, w1, b1, w2, b2):
+        h = F.layer_norm(x, (self.width,), g, b)
+        return x + F.linear(F.gelu(F.linear(h, w1, b1), approximate=self.approximate), w2, b2)
+
+
+@pytest.mark.parametrize("dtype,tokens,width,approximate", [(torch.float32, 96, 64, "none"), (torch.bfloat16, 200, 128, "tanh"), (torch.bfloat16, 1, 64, "none"),
+                                                            (torch.bfloat16, 8, 2048, "none"), (torch.float32, 5, 100, "tanh")])
+def test_block_program(dtype, tokens, width, approximate):
+    import docc_amd.torch as docc_torch
+
+    gen = torch.Generator().manual_seed(width)
+    rand = lambda *s, scale=1.0: (torch.randn(*s, generator=gen) * scale).to(dtype).cuda()
+    args = (rand(tokens, width), rand(width), rand(width), rand(4 * width, width, scale=width ** -0.5), rand(4 * width), rand(width, 4 * width, scale=0.5 * width ** -0.5), rand(width))
+    got = docc_torch.compile_torch(Block(width, approximate), None, target="rocm")(*args)
+    ref = Block(width, approximate)(*[t.double().cpu() for t in args])
+    assert got.dtype == dtype and got.shape == ref.shape
+    err = float((got.double().cpu() - ref).norm() / ref.norm())
+    assert err <= (1e-5 if dtype == torch.float32 else 1e-2), err     # bf16: the three intermediate tensors are rounded to bf16

@@ -1,0 +1,77 @@
+"""Launches merged when host code is generated: what is emitted for a layer and for a layer norm spelled with tensor nodes, and what
+keeps its separate launches."""
+import re
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+import docc_amd.torch as docc_torch
+from docc_amd.sdfg import Pointer, PrimitiveType, Scalar, StructuredSDFGBuilder
+
+F32, F64 = Pointer(Scalar(PrimitiveType.Float)), Pointer(Scalar(PrimitiveType.Double))
+
+
+def calls(sdfg, folder, mode=""):
+    report = sdfg.generate(str(folder), mode)
+    text = re.sub(r"\s+", " ", open(report["source"]).read())
+    return [c for c in re.findall(r"DOCC_ROCM_CHECK\((docc_rocm_(?:linear|layer_norm|\w*gemm\w*|reduce|elementwise\w*|cast|launch)\(.*?\))\);", text)]
+
+
+class Block(torch.nn.Module):
+    def forward(self, x, g, b, w1, b1, w2, b2):
+        return x + F.linear(F.gelu(F.linear(F.layer_norm(x, (16,), g, b), w1, b1)), w2, b2)
+
+
+def block_sdfg(dtype, rows):
+    t = lambda *s: torch.randn(*s).to(dtype)
+    return docc_torch.compile_torch(Block(), None, target="rocm").to_sdfg(t(rows, 16), t(16), t(16), t(64, 16), t(64), t(16, 64), t(16))
+
+
+@pytest.mark.parametrize("rows", [5, 1])
+@pytest.mark.parametrize("dtype,code", [(torch.float32, 2), (torch.bfloat16, 1)])
+def test_a_feed_forward_block_is_three_calls(tmp_path, dtype, code, rows):
+    s = block_sdfg(dtype, rows)
+    s.schedule("rocm", options={"offload": "none"})
+    assert [n["code"] for n in s.library_nodes()].count("GEMM") == 2      # the scheduled form keeps its nodes
+    got = calls(s, tmp_path)
+    rounds = (1, 2) if dtype == torch.bfloat16 else (0, 0)
+    assert got == [f"docc_rocm_layer_norm(nullptr, {code}, {rows}, 16, (float) (1e-05), _x, _weight, _bias, _y)",
+                   f"docc_rocm_linear(nullptr, {code}, 111, 112, {rows}, 64, 16, (float) __alpha, _a, 16, _b, 16, _bias, {code}, 16, nullptr, 2, {rounds[0]}, _y, {code})",
+                   f"docc_rocm_linear(nullptr, {code}, 111, 112, {rows}, 16, 64, (float) __alpha, _a, 64, _b, 64, _bias, {code}, -1, _residual, {code}, {rounds[1]}, _y, {code})"]
+    # every transient that is left is allocated before and freed behind its uses
+    text = open(next(tmp_path.glob("*.cpp"))).read()
+    assert text.count("docc_rocm_malloc_async(") == text.count("docc_rocm_free_async(") == 2
+
+
+def test_instrumented_and_unfused_programs_keep_their_launches(tmp_path):
+    s = block_sdfg(torch.float32, 5)
+    s.schedule("rocm", options={"offload": "none"})
+    assert "docc_rocm_linear" not in " ".join(calls(s, tmp_path / "ols", "ols"))
+    s = block_sdfg(torch.float32, 5)
+    s.schedule("rocm", options={"offload": "none", "fuse": False})
+    assert "docc_rocm_linear" not in " ".join(calls(s, tmp_path / "apart"))
+
+
+def two_layers(element, second_reader=False, factor="0.5"):
+    b = StructuredSDFGBuilder("layers")
+    for n in ("X", "W", "R", "Y", "Z"):
+        b.add_container(n, element, True)
+    for n in ("T0", "T1", "T2"):
+        b.add_container(n, element, False, transient_bytes=32 * 16 * 8)
+    b.add_gemm("X", "W", "T0", "1.0", "0.0", 32, 16, 8)
+    b.add_elementwise_unary_op("sigmoid", "T0", "T1", [32, 16])
+    b.add_elementwise_op("mul", "T0", "T1", "T2", [32, 16])
+    b.add_elementwise_op("add", "T2", "R", "Y", [32, 16])
+    if second_reader:
+        b.add_elementwise_op("mul", "T0", factor, "Z", [32, 16])
+    s = b.move()
+    s.schedule("rocm", options={"offload": "none"})
+    return s
+
+
+def test_only_float_products_with_one_reader_are_merged(tmp_path):
+    got = calls(two_layers(F32), tmp_path / "a")
+    assert got == ["docc_rocm_linear(nullptr, 2, 111, 111, 32, 16, 8, (float) __alpha, _a, 8, _b, 16, nullptr, 2, 18, _residual, 2, 0, _y, 2)"]
+    assert "docc_rocm_linear" not in " ".join(calls(two_layers(F64), tmp_path / "b"))
+    assert "docc_rocm_linear" not in " ".join(calls(two_layers(F32, second_reader=True), tmp_path / "c"))
