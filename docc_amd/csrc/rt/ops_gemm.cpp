@@ -30,6 +30,23 @@ size_t gemm_lds_bytes(const TileConfig& c, bool ta, bool tb, size_t elem) {
     return 2 * (a_elems + b_elems) * elem;
 }
 
+// Seconds a bf16 product of `count` matrices takes on tile `c`, fitted to 26 products from 64 x 2048 x 8192 to 8192 x 3072 x 768 and
+// 6144 x 4096 x 4096 (within 15 % on most): a launch, and for every round of tiles over the CUs the fp32 store of the tiles (all of
+// them at once: 11 us for 256 x 256) and their products at what the tile sustains. A last round that leaves CUs idle runs
+// faster (less traffic, higher clocks), but not in proportion, the smallest tile's, which waits for its copies, least of all.
+double bgemm_seconds(const TileConfig& c, int64_t m, int64_t n, int64_t k, bool tb, int64_t count) {
+    int cus = compute_units();
+    if (cus <= 0) cus = 256;
+    const int64_t tiles = ((m + c.bm - 1) / c.bm) * ((n + c.bn - 1) / c.bn) * count, last = tiles % cus;
+    const double part = (double) last / cus;
+    const double rounds = (double) (tiles / cus) + (!last ? 0.0 : tiles < cus && c.bn == 128 ? 0.7 + 0.2 * part : 0.5 + 0.4 * part);
+    // relative to the 256 x 256 tile on the 16x16x32 MFMA (which takes K in whole pairs of 32): the 128 x 256 one reads a k-major B from
+    // LDS at half the width; 128 x 128 tiles in several rounds read the operands from further away than L2
+    const double rel = c.bm == 256 ? (k % 64 == 0 ? 1.0 : 0.93) : c.bn == 256 ? (tb ? 0.88 : 0.80) : tiles > cus ? 0.75 : 0.86;
+    const double area = (double) c.bm * c.bn;
+    return 1e-6 * (4.0 + rounds * (area * (11.0 / 65536) + area * (double) k * 3.6e-7 / rel));
+}
+
 // What GemmFinish of csrc/kernels/gemm_finish.h holds: the rest of a layer behind a product.
 struct LinearFinish {
     const void *bias, *residual;
@@ -204,7 +221,7 @@ int gemv_launch(const char* prefix, hipStream_t s, bool ta, bool tb, int64_t m, 
 template <typename T, typename S = T>
 int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int trans_b, int64_t m, int64_t n,
                 int64_t k, S alpha, const T* A, int64_t lda, const T* B, int64_t ldb, S beta, S* C, int64_t ldc,
-                TileConfig (*pick)(int64_t m, int64_t n, int64_t batch, bool aligned, int force), const S* bias = nullptr,
+                TileConfig (*pick)(int64_t m, int64_t n, int64_t k, bool tb, int64_t batch, bool aligned, int force), const S* bias = nullptr,
                 int activation = -1, int64_t batch = 1, int64_t batch_a = 0, int64_t batch_b = 0, int64_t batch_c = 0,
                 const LinearFinish* fin = nullptr) {
     if ((trans_a != DOCC_ROCM_NO_TRANS && trans_a != DOCC_ROCM_TRANS) ||
@@ -400,7 +417,7 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
     }
     // DOCC_ROCM_GEMM_TILE=big|small overrides the size heuristic (tests, tuning)
     const char* force = std::getenv("DOCC_ROCM_GEMM_TILE");
-    TileConfig cfg = pick(m, n, batch, aligned, force && force[0] == 'b' ? 1 : force && force[0] == 's' ? -1 : 0);
+    TileConfig cfg = pick(m, n, k, tb, batch, aligned, force && force[0] == 'b' ? 1 : force && force[0] == 's' ? -1 : 0);
     // DOCC_ROCM_GEMM_CFG=BMxBNxBKxWAVES[xSTAGES[p|q]] selects a built configuration directly (tuning)
     if (const char* c = std::getenv("DOCC_ROCM_GEMM_CFG")) {
         TileConfig t{};
@@ -415,7 +432,7 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
     // the asynchronous kernels need aligned operands and address a tile with 32-bit byte offsets
     const int64_t max_edge = cfg.bm > cfg.bn ? (cfg.bm > cfg.bk ? cfg.bm : cfg.bk) : (cfg.bn > cfg.bk ? cfg.bn : cfg.bk);
     const bool offsets_fit = max_edge * (lda > ldb ? lda : ldb) * (int64_t) sizeof(T) < (int64_t(1) << 32);
-    if (cfg.stages > 0 && !(aligned && offsets_fit)) cfg = pick(m, n, batch, false, 0);
+    if (cfg.stages > 0 && !(aligned && offsets_fit)) cfg = pick(m, n, k, tb, batch, false, 0);
     const int64_t tiles = ((m + cfg.bm - 1) / cfg.bm) * ((n + cfg.bn - 1) / cfg.bn);
     if (tiles > 0x7fffffffLL) return fail(DOCC_ROCM_ERR_UNSUPPORTED, "%s: too many tiles", prefix);
     // Few output tiles and a long K extent (a handful of rows against a wide matrix: the product is bound by reading
@@ -437,6 +454,8 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
         // the padded tiles at what the tile sustains (relative to the 128 x 256 one) on the share of the CUs that get a
         // work-group, plus writing and reading the parts at 5 TB/s and a second launch.
         auto seconds = [&](const TileConfig& c, int64_t parts) {
+            if (sizeof(T) == 2)
+                return bgemm_seconds(c, m, n, k / parts, tb, parts) + (parts > 1 ? 2.0 * (double) parts * (double) m * (double) n * sizeof(S) / 5e12 + 3e-6 : 0.0);
             const double tm = (double) ((m + c.bm - 1) / c.bm), tn = (double) ((n + c.bn - 1) / c.bn);
             const double area = (double) c.bm * c.bn;
             const double rel = area >= 65536 ? 1.03 : area >= 32768 ? 1.0 : area >= 16384 ? 0.97 : 0.75;
@@ -444,7 +463,7 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
             // whole rounds (344 work-groups on 256 CUs take as long as 512)
             const double per_cu = tm * tn * (double) parts / cus;
             const double fill = per_cu < 1.0 ? per_cu : per_cu / (double) (int64_t) (per_cu + 0.999999);
-            const double rate = sizeof(T) == 8 ? 68e12 : sizeof(T) == 4 ? 141e12 : 1.25e15;
+            const double rate = sizeof(T) == 8 ? 68e12 : 141e12;
             double t = 2.0 * tm * c.bm * tn * c.bn * (double) k / (rate * rel * fill);
             if (parts > 1) t += 2.0 * (double) parts * (double) m * (double) n * sizeof(S) / 5e12 + 3e-6;
             return t;
@@ -456,7 +475,7 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
         } else if (tiles < cus) {   // CUs without a work-group: the case parts are for
             double best = seconds(cfg, 1);
             for (int64_t parts = 2; allowed(parts); parts *= 2) {
-                const TileConfig c = pick(m, n, parts, true, 0);
+                const TileConfig c = pick(m, n, k / parts, tb, parts, true, 0);
                 if (c.stages == 0) break;
                 const double t = seconds(c, parts);
                 if (t < 0.9 * best) {   // only for a clear gain: the estimate is rough
@@ -502,7 +521,7 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
     size_t lds;
     if (fin) {
         // kernels with the chain in their store: the asynchronous ones the picker chooses from, A stored by rows
-        const bool built = cfg.stages > 0 && !ta && sizeof(T) <= 4 && (sizeof(T) == 4 || cfg.bm == 128 || cfg.small) && n % 8 == 0 &&
+        const bool built = cfg.stages > 0 && !ta && sizeof(T) <= 4 && (sizeof(T) == 4 || !cfg.spread || cfg.small) && n % 8 == 0 &&
                            ((uintptr_t) fin->bias | (uintptr_t) fin->residual | (uintptr_t) fin->out) % 16 == 0;
         if (!built) return through_memory(plain_product);
         std::snprintf(name, sizeof(name), "docc_%sa_%dx%dx%d%c%d_n%c_f", prefix, cfg.bm, cfg.bn, cfg.bk, cfg.small ? 'q' : 's', cfg.stages, tb ? 't' : 'n');
@@ -535,7 +554,7 @@ template <typename T, typename S>
 static int gemm_batched(const char* prefix, docc_rocm_stream_t stream, int trans_a, int trans_b, int64_t m, int64_t n, int64_t k,
                         S alpha, const T* A, int64_t lda, int64_t stride_a, const T* B, int64_t ldb, int64_t stride_b, S beta, S* C,
                         int64_t ldc, int64_t stride_c, int64_t batch,
-                        TileConfig (*pick)(int64_t m, int64_t n, int64_t batch, bool aligned, int force)) {
+                        TileConfig (*pick)(int64_t m, int64_t n, int64_t k, bool tb, int64_t batch, bool aligned, int force)) {
     if (batch < 0) return fail(DOCC_ROCM_ERR_INVALID_ARGUMENT, "%s: negative batch", prefix);
     const int64_t kMaxGridY = 65535;
     for (int64_t b0 = 0; b0 < batch; b0 += kMaxGridY) {
@@ -555,7 +574,7 @@ extern "C" {
 // tiles of one matrix times the number of matrices: what there is to spread over the compute units
 static int64_t tiles_of(int64_t m, int64_t n, int bm, int bn, int64_t batch = 1) { return ((m + bm - 1) / bm) * ((n + bn - 1) / bn) * batch; }
 
-static TileConfig pick_sgemm(int64_t m, int64_t n, int64_t batch, bool aligned, int force) {
+static TileConfig pick_sgemm(int64_t m, int64_t n, int64_t, bool, int64_t batch, bool aligned, int force) {
     const TileConfig huge{256, 256, 32, 4, 2}, wide{128, 256, 32, 4, 2}, big{128, 128, 32, 4, 3}, small{64, 64, 16, 4, 4};
     const TileConfig plain_big{128, 128, 16, 4, 0}, plain_small{64, 64, 16, 4, 0};
     if (!aligned) return force > 0 ? plain_big : force < 0 ? plain_small : (tiles_of(m, n, 128, 128, batch) >= 256 ? plain_big : plain_small);
@@ -578,7 +597,7 @@ static TileConfig pick_sgemm(int64_t m, int64_t n, int64_t batch, bool aligned, 
     return sw >= sb && sw >= ss ? wide : sb >= ss ? big : small;
 }
 
-static TileConfig pick_dgemm(int64_t m, int64_t n, int64_t batch, bool aligned, int force) {
+static TileConfig pick_dgemm(int64_t m, int64_t n, int64_t, bool, int64_t batch, bool aligned, int force) {
     const TileConfig big{128, 128, 16, 4, 3}, mid{64, 64, 16, 4, 4}, small{64, 32, 16, 4, 4};
     const TileConfig plain_big{128, 128, 16, 4, 0}, plain_small{64, 64, 16, 4, 0};
     if (!aligned) return force > 0 ? plain_big : plain_small;
@@ -587,13 +606,22 @@ static TileConfig pick_dgemm(int64_t m, int64_t n, int64_t batch, bool aligned, 
     return t >= 2048 ? big : t > 512 ? mid : small;   // few tiles: halve them so that two work-groups share a CU
 }
 
-static TileConfig pick_bgemm(int64_t m, int64_t n, int64_t batch, bool aligned, int force) {
+static TileConfig pick_bgemm(int64_t m, int64_t n, int64_t k, bool tb, int64_t batch, bool aligned, int force) {
     // big: on the 16x16x32 MFMA where K allows it (see gemm_launch), else on the 32x32x16 one with the copies dealt out
-    const TileConfig big{256, 256, 32, 4, 4, true, true}, small{128, 128, 32, 4, 4};
+    const TileConfig big{256, 256, 32, 4, 4, true, true}, wide{128, 256, 64, 4, 3}, deep{128, 128, 64, 4, 4}, small{128, 128, 32, 4, 4};
     const TileConfig plain_big{256, 256, 64, 4, 0}, plain_small{128, 128, 64, 4, 0};
     if (!aligned) return force > 0 ? plain_big : force < 0 ? plain_small : (tiles_of(m, n, 256, 256, batch) >= 256 ? plain_big : plain_small);
     if (force) return force > 0 ? big : small;
-    return tiles_of(m, n, 256, 256, batch) >= 192 ? big : small;
+    const TileConfig* best = &big;
+    double least = bgemm_seconds(big, m, n, k, tb, batch);
+    for (const TileConfig* c : {&wide, k >= 1024 ? &deep : &small}) {
+        const double t = bgemm_seconds(*c, m, n, k, tb, batch);
+        if (t < least) {
+            least = t;
+            best = c;
+        }
+    }
+    return *best;
 }
 
 int docc_rocm_sgemm(docc_rocm_stream_t stream, int trans_a, int trans_b, int64_t m, int64_t n, int64_t k, float alpha,

@@ -69,6 +69,22 @@ def test_linear_over_the_launchers_forms(dtype, m, n, k):
         assert bool((err <= bound).all()), (act, float((err / bound).max()))
 
 
+# every tile with the chain in its store, ragged at both edges and along K where the tile allows it
+@pytest.mark.parametrize("cfg,dtype,k", [("128x128x32x4x4", torch.bfloat16, 104), ("128x128x64x4x4", torch.bfloat16, 328), ("128x256x64x4x3", torch.bfloat16, 328),
+                                         ("256x256x32x4x4q", torch.bfloat16, 192), ("64x64x16x4x4", torch.float32, 84), ("128x128x32x4x3", torch.float32, 84),
+                                         ("128x256x32x4x2", torch.float32, 84), ("256x256x32x4x2", torch.float32, 84)])
+@pytest.mark.parametrize("trans_b", [True, False])
+def test_linear_tiles(monkeypatch, cfg, dtype, k, trans_b):
+    monkeypatch.setenv("DOCC_ROCM_GEMM_CFG", cfg)
+    gen = torch.Generator().manual_seed(k)
+    for m, n in ((256, 256), (259, 520), (65, 264)):
+        a = torch.randn(m, k, generator=gen).to(dtype).cuda()
+        w = (torch.randn(*((n, k) if trans_b else (k, n)), generator=gen) * k ** -0.5).to(dtype).cuda()
+        bias, res = torch.randn(n, generator=gen).to(dtype).cuda(), torch.randn(m, n, generator=gen).to(dtype).cuda()
+        got = linear(a, w, trans_b, bias, "silu", res, 0, torch.float32).double().cpu()
+        assert float((got - reference(a, w, trans_b, bias, "silu", res, 0)).abs().max()) <= 2e-5     # fp32 throughout: sums of at most 328 terms
+
+
 @pytest.mark.parametrize("act", list(ACTS))
 @pytest.mark.parametrize("trans_b", [True, False])
 def test_linear_activations(act, trans_b):
