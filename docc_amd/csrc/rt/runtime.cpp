@@ -75,13 +75,25 @@ std::vector<DeviceState> g_devices;
 // records an event on the stream the owner worked on instead of waiting for the device, and the next owner either
 // continues on that same stream (stream order keeps it behind the old work), makes its own stream wait for the event
 // (docc_rocm_malloc_async), or waits for it on the host (docc_rocm_malloc). docc_rocm_free has waited for the whole
-// device and leaves `pending` false.
+// device and leaves `pending` false. On the null stream, which lives as long as the process, the event is not recorded until somebody
+// has to wait for it: between two launches a recorded event is a packet of its own on the device and a call on the host, which the
+// usual next owner - the next call of the same generated function, on the same stream - never looks at. Recorded later it stands
+// behind more work than the owner's, never behind less.
 struct CachedBlock {
     void* ptr = nullptr;
     hipEvent_t released = nullptr;   // created the first time the block is freed on a stream, reused afterwards
     hipStream_t stream = nullptr;    // the stream `released` was recorded on
     bool pending = false;            // `released` may not have happened yet
+    bool recorded = false;           // pending, and `released` has been recorded
 };
+
+// records the release of a pending block that has not been (see above)
+int record_release(CachedBlock* b) {
+    if (b->recorded) return 0;
+    if (!b->released)
+        if (int rc = check(hipEventCreateWithFlags(&b->released, hipEventDisableTiming), "hipEventCreate(block release)")) return rc;
+    return check(hipEventRecord(b->released, b->stream), "hipEventRecord(block release)");
+}
 
 struct BlockCache {
     std::mutex mutex;
@@ -605,8 +617,14 @@ int pool_malloc(void** dev_ptr, size_t bytes, bool ordered, hipStream_t stream) 
     }
     if (got.ptr) {
         if (got.pending && !(ordered && got.stream == stream)) {
-            rc = ordered ? check(hipStreamWaitEvent(stream, got.released, 0), "hipStreamWaitEvent(block release)")
-                         : check(hipEventSynchronize(got.released), "hipEventSynchronize(block release)");
+            rc = record_release(&got);
+            {
+                std::lock_guard<std::mutex> lock(c.mutex);
+                c.live[got.ptr].released = got.released;
+            }
+            if (!rc)
+                rc = ordered ? check(hipStreamWaitEvent(stream, got.released, 0), "hipStreamWaitEvent(block release)")
+                             : check(hipEventSynchronize(got.released), "hipEventSynchronize(block release)");
             if (rc) return rc;   // the block stays in `live`; its owner-to-be never sees it
         }
         *dev_ptr = got.ptr;
@@ -666,10 +684,12 @@ int pool_free(void* dev_ptr, bool ordered, hipStream_t stream) {
     blk.released = info.released;
     int rc = 0;
     if (ordered) {
-        if (!blk.released) rc = check(hipEventCreateWithFlags(&blk.released, hipEventDisableTiming), "hipEventCreate(block release)");
-        if (!rc) rc = check(hipEventRecord(blk.released, stream), "hipEventRecord(block release)");
         blk.stream = stream;
         blk.pending = true;
+        if (stream) {
+            rc = record_release(&blk);
+            blk.recorded = true;
+        }
     } else {
         // hipFree waits for the device before it releases memory; a block that stays allocated must do the same
         // before another caller can get it
