@@ -510,12 +510,21 @@ struct AsyncGemmKernel {
 
 } // namespace docc_k
 
-// extern "C" kernels docc_<prefix>a_<BM>x<BN>x<BK>s<STAGES>_<nn|nt|tn|tt>
+namespace docc_k {
+// k of part z of a product whose K is cut: `kpart` each, the last part what is left
+__device__ __forceinline__ long gemm_part(long K, long kpart, long z) {
+    const long left = K - z * kpart;
+    return left < kpart ? left : kpart;
+}
+} // namespace docc_k
+
+// extern "C" kernels docc_<prefix>a_<BM>x<BN>x<BK>s<STAGES>_<nn|nt|tn|tt>; kpart > 0: entry z of the batch is part z of K
 #define DOCC_AGEMM_ONE(PREFIX, T, OT, BM, BN, BK, WM, WN, ST, TA, TB, TAG)                                          \
     extern "C" __global__ __launch_bounds__(64 * WM * WN) void DOCC_GEMM_NAME(docc_##PREFIX##a_##BM##x##BN##x##BK##s##ST##_##TAG)(  \
         const T* A, const T* B, OT* C, long M, long N, long K, long lda, long ldb, long ldc, OT alpha, OT beta,    \
-        const OT* bias, int act, long batch_a, long batch_b, long batch_c) {                                       \
+        const OT* bias, int act, long batch_a, long batch_b, long batch_c, long kpart) {                                       \
         const long z = blockIdx.y;                                                                                 \
+        if (kpart > 0) K = docc_k::gemm_part(K, kpart, z);                                                            \
         docc_k::AsyncGemmKernel<T, BM, BN, BK, WM, WN, ST, TA, TB>::run(A + z * batch_a, B + z * batch_b, C + z * batch_c, M, N, \
                                                                         K, lda, ldb, ldc, alpha, beta, bias, act); \
     }
@@ -524,8 +533,9 @@ struct AsyncGemmKernel {
 #define DOCC_AGEMM_SPREAD_ONE(PREFIX, T, OT, BM, BN, BK, WM, WN, ST, TA, TB, TAG)                                   \
     extern "C" __global__ __launch_bounds__(64 * WM * WN) void DOCC_GEMM_NAME(docc_##PREFIX##a_##BM##x##BN##x##BK##p##ST##_##TAG)(  \
         const T* A, const T* B, OT* C, long M, long N, long K, long lda, long ldb, long ldc, OT alpha, OT beta,    \
-        const OT* bias, int act, long batch_a, long batch_b, long batch_c) {                                       \
+        const OT* bias, int act, long batch_a, long batch_b, long batch_c, long kpart) {                                       \
         const long z = blockIdx.y;                                                                                 \
+        if (kpart > 0) K = docc_k::gemm_part(K, kpart, z);                                                            \
         docc_k::AsyncGemmKernel<T, BM, BN, BK, WM, WN, ST, TA, TB, true>::run(A + z * batch_a, B + z * batch_b, C + z * batch_c, \
                                                                               M, N, K, lda, ldb, ldc, alpha, beta, bias, act);  \
     }

@@ -188,8 +188,9 @@ struct AsyncGemm16Kernel {
 #define DOCC_AGEMM16_ONE(BM, BN, WM, WN, ST, TA, TB, TAG)                                                                       \
     extern "C" __global__ __launch_bounds__(64 * WM * WN) void DOCC_GEMM_NAME(docc_bgemma_##BM##x##BN##x32q##ST##_##TAG)(       \
         const uint16_t* A, const uint16_t* B, float* C, long M, long N, long K, long lda, long ldb, long ldc, float alpha,     \
-        float beta, const float* bias, int act, long batch_a, long batch_b, long batch_c) {                                    \
+        float beta, const float* bias, int act, long batch_a, long batch_b, long batch_c, long kpart) {                                    \
         const long z = blockIdx.y;                                                                                             \
+        if (kpart > 0) K = docc_k::gemm_part(K, kpart, z);                                                            \
         docc_k::AsyncGemm16Kernel<BM, BN, WM, WN, ST, TA, TB>::run(A + z * batch_a, B + z * batch_b, C + z * batch_c, M, N, K, \
                                                                    lda, ldb, ldc, alpha, beta, bias, act);                    \
     }

@@ -41,10 +41,10 @@ double bgemm_seconds(const TileConfig& c, int64_t m, int64_t n, int64_t k, bool 
     const double part = (double) last / cus;
     const double rounds = (double) (tiles / cus) + (!last ? 0.0 : tiles < cus && c.bn == 128 ? 0.7 + 0.2 * part : 0.5 + 0.4 * part);
     // relative to the 256 x 256 tile on the 16x16x32 MFMA (which takes K in whole pairs of 32): the 128 x 256 one reads a k-major B from
-    // LDS at half the width; 128 x 128 tiles in several rounds read the operands from further away than L2
+    // LDS at half the width (and has the deepest pipeline to fill); 128 x 128 tiles in several rounds read the operands from further away than L2
     const double rel = c.bm == 256 ? (k % 64 == 0 ? 1.0 : 0.93) : c.bn == 256 ? (tb ? 0.88 : 0.80) : tiles > cus ? 0.75 : 0.86;
-    const double area = (double) c.bm * c.bn;
-    return 1e-6 * (4.0 + rounds * (area * (11.0 / 65536) + area * (double) k * 3.6e-7 / rel));
+    const double area = (double) c.bm * c.bn, fill = c.bm < c.bn ? (tb ? 1.5 : 3.0) : 0.0;
+    return 1e-6 * (4.0 + rounds * (fill + area * (11.0 / 65536) + area * (double) k * 3.6e-7 / rel));
 }
 
 // What GemmFinish of csrc/kernels/gemm_finish.h holds: the rest of a layer behind a product.
@@ -68,8 +68,8 @@ int finish_parts(hipStream_t s, const void* P, int64_t m, int64_t n, int parts, 
 // shape is not one of theirs (the caller goes on to the tiled kernels), 0 or an error code otherwise.
 template <typename T, typename S>
 int gemv_launch(const char* prefix, hipStream_t s, bool ta, bool tb, int64_t m, int64_t n, int64_t k, S alpha, const T* A, int64_t lda,
-                const T* B, int64_t ldb, S beta, S* C, int64_t ldc) {
-    if (std::getenv("DOCC_ROCM_GEMV_OFF")) return 1;   // tuning and tests: always the tiled kernels
+                const T* B, int64_t ldb, S beta, S* C, int64_t ldc, bool tuned) {
+    if (tuned && std::getenv("DOCC_ROCM_GEMV_OFF")) return 1;   // tuning and tests: always the tiled kernels
     const T *M, *x;
     int64_t ld, incx, incy, rows, cols;
     bool by_rows;
@@ -108,7 +108,7 @@ int gemv_launch(const char* prefix, hipStream_t s, bool ta, bool tb, int64_t m, 
             const int64_t fit = (int64_t) kPartialsBytes / ((int64_t) sizeof(S) * cols * group);
             if (slices > fit) slices = fit;
             if (slices > 256) slices = 256;
-            if (const char* e = std::getenv("DOCC_ROCM_GEMV_SLICES")) {   // tuning: a cap on the slices
+            if (const char* e = tuned ? std::getenv("DOCC_ROCM_GEMV_SLICES") : nullptr) {   // tuning: a cap on the slices
                 const int64_t cap = std::atoi(e);
                 if (cap >= 1 && cap < slices) slices = cap;
             }
@@ -198,7 +198,7 @@ int gemv_launch(const char* prefix, hipStream_t s, bool ta, bool tb, int64_t m, 
     const int64_t fit = (int64_t) kPartialsBytes / ((int64_t) sizeof(S) * cols);
     if (slices > fit) slices = fit;
     if (slices > 256) slices = 256;
-    if (const char* e = std::getenv("DOCC_ROCM_GEMV_SLICES")) {   // tuning: a cap on the slices
+    if (const char* e = tuned ? std::getenv("DOCC_ROCM_GEMV_SLICES") : nullptr) {   // tuning: a cap on the slices
         const int64_t cap = std::atoi(e);
         if (cap >= 1 && cap < slices) slices = cap;
     }
@@ -217,13 +217,14 @@ int gemv_launch(const char* prefix, hipStream_t s, bool ta, bool tb, int64_t m, 
                   alpha, beta);
 }
 
-// T: element type of A and B; S: type of C, alpha and beta
+// T: element type of A and B; S: type of C, alpha and beta. k_total > 0: the `batch` entries are the parts of a product of that k,
+// `k` each and the last one what is left.
 template <typename T, typename S = T>
 int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int trans_b, int64_t m, int64_t n,
                 int64_t k, S alpha, const T* A, int64_t lda, const T* B, int64_t ldb, S beta, S* C, int64_t ldc,
                 TileConfig (*pick)(int64_t m, int64_t n, int64_t k, bool tb, int64_t batch, bool aligned, int force), const S* bias = nullptr,
                 int activation = -1, int64_t batch = 1, int64_t batch_a = 0, int64_t batch_b = 0, int64_t batch_c = 0,
-                const LinearFinish* fin = nullptr) {
+                const LinearFinish* fin = nullptr, int64_t k_total = 0) {
     if ((trans_a != DOCC_ROCM_NO_TRANS && trans_a != DOCC_ROCM_TRANS) ||
         (trans_b != DOCC_ROCM_NO_TRANS && trans_b != DOCC_ROCM_TRANS))
         return fail(DOCC_ROCM_ERR_INVALID_ARGUMENT, "%s: transpose code must be 111 or 112", prefix);
@@ -246,6 +247,8 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
     if (rc) return rc;
     hipStream_t s = (hipStream_t) stream;
     char name[96];
+    const bool tuned = gemm_tuning_set();
+    auto tuning = [&](const char* variable) -> const char* { return tuned ? std::getenv(variable) : nullptr; };
     // with a finish (docc_rocm_linear): where no kernel has it in its store, the product goes to a block of the device block
     // cache and the chain runs as one pass over it. `product(C)` returns 1 where it does not take the shape.
     auto through_memory = [&](auto&& product) -> int {
@@ -281,7 +284,7 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
     // ninth of the rate) and the matrix-vector kernels want the vectors contiguous along k. B is small: it is transposed
     // into a block of the device block cache first (k x n elements), and the product runs as A B'^T.
     if (!tb && batch == 1 && n >= 2 && n <= 64 && ldb == n && m >= 1024 && k >= 256 && k % (16 / (int64_t) sizeof(T)) == 0 &&
-        (n <= 4 || n % (16 / (int64_t) sizeof(T)) != 0) && !std::getenv("DOCC_ROCM_GEMV_OFF")) {
+        (n <= 4 || n % (16 / (int64_t) sizeof(T)) != 0) && !tuning("DOCC_ROCM_GEMV_OFF")) {
         if (fin) return through_memory(plain_product);
         void* bt = nullptr;
         if ((rc = docc_rocm_malloc_async(&bt, (size_t) (n * k) * sizeof(T), stream))) return rc;
@@ -295,7 +298,7 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
     // Five to 32 rows of fp32 against a wide matrix go to the kernels of csrc/kernels/gemm_skinny.hip (below); measured against
     // the tiles with K in parts and the matrix-vector forms, they pay from 8 M elements of B (16 M above 16 rows).
     // DOCC_ROCM_GEMM_SKINNY=1 takes them for smaller ones too (tests).
-    const char* skinny_env = std::getenv("DOCC_ROCM_GEMM_SKINNY");
+    const char* skinny_env = tuning("DOCC_ROCM_GEMM_SKINNY");
     const bool skinny_on = !(skinny_env && skinny_env[0] == '0'), skinny_any_size = skinny_env && skinny_env[0] == '1';
     // (a lane's offset from the chunk's base, up to 31 rows of either operand, is held in 32 bits)
     const bool skinny_base = batch == 1 && !ta && (!epilogue || ldc == n) && n >= 512 && k >= 512 && skinny_on && (uintptr_t) A % 16 == 0 &&
@@ -314,10 +317,10 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
                             lda % 2 == 0 && ldb % 2 == 0 && k % 2 == 0 && n % 2 == 0;
     const bool skinny = skinny_f32 || skinny_bf16 || skinny_f64;
     if (fin && (m <= 8 || n <= 8) && !skinny && batch == 1) {
-        rc = through_memory([&](S* to) { return gemv_launch<T, S>(prefix, s, ta, tb, m, n, k, alpha, A, lda, B, ldb, (S) 0, to, n); });
+        rc = through_memory([&](S* to) { return gemv_launch<T, S>(prefix, s, ta, tb, m, n, k, alpha, A, lda, B, ldb, (S) 0, to, n, tuned); });
         if (rc != 1) return rc;
     } else if ((m <= 8 || n <= 8) && !skinny && batch == 1 && (!epilogue || ldc == n)) {
-        rc = gemv_launch<T, S>(prefix, s, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc);
+        rc = gemv_launch<T, S>(prefix, s, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, tuned);
         if (rc == 0 && epilogue) {
             // the few rows or columns of output are a small tensor: bias and activation as one elementwise pass over it,
             // the same roundings as the fused store
@@ -367,7 +370,7 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
                     parts = p;
                 }
             }
-            if (const char* e = std::getenv("DOCC_ROCM_GEMM_SPLITK"))
+            if (const char* e = tuning("DOCC_ROCM_GEMM_SPLITK"))
                 if (std::atoll(e) > 0 && part_length(std::atoll(e)) >= unit) parts = std::atoll(e);
             const int64_t kpart = part_length(parts);
             parts = (k + kpart - 1) / kpart;
@@ -415,11 +418,61 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
             }
         }
     }
+    // Operands the vectors of the asynchronous kernels do not fit are packed first (csrc/kernels/gemm_pack.hip): those that are
+    // off, both of them where k itself is no whole number of vectors. That costs a launch of 4-5 us and reading and writing the operands
+    // once; the element-wise tiles sustain a tenth (bf16 read along m or n) to nine tenths (fp64) of the others' rate, and wait for every
+    // step of a long k. Measured, k one off the vector: bf16 4096^3 649-1195 us plain against 134-208 packed, 512^3 13-27 against 12;
+    // fp32 2048^3 190-310 against 148-272, 512^3 read along n 23.6 against 15.8, otherwise 15.3 against 15.2, 3000 x 500 x 300 16-19
+    // against 21 (few steps, enough tiles: plain); fp64 2048^3 read along n 365 against 329, otherwise 279 against 286 (plain), 512^3 25
+    // against 20, 128 x 2048 x 8192 362 against 135. DOCC_ROCM_GEMM_PACK=0 switches it off, =1 packs whatever the size (tests, tuning).
+    const char* pack_env = tuning("DOCC_ROCM_GEMM_PACK");
+    if (!aligned && batch == 1 && !(pack_env && pack_env[0] == '0')) {
+        const int64_t v = (int64_t) vec;
+        const bool whole_k = k % v == 0;
+        auto off = [&](const T* p, int64_t ld, int64_t contiguous) { return (uintptr_t) p % 16 != 0 || ld % v != 0 || contiguous % v != 0; };
+        const bool pack_a = !whole_k || off(A, lda, a_contig), pack_b = !whole_k || off(B, ldb, b_contig);
+        const bool turned = (pack_a && ta) || (pack_b && !tb);   // an operand would be read along m or n
+        const double work = (double) m * (double) n * (double) k;
+        const int64_t kp = pack_a && pack_b ? (k + 63) / 64 * 64 : k;
+        const int64_t bytes_a = pack_a ? m * kp * (int64_t) sizeof(T) : 0, bytes_b = pack_b ? n * kp * (int64_t) sizeof(T) : 0;
+        // the plain tiles: the chain of K-steps of one tile, or all of them at the rate they sustain; against the copies and the rate of the
+        // asynchronous ones (flop per us)
+        const double step_us = sizeof(T) == 2 ? (turned ? 2.3 : 0.95) : sizeof(T) == 4 ? (turned ? 0.58 : 0.31) : turned ? 0.7 : 0.63;
+        const double plain_rate = sizeof(T) == 2 ? (turned ? 1.2e8 : 4.2e8) : sizeof(T) == 4 ? 1.0e8 : turned ? 4.8e7 : 6.2e7;
+        const double packed_rate = sizeof(T) == 2 ? 1.1e9 : sizeof(T) == 4 ? 1.4e8 : 6.6e7;
+        const double chain_us = step_us * (double) k / (sizeof(T) == 2 ? 64 : 16), all_us = 2.0 * work / plain_rate;
+        // (below k = 192 both are bound by storing C)
+        bool pays = (chain_us > 14.0 || k >= 192) && 5.0 + (chain_us > all_us ? chain_us : all_us) >
+                                                         14.0 + 2e-6 / 4.0 * (double) (bytes_a + bytes_b) + 2.0 * work / packed_rate;
+        if (pack_env && pack_env[0] == '1') pays = true;
+        if (pays && bytes_a + bytes_b <= (int64_t(1) << 31)) {
+            const int64_t at_b = (bytes_a + 255) / 256 * 256;
+            void* packed = nullptr;
+            if ((rc = docc_rocm_malloc_async(&packed, (size_t) (at_b + bytes_b), stream))) return rc;
+            struct {
+                const void* src;
+                void* dst;
+                long ld, rows;
+                int k_major;
+            } pa{A, packed, (long) lda, (long) m, ta}, pb{B, (char*) packed + at_b, (long) ldb, (long) n, !tb};
+            const int64_t tiles_k = (kp + 63) / 64;
+            const int64_t groups_a = pack_a ? (m + 63) / 64 * tiles_k : 0, groups_b = pack_b ? (n + 63) / 64 * tiles_k : 0;
+            if (groups_a + groups_b > 0x7fffffffLL) return fail(DOCC_ROCM_ERR_UNSUPPORTED, "%s: too many tiles", prefix);
+            rc = launch(sizeof(T) == 2 ? "docc_gemm_pack_b2" : sizeof(T) == 4 ? "docc_gemm_pack_b4" : "docc_gemm_pack_b8",
+                        (uint32_t) (groups_a + groups_b), 1, 1, 256, 0, s, pa, pb, (long) groups_a, (long) k, (long) kp);
+            if (!rc)
+                rc = gemm_launch<T, S>(prefix, stream, pack_a ? DOCC_ROCM_NO_TRANS : trans_a, pack_b ? DOCC_ROCM_TRANS : trans_b, m, n, kp, alpha,
+                                       pack_a ? (const T*) pa.dst : A, pack_a ? kp : lda, pack_b ? (const T*) pb.dst : B, pack_b ? kp : ldb, beta, C, ldc,
+                                       pick, bias, activation, 1, 0, 0, 0, fin);
+            const int rc2 = docc_rocm_free_async(packed, stream);
+            return rc ? rc : rc2;
+        }
+    }
     // DOCC_ROCM_GEMM_TILE=big|small overrides the size heuristic (tests, tuning)
-    const char* force = std::getenv("DOCC_ROCM_GEMM_TILE");
+    const char* force = tuning("DOCC_ROCM_GEMM_TILE");
     TileConfig cfg = pick(m, n, k, tb, batch, aligned, force && force[0] == 'b' ? 1 : force && force[0] == 's' ? -1 : 0);
     // DOCC_ROCM_GEMM_CFG=BMxBNxBKxWAVES[xSTAGES[p|q]] selects a built configuration directly (tuning)
-    if (const char* c = std::getenv("DOCC_ROCM_GEMM_CFG")) {
+    if (const char* c = tuning("DOCC_ROCM_GEMM_CFG")) {
         TileConfig t{};
         char tag = 0;
         const int got = std::sscanf(c, "%dx%dx%dx%dx%d%c", &t.bm, &t.bn, &t.bk, &t.waves, &t.stages, &tag);
@@ -427,8 +480,10 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
         t.small = got == 6 && tag == 'q';
         if (got >= 4 && t.bm > 0 && t.bn > 0 && t.bk > 0 && t.waves > 0) cfg = t;
     }
-    // the 16x16x32 kernels (gemm_async16.h) take whole pairs of K-steps, at least a ring of them
-    if (cfg.small && !(k % (2 * cfg.bk) == 0 && k >= (int64_t) cfg.stages * cfg.bk)) cfg.small = false;
+    // the 16x16x32 kernels (gemm_async16.h) take whole pairs of K-steps, at least a ring of them, in the last part too
+    const int64_t k_last = k_total > 0 ? k_total - (batch - 1) * k : k;
+    for (int64_t kk : {k, k_last})
+        if (cfg.small && !(kk % (2 * cfg.bk) == 0 && kk >= (int64_t) cfg.stages * cfg.bk)) cfg.small = false;
     // the asynchronous kernels need aligned operands and address a tile with 32-bit byte offsets
     const int64_t max_edge = cfg.bm > cfg.bn ? (cfg.bm > cfg.bk ? cfg.bm : cfg.bk) : (cfg.bn > cfg.bk ? cfg.bn : cfg.bk);
     const bool offsets_fit = max_edge * (lda > ldb ? lda : ldb) * (int64_t) sizeof(T) < (int64_t(1) << 32);
@@ -440,22 +495,26 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
     // one entry of a batched launch into the stream's buffer of partial results, and a second launch adds the parts
     // (in order: the result does not depend on the device's scheduling). DOCC_ROCM_GEMM_SPLITK=0 switches it off,
     // another number forces that many parts where K allows it (tests, tuning).
-    if (batch == 1 && (!epilogue || ldc == n) && aligned && k >= 1024) {
+    const bool largest_fits = 256 * (lda > ldb ? lda : ldb) * (int64_t) sizeof(T) < (int64_t(1) << 32);   // whatever tile the parts take
+    if (batch == 1 && (!epilogue || ldc == n) && cfg.stages > 0 && largest_fits && k >= 512) {
         int cus = compute_units();
         if (cus <= 0) cus = 256;
-        const char* env = std::getenv("DOCC_ROCM_GEMM_SPLITK");
+        const char* env = tuning("DOCC_ROCM_GEMM_SPLITK");
         // the parts' products: in the stream's buffer of partial results where they fit, else in a block of the device
         // block cache (taken and returned in stream order), up to 64 MiB
         constexpr int64_t kMaxPartBytes = int64_t(64) << 20;
+        // k of a part: whole steps of 64 of every tile; the last part takes what is left
+        auto part_of = [&](int64_t parts) { return ((k + parts - 1) / parts + 63) / 64 * 64; };
         auto allowed = [&](int64_t parts) {
-            return parts <= 64 && k % parts == 0 && (k / parts) % 64 == 0 && k / parts >= 256 && parts * m * n * (int64_t) sizeof(S) <= kMaxPartBytes;
+            const int64_t part = part_of(parts);
+            return parts <= 64 && (k + part - 1) / part == parts && part >= 256 && parts * m * n * (int64_t) sizeof(S) <= kMaxPartBytes;
         };
         // Estimated seconds of the product in `parts` parts on the tile the picker gives that many matrices: the work of
         // the padded tiles at what the tile sustains (relative to the 128 x 256 one) on the share of the CUs that get a
         // work-group, plus writing and reading the parts at 5 TB/s and a second launch.
         auto seconds = [&](const TileConfig& c, int64_t parts) {
             if (sizeof(T) == 2)
-                return bgemm_seconds(c, m, n, k / parts, tb, parts) + (parts > 1 ? 2.0 * (double) parts * (double) m * (double) n * sizeof(S) / 5e12 + 3e-6 : 0.0);
+                return bgemm_seconds(c, m, n, part_of(parts), tb, parts) + (parts > 1 ? 2.0 * (double) parts * (double) m * (double) n * sizeof(S) / 5e12 + 2e-6 : 0.0);
             const double tm = (double) ((m + c.bm - 1) / c.bm), tn = (double) ((n + c.bn - 1) / c.bn);
             const double area = (double) c.bm * c.bn;
             const double rel = area >= 65536 ? 1.03 : area >= 32768 ? 1.0 : area >= 16384 ? 0.97 : 0.75;
@@ -474,11 +533,12 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
             while (splits * 2 <= wanted && allowed(splits * 2)) splits *= 2;
         } else if (tiles < cus) {   // CUs without a work-group: the case parts are for
             double best = seconds(cfg, 1);
-            for (int64_t parts = 2; allowed(parts); parts *= 2) {
-                const TileConfig c = pick(m, n, k / parts, tb, parts, true, 0);
+            for (int64_t parts : {2, 3, 4, 5, 6, 8, 10, 12, 16, 20, 24, 32, 48, 64}) {
+                if (!allowed(parts)) continue;
+                const TileConfig c = pick(m, n, part_of(parts), tb, parts, true, 0);
                 if (c.stages == 0) break;
                 const double t = seconds(c, parts);
-                if (t < 0.9 * best) {   // only for a clear gain: the estimate is rough
+                if (t < (splits > 1 ? 1.0 : sizeof(T) == 2 ? 0.95 : 0.9) * best) {   // cut for a clear gain only: the estimate is rough
                     best = t;
                     splits = parts;
                 }
@@ -495,9 +555,9 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
                 if ((rc = partials_for(s, &lease))) return rc;
                 parts = lease.ptr;
             }
-            const int64_t part = k / splits;
+            const int64_t part = part_of(splits);
             rc = gemm_launch<T, S>(prefix, stream, trans_a, trans_b, m, n, part, (S) 1, A, lda, B, ldb, (S) 0, (S*) parts, n, pick, nullptr, -1, splits,
-                                   ta ? part * lda : part, tb ? part : part * ldb, m * n);
+                                   ta ? part * lda : part, tb ? part : part * ldb, m * n, nullptr, k);
             if (!rc && fin) {
                 rc = finish_parts(s, parts, m, n, (int) splits, (float) alpha, *fin);
             } else if (!rc) {
@@ -542,6 +602,11 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
     }
     // the variants with bias / activation in the store carry the suffix "_e"
     if (bias || activation >= 0) std::strncat(name, "_e", sizeof(name) - std::strlen(name) - 1);
+    if (cfg.stages > 0)
+        return launch(name, (uint32_t) tiles, (uint32_t) batch, 1, 64 * cfg.waves, (uint32_t) lds, s, A, B, C, (long) m, (long) n,
+                      (long) (k_total > 0 ? k_total : k), (long) lda, (long) ldb, (long) ldc, alpha, beta, bias, activation, (long) batch_a,
+                      (long) batch_b, (long) batch_c, (long) (k_total > 0 ? k : 0));
+    if (k_total > 0) return fail(DOCC_ROCM_ERR_UNSUPPORTED, "%s: K in parts needs the asynchronous tiles", prefix);
     return launch(name, (uint32_t) tiles, (uint32_t) batch, 1, 64 * cfg.waves, (uint32_t) lds, s, A, B, C, (long) m, (long) n,
                   (long) k, (long) lda, (long) ldb, (long) ldc, alpha, beta, bias, activation, (long) batch_a, (long) batch_b,
                   (long) batch_c);

@@ -14,6 +14,8 @@
 #include <map>
 #include <mutex>
 #include <thread>
+
+#include <unistd.h>
 #include <unordered_map>
 #include <vector>
 
@@ -42,6 +44,7 @@ const char* const kKernelImages[] = {
     "docc_rocm_gemm_f32_big.hsaco",
     "docc_rocm_gemm_f32_big_epilogue.hsaco",
     "docc_rocm_gemm_finish.hsaco",
+    "docc_rocm_gemm_pack.hsaco",
     "docc_rocm_gemm_bf16_async_finish.hsaco",
     "docc_rocm_gemm_bf16_async_big_finish.hsaco",
     "docc_rocm_gemm_f32_finish.hsaco",
@@ -339,6 +342,12 @@ void release_partials(hipStream_t stream) {
         }
         delete slot;
     }
+}
+
+bool gemm_tuning_set() {
+    for (char** e = environ; e && *e; e++)
+        if ((*e)[0] == 'D' && std::strncmp(*e, "DOCC_ROCM_GEM", 13) == 0) return true;
+    return false;
 }
 
 int compute_units() {
