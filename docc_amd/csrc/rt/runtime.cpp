@@ -5,6 +5,7 @@
 // that owns the loaded kernel image, with the image located next to the
 // library unless an environment variable points elsewhere
 // (reference runtime.cpp:129-143).
+#include <algorithm>
 #include <dlfcn.h>
 
 #include <cstdio>
@@ -992,8 +993,9 @@ int docc_rocm_take_failure(char* message, size_t message_len) {
     std::lock_guard<std::mutex> lock(g_failure_mutex);
     const int code = g_failure_code;
     if (message && message_len) {
-        std::strncpy(message, g_failure_message.c_str(), message_len - 1);
-        message[message_len - 1] = 0;
+        const size_t n = std::min(g_failure_message.size(), message_len - 1);
+        std::memcpy(message, g_failure_message.data(), n);
+        message[n] = 0;
     }
     g_failure_code = 0;
     g_failure_message.clear();

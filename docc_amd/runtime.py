@@ -7,6 +7,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import threading
 from pathlib import Path
 from typing import Optional
 
@@ -151,11 +152,16 @@ def call(name: str, *args) -> None:
         raise RocmRuntimeError(name, rc, last_error())
 
 
+_failure = threading.local()
+
+
 def take_failure() -> tuple[int, str]:
     """Collects (and clears) the failure reported by generated code, if any."""
-    buf = ctypes.create_string_buffer(1024)
+    buf = getattr(_failure, "text", None)
+    if buf is None:
+        buf = _failure.text = ctypes.create_string_buffer(1024)
     code = lib().docc_rocm_take_failure(buf, 1024)
-    return int(code), buf.value.decode()
+    return code, buf.value.decode()
 
 
 def version() -> str:

@@ -797,10 +797,12 @@ class _CompiledTorch:
         self.func.argtypes = [ctypes.c_void_p] * len(sdfg.arguments)
         self.func.restype = None
         self.inputs, self.outputs, self.gm, self.on_device = inputs, outputs, gm, on_device
+        self._ready = set()      # device indices the runtime has been initialised on
 
     def _operands(self, args, device):
         """The tensors the generated function reads (kept alive by the caller) and their addresses."""
         keep, ptrs = [], []
+        on_gpu = device.type == "cuda"
         for name, (kind, ref) in self.inputs:
             if kind == "arg":
                 t = args[ref]
@@ -808,10 +810,10 @@ class _CompiledTorch:
                 t = self.gm
                 for part in ref.split("."):
                     t = getattr(t, part)
-            t = t.detach()
-            if t.device.type != device.type:
+            if t.is_cuda != on_gpu:
                 raise ValueError(f"input '{name}' is on {t.device}, the program was compiled for {device.type} tensors")
-            t = t.contiguous()
+            if not t.is_contiguous():
+                t = t.detach().contiguous()
             keep.append(t)
             ptrs.append(t.data_ptr())
         return keep, ptrs
@@ -860,16 +862,20 @@ class _CompiledTorch:
         pin = lambda shape, dtype: (not self.on_device and torch.cuda.is_available() and
                                     math.prod(shape) * torch.empty((), dtype=dtype).element_size() >= (1 << 20))
         outs = [torch.empty(shape, dtype=dtype, device=device, pin_memory=pin(shape, dtype)) for _, shape, dtype in self.outputs]
+        side = None
         if self.on_device:
-            runtime.init(device.index or 0)
+            if device.index not in self._ready:      # loads the kernel images; the device is the caller's current one already
+                runtime.init(device.index or 0)
+                self._ready.add(device.index)
             current = torch.cuda.current_stream()
-            if current != torch.cuda.default_stream():
-                current.synchronize()  # the kernels run on the null stream
+            if current.cuda_stream != 0:
+                side = current
+                side.synchronize()  # the kernels run on the null stream
         self.func(*ptrs, *[o.data_ptr() for o in outs])
         code, message = runtime.take_failure()
         if code != 0:
             raise runtime.RocmRuntimeError(self.sdfg.name, code, message)
-        if self.on_device and torch.cuda.current_stream() != torch.cuda.default_stream():
+        if side is not None:
             torch.cuda.default_stream().synchronize()
         return outs[0] if len(outs) == 1 else tuple(outs)
 
@@ -941,6 +947,13 @@ class TorchProgram(DoccProgram):
             self._gm = self.model if isinstance(self.model, torch.fx.GraphModule) else torch.fx.symbolic_trace(self.model)
         return self._gm
 
+    def _shapes(self, args: Sequence[Any]):
+        """What the cache of compiled programs goes by on a call: the same distinctions as _get_cache_key, as a tuple (building the
+        text for seven tensors takes longer than the call of the compiled function)."""
+        import torch
+
+        return tuple([(a.shape, a.dtype, a.is_cuda) if isinstance(a, torch.Tensor) else type(a) for a in args])
+
     def _get_cache_key(self, *args: Any) -> str:
         import torch
 
@@ -975,9 +988,12 @@ class TorchProgram(DoccProgram):
         import torch
 
         examples = self._examples(args)
+        shapes = self._shapes(examples)
+        if output_folder is None:
+            compiled = self.cache.get(shapes)
+            if compiled is not None:
+                return compiled
         key = self._get_cache_key(*examples)
-        if output_folder is None and key in self.cache:
-            return self.cache[key]
         on_device = any(isinstance(a, torch.Tensor) and a.device.type == "cuda" for a in examples)
         sdfg, lowering = self._lower(examples)
         self._sdfg = sdfg
@@ -1016,7 +1032,7 @@ class TorchProgram(DoccProgram):
         compiled = _CompiledTorch(lib_path, sdfg, lowering.inputs, lowering.outputs, self._graph_module(), on_device)
         self._output_info = [{"shape": tuple(shape)} for _, shape, _ in lowering.outputs]
         if output_folder is None:
-            self.cache[key] = compiled
+            self.cache[shapes] = compiled
         self._compiled = compiled
         return compiled
 
