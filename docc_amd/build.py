@@ -55,6 +55,7 @@ KERNEL_FAMILIES = {
     "layernorm": "layernorm.hip",
     "conv2d": "conv2d.hip",
     "attention": "attention.hip",
+    "attention_split": "attention_split.hip",
     "elementwise": "elementwise.hip",
     "reduce": "reduce.hip",
     "transpose": "transpose.hip",
@@ -78,6 +79,7 @@ FAMILY_FLAGS = {
     "gemm_f32_finish": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "conv2d": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "attention": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+    "attention_split": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "gemm_skinny": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
 }
 

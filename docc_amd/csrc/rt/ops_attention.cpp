@@ -10,6 +10,90 @@ using namespace docc::rt::rocm;
 
 namespace {
 
+// The kernels of attention_split.hip: 32 queries a work-group, the keys cut between its four wavefronts and into `parts` between
+// work-groups. `parts` > 1 needs the parts' results in memory and a second launch that adds them.
+constexpr int kSplitQueries = 32, kSplitBlock = 32 /* keys */, kSplitWaves = 4;
+
+int64_t split_lds_bytes(int64_t D) { return kSplitWaves * (D == 32 ? 4 : 2) * kSplitBlock * D * 4; }   // wavefronts x blocks in the ring x K and V
+
+// Estimates in microseconds of a launch of either form, fitted to 36 shapes of head dims 32, 64 and 128 (within 15 % of them). A step is
+// what a wavefront of the split form (32 keys) or a work-group of the other one (64 keys) needs per block with its CU to itself; work-groups
+// beyond what the CUs hold queue. K and V come from memory once per head, at kMemory.
+struct AttentionRates { double split_step, split_start, step, start; };
+AttentionRates attention_rates(int64_t D) {
+    return D == 32 ? AttentionRates{0.5, 2.2, 0.48, 3.2} : D == 64 ? AttentionRates{0.75, 2.2, 0.8, 3.2} : AttentionRates{0.97, 3.5, 1.2, 5.0};
+}
+constexpr double kMemory = 6.0e6, kCombine = 2.5;   // bytes / us; us of the second launch
+
+// the split form with the best number of parts: its time, and the number in *best
+double attention_split_us(int64_t BH, int64_t SQ, int64_t SKV, int64_t D, int64_t* best) {
+    const AttentionRates r = attention_rates(D);
+    const int64_t tiles = (SQ + kSplitQueries - 1) / kSplitQueries, blocks = (SKV + kSplitBlock - 1) / kSplitBlock;
+    const int64_t cus = compute_units(), slots = cus * (D == 128 ? 1 : 2);   // what the rings' LDS lets a CU hold
+    double best_us = 0;
+    for (const int64_t parts : {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64}) {
+        if (parts > 1 && (parts * kSplitWaves > blocks || BH > 65535)) break;
+        const int64_t groups = tiles * BH * parts, each = (blocks + kSplitWaves * parts - 1) / (kSplitWaves * parts);
+        auto round = [&](int64_t resident) {   // that many work-groups at once, start to end
+            const bool shared = resident > cus;   // two on a CU slow each other
+            const double bound = each * (shared ? 1.33 : 1.0) * r.split_step + (shared ? 1.5 : 1.0) * r.split_start;
+            const double memory = (double) each * resident * kSplitWaves * kSplitBlock * D * 4 / kMemory / tiles;
+            return bound > memory ? bound : memory;
+        };
+        double us = 1.9 + (double) (groups / slots) * round(slots) + (groups % slots ? round(groups % slots) : 0.0);
+        if (parts > 1) us += kCombine + 0.03 * parts + (double) (BH * SQ * parts * D * 8) / (kMemory / 2);
+        if (parts == 1 || us < best_us) *best = parts, best_us = us;
+    }
+    return best_us;
+}
+
+// the form of 128 queries per work-group (the causal one takes a long and a short block of queries together)
+double attention_us(int64_t BH, int64_t SQ, int64_t SKV, int64_t D, bool causal) {
+    const AttentionRates r = attention_rates(D);
+    const int64_t tiles = (SQ + 127) / 128, blocks = (SKV + 63) / 64, cus = compute_units();
+    const int64_t groups = BH * (causal ? (tiles + 1) / 2 : tiles);
+    const int64_t each = causal && 2 * tiles < blocks ? 2 * tiles + 2 : causal && tiles > 1 ? blocks + 2 : blocks;
+    const double memory = (double) (BH * SKV * D * 4) / kMemory * 1.2, bound = (double) each * ((groups + cus - 1) / cus) * r.step;
+    return r.start + (bound > memory ? bound : memory);
+}
+
+int attention_split(hipStream_t s, int64_t BH, int64_t SQ, int64_t SKV, int64_t D, float scale_log2e, const uint16_t* Q, const uint16_t* K,
+                    const uint16_t* V, void* O, int out_bf16, bool causal, int64_t parts) {
+    const int64_t tiles = (SQ + kSplitQueries - 1) / kSplitQueries;
+    float* po = nullptr;
+    if (parts > 1) {
+        // a capture that is not the runtime's own keeps no block for its graph: one part then, and no memory
+        hipStream_t on = resolve_stream(s);
+        hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+        if (on && !capturing() && (hipStreamIsCapturing(on, &status) != hipSuccess || status != hipStreamCaptureStatusNone)) parts = 1;
+        if (parts > 1 && docc_rocm_malloc_async((void**) &po, (size_t) (BH * SQ * parts * (D + 2) * 4), (docc_rocm_stream_t) s) != 0) {
+            po = nullptr;
+            parts = 1;
+        }
+    }
+    float* pm = po ? po + BH * SQ * parts * D : nullptr;
+    char kernel[64];
+    std::snprintf(kernel, sizeof(kernel), "docc_attention_split_d%d_%s%s", (int) D, out_bf16 ? "bf16out" : "f32out", causal ? "_causal" : "");
+    int rc = 0;
+    for (int64_t h0 = 0; h0 < BH && !rc; h0 += 65535) {
+        const int64_t nh = BH - h0 < 65535 ? BH - h0 : 65535;
+        rc = launch(kernel, (uint32_t) tiles, (uint32_t) nh, (uint32_t) parts, 64 * kSplitWaves, (uint32_t) split_lds_bytes(D), s, Q + h0 * SQ * D,
+                    K + h0 * SKV * D, V + h0 * SKV * D, (void*) ((char*) O + h0 * SQ * D * (out_bf16 ? 2 : 4)), po, pm, (int) SQ, (int) SKV, scale_log2e);
+    }
+    if (!rc && parts > 1) {
+        int G = 1;   // threads that share the parts of four values: four parts each, as long as a work-group holds a row
+        while (G * 4 < parts && G * 2 * (D / 4) <= 256) G *= 2;
+        const int64_t rows_per_group = 256 / (G * (D / 4));
+        rc = launch(out_bf16 ? "docc_attention_combine_bf16out" : "docc_attention_combine_f32out", (uint32_t) ((BH * SQ + rows_per_group - 1) / rows_per_group), 1, 1,
+                    256, 0, s, (const float*) po, (const float*) pm, O, (long) (BH * SQ), (int) D, (int) parts, G);
+    }
+    if (po) {
+        const int freed = docc_rocm_free_async(po, (docc_rocm_stream_t) s);
+        rc = rc ? rc : freed;
+    }
+    return rc;
+}
+
 int attention_fused(docc_rocm_stream_t stream, int64_t B, int64_t H, int64_t SQ, int64_t SKV, int64_t D, float scale, const uint16_t* Q,
                     const uint16_t* K, const uint16_t* V, void* O, int out_bf16, bool causal) {
     if (B < 0 || H < 0 || SQ < 0 || SKV < 0 || D < 0) return fail(DOCC_ROCM_ERR_INVALID_ARGUMENT, "attention: negative shape");
@@ -29,18 +113,28 @@ int attention_fused(docc_rocm_stream_t stream, int64_t B, int64_t H, int64_t SQ,
     const float scale_log2e = scale * 1.4426950408889634f;
     // Two forms: 256 queries per work-group (a wavefront takes 64, so each K/V operand read from LDS serves two
     // MFMAs: fewer instructions per flop) once that still gives every CU its two resident work-groups, else 128
-    // per work-group (more, smaller work-groups). DOCC_ROCM_ATTENTION_Q=128|256 forces one (tuning and tests).
+    // per work-group (more, smaller work-groups). DOCC_ROCM_ATTENTION_Q=32|128|256 forces one (tuning and tests).
     const int64_t BH = B * H, out_bytes = out_bf16 ? 2 : 4;
     // ... and only where the larger groups do not add padded queries: a wavefront multiplies its 64 queries whether they
     // exist or not (SQ = 100 would run 256 queries in the large form and 128 in the small one)
     const bool no_extra_padding = (SQ + 255) / 256 * 256 <= (SQ + 127) / 128 * 128 || SQ >= 1024;
     int per_group = ((SQ + 255) / 256) * BH >= 2 * compute_units() && no_extra_padding ? 256 : 128;
+    // head dim 128: the large form is eight wavefronts of 32 queries (one work-group per CU), the small one four
+    if (D == 128) per_group = ((SQ + 255) / 256) * BH >= compute_units() && no_extra_padding ? 256 : 128;
+    // Few queries, or few work-groups: the form that cuts the keys, where the estimates say so by more than they are off. Both forms,
+    // measured (B, H, SQ, SKV, D, us of 128 queries a group / cut keys): 1,4,1,32768,128 609 / 17; 4,8,4,8192,64 104 / 16; 16,16,1,4096,128
+    // 96-106 / 93; 32,32,1,1024,128 115 / 94; 1,4,2048,2048,64 28 / 15; 1,16,1024,1024,64 16 / 12; on the other side 2,16,1024,1024,64 17 / 23;
+    // 4,16,256,256,128 10 / 14; 16,16,128,128,64 6 / 10
+    int64_t parts = 1;
+    if (per_group == 128) {
+        const double split = attention_split_us(BH, SQ, SKV, D, &parts);
+        if (split < 0.92 * attention_us(BH, SQ, SKV, D, causal)) per_group = kSplitQueries;
+    }
     if (const char* force = std::getenv("DOCC_ROCM_ATTENTION_Q")) {
         const int v = std::atoi(force);
-        if (v == 128 || v == 256) per_group = v;
+        if (v == 32 || v == 128 || v == 256) per_group = v;
     }
-    // head dim 128: the large form is eight wavefronts of 32 queries (one work-group per CU), the small one four
-    if (D == 128 && !std::getenv("DOCC_ROCM_ATTENTION_Q")) per_group = ((SQ + 255) / 256) * BH >= compute_units() && no_extra_padding ? 256 : 128;
+    if (per_group == kSplitQueries) return attention_split((hipStream_t) stream, BH, SQ, SKV, D, scale_log2e, Q, K, V, O, out_bf16, causal, parts);
     char kernel[64];
     std::snprintf(kernel, sizeof(kernel), "docc_attention_bf16_d%d_q%d_%s%s", (int) D, per_group, out_bf16 ? "bf16out" : "f32out",
                   causal ? "_causal" : "");

@@ -53,6 +53,7 @@ const char* const kKernelImages[] = {
     "docc_rocm_layernorm.hsaco",
     "docc_rocm_conv2d.hsaco",
     "docc_rocm_attention.hsaco",
+    "docc_rocm_attention_split.hsaco",
     "docc_rocm_elementwise.hsaco",
     "docc_rocm_reduce.hsaco",
     "docc_rocm_transpose.hsaco",
