@@ -253,7 +253,7 @@ DOCC_CONV_GATHER(64, 128, 16, 2, 2, false, u)
 
 namespace docc_k {
 
-template <int KH, int KW, bool SPLIT = false, bool NARROW = false, int TILES = 7, bool MULTI = false>
+template <int KH, int KW, bool SPLIT = false, bool NARROW = false, int TILES = 7, bool MULTI = false, bool PARTS = false>
 struct ConvHaloKernel {
     static_assert(!MULTI || !SPLIT, "several images per work-group: the plain strips only");
     static_assert(!NARROW || SPLIT, "the narrow tile is the shared tile of a split strip");
@@ -271,7 +271,8 @@ struct ConvHaloKernel {
     // MULTI: a work-group takes G whole images (TH == OH; images of a few pixels, which alone would fill a fraction of
     // the smallest strip): the patch buffer holds their G patches one after the other, pixel q of the strip is pixel
     // q % (OH * OW) of image q / (OH * OW).
-    static __device__ __forceinline__ void run(const ConvParams& p, int TH, int G = 1) {
+    // PARTS: X and W start at the channels of this work-group's part, of which there are `chunks` chunks.
+    static __device__ __forceinline__ void run(const ConvParams& p, int TH, int G = 1, int chunks = 0) {
         extern __shared__ __attribute__((aligned(16))) unsigned char docc_conv_lds[];
         float* const lds = reinterpret_cast<float*>(docc_conv_lds);
         const int tid = threadIdx.x, lane = tid & 63, wave = SPLIT ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6;   // SPLIT: the mirrored tap is a scalar
@@ -679,7 +680,7 @@ struct ConvHaloKernel {
             }
         };
 
-        const int nch = p.C / CI;
+        const int nch = PARTS ? chunks : p.C / CI;
         gload(0);
         // the index arithmetic nothing needs before the first operand read goes here, under the loads' way to memory and back
         // (left to the compiler it lands behind the barrier, in front of the first MFMA)
@@ -904,6 +905,56 @@ extern "C" __global__ __launch_bounds__(256) void docc_conv2d_f32_halo_1x1_t2m(d
 extern "C" __global__ __launch_bounds__(256) void docc_conv2d_f32_halo_1x1_t2m_g(docc_k::ConvParams p, int TH, int G) {
     docc_k::conv_select_group(p);
     docc_k::ConvHaloKernel<1, 1, false, false, 2, true>::run(p, TH, G);
+}
+
+// The channels cut into gridDim.z parts, one work-group each: a few images of many channels are a handful of strips whose chunks
+// follow one another (1 x 256 x 14 x 14, 256 channels out: 8 work-groups, 85 us). A part's sums, without the bias, lie in
+// sums[part][N][OC][OH][OW]; docc_conv2d_add_parts_f32 adds them up.
+#define DOCC_CONV_PARTS(K, FORM, TILES, MULTI)                                                                                              \
+    extern "C" __global__ __launch_bounds__(256) void docc_conv2d_f32_halo_##K##x##K##_##FORM##_parts(docc_k::ConvParams p, int TH, int G,   \
+                                                                                                      float* sums) {                        \
+        typedef docc_k::ConvHaloKernel<K, K, false, false, TILES, MULTI, true> Kernel;                                                      \
+        const int all = p.C / Kernel::CI, parts = gridDim.z, part = blockIdx.z;                                                             \
+        const int first = (int) ((long) all * part / parts), next = (int) ((long) all * (part + 1) / parts);                                \
+        p.X += (long) first * Kernel::CI * p.H * p.W;                                                                                       \
+        p.Wt += (long) first * Kernel::KC;                                                                                                  \
+        p.bias = nullptr;                                                                                                                   \
+        p.Y = sums + (long) part * p.N * p.OC * p.OH * p.OW;                                                                                \
+        Kernel::run(p, TH, G, next - first);                                                                                                \
+    }
+DOCC_CONV_PARTS(3, t4, 4, false)
+DOCC_CONV_PARTS(3, t2, 2, false)
+DOCC_CONV_PARTS(3, t4m, 4, true)
+DOCC_CONV_PARTS(3, t2m, 2, true)
+DOCC_CONV_PARTS(1, t4, 4, false)
+DOCC_CONV_PARTS(1, t2, 2, false)
+DOCC_CONV_PARTS(1, t4m, 4, true)
+DOCC_CONV_PARTS(1, t2m, 2, true)
+
+// Y = bias + the parts' sums, in the order of the parts; `total` values, a plane of them per channel. A thread takes four
+// consecutive ones where `total` is a multiple of four (VEC), which may lie in two planes.
+template <int VEC>
+__device__ __forceinline__ void conv_add_parts(const float* __restrict__ sums, const float* __restrict__ bias, float* __restrict__ Y, long total,
+                                               int plane, int OC, int parts) {
+    typedef float vec_t __attribute__((ext_vector_type(VEC)));
+    for (long e = ((long) blockIdx.x * 256 + threadIdx.x) * VEC; e < total; e += (long) gridDim.x * 256 * VEC) {
+        vec_t v = *reinterpret_cast<const vec_t*>(sums + e);
+#pragma unroll 4
+        for (int k = 1; k < parts; k++) v += *reinterpret_cast<const vec_t*>(sums + k * total + e);
+        if (bias) {
+#pragma unroll
+            for (int i = 0; i < VEC; i++) v[i] += bias[(e + i) / plane % OC];
+        }
+        *reinterpret_cast<vec_t*>(Y + e) = v;
+    }
+}
+extern "C" __global__ __launch_bounds__(256) void docc_conv2d_add_parts_f32_v4(const float* sums, const float* bias, float* Y, long total, int plane, int OC,
+                                                                              int parts) {
+    conv_add_parts<4>(sums, bias, Y, total, plane, OC, parts);
+}
+extern "C" __global__ __launch_bounds__(256) void docc_conv2d_add_parts_f32(const float* sums, const float* bias, float* Y, long total, int plane, int OC,
+                                                                           int parts) {
+    conv_add_parts<1>(sums, bias, Y, total, plane, OC, parts);
 }
 
 extern "C" __global__ __launch_bounds__(256) void docc_conv2d_f32_halo_3x3_split(docc_k::ConvParams p, int TH) {

@@ -51,6 +51,7 @@ struct HaloPlan {
     int64_t TH = 1;       // output rows per strip
     int64_t images = 1;   // whole images per work-group (then TH == OH): images of a few pixels share a strip
     bool split = false, narrow = false;
+    int64_t parts = 1;    // the channels cut into that many launches' worth of work-groups (forms of 4 and 2 tiles)
     double cost = 0;      // rounds x tiles per wave x overhead
 };
 
@@ -61,8 +62,11 @@ bool halo_strip_fits(int64_t th, int64_t OW, int64_t KH, int64_t KW, int64_t str
     return PS <= 3 * 256 && 3 * stage * 4 <= 160 * 1024;
 }
 
-// cost 0: no form of the kernel fits the layer
-HaloPlan plan_halo(int64_t N, int64_t OC, int64_t OH, int64_t OW, int64_t KH, int64_t KW, int64_t stride_h, int64_t stride_w, int cus) {
+// us per unit of HaloPlan::cost for a filter of K values: the kernel does about 490 GFLOP/s per CU on the tiles it computes
+double halo_unit_us(int64_t K) { return (2.0 * 64 * 64 * (double) K) / 490e3; }
+
+// cost 0: no form of the kernel fits the layer. C = 0: not cut into parts (a group of a grouped convolution, a caller that cannot)
+HaloPlan plan_halo(int64_t N, int64_t C, int64_t OC, int64_t OH, int64_t OW, int64_t KH, int64_t KW, int64_t stride_h, int64_t stride_w, int cus) {
     const int64_t ocb = (OC + 63) / 64;
     auto fits = [&](int64_t th) { return th >= 1 && halo_strip_fits(th, OW, KH, KW, stride_h, stride_w); };
     auto rows_for = [&](int64_t pixels) {
@@ -131,6 +135,35 @@ HaloPlan plan_halo(int64_t N, int64_t OC, int64_t OH, int64_t OW, int64_t KH, in
             plan.cost = cost;
         }
     }
+    // Few work-groups with a long chain of chunks each: the channels go to several of them, whose sums a second launch adds. Measured
+    // that launch takes about 3 us and moves its parts at 3 TB/s, and a part needs 4 us around its chunks; taken where the whole is a
+    // sixth faster by these figures. 8 x 256 x 14 x 14 (3x3, 256 out): 64 work-groups in 85 us, in four parts 31.
+    if (C >= 16 && !forced && plan.cost > 0.0) {
+        const double unit = halo_unit_us(C * KH * KW), chunks = (double) (C / 8), bytes = (double) (N * OC * OH * OW * 4);
+        double best = (plan.cost * unit + 4.0) / 1.2;
+        auto consider = [&](int tiles, double overhead, int64_t th, int64_t images, int64_t groups) {
+            for (const int64_t parts : {2, 3, 4, 6, 8, 12, 16, 24, 32}) {
+                if (parts * 2 > C / 8 || groups * parts > 2 * cus || parts * N * OC * OH * OW > (int64_t(1) << 26)) break;
+                const double each = (double) ((C / 8 + parts - 1) / parts) / chunks;
+                const double us = (double) ((groups * parts + cus - 1) / cus) * (tiles * overhead * unit * each + 4.0) + 3.0 + (double) (parts + 1) * bytes / 3e6;
+                if (us >= best) continue;
+                best = us;
+                plan.tiles = tiles, plan.TH = th, plan.images = images, plan.parts = parts;
+                plan.split = plan.narrow = false;
+                plan.cost = us / unit;
+            }
+        };
+        for (const auto& form : small) {
+            int64_t th = rows_for(64 * form.tiles);
+            while (th > 1 && !fits(th)) th--;
+            if (fits(th)) consider(form.tiles, form.overhead, th, 1, N * ((OH + th - 1) / th) * ocb);
+            int64_t g = 64 * form.tiles / (OH * OW);
+            const int64_t patch = ((OH - 1) * stride_h + KH) * ((OW - 1) * stride_w + KW);
+            if (g > N) g = N;
+            while (g >= 2 && !(g * patch <= 3 * 256 && 3 * (64 * (8 * KH * KW + 4) + 8 * (g * patch + 1)) * 4 <= 160 * 1024)) g--;
+            if (g >= 2) consider(form.tiles, form.overhead, OH, g, (N + g - 1) / g * ocb);
+        }
+    }
     return plan;
 }
 
@@ -139,8 +172,8 @@ HaloPlan plan_halo(int64_t N, int64_t OC, int64_t OH, int64_t OW, int64_t KH, in
 // tiles fill the CUs evenly. The GEMM on a column matrix runs at
 // about 75 TFLOP/s on these shapes; the columns are written and read once at about 5 TB/s, and the extra launches
 // (columns, bias, transpose) cost about 15 us.
-double halo_time_us(int64_t N, int64_t OC, int64_t OH, int64_t OW, int64_t KH, int64_t KW, int64_t stride_h, int64_t stride_w, int64_t K, int cus) {
-    return plan_halo(N, OC, OH, OW, KH, KW, stride_h, stride_w, cus).cost * (2.0 * 64 * 64 * (double) K) / 490e3;
+double halo_time_us(int64_t N, int64_t C, int64_t OC, int64_t OH, int64_t OW, int64_t KH, int64_t KW, int64_t stride_h, int64_t stride_w, int64_t K, int cus) {
+    return plan_halo(N, C, OC, OH, OW, KH, KW, stride_h, stride_w, cus).cost * halo_unit_us(K);
 }
 
 double gather_time_us(int64_t N, int64_t OC, int64_t P, int64_t K, int cus) {
@@ -169,7 +202,7 @@ bool halo_shape_ok(int64_t C, int64_t KH, int64_t KW, int64_t OW, int64_t stride
 }
 
 ConvPath choose_path(int64_t N, int64_t C, int64_t OC, int64_t KH, int64_t KW, int64_t OH, int64_t OW, int64_t stride_h, int64_t stride_w,
-                     int64_t pad_h, int64_t pad_w, bool halo_ok, bool have_workspace) {
+                     int64_t pad_h, int64_t pad_w, bool halo_ok, bool have_workspace, bool parts_ok) {
     const char* force = std::getenv("DOCC_ROCM_CONV");   // halo | gather | gemm (tuning and tests)
     const bool pointwise = KH == 1 && KW == 1 && stride_h == 1 && stride_w == 1 && pad_h == 0 && pad_w == 0;
     const ConvPath gemm = pointwise ? ConvPath::Gemm1x1 : ConvPath::GemmColumns;
@@ -185,7 +218,7 @@ ConvPath choose_path(int64_t N, int64_t C, int64_t OC, int64_t KH, int64_t KW, i
     // 1x1 layers move more bytes than they compute, which the models above do not see: measured, the batched GEMM
     // wins from 128 input channels on (C 256 -> 64 on 56 x 56: 50 against 65 us; C 64 -> 256: 99 against 74)
     if (pointwise) return gemm_fast && C >= 128 ? gemm : halo_ok ? ConvPath::Halo : ConvPath::Gather;
-    const double direct = halo_ok ? halo_time_us(N, OC, OH, OW, KH, KW, stride_h, stride_w, K, cus) : gather_time_us(N, OC, P, K, cus);
+    const double direct = halo_ok ? halo_time_us(N, parts_ok ? C : 0, OC, OH, OW, KH, KW, stride_h, stride_w, K, cus) : gather_time_us(N, OC, P, K, cus);
     if (gemm_fast && gemm_time_us(N, OC, P, K, true) < 0.75 * direct) return gemm;
     return halo_ok ? ConvPath::Halo : ConvPath::Gather;
 }
@@ -203,9 +236,10 @@ extern "C" int64_t docc_rocm_conv2d_f32_pads_workspace_bytes(int64_t N, int64_t 
     pad_h = pad_h > pad_h_end ? pad_h : pad_h_end;
     pad_w = pad_w > pad_w_end ? pad_w : pad_w_end;
     if (KH == 1 && KW == 1 && stride_h == 1 && stride_w == 1 && pad_h == 0 && pad_w == 0) return 0;   // the input is the column matrix
-    // nothing either when one of the direct kernels would be chosen anyway (operands assumed aligned)
+    // nothing either when one of the direct kernels would be chosen anyway (operands assumed aligned, the channels in one
+    // piece: cutting them takes memory of its own, which the call may not get)
     const bool halo_ok = halo_shape_ok(C, KH, KW, OW, stride_h, stride_w, dil_h, dil_w);
-    if (choose_path(N, C, OC, KH, KW, OH, OW, stride_h, stride_w, pad_h, pad_w, halo_ok, true) != ConvPath::GemmColumns) return 0;
+    if (choose_path(N, C, OC, KH, KW, OH, OW, stride_h, stride_w, pad_h, pad_w, halo_ok, true, false) != ConvPath::GemmColumns) return 0;
     const int64_t per_image = conv_bytes_per_image(OC, C * KH * KW, OH * OW);
     int64_t images = kConvWorkspaceCap / per_image;
     if (images < 1) images = 1;
@@ -257,7 +291,7 @@ static int conv2d_run(docc_rocm_stream_t stream, int64_t N, int64_t C, int64_t H
                                                                    dil_h, dil_w);
     const bool have_workspace = workspace && workspace_bytes >= need && need > 0 && ((uintptr_t) workspace % 256) == 0;
     ConvPath path = C == 0 ? ConvPath::Gather
-                           : choose_path(N, C, OC, KH, KW, OH, OW, stride_h, stride_w, any_pad_h, any_pad_w, halo_shape, have_workspace);
+                           : choose_path(N, C, OC, KH, KW, OH, OW, stride_h, stride_w, any_pad_h, any_pad_w, halo_shape, have_workspace, !slice);
     // one group of a grouped convolution: the direct kernels, which take the distance between the images as it is (the
     // GEMM paths write whole [N, OC, P] tensors)
     if (slice && (path == ConvPath::Gemm1x1 || path == ConvPath::GemmColumns)) path = halo_shape ? ConvPath::Halo : ConvPath::Gather;
@@ -306,11 +340,38 @@ static int conv2d_run(docc_rocm_stream_t stream, int64_t N, int64_t C, int64_t H
     if (path == ConvPath::Halo) {
         int cus = compute_units();
         if (cus <= 0) cus = 256;
-        const HaloPlan plan = plan_halo(N, OC, OH, OW, KH, KW, stride_h, stride_w, cus);
+        HaloPlan plan = plan_halo(N, slice ? 0 : C, OC, OH, OW, KH, KW, stride_h, stride_w, cus);
+        float* sums = nullptr;
+        if (plan.parts > 1 && !(OC * C * KH * KW < (int64_t(1) << 29) && plan.images * C * H * W < (int64_t(1) << 29) && (OC + 63) / 64 <= 65535))
+            plan = plan_halo(N, 0, OC, OH, OW, KH, KW, stride_h, stride_w, cus);   // the lane offsets are 32 bits
+        if (plan.parts > 1) {
+            // a capture that is not the runtime's own keeps no block for its graph; without memory for the sums the layer runs whole too
+            hipStream_t on = resolve_stream((hipStream_t) stream);
+            hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+            const bool foreign = on && !capturing() && (hipStreamIsCapturing(on, &status) != hipSuccess || status != hipStreamCaptureStatusNone);
+            if (foreign || docc_rocm_malloc_async((void**) &sums, (size_t) (plan.parts * N * OC * OH * OW * 4), stream) != 0) {
+                sums = nullptr;
+                plan = plan_halo(N, 0, OC, OH, OW, KH, KW, stride_h, stride_w, cus);
+            }
+        }
         const int64_t TH = plan.TH;
         const int64_t PS = plan.images * ((TH - 1) * stride_h + KH) * ((OW - 1) * stride_w + KW);   // patch pixels
         const int64_t stage = 64 * (8 * KH * KW + 4) + 8 * (PS + 1);  // weights + patch + spare pixel, floats
         const int64_t strips = (OH + TH - 1) / TH;
+        if (sums) {
+            char name[64];
+            std::snprintf(name, sizeof(name), "docc_conv2d_f32_halo_%s_t%d%s_parts", KH == 3 ? "3x3" : "1x1", plan.tiles, plan.images > 1 ? "m" : "");
+            const int64_t total = N * OC * OH * OW;
+            rc = launch(name, (uint32_t) (plan.images > 1 ? (N + plan.images - 1) / plan.images : N * strips), (uint32_t) ((OC + 63) / 64),
+                        (uint32_t) plan.parts, 256, (uint32_t) (3 * stage * 4), (hipStream_t) stream, p, (int) TH, (int) plan.images, sums);
+            const bool vectors = total % 4 == 0 && (uintptr_t) Y % 16 == 0;
+            const int64_t items = vectors ? total / 4 : total, blocks = (items + 255) / 256;
+            if (!rc)
+                rc = launch(vectors ? "docc_conv2d_add_parts_f32_v4" : "docc_conv2d_add_parts_f32", (uint32_t) (blocks < 2048 ? blocks : 2048), 1, 1, 256, 0,
+                            (hipStream_t) stream, (const float*) sums, bias, Y, (long) total, (int) (OH * OW), (int) OC, (int) plan.parts);
+            const int freed = docc_rocm_free_async(sums, stream);
+            return rc ? rc : freed;
+        }
         if (plan.images > 1 && plan.cost > 0.0 && PS <= 3 * 256 && 3 * stage * 4 <= 160 * 1024 && OC * C * KH * KW < (int64_t(1) << 29) &&
             plan.images * x_channels * H * W < (int64_t(1) << 29) && (OC + 63) / 64 <= 65535) {
             char name[64];
