@@ -79,12 +79,21 @@ public:
         auto it = scalars_.find(v);
         return it != scalars_.end() && it->second->source.is_constant ? it->second->source.data : "";
     }
-    bool is(const std::string& v, double value) const {
+    // the value of a constant that is a plain number; other text (FLT_MAX, an expression) is compiled as it stands and says nothing here
+    bool number(const std::string& v, double* value) const {
         const std::string text = constant(v);
-        if (text.empty()) return false;
         char* end = nullptr;
-        const double got = std::strtod(text.c_str(), &end);
-        return end != text.c_str() && std::fabs(got - value) <= 1e-7 * std::fabs(value);
+        *value = std::strtod(text.c_str(), &end);
+        if (end != text.c_str() && (*end == 'f' || *end == 'F')) end++;
+        return end != text.c_str() && *end == 0;
+    }
+    bool is(const std::string& v, double value) const {
+        double got = 0;
+        return number(v, &got) && std::fabs(got - value) <= 1e-7 * std::fabs(value);
+    }
+    bool is_zero(const std::string& v) const {   // +0: the larger of x and -0 is another zero
+        double got = 0;
+        return number(v, &got) && got == 0.0 && !std::signbit(got);
     }
     // `v` without the conversions it passed through; *rounded: one of them was to bf16
     std::string through_casts(std::string v, bool* rounded) const {
@@ -155,7 +164,7 @@ std::string activation_of(const Values& v, const std::string& name, int* act) {
     *act = -1;
     if (const Statement* s = v.statement(name, "fabs")) return *act = 0, s->args[0];
     if (const Statement* s = v.statement(name, "tanh")) return *act = 5, s->args[0];
-    const std::string r = v.other(name, "fmax", [&](const std::string& a) { return v.constant(a) != "" && std::strtod(v.constant(a).c_str(), nullptr) == 0.0; });
+    const std::string r = v.other(name, "fmax", [&](const std::string& a) { return v.is_zero(a); });
     if (!r.empty()) return *act = 2, r;
     const std::string sg = sigmoid_of(v, name);
     if (!sg.empty()) return *act = 3, sg;

@@ -75,3 +75,42 @@ def test_only_float_products_with_one_reader_are_merged(tmp_path):
     assert got == ["docc_rocm_linear(nullptr, 2, 111, 111, 32, 16, 8, (float) __alpha, _a, 8, _b, 16, nullptr, 2, 18, _residual, 2, 0, _y, 2)"]
     assert "docc_rocm_linear" not in " ".join(calls(two_layers(F64), tmp_path / "b"))
     assert "docc_rocm_linear" not in " ".join(calls(two_layers(F32, second_reader=True), tmp_path / "c"))
+
+
+def bounded_product(bound):
+    b = StructuredSDFGBuilder("bounded")
+    for n in ("X", "W", "Y"):
+        b.add_container(n, F32, True)
+    b.add_container("T0", F32, False, transient_bytes=32 * 16 * 4)
+    b.add_gemm("X", "W", "T0", "1.0", "0.0", 32, 16, 8)
+    b.add_elementwise_op("maximum", "T0", bound, "Y", [32, 16])
+    s = b.move()
+    s.schedule("rocm", options={"offload": "none"})
+    return s
+
+
+# a bound is zero only where its text is the number: any other text goes into the code as it is written
+@pytest.mark.parametrize("bound,relu", [("0.0", True), ("0", True), ("0.0f", True), ("-0.0", False), ("FLT_MAX", False), ("M_PI", False), ("(-1.5)", False),
+                                        ("0.0 + 1.5", False), ("1.5", False)])
+def test_the_larger_of_a_product_and_a_bound(tmp_path, bound, relu):
+    got = " ".join(calls(bounded_product(bound), tmp_path))
+    assert ("docc_rocm_linear" in got) == relu
+    if not relu:
+        assert bound in open(next(tmp_path.glob("*.cpp"))).read()
+
+
+def test_factors_are_read_as_whole_numbers_only(tmp_path):
+    b = StructuredSDFGBuilder("factors")
+    for n in ("X", "W", "Y"):
+        b.add_container(n, F32, True)
+    for n in ("T0", "T1", "T2", "T3", "T4"):
+        b.add_container(n, F32, False, transient_bytes=32 * 16 * 4)
+    b.add_gemm("X", "W", "T0", "1.0", "0.0", 32, 16, 8)
+    b.add_elementwise_op("mul", "T0", "0.7071067811865476 * 2", "T1", [32, 16])
+    b.add_elementwise_unary_op("erf", "T1", "T2", [32, 16])
+    b.add_elementwise_op("add", "T2", "1.0", "T3", [32, 16])
+    b.add_elementwise_op("mul", "T0", "0.5", "T4", [32, 16])
+    b.add_elementwise_op("mul", "T4", "T3", "Y", [32, 16])
+    s = b.move()
+    s.schedule("rocm", options={"offload": "none"})
+    assert "docc_rocm_linear" not in " ".join(calls(s, tmp_path))
