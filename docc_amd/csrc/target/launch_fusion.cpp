@@ -587,7 +587,8 @@ public:
     void dispatch_code(codegen::PrettyPrinter& s, codegen::PrettyPrinter& globals, codegen::CodeSnippetFactory&) override {
         emit_runtime_preamble(globals, function_);
         if (const auto* l = dynamic_cast<const LinearLaunch*>(&node_)) {
-            s << "DOCC_ROCM_CHECK(docc_rocm_linear(nullptr, " << type_code(l->type) << ", " << (l->trans_a ? 112 : 111) << ", " << (l->trans_b ? 112 : 111)
+            // an empty product is not launched, as the GEMM's dispatcher has it (a leading dimension of 0 is an error to the launcher)
+            s << "if ((" << l->m << ") != 0 && (" << l->n << ") != 0) DOCC_ROCM_CHECK(docc_rocm_linear(nullptr, " << type_code(l->type) << ", " << (l->trans_a ? 112 : 111) << ", " << (l->trans_b ? 112 : 111)
               << ", " << l->m << ", " << l->n << ", " << l->k << ", (float) __alpha, _a, " << l->lda << ", _b, " << l->ldb << ", "
               << (l->has_bias ? "_bias" : "nullptr") << ", " << type_code(l->bias_type) << ", " << l->activation << ", "
               << (l->has_residual ? "_residual" : "nullptr") << ", " << type_code(l->residual_type) << ", " << l->rounding << ", _y, " << type_code(l->y_type)

@@ -114,3 +114,19 @@ def test_factors_are_read_as_whole_numbers_only(tmp_path):
     s = b.move()
     s.schedule("rocm", options={"offload": "none"})
     assert "docc_rocm_linear" not in " ".join(calls(s, tmp_path))
+
+
+def test_an_empty_product_is_not_launched(tmp_path):
+    # no columns: the leading dimension of W and Y is 0, which the launcher refuses; the GEMM node alone has always been guarded
+    b = StructuredSDFGBuilder("empty")
+    b.add_container("n", Scalar(PrimitiveType.Int64), True)
+    for name in ("X", "W", "Y"):
+        b.add_container(name, F32, True)
+    b.add_container("T", F32, False, transient_bytes="32*n*4")
+    b.add_gemm("X", "W", "T", "1.0", "0.0", 32, "n", 8)
+    b.add_elementwise_unary_op("sigmoid", "T", "Y", [32, "n"])
+    s = b.move()
+    s.schedule("rocm", options={"offload": "none"})
+    assert "docc_rocm_linear" in " ".join(calls(s, tmp_path))
+    text = re.sub(r"\s+", " ", open(next(tmp_path.glob("*.cpp"))).read())
+    assert "if ((32) != 0 && (n) != 0) DOCC_ROCM_CHECK(docc_rocm_linear(" in text
