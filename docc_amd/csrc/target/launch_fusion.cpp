@@ -274,10 +274,16 @@ private:
     // ---- what may move -------------------------------------------------------------------------------
     bool ours(size_t i) const { return blocks_[i].node->implementation_type() == ImplementationType_ROCMWithoutTransfers; }
 
-    bool written_between(const std::string& name, size_t from, size_t to) const {
-        for (size_t i = from + 1; i < to; i++)
-            for (auto& out : blocks_[i].outputs)
+    // whether what stands between two blocks writes `name` or releases it (a download that frees its buffer has stayed in place)
+    bool lost_between(const std::string& name, size_t from, size_t to) const {
+        for (size_t i = from + 1; i < to; i++) {
+            const Block& b = blocks_[i];
+            for (auto& out : b.outputs)
                 if (out.data == name) return true;
+            if (!is_offloading(b) || !static_cast<const ROCMDataOffloadingNode&>(*b.node).is_free()) continue;
+            for (auto& in : b.inputs)
+                if (!in.is_constant && in.data == name) return true;
+        }
         return false;
     }
 
@@ -403,10 +409,10 @@ private:
         const std::string result = f.results[0].data, a = product.input("__A")->data, b = product.input("__B")->data;
         // what the product reads it now reads where block j stands; what block j reads of its own it reads there already
         for (const std::string& name : {a, b, bias ? std::string() : bias_name})
-            if (!name.empty() && written_between(name, i, j)) return false;
+            if (!name.empty() && lost_between(name, i, j)) return false;
         if (result == a || result == b || result == bias_name) return false;
         const ConnectorBinding alpha = *product.input("__alpha");
-        if (!alpha.is_constant && written_between(alpha.data, i, j)) return false;
+        if (!alpha.is_constant && lost_between(alpha.data, i, j)) return false;
 
         std::vector<std::string> connectors{"_a", "_b", "__alpha"};
         std::vector<ConnectorBinding> inputs{bind("_a", a), bind("_b", b), alpha};
@@ -555,7 +561,7 @@ private:
         for (auto& name : links)
             if (!private_to(name, users)) return false;
         const std::string result = f->results[0].data;
-        if (written_between(source, *gone.begin(), q)) return false;
+        if (lost_between(source, *gone.begin(), q)) return false;
         for (auto* r : {weight, bias})   // (X in place is fine: a row is read before it is written)
             if (r && r->data == result) return false;
 

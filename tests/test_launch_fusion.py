@@ -1,5 +1,6 @@
 """Launches merged when host code is generated: what is emitted for a layer and for a layer norm spelled with tensor nodes, and what
 keeps its separate launches."""
+import json
 import re
 
 import pytest
@@ -7,7 +8,7 @@ import torch
 import torch.nn.functional as F
 
 import docc_amd.torch as docc_torch
-from docc_amd.sdfg import Pointer, PrimitiveType, Scalar, StructuredSDFGBuilder
+from docc_amd.sdfg import Pointer, PrimitiveType, Scalar, StructuredSDFG, StructuredSDFGBuilder
 
 F32, F64 = Pointer(Scalar(PrimitiveType.Float)), Pointer(Scalar(PrimitiveType.Double))
 
@@ -130,3 +131,34 @@ def test_an_empty_product_is_not_launched(tmp_path):
     assert "docc_rocm_linear" in " ".join(calls(s, tmp_path))
     text = re.sub(r"\s+", " ", open(next(tmp_path.glob("*.cpp"))).read())
     assert "if ((32) != 0 && (n) != 0) DOCC_ROCM_CHECK(docc_rocm_linear(" in text
+
+
+@pytest.mark.parametrize("between", [False, True])
+def test_an_operand_that_a_download_frees_stays_with_its_product(tmp_path, between):
+    # H is computed, multiplied and copied back; the copy releases its device buffer. Where that happens between the product and the
+    # elementwise node behind it, the product must not move down to that node
+    b = StructuredSDFGBuilder("download")
+    for n in ("X", "W", "H", "Y"):
+        b.add_container(n, F32, True)
+    for n in ("T0", "T1"):
+        b.add_container(n, F32, False, transient_bytes=32 * 16 * 4)
+    b.add_elementwise_unary_op("relu", "X", "H", [32, 8])
+    b.add_gemm("H", "W", "T0", "1.0", "0.0", 32, 16, 8)
+    b.add_elementwise_unary_op("sigmoid", "T0", "T1", [32, 16])
+    b.add_elementwise_op("mul", "T0", "T1", "Y", [32, 16])
+    s = b.move()
+    s.schedule("rocm")
+    form = json.loads(s.to_json())
+    blocks = form["root"]["children"]
+    node = lambda e: e["dataflow"]["library_node"]
+    reads = lambda e, name: any(i.get("data", "").endswith(name) for i in e["dataflow"]["inputs"])
+    copy = next(e for e in blocks if node(e).get("transfer_direction") == -1 and reads(e, "_H"))
+    free = next(e for e in blocks if node(e).get("transfer_direction") == 0 and node(e).get("buffer_lifecycle") == -1 and reads(e, "_H"))
+    if between:
+        node(copy)["buffer_lifecycle"] = -1
+        blocks.remove(copy)
+        blocks[blocks.index(free)] = copy
+    names = [node(e)["code"] for e in blocks]
+    assert blocks.index(copy) > names.index("GEMM") if between else blocks.index(copy) < names.index("GEMM")
+    got = calls(StructuredSDFG.parse(json.dumps(form)), tmp_path)
+    assert ("docc_rocm_linear" in " ".join(got)) == (not between)
