@@ -300,7 +300,13 @@ Expression GEMMNode::connector_bytes(const std::string& connector) const {
 bool GEMMNode::reads(const std::string& connector, const std::vector<data_flow::ConnectorBinding>& inputs) const {
     if (connector != "__C") return true;
     for (auto& b : inputs)
-        if (b.connector == "__beta" && b.is_constant) return std::strtod(b.data.c_str(), nullptr) != 0.0;
+        if (b.connector == "__beta" && b.is_constant) {
+            // zero only where the whole text is the number: FLT_EPSILON or an expression is compiled as it stands
+            char* end = nullptr;
+            const double beta = std::strtod(b.data.c_str(), &end);
+            if (end != b.data.c_str() && (*end == 'f' || *end == 'F')) end++;
+            return end == b.data.c_str() || *end != 0 || beta != 0.0;
+        }
     return true;
 }
 

@@ -162,3 +162,15 @@ def test_an_operand_that_a_download_frees_stays_with_its_product(tmp_path, betwe
     assert blocks.index(copy) > names.index("GEMM") if between else blocks.index(copy) < names.index("GEMM")
     got = calls(StructuredSDFG.parse(json.dumps(form)), tmp_path)
     assert ("docc_rocm_linear" in " ".join(got)) == (not between)
+
+
+@pytest.mark.parametrize("beta,read", [("0.0", False), ("0", False), ("0.0f", False), ("0.5", True), ("M_PI", True), ("0.0 + 1.0", True)])
+def test_c_is_read_unless_beta_is_the_number_zero(tmp_path, beta, read):
+    b = StructuredSDFGBuilder("beta")
+    for n in ("X", "W", "C", "Y"):
+        b.add_container(n, F32, True)
+    b.add_gemm("X", "W", "C", "1.0", beta, 32, 16, 8)
+    b.add_elementwise_unary_op("sigmoid", "C", "Y", [32, 16])
+    s = b.move()
+    s.schedule("rocm")
+    assert s.loop_report()["H2D"] == (3 if read else 2)
