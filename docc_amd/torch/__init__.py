@@ -810,7 +810,7 @@ class _CompiledTorch:
                 t = self.gm
                 for part in ref.split("."):
                     t = getattr(t, part)
-            if t.is_cuda != on_gpu:
+            if not (t.is_cuda if on_gpu else t.is_cpu):
                 raise ValueError(f"input '{name}' is on {t.device}, the program was compiled for {device.type} tensors")
             if not t.is_contiguous():
                 t = t.detach().contiguous()
@@ -948,11 +948,11 @@ class TorchProgram(DoccProgram):
         return self._gm
 
     def _shapes(self, args: Sequence[Any]):
-        """What the cache of compiled programs goes by on a call: the same distinctions as _get_cache_key, as a tuple (building the
-        text for seven tensors takes longer than the call of the compiled function)."""
+        """What the cache of compiled programs goes by on a call: the distinctions of _get_cache_key, as a tuple (building the text
+        for seven tensors takes longer than the call of the compiled function). Neither host nor GPU memory: no program runs on those."""
         import torch
 
-        return tuple([(a.shape, a.dtype, a.is_cuda) if isinstance(a, torch.Tensor) else type(a) for a in args])
+        return tuple([(a.shape, a.dtype, a.is_cuda, a.is_cpu) if isinstance(a, torch.Tensor) else type(a) for a in args])
 
     def _get_cache_key(self, *args: Any) -> str:
         import torch

@@ -437,6 +437,24 @@ def test_a_torch_program_is_lowered_for_the_shapes_of_each_call():
         assert node["code"] == "GEMM" and int(node["m"]) == rows
 
 
+def test_a_program_for_host_tensors_takes_no_others():
+    class Relu(torch.nn.Module):
+        def forward(self, x):
+            return torch.relu(x)
+
+    program = docc_torch.compile_torch(Relu(), None, target="rocm")
+    x = torch.randn(4, 8)
+    compiled = program.compile(x)
+    assert program.compile(torch.randn(4, 8)) is compiled
+    # a tensor without memory: its address is 0
+    meta = x.to("meta")
+    assert program._shapes([x]) != program._shapes([meta])
+    with pytest.raises(ValueError, match="is on meta"):
+        compiled._operands([meta], torch.device("cpu"))
+    with pytest.raises(ValueError, match="is on cpu"):
+        compiled._operands([x], torch.device("cuda", 0))
+
+
 def test_reductions_and_softmax_pieces_used_on_their_own():
     @native
     def stats(x):
