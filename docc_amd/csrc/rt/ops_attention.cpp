@@ -62,11 +62,8 @@ int attention_split(hipStream_t s, int64_t BH, int64_t SQ, int64_t SKV, int64_t 
     const int64_t tiles = (SQ + kSplitQueries - 1) / kSplitQueries;
     float* po = nullptr;
     if (parts > 1) {
-        // a capture that is not the runtime's own keeps no block for its graph: one part then, and no memory
-        hipStream_t on = resolve_stream(s);
-        hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-        if (on && !capturing() && (hipStreamIsCapturing(on, &status) != hipSuccess || status != hipStreamCaptureStatusNone)) parts = 1;
-        if (parts > 1 && docc_rocm_malloc_async((void**) &po, (size_t) (BH * SQ * parts * (D + 2) * 4), (docc_rocm_stream_t) s) != 0) {
+        // no block can be had: one part
+        if (foreign_capture(s) || docc_rocm_malloc_async((void**) &po, (size_t) (BH * SQ * parts * (D + 2) * 4), (docc_rocm_stream_t) s) != 0) {
             po = nullptr;
             parts = 1;
         }

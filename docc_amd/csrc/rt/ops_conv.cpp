@@ -290,8 +290,9 @@ static int conv2d_run(docc_rocm_stream_t stream, int64_t N, int64_t C, int64_t H
     const int64_t need = docc_rocm_conv2d_f32_pads_workspace_bytes(N, C, H, W, OC, KH, KW, stride_h, stride_w, pad_h, pad_w, pad_h_end, pad_w_end,
                                                                    dil_h, dil_w);
     const bool have_workspace = workspace && workspace_bytes >= need && need > 0 && ((uintptr_t) workspace % 256) == 0;
+    const bool parts_ok = !slice && !foreign_capture((hipStream_t) stream);   // cutting the channels takes a block of the cache
     ConvPath path = C == 0 ? ConvPath::Gather
-                           : choose_path(N, C, OC, KH, KW, OH, OW, stride_h, stride_w, any_pad_h, any_pad_w, halo_shape, have_workspace, !slice);
+                           : choose_path(N, C, OC, KH, KW, OH, OW, stride_h, stride_w, any_pad_h, any_pad_w, halo_shape, have_workspace, parts_ok);
     // one group of a grouped convolution: the direct kernels, which take the distance between the images as it is (the
     // GEMM paths write whole [N, OC, P] tensors)
     if (slice && (path == ConvPath::Gemm1x1 || path == ConvPath::GemmColumns)) path = halo_shape ? ConvPath::Halo : ConvPath::Gather;
@@ -340,19 +341,13 @@ static int conv2d_run(docc_rocm_stream_t stream, int64_t N, int64_t C, int64_t H
     if (path == ConvPath::Halo) {
         int cus = compute_units();
         if (cus <= 0) cus = 256;
-        HaloPlan plan = plan_halo(N, slice ? 0 : C, OC, OH, OW, KH, KW, stride_h, stride_w, cus);
+        HaloPlan plan = plan_halo(N, parts_ok ? C : 0, OC, OH, OW, KH, KW, stride_h, stride_w, cus);
         float* sums = nullptr;
         if (plan.parts > 1 && !(OC * C * KH * KW < (int64_t(1) << 29) && plan.images * C * H * W < (int64_t(1) << 29) && (OC + 63) / 64 <= 65535))
             plan = plan_halo(N, 0, OC, OH, OW, KH, KW, stride_h, stride_w, cus);   // the lane offsets are 32 bits
-        if (plan.parts > 1) {
-            // a capture that is not the runtime's own keeps no block for its graph; without memory for the sums the layer runs whole too
-            hipStream_t on = resolve_stream((hipStream_t) stream);
-            hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-            const bool foreign = on && !capturing() && (hipStreamIsCapturing(on, &status) != hipSuccess || status != hipStreamCaptureStatusNone);
-            if (foreign || docc_rocm_malloc_async((void**) &sums, (size_t) (plan.parts * N * OC * OH * OW * 4), stream) != 0) {
-                sums = nullptr;
-                plan = plan_halo(N, 0, OC, OH, OW, KH, KW, stride_h, stride_w, cus);
-            }
+        if (plan.parts > 1 && docc_rocm_malloc_async((void**) &sums, (size_t) (plan.parts * N * OC * OH * OW * 4), stream) != 0) {
+            sums = nullptr;   // without memory for the sums the layer runs whole
+            plan = plan_halo(N, 0, OC, OH, OW, KH, KW, stride_h, stride_w, cus);
         }
         const int64_t TH = plan.TH;
         const int64_t PS = plan.images * ((TH - 1) * stride_h + KH) * ((OW - 1) * stride_w + KW);   // patch pixels

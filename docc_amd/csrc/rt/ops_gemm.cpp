@@ -249,9 +249,14 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
     char name[96];
     const bool tuned = gemm_tuning_set();
     auto tuning = [&](const char* variable) -> const char* { return tuned ? std::getenv(variable) : nullptr; };
+    // A block of the device block cache for this call, given back behind its last launch. False: there is none (no memory, or a
+    // capture it could not be kept for), and the product runs in a form without it.
+    auto block = [&](void** ptr, int64_t bytes) { return !foreign_capture(s) && docc_rocm_malloc_async(ptr, (size_t) bytes, stream) == 0; };
     // with a finish (docc_rocm_linear): where no kernel has it in its store, the product goes to a block of the device block
     // cache and the chain runs as one pass over it. `product(C)` returns 1 where it does not take the shape.
     auto through_memory = [&](auto&& product) -> int {
+        if (foreign_capture(s))
+            return fail(DOCC_ROCM_ERR_UNSUPPORTED, "linear: this shape needs device memory between its launches, which a capture that the runtime did not begin cannot keep");
         void* wide = nullptr;
         if (int r = docc_rocm_malloc_async(&wide, (size_t) (m * n) * sizeof(S), stream)) return r;
         int r = product((S*) wide);
@@ -287,13 +292,14 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
         (n <= 4 || n % (16 / (int64_t) sizeof(T)) != 0) && !tuning("DOCC_ROCM_GEMV_OFF")) {
         if (fin) return through_memory(plain_product);
         void* bt = nullptr;
-        if ((rc = docc_rocm_malloc_async(&bt, (size_t) (n * k) * sizeof(T), stream))) return rc;
-        const int64_t shape[2] = {k, n}, perm[2] = {1, 0};
-        rc = docc_rocm_transpose(stream, (int) sizeof(T), 2, shape, perm, B, bt);
-        if (!rc)
-            rc = gemm_launch<T, S>(prefix, stream, trans_a, DOCC_ROCM_TRANS, m, n, k, alpha, A, lda, (const T*) bt, k, beta, C, ldc, pick, bias, activation);
-        const int rc2 = docc_rocm_free_async(bt, stream);
-        return rc ? rc : rc2;
+        if (block(&bt, n * k * (int64_t) sizeof(T))) {
+            const int64_t shape[2] = {k, n}, perm[2] = {1, 0};
+            rc = docc_rocm_transpose(stream, (int) sizeof(T), 2, shape, perm, B, bt);
+            if (!rc)
+                rc = gemm_launch<T, S>(prefix, stream, trans_a, DOCC_ROCM_TRANS, m, n, k, alpha, A, lda, (const T*) bt, k, beta, C, ldc, pick, bias, activation);
+            const int rc2 = docc_rocm_free_async(bt, stream);
+            return rc ? rc : rc2;
+        }
     }
     // Five to 32 rows of fp32 against a wide matrix go to the kernels of csrc/kernels/gemm_skinny.hip (below); measured against
     // the tiles with K in parts and the matrix-vector forms, they pay from 8 M elements of B (16 M above 16 rows).
@@ -316,10 +322,10 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
     const bool skinny_f64 = sizeof(T) == 8 && skinny_base && !tb && m >= 5 && m <= 16 && (n * k >= (int64_t(4) << 20) || skinny_any_size) &&
                             lda % 2 == 0 && ldb % 2 == 0 && k % 2 == 0 && n % 2 == 0;
     const bool skinny = skinny_f32 || skinny_bf16 || skinny_f64;
-    if (fin && (m <= 8 || n <= 8) && !skinny && batch == 1) {
+    if (fin && (m <= 8 || n <= 8) && !skinny && batch == 1 && !foreign_capture(s)) {
         rc = through_memory([&](S* to) { return gemv_launch<T, S>(prefix, s, ta, tb, m, n, k, alpha, A, lda, B, ldb, (S) 0, to, n, tuned); });
         if (rc != 1) return rc;
-    } else if ((m <= 8 || n <= 8) && !skinny && batch == 1 && (!epilogue || ldc == n)) {
+    } else if (!fin && (m <= 8 || n <= 8) && !skinny && batch == 1 && (!epilogue || ldc == n)) {
         rc = gemv_launch<T, S>(prefix, s, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, tuned);
         if (rc == 0 && epilogue) {
             // the few rows or columns of output are a small tensor: bias and activation as one elementwise pass over it,
@@ -376,13 +382,11 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
             parts = (k + kpart - 1) / kpart;
             const int64_t bytes = parts * m * n * (int64_t) sizeof(S);
             const bool direct = !fin && parts == 1 && (tb || ((uintptr_t) C % 16 == 0 && ldc % (skinny_f64 ? 2 : 4) == 0));
-            if (direct || bytes <= (int64_t(64) << 20)) {
+            const bool own_block = !direct && bytes > (int64_t) kPartialsBytes;
+            void* buf = nullptr;
+            if (direct || (bytes <= (int64_t(64) << 20) && (!own_block || block(&buf, bytes)))) {
                 PartialsLease lease;
-                void* buf = nullptr;
-                const bool own_block = !direct && bytes > (int64_t) kPartialsBytes;
-                if (own_block) {
-                    if ((rc = docc_rocm_malloc_async(&buf, (size_t) bytes, stream))) return rc;
-                } else if (!direct) {
+                if (!direct && !own_block) {
                     if ((rc = partials_for(s, &lease))) return rc;
                     buf = lease.ptr;
                 }
@@ -445,19 +449,17 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
         bool pays = (chain_us > 14.0 || k >= 192) && 5.0 + (chain_us > all_us ? chain_us : all_us) >
                                                          14.0 + 2e-6 / 4.0 * (double) (bytes_a + bytes_b) + 2.0 * work / packed_rate;
         if (pack_env && pack_env[0] == '1') pays = true;
-        if (pays && bytes_a + bytes_b <= (int64_t(1) << 31)) {
-            const int64_t at_b = (bytes_a + 255) / 256 * 256;
-            void* packed = nullptr;
-            if ((rc = docc_rocm_malloc_async(&packed, (size_t) (at_b + bytes_b), stream))) return rc;
+        const int64_t tiles_k = (kp + 63) / 64;
+        const int64_t groups_a = pack_a ? (m + 63) / 64 * tiles_k : 0, groups_b = pack_b ? (n + 63) / 64 * tiles_k : 0;
+        const int64_t at_b = (bytes_a + 255) / 256 * 256;
+        void* packed = nullptr;
+        if (pays && bytes_a + bytes_b <= (int64_t(1) << 31) && groups_a + groups_b < (int64_t(1) << 24) && block(&packed, at_b + bytes_b)) {
             struct {
                 const void* src;
                 void* dst;
                 long ld, rows;
                 int k_major;
             } pa{A, packed, (long) lda, (long) m, ta}, pb{B, (char*) packed + at_b, (long) ldb, (long) n, !tb};
-            const int64_t tiles_k = (kp + 63) / 64;
-            const int64_t groups_a = pack_a ? (m + 63) / 64 * tiles_k : 0, groups_b = pack_b ? (n + 63) / 64 * tiles_k : 0;
-            if (groups_a + groups_b > 0x7fffffffLL) return fail(DOCC_ROCM_ERR_UNSUPPORTED, "%s: too many tiles", prefix);
             rc = launch(sizeof(T) == 2 ? "docc_gemm_pack_b2" : sizeof(T) == 4 ? "docc_gemm_pack_b4" : "docc_gemm_pack_b8",
                         (uint32_t) (groups_a + groups_b), 1, 1, 256, 0, s, pa, pb, (long) groups_a, (long) k, (long) kp);
             if (!rc)
@@ -501,8 +503,8 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
         if (cus <= 0) cus = 256;
         const char* env = tuning("DOCC_ROCM_GEMM_SPLITK");
         // the parts' products: in the stream's buffer of partial results where they fit, else in a block of the device
-        // block cache (taken and returned in stream order), up to 64 MiB
-        constexpr int64_t kMaxPartBytes = int64_t(64) << 20;
+        // block cache (taken and returned in stream order), up to 64 MiB; in a capture that keeps no blocks only in a buffer that is there
+        const int64_t kMaxPartBytes = !foreign_capture(s) ? int64_t(64) << 20 : partials_held(s) ? (int64_t) kPartialsBytes : 0;
         // k of a part: whole steps of 64 of every tile; the last part takes what is left
         auto part_of = [&](int64_t parts) { return ((k + parts - 1) / parts + 63) / 64 * 64; };
         auto allowed = [&](int64_t parts) {
@@ -544,17 +546,12 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
                 }
             }
         }
-        if (splits >= 2) {
-            const int64_t bytes = splits * m * n * (int64_t) sizeof(S);
-            PartialsLease lease;
-            void* parts = nullptr;
-            const bool own_block = bytes > (int64_t) kPartialsBytes;
-            if (own_block) {
-                if ((rc = docc_rocm_malloc_async(&parts, (size_t) bytes, stream))) return rc;
-            } else {
-                if ((rc = partials_for(s, &lease))) return rc;
-                parts = lease.ptr;
-            }
+        const int64_t bytes = splits * m * n * (int64_t) sizeof(S);
+        const bool own_block = bytes > (int64_t) kPartialsBytes;
+        PartialsLease lease;
+        void* parts = nullptr;
+        if (splits >= 2 && (own_block ? block(&parts, bytes) : partials_for(s, &lease) == 0)) {
+            if (!own_block) parts = lease.ptr;
             const int64_t part = part_of(splits);
             rc = gemm_launch<T, S>(prefix, stream, trans_a, trans_b, m, n, part, (S) 1, A, lda, B, ldb, (S) 0, (S*) parts, n, pick, nullptr, -1, splits,
                                    ta ? part * lda : part, tb ? part : part * ldb, m * n, nullptr, k);

@@ -38,12 +38,18 @@ struct PartialsLease {
     std::unique_lock<std::mutex> lock;
 };
 int partials_for(hipStream_t stream, PartialsLease* lease);
+// True if the stream has its buffer already: partials_for() then allocates nothing.
+bool partials_held(hipStream_t stream);
 
 // The stream work is enqueued on: `stream` itself, or - where generated code and callers pass the null stream -
 // the stream the calling thread has named with docc_rocm_set_default_stream (the null stream if none).
 hipStream_t resolve_stream(hipStream_t stream);
 // True while the calling thread has a graph capture open: calls that must wait for the device refuse then.
 bool capturing();
+// True while the stream (as resolve_stream has it) is being captured by somebody else: that graph goes on using, at every replay, the
+// device memory its launches were given, and no block of the cache can be kept for it. A launcher that would take one runs in its
+// form without one, or refuses.
+bool foreign_capture(hipStream_t stream);
 
 // The launchers' switches (tests, tuning) are environment variables read on every call: whether any DOCC_ROCM_GEM... variable is set at
 // all, in one walk over the environment instead of one per variable (seven for a GEMM, 0.2-0.3 us each).

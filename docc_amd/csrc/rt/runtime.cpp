@@ -175,6 +175,15 @@ hipStream_t resolve_stream(hipStream_t stream) { return stream ? stream : t_defa
 
 bool capturing() { return t_capture != nullptr; }
 
+bool foreign_capture(hipStream_t stream) {
+    stream = resolve_stream(stream);
+    if (!stream || t_capture) return false;   // the null stream cannot be captured
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &status) == hipSuccess) return status != hipStreamCaptureStatusNone;
+    (void) hipGetLastError();
+    return true;
+}
+
 int fail(int code, const char* fmt, ...) {
     char buf[512];
     va_list ap;
@@ -312,6 +321,7 @@ int partials_for(hipStream_t stream, PartialsLease* lease) {
     if (!slot->ptr) {
         rc = check(hipMalloc(&slot->ptr, kPartialsBytes), "hipMalloc (partial results)");
         if (rc) {
+            (void) hipGetLastError();
             slot->ptr = nullptr;
             return rc;
         }
@@ -319,6 +329,14 @@ int partials_for(hipStream_t stream, PartialsLease* lease) {
     lease->ptr = slot->ptr;
     lease->lock = std::move(busy);
     return 0;
+}
+
+bool partials_held(hipStream_t stream) {
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return false;
+    std::lock_guard<std::mutex> lock(g_partials_mutex);
+    auto it = partials_slots().find({dev, resolve_stream(stream)});
+    return it != partials_slots().end() && it->second->ptr;
 }
 
 // The stream goes away: its partial-results buffers (one per device it was used on) go with it. A launcher still
@@ -589,7 +607,11 @@ int pool_malloc(void** dev_ptr, size_t bytes, bool ordered, hipStream_t stream) 
     *dev_ptr = nullptr;
     if (bytes == 0) return 0;
     BlockCache& c = block_cache();
-    if (c.limit == 0) return check(hipMalloc(dev_ptr, bytes), "hipMalloc");
+    if (c.limit == 0) {
+        const int failed = check(hipMalloc(dev_ptr, bytes), "hipMalloc");
+        if (failed) (void) hipGetLastError();
+        return failed;
+    }
     const size_t rounded = (bytes + 255) & ~size_t(255);
     int dev = 0;
     int rc = check(hipGetDevice(&dev), "hipGetDevice");
@@ -649,7 +671,10 @@ int pool_malloc(void** dev_ptr, size_t bytes, bool ordered, hipStream_t stream) 
         e = hipMalloc(dev_ptr, rounded);
     }
     rc = check(e, "hipMalloc");
-    if (rc) return rc;
+    if (rc) {
+        (void) hipGetLastError();   // reported here; a launcher may go on without the block
+        return rc;
+    }
     std::lock_guard<std::mutex> lock(c.mutex);
     c.live[*dev_ptr] = {dev, rounded, nullptr};
     if (capture) capture->blocks.push_back({*dev_ptr, rounded});

@@ -96,6 +96,8 @@ int docc_rocm_bf16gemm_f32_epilogue(docc_rocm_stream_t stream, int trans_a, int 
  * `rounding`: DOCC_ROCM_ROUND_* bits, where a chain of bf16 nodes rounds in between (round1: before the activation, round2: before
  * the residual). Y may be the residual itself. What the code generator emits for a GEMM node and the elementwise node that alone
  * reads its result; the reference expands the latter to a Map of its own (python/bindings/py_structured_sdfg.cpp:258-260).
+ * Shapes whose product goes through memory are refused (DOCC_ROCM_ERR_UNSUPPORTED) on a stream that is being captured by other means
+ * than docc_rocm_graph_capture_begin: that graph could not keep the memory.
  */
 #define DOCC_ROCM_ACT_GELU 16      /* x Phi(x) */
 #define DOCC_ROCM_ACT_GELU_TANH 17 /* 0.5 x (1 + tanh(sqrt(2 / pi) (x + 0.044715 x^3))) */

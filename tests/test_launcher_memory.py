@@ -1,0 +1,127 @@
+"""What the launchers ask of the HIP runtime, on the CPU: the library runs in a process of its own on a recorder of the HIP host API
+(hip_recorder.c), which writes down allocations, events, waits and launches. No kernel runs, so what is checked is the order of
+the calls: whose memory a launch uses, and what stands between a block's release and its next owner."""
+import os
+import subprocess
+import sys
+from pathlib import Path
+
+import pytest
+
+HERE = Path(__file__).resolve().parent
+PRELUDE = f"""
+import ctypes, sys
+sys.path.insert(0, {str(HERE.parent)!r})
+recorder = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+recorder.recorder_take.restype = ctypes.c_char_p
+recorder.recorder_capture.argtypes = [ctypes.c_void_p]
+recorder.recorder_no_memory_from.argtypes = [ctypes.c_size_t]
+from docc_amd import runtime as rt
+rt.init(0)
+A, B, C, D = 0x10000000, 0x20000000, 0x30000000, 0x40000000     # operands: numbers, nothing reads them
+def take():
+    return recorder.recorder_take().decode().splitlines()
+"""
+
+
+@pytest.fixture(scope="module")
+def recorded(tmp_path_factory):
+    """Runs a script behind PRELUDE; what it prints, as lines."""
+    lib = tmp_path_factory.mktemp("recorder") / "librecorder.so"
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-O1", "-I", f"{rocm}/include", str(HERE / "hip_recorder.c"), "-o", str(lib)], check=True)
+
+    def run(script, **env):
+        clean = {k: v for k, v in os.environ.items() if not k.startswith("DOCC_ROCM_")}
+        done = subprocess.run([sys.executable, "-c", PRELUDE + script, str(lib)], capture_output=True, text=True, env={**clean, **env}, timeout=60)
+        assert done.returncode == 0, done.stderr
+        return done.stdout.splitlines()
+
+    return run
+
+
+# a packed product; K in parts whose sums exceed the stream's buffer; few rows in parts of the same size; a few columns held row by row
+GEMMS = {"packed": "rt.bf16gemm_f32(4096, 4096, 4097, 1.0, A, 4097, B, 4096, 0.0, C, 4096, stream=s)",
+         "parts": "rt.sgemm(512, 1024, 8192, 1.0, A, 8192, B, 1024, 0.0, C, 1024, stream=s)",
+         "few rows": "rt.sgemm(32, 16384, 16384, 1.0, A, 16384, B, 16384, 0.0, C, 16384, stream=s)",
+         "few columns": "rt.sgemm(4096, 9, 4096, 1.0, A, 4096, B, 9, 0.0, C, 9, stream=s)"}
+
+
+@pytest.mark.parametrize("what", list(GEMMS))
+def test_a_product_takes_no_block_where_none_can_be_kept_for_it(recorded, what):
+    script = f"""
+def gemm(s): {GEMMS[what]}
+s = rt.stream_create()
+gemm(s)
+usual = take()
+assert any(l.startswith("malloc") and l != "malloc 8388608" for l in usual), usual      # (that size: the stream's own buffer, kept)
+rt.pool_trim()
+take()
+# a graph that another library records would go on writing to a block that has been given back
+recorder.recorder_capture(s)
+gemm(s)
+got = take()
+assert got and all(l.startswith("launch") for l in got), got
+recorder.recorder_capture(None)
+# without memory the product runs on what it has, and leaves no error behind for other users of the HIP runtime
+recorder.recorder_no_memory_from(1)
+gemm(s)
+got = take()
+assert all(l.startswith("launch") or l.endswith("refused") for l in got) and got[-1].startswith("launch"), got
+assert recorder.hipGetLastError() == 0
+"""
+    recorded(script, **({"DOCC_ROCM_GEMM_SPLITK": "16"} if what == "few rows" else {}))
+
+
+def test_a_layer_that_needs_a_block_is_refused_in_a_foreign_capture(recorded):
+    recorded("""
+s = rt.stream_create()
+def linear(n): rt.call("docc_rocm_linear", s, 2, 111, 112, 256, n, 64, 1.0, A, 64, B, 64, None, 2, 16, None, 2, 0, D, 2)
+linear(100)
+assert any(l.startswith("malloc") for l in take())
+recorder.recorder_capture(s)
+linear(128)                       # the chain is in the product's store
+assert [l.split()[0] for l in take()] == ["launch"]
+try:
+    linear(100)                   # no whole vectors: through memory
+    assert False
+except rt.RocmRuntimeError as e:
+    assert "capture" in str(e), e
+assert take() == []
+""")
+
+
+def test_attention_and_convolution_run_whole_in_a_foreign_capture_or_without_memory(recorded):
+    recorded("""
+s = rt.stream_create()
+def attention(): rt.attention_bf16(1, 4, 1, 32768, 128, 0.1, A, B, C, D, stream=s)
+W = 0x50000000
+def conv(): rt.conv2d_f32(1, 256, 14, 14, 256, 3, 3, (1, 1), (1, 1), (1, 1), A, B, C, D, stream=s)
+for call in (attention, conv):
+    call()
+    usual = take()
+    assert any(l.startswith("malloc") for l in usual) and len([l for l in usual if l.startswith("launch")]) == 2, usual
+    rt.pool_trim()
+    take()
+    recorder.recorder_capture(s)
+    call()
+    got = take()
+    assert [l.split()[0] for l in got] == ["launch"], got
+    recorder.recorder_capture(None)
+    recorder.recorder_no_memory_from(1)
+    call()
+    got = take()
+    assert got[0].endswith("refused") and [l.split()[0] for l in got if not l.endswith("refused")] == ["launch"], got
+    assert recorder.hipGetLastError() == 0
+    recorder.recorder_no_memory_from(ctypes.c_size_t(-1))
+# with a workspace a convolution that cannot be cut takes the form that was the fastest before
+size = (8, 256, 14, 14, 256, 3, 3, (1, 1), (1, 1), (1, 1))
+need = rt.conv2d_f32_workspace_bytes(*size)
+assert need > 0
+rt.conv2d_f32_ws(*size, A, B, C, D, W, need, stream=s)
+assert "_parts" in " ".join(take())
+recorder.recorder_capture(s)
+rt.conv2d_f32_ws(*size, A, B, C, D, W, need, stream=s)
+got = " ".join(take())
+assert "im2col" in got and "sgemm" in got and "malloc" not in got, got
+""")
