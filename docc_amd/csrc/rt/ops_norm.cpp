@@ -12,7 +12,6 @@ extern "C" int docc_rocm_layer_norm(docc_rocm_stream_t stream, int type, int64_t
     if (rows < 0 || cols < 0) return fail(DOCC_ROCM_ERR_INVALID_ARGUMENT, "layer_norm: negative dimension");
     if (rows == 0 || cols == 0) return 0;
     if (!X || !Y) return fail(DOCC_ROCM_ERR_INVALID_ARGUMENT, "layer_norm: null pointer");
-    if (rows > 0x7fffffffLL) return fail(DOCC_ROCM_ERR_UNSUPPORTED, "layer_norm: too many rows");
     if (int rc = ensure_device()) return rc;
     int cus = compute_units();
     if (cus <= 0) cus = 256;
@@ -30,10 +29,17 @@ extern "C" int docc_rocm_layer_norm(docc_rocm_stream_t stream, int type, int64_t
     const int w = held(64), b = held(256);
     const bool wave = w != 0 && (rows >= 4 * (int64_t) cus || cols <= 64 * lane);
     char name[64];
-    if (!wave && !b) {
-        std::snprintf(name, sizeof(name), "docc_layernorm_%s_long", bf16 ? "bf16" : "f32");
-        return launch(name, (uint32_t) rows, 1, 1, 1024, 0, (hipStream_t) stream, (long) rows, (long) cols, eps, X, weight, bias, Y);
+    const bool one = !wave && !b;   // a work-group of 1024 a row
+    if (one) std::snprintf(name, sizeof(name), "docc_layernorm_%s_long", bf16 ? "bf16" : "f32");
+    else std::snprintf(name, sizeof(name), "docc_layernorm_%s_%c_%c%d", bf16 ? "bf16" : "f32", vec ? 'v' : 's', wave ? 'w' : 'b', wave ? w : b);
+    // a launch holds fewer than 2^32 threads: more rows than that takes go in several
+    const int64_t threads = one ? 1024 : 256, per_group = wave ? 4 : 1, most = ((int64_t(1) << 32) / threads - 1) * per_group;
+    const int64_t row_bytes = cols * (bf16 ? 2 : 4);
+    for (int64_t r0 = 0; r0 < rows; r0 += most) {
+        const int64_t n = rows - r0 < most ? rows - r0 : most;
+        const int rc = launch(name, (uint32_t) ((n + per_group - 1) / per_group), 1, 1, (uint32_t) threads, 0, (hipStream_t) stream, (long) n, (long) cols,
+                              eps, (const void*) ((const char*) X + r0 * row_bytes), weight, bias, (void*) ((char*) Y + r0 * row_bytes));
+        if (rc) return rc;
     }
-    std::snprintf(name, sizeof(name), "docc_layernorm_%s_%c_%c%d", bf16 ? "bf16" : "f32", vec ? 'v' : 's', wave ? 'w' : 'b', wave ? w : b);
-    return launch(name, (uint32_t) (wave ? (rows + 3) / 4 : rows), 1, 1, 256, 0, (hipStream_t) stream, (long) rows, (long) cols, eps, X, weight, bias, Y);
+    return 0;
 }

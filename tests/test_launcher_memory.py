@@ -125,3 +125,13 @@ rt.conv2d_f32_ws(*size, A, B, C, D, W, need, stream=s)
 got = " ".join(take())
 assert "im2col" in got and "sgemm" in got and "malloc" not in got, got
 """)
+
+
+@pytest.mark.parametrize("rows,cols,launches", [(2 ** 24 + 5, 2000, 2), (2 ** 26 + 1, 64, 2), (2 ** 22, 20000, 2), (2 ** 24 - 1, 2000, 1)])
+def test_layer_norm_of_more_rows_than_a_launch_holds(recorded, rows, cols, launches):
+    # 2^32 threads are one too many for a launch (the recorder refuses them as the device does)
+    got = recorded(f"""
+rt.call("docc_rocm_layer_norm", 0, 2, {rows}, {cols}, 1e-5, A, None, None, B)
+print("\\n".join(take()))
+""")
+    assert len(got) == launches and all(l.startswith("launch docc_layernorm_f32") for l in got)
