@@ -34,9 +34,7 @@ size_t gemm_lds_bytes(const TileConfig& c, bool ta, bool tb, size_t elem) {
 // 6144 x 4096 x 4096 (within 15 % on most): a launch, and for every round of tiles over the CUs the fp32 store of the tiles (all of
 // them at once: 11 us for 256 x 256) and their products at what the tile sustains. A last round that leaves CUs idle runs
 // faster (less traffic, higher clocks), but not in proportion, the smallest tile's, which waits for its copies, least of all.
-double bgemm_seconds(const TileConfig& c, int64_t m, int64_t n, int64_t k, bool tb, int64_t count) {
-    int cus = compute_units();
-    if (cus <= 0) cus = 256;
+double bgemm_seconds(const TileConfig& c, int64_t m, int64_t n, int64_t k, bool tb, int64_t count, int cus) {
     const int64_t tiles = ((m + c.bm - 1) / c.bm) * ((n + c.bn - 1) / c.bn) * count, last = tiles % cus;
     const double part = (double) last / cus;
     const double rounds = (double) (tiles / cus) + (!last ? 0.0 : tiles < cus && c.bn == 128 ? 0.7 + 0.2 * part : 0.5 + 0.4 * part);
@@ -45,6 +43,12 @@ double bgemm_seconds(const TileConfig& c, int64_t m, int64_t n, int64_t k, bool 
     const double rel = c.bm == 256 ? (k % 64 == 0 ? 1.0 : 0.93) : c.bn == 256 ? (tb ? 0.88 : 0.80) : tiles > cus ? 0.75 : 0.86;
     const double area = (double) c.bm * c.bn, fill = c.bm < c.bn ? (tb ? 1.5 : 3.0) : 0.0;
     return 1e-6 * (4.0 + rounds * (fill + area * (11.0 / 65536) + area * (double) k * 3.6e-7 / rel));
+}
+
+// the number of CUs, asked for once per call of an entry point: a product with fewer tiles than CUs weighs up to 60 forms by it
+int cu_count() {
+    const int cus = compute_units();
+    return cus > 0 ? cus : 256;
 }
 
 // What GemmFinish of csrc/kernels/gemm_finish.h holds: the rest of a layer behind a product.
@@ -68,7 +72,7 @@ int finish_parts(hipStream_t s, const void* P, int64_t m, int64_t n, int parts, 
 // shape is not one of theirs (the caller goes on to the tiled kernels), 0 or an error code otherwise.
 template <typename T, typename S>
 int gemv_launch(const char* prefix, hipStream_t s, bool ta, bool tb, int64_t m, int64_t n, int64_t k, S alpha, const T* A, int64_t lda,
-                const T* B, int64_t ldb, S beta, S* C, int64_t ldc, bool tuned) {
+                const T* B, int64_t ldb, S beta, S* C, int64_t ldc, bool tuned, int cus) {
     if (tuned && std::getenv("DOCC_ROCM_GEMV_OFF")) return 1;   // tuning and tests: always the tiled kernels
     const T *M, *x;
     int64_t ld, incx, incy, rows, cols;
@@ -77,8 +81,6 @@ int gemv_launch(const char* prefix, hipStream_t s, bool ta, bool tb, int64_t m, 
         // two to eight rows or columns of output with both operands stored row by row along k (op(A) = A, op(B) = B^T,
         // the product of a small batch with a weight matrix): the larger operand moves once
         if (m > 8 && n > 8) return 1;
-        int cusm = compute_units();
-        if (cusm <= 0) cusm = 256;
         // five to eight vectors would be two passes over the matrix: the tiles with K in parts are faster (fp32 8 x 4096 x 4096:
         // 39 us here, 26 there; 8 x 8192 x 8192: 95 against 81; fp64 8 x 8192 x 8192: 296 against 172)
         const int64_t max_vectors = 4;
@@ -98,12 +100,12 @@ int gemv_launch(const char* prefix, hipStream_t s, bool ta, bool tb, int64_t m, 
             const int64_t col_blocks = (cols / lanes + 255) / 256;
             // 1.75 work-groups per CU (measured against 0.75 .. 6 per CU on five shapes: 4 x 8192 x 8192 in 46.9 us against
             // 51.7 with two, 8 x 8192 x 8192 in 93.9 against 102.3, 4 x 4096 x 11008 in 32.9 against 35.3)
-            int64_t slices = (7 * (int64_t) cusm / 4 + col_blocks - 1) / col_blocks;
+            int64_t slices = (7 * (int64_t) cus / 4 + col_blocks - 1) / col_blocks;
             if (slices > k / 16) slices = k / 16;
             // the partial sums are written and read back: keep them under a sixteenth of the matrix's bytes
             const int64_t group = nv < 4 ? nv : 4;                                     // vectors per pass
             int64_t cheap = k * (int64_t) sizeof(T) / (16 * (int64_t) sizeof(S) * group);
-            if (cheap * col_blocks < 4 * (int64_t) cusm) cheap *= 2;      // ... unless that leaves the chip short of work-groups
+            if (cheap * col_blocks < 4 * (int64_t) cus) cheap *= 2;      // ... unless that leaves the chip short of work-groups
             if (slices > cheap) slices = cheap;
             const int64_t fit = (int64_t) kPartialsBytes / ((int64_t) sizeof(S) * cols * group);
             if (slices > fit) slices = fit;
@@ -136,8 +138,6 @@ int gemv_launch(const char* prefix, hipStream_t s, bool ta, bool tb, int64_t m, 
         if (ta || !tb) return 1;
         const bool small_a = m <= n;                  // the vectors: A's rows (m of them) or B's rows (n of them)
         const int64_t nv = small_a ? m : n, big = small_a ? n : m;
-        int cus0 = compute_units();
-        if (cus0 <= 0) cus0 = 256;
         // five to eight vectors: fp64 is faster through the MFMA tiles (8 x 8192 x 8192: 166 us against 218 here), bf16 too
         // once the matrix is large (8 x 28672 x 8192: 111 us against 137; 8 x 8192 x 8192: 56 against 46 here)
         const int64_t max_nv = sizeof(T) == 8 || (sizeof(T) == 2 && big * k > (int64_t(1) << 27)) ? 4 : 8;
@@ -146,9 +146,9 @@ int gemv_launch(const char* prefix, hipStream_t s, bool ta, bool tb, int64_t m, 
                              (small_a ? lda : ldb) % vecw == 0;
         // a wavefront takes four matrix rows, or eight where that still leaves a work-group per CU (fp32 4 x 8192 x 8192:
         // 79 -> 68 us; bf16 gains nothing from it)
-        const bool eight = nv <= 4 && aligned && sizeof(T) != 2 && big >= 32 * (int64_t) cus0;
+        const bool eight = nv <= 4 && aligned && sizeof(T) != 2 && big >= 32 * (int64_t) cus;
         const int64_t wg_rows = eight ? 32 : 16;
-        if (nv > max_nv || big < 16 * (int64_t) cus0 || (big + wg_rows - 1) / wg_rows > 0x7fffffffLL) return 1;
+        if (nv > max_nv || big < 16 * (int64_t) cus || (big + wg_rows - 1) / wg_rows > 0x7fffffffLL) return 1;
         const T* mat = small_a ? B : A;
         const T* vecs = small_a ? A : B;
         const int64_t ldm = small_a ? ldb : lda, ldx = small_a ? lda : ldb;
@@ -173,8 +173,6 @@ int gemv_launch(const char* prefix, hipStream_t s, bool ta, bool tb, int64_t m, 
     const int vec = 16 / (int) sizeof(T);
     const char* type = sizeof(T) == 2 ? "bf16" : sizeof(T) == 4 ? "f32" : "f64";   // elements of the matrix
     const int bits = (int) sizeof(S) * 8;                                        // of the sums and of y
-    int cus = compute_units();
-    if (cus <= 0) cus = 256;
     char name[64];
     if (by_rows) {
         // one wavefront per row: worth it from a few rows per SIMD on
@@ -222,7 +220,7 @@ int gemv_launch(const char* prefix, hipStream_t s, bool ta, bool tb, int64_t m, 
 template <typename T, typename S = T>
 int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int trans_b, int64_t m, int64_t n,
                 int64_t k, S alpha, const T* A, int64_t lda, const T* B, int64_t ldb, S beta, S* C, int64_t ldc,
-                TileConfig (*pick)(int64_t m, int64_t n, int64_t k, bool tb, int64_t batch, bool aligned, int force), const S* bias = nullptr,
+                TileConfig (*pick)(int64_t m, int64_t n, int64_t k, bool tb, int64_t batch, bool aligned, int force, int cus), const S* bias = nullptr,
                 int activation = -1, int64_t batch = 1, int64_t batch_a = 0, int64_t batch_b = 0, int64_t batch_c = 0,
                 const LinearFinish* fin = nullptr, int64_t k_total = 0) {
     if ((trans_a != DOCC_ROCM_NO_TRANS && trans_a != DOCC_ROCM_TRANS) ||
@@ -248,6 +246,7 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
     hipStream_t s = (hipStream_t) stream;
     char name[96];
     const bool tuned = gemm_tuning_set();
+    const int cus = cu_count();
     auto tuning = [&](const char* variable) -> const char* { return tuned ? std::getenv(variable) : nullptr; };
     // A block of the device block cache for this call, given back behind its last launch. False: there is none (no memory, or a
     // capture it could not be kept for), and the product runs in a form without it.
@@ -323,10 +322,10 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
                             lda % 2 == 0 && ldb % 2 == 0 && k % 2 == 0 && n % 2 == 0;
     const bool skinny = skinny_f32 || skinny_bf16 || skinny_f64;
     if (fin && (m <= 8 || n <= 8) && !skinny && batch == 1 && !foreign_capture(s)) {
-        rc = through_memory([&](S* to) { return gemv_launch<T, S>(prefix, s, ta, tb, m, n, k, alpha, A, lda, B, ldb, (S) 0, to, n, tuned); });
+        rc = through_memory([&](S* to) { return gemv_launch<T, S>(prefix, s, ta, tb, m, n, k, alpha, A, lda, B, ldb, (S) 0, to, n, tuned, cus); });
         if (rc != 1) return rc;
     } else if (!fin && (m <= 8 || n <= 8) && !skinny && batch == 1 && (!epilogue || ldc == n)) {
-        rc = gemv_launch<T, S>(prefix, s, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, tuned);
+        rc = gemv_launch<T, S>(prefix, s, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, tuned, cus);
         if (rc == 0 && epilogue) {
             // the few rows or columns of output are a small tensor: bias and activation as one elementwise pass over it,
             // the same roundings as the fused store
@@ -350,8 +349,6 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
     // parts (tests, tuning).
     if (skinny) {
         {
-            int cus = compute_units();
-            if (cus <= 0) cus = 256;
             // fp32: 16 or 32 rows per MFMA, 128 columns per work-group; bf16: 1, 2 or 4 blocks of 16 rows, 64 columns
             const int nw = 4, nbuf = 2;
             const int ch = skinny_bf16 ? 64 : tb ? 32 : 16, mt = skinny_bf16 ? (m <= 16 ? 1 : 2) : m <= 16 ? 16 : 32;
@@ -472,7 +469,7 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
     }
     // DOCC_ROCM_GEMM_TILE=big|small overrides the size heuristic (tests, tuning)
     const char* force = tuning("DOCC_ROCM_GEMM_TILE");
-    TileConfig cfg = pick(m, n, k, tb, batch, aligned, force && force[0] == 'b' ? 1 : force && force[0] == 's' ? -1 : 0);
+    TileConfig cfg = pick(m, n, k, tb, batch, aligned, force && force[0] == 'b' ? 1 : force && force[0] == 's' ? -1 : 0, cus);
     // DOCC_ROCM_GEMM_CFG=BMxBNxBKxWAVES[xSTAGES[p|q]] selects a built configuration directly (tuning)
     if (const char* c = tuning("DOCC_ROCM_GEMM_CFG")) {
         TileConfig t{};
@@ -489,7 +486,7 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
     // the asynchronous kernels need aligned operands and address a tile with 32-bit byte offsets
     const int64_t max_edge = cfg.bm > cfg.bn ? (cfg.bm > cfg.bk ? cfg.bm : cfg.bk) : (cfg.bn > cfg.bk ? cfg.bn : cfg.bk);
     const bool offsets_fit = max_edge * (lda > ldb ? lda : ldb) * (int64_t) sizeof(T) < (int64_t(1) << 32);
-    if (cfg.stages > 0 && !(aligned && offsets_fit)) cfg = pick(m, n, k, tb, batch, false, 0);
+    if (cfg.stages > 0 && !(aligned && offsets_fit)) cfg = pick(m, n, k, tb, batch, false, 0, cus);
     const int64_t tiles = ((m + cfg.bm - 1) / cfg.bm) * ((n + cfg.bn - 1) / cfg.bn);
     if (tiles > 0x7fffffffLL) return fail(DOCC_ROCM_ERR_UNSUPPORTED, "%s: too many tiles", prefix);
     // Few output tiles and a long K extent (a handful of rows against a wide matrix: the product is bound by reading
@@ -499,8 +496,6 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
     // another number forces that many parts where K allows it (tests, tuning).
     const bool largest_fits = 256 * (lda > ldb ? lda : ldb) * (int64_t) sizeof(T) < (int64_t(1) << 32);   // whatever tile the parts take
     if (batch == 1 && (!epilogue || ldc == n) && cfg.stages > 0 && largest_fits && k >= 512) {
-        int cus = compute_units();
-        if (cus <= 0) cus = 256;
         const char* env = tuning("DOCC_ROCM_GEMM_SPLITK");
         // the parts' products: in the stream's buffer of partial results where they fit, else in a block of the device
         // block cache (taken and returned in stream order), up to 64 MiB; in a capture that keeps no blocks only in a buffer that is there
@@ -516,7 +511,7 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
         // work-group, plus writing and reading the parts at 5 TB/s and a second launch.
         auto seconds = [&](const TileConfig& c, int64_t parts) {
             if (sizeof(T) == 2)
-                return bgemm_seconds(c, m, n, part_of(parts), tb, parts) + (parts > 1 ? 2.0 * (double) parts * (double) m * (double) n * sizeof(S) / 5e12 + 2e-6 : 0.0);
+                return bgemm_seconds(c, m, n, part_of(parts), tb, parts, cus) + (parts > 1 ? 2.0 * (double) parts * (double) m * (double) n * sizeof(S) / 5e12 + 2e-6 : 0.0);
             const double tm = (double) ((m + c.bm - 1) / c.bm), tn = (double) ((n + c.bn - 1) / c.bn);
             const double area = (double) c.bm * c.bn;
             const double rel = area >= 65536 ? 1.03 : area >= 32768 ? 1.0 : area >= 16384 ? 0.97 : 0.75;
@@ -537,7 +532,7 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
             double best = seconds(cfg, 1);
             for (int64_t parts : {2, 3, 4, 5, 6, 8, 10, 12, 16, 20, 24, 32, 48, 64}) {
                 if (!allowed(parts)) continue;
-                const TileConfig c = pick(m, n, part_of(parts), tb, parts, true, 0);
+                const TileConfig c = pick(m, n, part_of(parts), tb, parts, true, 0, cus);
                 if (c.stages == 0) break;
                 const double t = seconds(c, parts);
                 if (t < (splits > 1 ? 1.0 : sizeof(T) == 2 ? 0.95 : 0.9) * best) {   // cut for a clear gain only: the estimate is rough
@@ -616,7 +611,7 @@ template <typename T, typename S>
 static int gemm_batched(const char* prefix, docc_rocm_stream_t stream, int trans_a, int trans_b, int64_t m, int64_t n, int64_t k,
                         S alpha, const T* A, int64_t lda, int64_t stride_a, const T* B, int64_t ldb, int64_t stride_b, S beta, S* C,
                         int64_t ldc, int64_t stride_c, int64_t batch,
-                        TileConfig (*pick)(int64_t m, int64_t n, int64_t k, bool tb, int64_t batch, bool aligned, int force)) {
+                        TileConfig (*pick)(int64_t m, int64_t n, int64_t k, bool tb, int64_t batch, bool aligned, int force, int cus)) {
     if (batch < 0) return fail(DOCC_ROCM_ERR_INVALID_ARGUMENT, "%s: negative batch", prefix);
     const int64_t kMaxGridY = 65535;
     for (int64_t b0 = 0; b0 < batch; b0 += kMaxGridY) {
@@ -636,7 +631,7 @@ extern "C" {
 // tiles of one matrix times the number of matrices: what there is to spread over the compute units
 static int64_t tiles_of(int64_t m, int64_t n, int bm, int bn, int64_t batch = 1) { return ((m + bm - 1) / bm) * ((n + bn - 1) / bn) * batch; }
 
-static TileConfig pick_sgemm(int64_t m, int64_t n, int64_t, bool, int64_t batch, bool aligned, int force) {
+static TileConfig pick_sgemm(int64_t m, int64_t n, int64_t, bool, int64_t batch, bool aligned, int force, int cus) {
     const TileConfig huge{256, 256, 32, 4, 2}, wide{128, 256, 32, 4, 2}, big{128, 128, 32, 4, 3}, small{64, 64, 16, 4, 4};
     const TileConfig plain_big{128, 128, 16, 4, 0}, plain_small{64, 64, 16, 4, 0};
     if (!aligned) return force > 0 ? plain_big : force < 0 ? plain_small : (tiles_of(m, n, 128, 128, batch) >= 256 ? plain_big : plain_small);
@@ -644,8 +639,6 @@ static TileConfig pick_sgemm(int64_t m, int64_t n, int64_t, bool, int64_t batch,
     // Score = share of a tile's area that is real output x share of the CUs that get a work-group x what the
     // tile sustains relative to the 128x256 one (146 / 141 / 138 / about 105 TFLOP/s on large problems): a 64-row
     // product wastes half of a 128-row tile, a 1000^2 one leaves most CUs idle with the large tiles.
-    int cus = compute_units();
-    if (cus <= 0) cus = 256;
     auto score = [&](const TileConfig& c, double rel) {
         const double padded = (double) ((m + c.bm - 1) / c.bm * c.bm) * (double) ((n + c.bn - 1) / c.bn * c.bn);
         const double fill = (double) tiles_of(m, n, c.bm, c.bn, batch) / cus;
@@ -659,7 +652,7 @@ static TileConfig pick_sgemm(int64_t m, int64_t n, int64_t, bool, int64_t batch,
     return sw >= sb && sw >= ss ? wide : sb >= ss ? big : small;
 }
 
-static TileConfig pick_dgemm(int64_t m, int64_t n, int64_t, bool, int64_t batch, bool aligned, int force) {
+static TileConfig pick_dgemm(int64_t m, int64_t n, int64_t, bool, int64_t batch, bool aligned, int force, int) {
     const TileConfig big{128, 128, 16, 4, 3}, mid{64, 64, 16, 4, 4}, small{64, 32, 16, 4, 4};
     const TileConfig plain_big{128, 128, 16, 4, 0}, plain_small{64, 64, 16, 4, 0};
     if (!aligned) return force > 0 ? plain_big : plain_small;
@@ -668,16 +661,16 @@ static TileConfig pick_dgemm(int64_t m, int64_t n, int64_t, bool, int64_t batch,
     return t >= 2048 ? big : t > 512 ? mid : small;   // few tiles: halve them so that two work-groups share a CU
 }
 
-static TileConfig pick_bgemm(int64_t m, int64_t n, int64_t k, bool tb, int64_t batch, bool aligned, int force) {
+static TileConfig pick_bgemm(int64_t m, int64_t n, int64_t k, bool tb, int64_t batch, bool aligned, int force, int cus) {
     // big: on the 16x16x32 MFMA where K allows it (see gemm_launch), else on the 32x32x16 one with the copies dealt out
     const TileConfig big{256, 256, 32, 4, 4, true, true}, wide{128, 256, 64, 4, 3}, deep{128, 128, 64, 4, 4}, small{128, 128, 32, 4, 4};
     const TileConfig plain_big{256, 256, 64, 4, 0}, plain_small{128, 128, 64, 4, 0};
     if (!aligned) return force > 0 ? plain_big : force < 0 ? plain_small : (tiles_of(m, n, 256, 256, batch) >= 256 ? plain_big : plain_small);
     if (force) return force > 0 ? big : small;
     const TileConfig* best = &big;
-    double least = bgemm_seconds(big, m, n, k, tb, batch);
+    double least = bgemm_seconds(big, m, n, k, tb, batch, cus);
     for (const TileConfig* c : {&wide, k >= 1024 ? &deep : &small}) {
-        const double t = bgemm_seconds(*c, m, n, k, tb, batch);
+        const double t = bgemm_seconds(*c, m, n, k, tb, batch, cus);
         if (t < least) {
             least = t;
             best = c;

@@ -135,3 +135,14 @@ rt.call("docc_rocm_layer_norm", 0, 2, {rows}, {cols}, 1e-5, A, None, None, B)
 print("\\n".join(take()))
 """)
     assert len(got) == launches and all(l.startswith("launch docc_layernorm_f32") for l in got)
+
+
+def test_a_product_asks_for_the_device_a_few_times_however_many_forms_it_weighs(recorded):
+    # 512 x 512 x 4096 has fewer tiles than CUs: a dozen numbers of parts on three tiles each
+    got = recorded("""
+for _ in range(2):
+    recorder.recorder_device_queries()
+    rt.bf16gemm_f32(512, 512, 4096, 1.0, A, 4096, B, 512, 0.0, C, 512)
+print(recorder.recorder_device_queries())
+""")
+    assert int(got[0]) <= 8
