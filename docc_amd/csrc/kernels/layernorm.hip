@@ -80,7 +80,7 @@ __device__ __forceinline__ void layernorm_row(long rows, long cols, float eps, c
                 sq += v[i][e] * v[i][e];
             }
         }
-    const float scale = 1.0f / sqrtf(ln_row_sum<TPR>(sq, slots[1]) / (float) cols + eps);
+    const float root = sqrtf(ln_row_sum<TPR>(sq, slots[1]) / (float) cols + eps);
 #pragma unroll
     for (int i = 0; i < NV; i++) {
         const long c = (long) (i * TPR + t) * V;
@@ -90,7 +90,7 @@ __device__ __forceinline__ void layernorm_row(long rows, long cols, float eps, c
         if (B) load(reinterpret_cast<const raw*>(B), c, b);
 #pragma unroll
         for (int e = 0; e < V; e++) {
-            float r = v[i][e] * scale;
+            float r = v[i][e] / root;
             if (W) r *= w[e];
             if (B) r += b[e];
             v[i][e] = r;
@@ -123,9 +123,9 @@ __device__ __forceinline__ void layernorm_long(long cols, float eps, const void*
         const float d = E::up(x[c]) - mean;
         sq += d * d;
     }
-    const float scale = 1.0f / sqrtf(ln_row_sum<1024>(sq, slots[1]) / (float) cols + eps);
+    const float root = sqrtf(ln_row_sum<1024>(sq, slots[1]) / (float) cols + eps);
     for (long c = threadIdx.x; c < cols; c += 1024) {
-        float r = (E::up(x[c]) - mean) * scale;
+        float r = (E::up(x[c]) - mean) / root;
         if (w) r *= E::up(w[c]);
         if (b) r += E::up(b[c]);
         y[c] = E::down(r);

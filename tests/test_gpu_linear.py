@@ -2,6 +2,7 @@
 the code generator emits them for. Against float64 on the CPU, with the roundings to bf16 that the chain asks for."""
 import ctypes
 
+import numpy as np
 import pytest
 import torch
 import torch.nn.functional as F
@@ -115,6 +116,22 @@ def test_layer_norm_over_row_lengths(dtype, rows, cols):
         err = (y.double().cpu() - ref).abs()
         bound = 1e-5 * (1 + ref.abs()) if dtype == torch.float32 else 2.0 ** -8 * (1e-3 + ref.abs())
         assert bool((err <= bound).all()), float((err / bound).max())
+
+
+@pytest.mark.parametrize("rows,cols", [(1100, 256), (3, 250), (5, 1024), (2, 4096), (3, 4097), (2, 16384)])
+def test_layer_norm_divides_by_the_root(rows, cols):
+    # small whole numbers whose mean is one too: both sums are exact in fp32 whatever their order, what is left is a division by cols, the
+    # root and one division an element, each rounded once
+    gen = torch.Generator().manual_seed(cols)
+    half = torch.randint(-7, 8, (rows, cols // 2), generator=gen).float()
+    x = 3 + torch.cat([half, -half, torch.zeros(rows, cols % 2)], 1)[:, torch.randperm(cols, generator=gen)]
+    d = x.numpy() - 3       # (numpy rounds each operation once; torch divides a tensor by a number through its reciprocal)
+    want = d / np.sqrt(np.square(d).sum(1, keepdims=True) / np.float32(cols) + np.float32(1e-5))
+    dx = x.cuda()
+    y = torch.full_like(dx, float("nan"))
+    rt.call("docc_rocm_layer_norm", 0, 2, rows, cols, 1e-5, ptr(dx), None, None, ptr(y))
+    torch.cuda.synchronize()
+    assert np.array_equal(y.cpu().numpy(), want)
 
 
 class Block(torch.nn.Module):
