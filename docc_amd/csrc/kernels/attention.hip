@@ -42,9 +42,8 @@
 //     keep their relative precision at any magnitude, so m stays what the first block set until a
 //     block's row sum shows growth beyond 2^40 (or inf, or NaN) - only then the block takes the slow
 //     path (scores recomputed, true block maximum, rescale of the output and the sum, p again). The usual
-//     block has no max pass and no rescale. A lane that has seen nothing but -inf scores so far keeps
-//     m = -inf, which makes its next block's sum inf or NaN and so leads it through the slow path until a
-//     finite score turns up;
+//     block has no max pass and no rescale. A query that has met nothing but -inf scores has the lowest finite
+//     float as m: p is 0 for those, and infinite for the first finite score, which leads through the slow path;
 //   - p is packed to bf16 with v_cvt_pk_bf16_f32 and the row sum is taken from the packed values with
 //     v_dot2c_f32_bf16: it sums exactly what the second product multiplies.
 // K/V blocks arrive in a ring of three LDS stages by asynchronous global->LDS copies, two blocks ahead.
@@ -163,7 +162,7 @@ __device__ __forceinline__ void attention_fwd(const uint16_t* __restrict__ Q, co
     };
 
     f32x16 ot[QT][DT];  // O^T tiles: d = 32*dt + acc_row(lane, r), column = this lane's query of tile qt
-    float m_run[QT];    // reference point of the exponentials (log2 domain); -inf: nothing finite seen yet
+    float m_run[QT];    // reference point of the exponentials (log2 domain), finite from the first block on (or +inf, a NaN)
     float l_part[QT];   // this lane's part of the running sum (its 32 keys per block)
 #pragma unroll
     for (int qt = 0; qt < QT; qt++) {
@@ -245,8 +244,8 @@ __device__ __forceinline__ void attention_fwd(const uint16_t* __restrict__ Q, co
             }
         return psum;
     };
-    // reference point a lane subtracts: 0 while it has seen no finite score (its scores are all -inf then, p = 0)
-    auto base_of = [&](float m) { return m == ninf ? 0.f : m; };
+    // the reference point where the first block has no finite score (see above)
+    const float lowest = -0x1.fffffep127f;
     // the maximum of the scaled scores of the lane pair's query (c > 0)
     auto scaled_max = [&](const f32x16 (&s)[2]) {
         float mx = s[0][0];
@@ -269,13 +268,13 @@ __device__ __forceinline__ void attention_fwd(const uint16_t* __restrict__ Q, co
         if (FIRST) {
             // the first block sets the reference point
 #pragma unroll
-            for (int qt = 0; qt < QT; qt++) m_run[qt] = scaled_max(st[qt]);
+            for (int qt = 0; qt < QT; qt++) m_run[qt] = fmaxf(scaled_max(st[qt]), lowest);
         }
         float psum[QT];
         bool slow = false;
 #pragma unroll
         for (int qt = 0; qt < QT; qt++) {
-            psum[qt] = exponentials(st[qt], pk[qt], base_of(m_run[qt]));
+            psum[qt] = exponentials(st[qt], pk[qt], m_run[qt]);
             // growth of the maximum beyond 2^40 over the reference point (or an overflow, or a NaN) shows in the sum
             slow = slow || !(psum[qt] < 0x1p40f);
         }
@@ -286,15 +285,14 @@ __device__ __forceinline__ void attention_fwd(const uint16_t* __restrict__ Q, co
 #pragma unroll
             for (int qt = 0; qt < QT; qt++) {
                 const float m_new = fmaxf(m_run[qt], scaled_max(st[qt]));     // fmaxf drops a NaN: it shows up in p instead
-                // exp2(-inf - -inf) would be NaN: a lane that still has nothing finite has nothing to rescale either
-                const float alpha = m_new == ninf ? 1.f : __builtin_amdgcn_exp2f(m_run[qt] - m_new);
+                const float alpha = __builtin_amdgcn_exp2f(m_run[qt] - m_new);
                 m_run[qt] = m_new;
                 l_part[qt] *= alpha;
 #pragma unroll
                 for (int dt = 0; dt < DT; dt++)
 #pragma unroll
                     for (int r = 0; r < 16; r++) ot[qt][dt][r] *= alpha;
-                psum[qt] = exponentials(st[qt], pk[qt], base_of(m_new));
+                psum[qt] = exponentials(st[qt], pk[qt], m_new);
             }
         }
 #pragma unroll

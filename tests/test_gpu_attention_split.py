@@ -69,6 +69,26 @@ def test_excluded_keys_and_growing_scores(rt, SKV):
     assert np.isnan(O[0, 1]).all() and np.isfinite(O[0, 0]).all()
 
 
+# whatever the form: the first 70 keys of a query score -inf, then come scores far below 0 (against a reference point of 0 every
+# exponential is 0), or scores near 0 and behind them some that are larger by more than 2^40 (a move of the reference point from 0 up)
+@pytest.mark.parametrize("form", ["32", "128", "256"])
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("causal", [False, True])
+def test_first_scores_that_are_not_finite(rt, monkeypatch, form, D, causal):
+    monkeypatch.setenv("DOCC_ROCM_ATTENTION_Q", form)
+    Q, K, V = draw(D, 1, 3, 300, 333, D)
+    Q[..., 0] = 1
+    K[0, :2, :70, 0] = -float("inf")
+    K[0, 0, 70:, 0] = -256.0 * D ** 0.5
+    K[0, 1, 200:, 0] = 64.0 * D ** 0.5
+    O, want = run(rt, Q, K, V, causal), expected(Q, K, V, causal)
+    first = 70 if causal else 0       # the queries before it see no finite score
+    assert np.isnan(O[0, :2, :first]).all()
+    for h in range(3):
+        rows = slice(first if h < 2 else 0, None)
+        assert rel_err_max(O[0, h, rows], want[0, h, rows]) <= TOL_BF16, h
+
+
 def test_captured_call_cut_into_parts_replays(rt):
     Q, K, V = draw(5, 1, 2, 1, 9000, 64)
     q, k, v = Q.cuda(), K.cuda(), V.cuda()
