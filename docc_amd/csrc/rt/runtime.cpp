@@ -83,13 +83,14 @@ std::vector<DeviceState> g_devices;
 // device and leaves `pending` false. On the null stream, which lives as long as the process, the event is not recorded until somebody
 // has to wait for it: between two launches a recorded event is a packet of its own on the device and a call on the host, which the
 // usual next owner - the next call of the same generated function, on the same stream - never looks at. Recorded later it stands
-// behind more work than the owner's, never behind less.
+// behind more work than the owner's, never behind less: a next owner on another stream, or on the host, waits for all that the null stream
+// has been given by then.
 struct CachedBlock {
     void* ptr = nullptr;
     hipEvent_t released = nullptr;   // created the first time the block is freed on a stream, reused afterwards
-    hipStream_t stream = nullptr;    // the stream `released` was recorded on
-    bool pending = false;            // `released` may not have happened yet
-    bool recorded = false;           // pending, and `released` has been recorded
+    hipStream_t stream = nullptr;    // the stream the last owner worked on, on which `released` is recorded
+    bool pending = false;            // that work may not be over yet
+    bool recorded = false;           // pending, and `released` has been recorded (at the release, but for the null stream)
 };
 
 // records the release of a pending block that has not been (see above)

@@ -68,6 +68,44 @@ def test_cached_blocks_hold_no_stale_work(rt):
     assert np.array_equal(out, np.arange(n, dtype=np.float32))
 
 
+def test_blocks_freed_on_the_null_stream_come_back_behind_its_work(rt):
+    """free_async on the null stream records nothing; the next owner elsewhere does, and waits for what the null stream has been given.
+    Twice: the second time the block brings its event along."""
+    import torch
+    n = 1 << 24
+    src = -torch.arange(n, dtype=torch.float32, device="cuda")
+    src2 = 2 * src
+    expected = np.arange(n, dtype=np.float32)
+    out = np.empty(n, np.float32)
+    b = rt.stream_create()
+    try:
+        torch.cuda.synchronize()
+        rt.pool_trim()
+        p = rt.malloc_async(n * 4)
+        for _ in range(2):
+            for _ in range(8):
+                rt.elementwise_unary("abs", 32, n, src.data_ptr(), p)
+            rt.free_async(p)
+            assert rt.malloc_async(n * 4) == p                       # the same stream: no wait
+            rt.free_async(p)
+            assert rt.malloc_async(n * 4, b) == p
+            rt.elementwise_unary("abs", 32, n, src2.data_ptr(), p, stream=b)      # must land after the eight launches
+            rt.memcpy_d2h(out.ctypes.data, p, n * 4, b)
+            rt.stream_sync(b)
+            rt.stream_sync()
+            assert np.array_equal(out, expected * 2)
+            for _ in range(8):
+                rt.elementwise_unary("abs", 32, n, src.data_ptr(), p)
+            rt.free_async(p)
+            assert rt.malloc(n * 4) == p                              # waits on the host
+            rt.memcpy_d2h(out.ctypes.data, p, n * 4, b)               # (b does not wait for the null stream by itself)
+            rt.stream_sync(b)
+            assert np.array_equal(out, expected)
+        rt.free(p)
+    finally:
+        rt.stream_destroy(b)
+
+
 def test_blocks_freed_on_a_stream_come_back_in_stream_order(rt):
     """free_async records the release on the stream and does not wait; the next owner sees the block only behind that
     release: on the same stream by stream order, on another stream through an event wait, on the host after a wait."""

@@ -146,3 +146,27 @@ for _ in range(2):
 print(recorder.recorder_device_queries())
 """)
     assert int(got[0]) <= 8
+
+
+def test_the_release_of_a_block_of_the_null_stream_is_recorded_when_somebody_else_takes_it(recorded):
+    recorded("""
+n, b = 1 << 20, rt.stream_create()
+p = rt.malloc_async(n)
+take()
+rt.free_async(p)
+assert rt.malloc_async(n) == p and take() == []                     # the same stream: nothing recorded, nothing waited for
+rt.free_async(p)
+assert rt.malloc_async(n, b) == p
+assert take() == ["event 1", "record 1 on (nil)", f"{b:#x} waits for 1"]
+rt.free_async(p, b)
+assert take() == ["record 1 on " + f"{b:#x}"]                        # any other stream may be gone by then: at once
+assert rt.malloc(n) == p
+assert take() == ["host waits for 1"]
+rt.free_async(p)
+assert take() == []
+assert rt.malloc(n) == p
+assert take() == ["record 1 on (nil)", "host waits for 1"]           # the event came along
+rt.set_default_stream(b)
+rt.free_async(p)                                                      # the null stream stands for b here
+assert take() == ["record 1 on " + f"{b:#x}"]
+""")
