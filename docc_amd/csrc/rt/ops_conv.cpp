@@ -45,7 +45,8 @@ constexpr int64_t kConvWorkspaceCap = int64_t(2) << 30;   // images are processe
 // with 7 tiles a wave, 67.0 us with 6.5); strips of 256 or 128 pixels (4 or 2 tiles per wave) for small images,
 // whose staging of weights per chunk is spread over fewer MFMAs (taken as 8 % and 20 %).
 // Images smaller than half the smallest strip go several to a work-group (`images`, the kernels with the suffix m).
-// DOCC_ROCM_CONV=halo-split / halo-split-wide / halo-whole / halo-t4 / halo-t2 / halo-t4m / halo-t2m force a form (tests, tuning).
+// DOCC_ROCM_CONV=halo-split / halo-split-wide / halo-whole / halo-t4 / halo-t2 / halo-t4m / halo-t2m force a form (tests, tuning), a form
+// followed by -parts<n> (halo-t4-parts3) that form with the channels in n parts.
 struct HaloPlan {
     int tiles = 7;        // column tiles per wave
     int64_t TH = 1;       // output rows per strip
@@ -137,16 +138,20 @@ HaloPlan plan_halo(int64_t N, int64_t C, int64_t OC, int64_t OH, int64_t OW, int
     }
     // Few work-groups with a long chain of chunks each: the channels go to several of them, whose sums a second launch adds. Measured
     // that launch takes about 3 us and moves its parts at 3 TB/s, and a part needs 4 us around its chunks; taken where the whole is a
-    // sixth faster by these figures. 8 x 256 x 14 x 14 (3x3, 256 out): 64 work-groups in 85 us, in four parts 31.
-    if (C >= 16 && !forced && plan.cost > 0.0) {
+    // sixth faster by these figures. 8 x 256 x 14 x 14 (3x3, 256 out): 64 work-groups in 85 us, in four parts 31. A part has two
+    // chunks of eight channels at least.
+    const char* cut = forced ? std::strstr(force, "-parts") : nullptr;
+    if (C >= 32 && (!forced || cut) && plan.cost > 0.0) {
         const double unit = halo_unit_us(C * KH * KW), chunks = (double) (C / 8), bytes = (double) (N * OC * OH * OW * 4);
         double best = (plan.cost * unit + 4.0) / 1.2;
-        auto consider = [&](int tiles, double overhead, int64_t th, int64_t images, int64_t groups) {
+        auto consider = [&](int tiles, double overhead, const char* name, int64_t th, int64_t images, int64_t groups) {
+            if (cut && (std::strncmp(force, name, std::strlen(name)) != 0 || std::strlen(name) + (images > 1) != (size_t) (cut - force))) return;
             for (const int64_t parts : {2, 3, 4, 6, 8, 12, 16, 24, 32}) {
+                if (cut && parts != std::atoi(cut + 6)) continue;
                 if (parts * 2 > C / 8 || groups * parts > 2 * cus || parts * N * OC * OH * OW > (int64_t(1) << 26)) break;
                 const double each = (double) ((C / 8 + parts - 1) / parts) / chunks;
                 const double us = (double) ((groups * parts + cus - 1) / cus) * (tiles * overhead * unit * each + 4.0) + 3.0 + (double) (parts + 1) * bytes / 3e6;
-                if (us >= best) continue;
+                if (us >= best && !cut) continue;
                 best = us;
                 plan.tiles = tiles, plan.TH = th, plan.images = images, plan.parts = parts;
                 plan.split = plan.narrow = false;
@@ -156,12 +161,12 @@ HaloPlan plan_halo(int64_t N, int64_t C, int64_t OC, int64_t OH, int64_t OW, int
         for (const auto& form : small) {
             int64_t th = rows_for(64 * form.tiles);
             while (th > 1 && !fits(th)) th--;
-            if (fits(th)) consider(form.tiles, form.overhead, th, 1, N * ((OH + th - 1) / th) * ocb);
+            if (fits(th)) consider(form.tiles, form.overhead, form.name, th, 1, N * ((OH + th - 1) / th) * ocb);
             int64_t g = 64 * form.tiles / (OH * OW);
             const int64_t patch = ((OH - 1) * stride_h + KH) * ((OW - 1) * stride_w + KW);
             if (g > N) g = N;
             while (g >= 2 && !(g * patch <= 3 * 256 && 3 * (64 * (8 * KH * KW + 4) + 8 * (g * patch + 1)) * 4 <= 160 * 1024)) g--;
-            if (g >= 2) consider(form.tiles, form.overhead, OH, g, (N + g - 1) / g * ocb);
+            if (g >= 2) consider(form.tiles, form.overhead, form.name, OH, g, (N + g - 1) / g * ocb);
         }
     }
     return plan;

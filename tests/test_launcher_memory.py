@@ -148,6 +148,29 @@ print(recorder.recorder_device_queries())
     assert int(got[0]) <= 8
 
 
+@pytest.mark.parametrize("form,channels,parts", [("t4-parts2", 32, 2), ("t2-parts2", 32, 2), ("t4m-parts3", 72, 3), ("t2m-parts4", 72, 4), ("t4-parts2", 24, 0)])
+def test_convolutions_in_a_given_form_and_number_of_parts(recorded, form, channels, parts):
+    got = recorded(f"""
+rt.conv2d_f32(5, {channels}, 9, 7, 70, 3, 3, (1, 1), (1, 1), (1, 1), A, B, C, D)
+print("\\n".join(l for l in take() if l.startswith("launch")))
+""", DOCC_ROCM_CONV="halo-" + form)
+    assert len(got) == (2 if parts else 1)          # fewer than four chunks of channels are not cut
+    if parts:
+        assert f"_{form.split('-')[0]}_parts " in got[0] and f",2,{parts} " in got[0] and "add_parts" in got[1]
+
+
+# what the planner takes by itself: the shapes of tests/test_gpu_conv_parts.py are products of the cut form
+def test_few_images_of_many_channels_are_cut(recorded):
+    from test_gpu_conv_parts import test_channels_in_parts as cases
+    rows = next(m for m in cases.pytestmark if m.name == "parametrize").args[1]
+    for N, C, OC, H, W, k, stride, pad, _ in rows:
+        got = recorded(f"""
+rt.conv2d_f32({N}, {C}, {H}, {W}, {OC}, {k}, {k}, ({stride}, {stride}), ({pad}, {pad}), (1, 1), A, B, C, D)
+print("\\n".join(l for l in take() if l.startswith("launch")))
+""")
+        assert ("_parts" in " ".join(got)) == (C > 16), (N, C, got)
+
+
 def test_the_release_of_a_block_of_the_null_stream_is_recorded_when_somebody_else_takes_it(recorded):
     recorded("""
 n, b = 1 << 20, rt.stream_create()
