@@ -49,3 +49,36 @@ def test_parts_of_different_lengths(kind, m, n, k):
     for tb in (False, True):
         check(kind, m, n, k, False, tb)
     check(kind, m, n, k, True, False, alpha=0.5, beta=1.0)
+
+
+@pytest.mark.parametrize("kind", list(KINDS))
+def test_a_packed_product_in_a_capture_replays(monkeypatch, kind):
+    """The packed operands' block belongs to the graph: replays between products of the program's own, which take blocks of that size too."""
+    monkeypatch.setenv("DOCC_ROCM_GEMM_PACK", "1")
+    dtype, gemm, _ = KINDS[kind]
+    out = torch.float32 if kind == "bf16" else dtype
+    m, n, k = 130, 67, 333
+    gen = torch.Generator().manual_seed(3)
+    draw = lambda r, c: torch.randint(-3, 4, (r, c), generator=gen).to(dtype)
+    pairs = [(draw(m, k), draw(k, n)) for _ in range(2)]
+    want = [a.double() @ b.double() for a, b in pairs]
+    (a, b), (a2, b2) = [[t.cuda() for t in pair] for pair in pairs]
+    c, c2 = torch.empty(m, n, device="cuda", dtype=out), torch.empty(m, n, device="cuda", dtype=out)
+    torch.cuda.synchronize()
+    call = lambda a, b, c, s: gemm(m, n, k, 1.0, a.data_ptr(), k, b.data_ptr(), n, 0.0, c.data_ptr(), n, stream=s)
+    s = rt.stream_create()
+    try:
+        call(a2, b2, c2, s)
+        with rt.Graph.capture(s) as graph:
+            call(a, b, c, s)
+        for _ in range(3):
+            c.fill_(float("nan"))
+            c2.fill_(float("nan"))
+            torch.cuda.synchronize()
+            graph.launch()
+            call(a2, b2, c2, s)
+            rt.stream_sync(s)
+            assert torch.equal(c.double().cpu(), want[0]) and torch.equal(c2.double().cpu(), want[1])
+        graph.destroy()
+    finally:
+        rt.stream_destroy(s)

@@ -11,8 +11,8 @@ from docc_amd import runtime as rt
 
 pytestmark = pytest.mark.gpu
 
-ACTS = {None: -1, "relu": 2, "sigmoid": 3, "tanh": 5, "gelu": 16, "gelu_tanh": 17, "silu": 18}
-REF = {None: lambda x: x, "relu": torch.relu, "sigmoid": torch.sigmoid, "tanh": torch.tanh, "gelu": F.gelu,
+ACTS = {None: -1, "abs": 0, "relu": 2, "sigmoid": 3, "tanh": 5, "gelu": 16, "gelu_tanh": 17, "silu": 18}
+REF = {None: lambda x: x, "abs": torch.abs, "relu": torch.relu, "sigmoid": torch.sigmoid, "tanh": torch.tanh, "gelu": F.gelu,
        "gelu_tanh": lambda x: F.gelu(x, approximate="tanh"), "silu": F.silu}
 TYPE = {torch.bfloat16: 1, torch.float32: 2}
 
@@ -21,10 +21,10 @@ def ptr(t):
     return ctypes.c_void_p(t.data_ptr() if t is not None else None)
 
 
-def linear(a, w, trans_b, bias, act, residual, rounding, out_dtype):
+def linear(a, w, trans_b, bias, act, residual, rounding, out_dtype, y=None):
     m, k = a.shape
     n = w.shape[0] if trans_b else w.shape[1]
-    y = torch.full((m, n), float("nan"), device="cuda", dtype=out_dtype)
+    y = y if y is not None else torch.full((m, n), float("nan"), device="cuda", dtype=out_dtype)
     rt.call("docc_rocm_linear", 0, TYPE[a.dtype], rt.NO_TRANS, rt.TRANS if trans_b else rt.NO_TRANS, m, n, k, 1.0, ptr(a), k, ptr(w), w.shape[1],
             ptr(bias), TYPE[bias.dtype] if bias is not None else 2, ACTS[act], ptr(residual), TYPE[residual.dtype] if residual is not None else 2,
             rounding, ptr(y), TYPE[out_dtype])
@@ -98,6 +98,71 @@ def test_linear_activations(act, trans_b):
     ref = reference(a, w, trans_b, bias, act, None, 0)
     # |x| up to about 15; sums of 64 terms in fp32 (2e-6) through slopes of at most 1.13
     assert float((got - ref).abs().max()) <= 1e-5
+
+
+# the chain in the store, behind parts of K, behind a matrix-vector product, and element by element (n = 77: no whole vectors)
+CHAINS = [(256, 256, "0"), (256, 256, "4"), (1, 4096, "0"), (130, 77, "0")]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("m,n,splits", CHAINS)
+def test_roundings_in_between(monkeypatch, dtype, m, n, splits):
+    """Whole numbers: every fp32 sum is exact, most of them have more bits than a bf16 value, and each rounding shows."""
+    monkeypatch.setenv("DOCC_ROCM_GEMM_SPLITK", splits)
+    gen = torch.Generator().manual_seed(m + n)
+    draw = lambda *shape: torch.randint(-7, 8, shape, generator=gen).float()
+    a, w, bias, res = draw(m, 512), draw(n, 512), draw(n), draw(m, n)
+    at = lambda t: t.to(dtype).cuda()
+    seen = []
+    for act in (None, "relu", "abs"):
+        for rounding in (0, 1, 2, 3):
+            want = reference(a, w, True, bias, act, res, rounding).float()
+            got = linear(at(a), at(w), True, at(bias), act, at(res), rounding, torch.float32).cpu()
+            assert torch.equal(got, want), (act, rounding)
+            seen.append(want)
+            # Y may be the residual itself
+            y = res.cuda()
+            assert torch.equal(linear(at(a), at(w), True, at(bias), act, y, rounding, torch.float32, y).cpu(), want)
+        assert not torch.equal(seen[-4], seen[-3]) and not torch.equal(seen[-4], seen[-2])
+
+
+@pytest.mark.parametrize("n,splits", [(256, "0"), (77, "0")])
+def test_activations_of_values_that_are_not_finite(monkeypatch, n, splits):
+    monkeypatch.setenv("DOCC_ROCM_GEMM_SPLITK", splits)
+    inf = float("inf")
+    x = torch.tensor([inf, -inf, float("nan"), 1e30, -1e30, 3e38, -3e38, 100.0, -100.0, 12.0, -12.0, 0.0])
+    a, w = torch.zeros(len(x), 64), torch.zeros(n, 64)
+    a[:, 0], w[:, 0] = x, 1
+    # as the nodes spell them, in fp32: -inf times a factor that is 0 is a NaN
+    spelled = {None: x, "abs": x.abs(), "relu": torch.fmax(x, torch.zeros(())), "sigmoid": 1 / (1 + torch.exp(-x)), "tanh": torch.tanh(x),
+               "gelu": 0.5 * x * (1 + torch.erf(x * 0.7071067811865476)), "gelu_tanh": 0.5 * x * (1 + torch.tanh(0.7978845608028654 * (x + 0.044715 * x * x * x))),
+               "silu": x * (1 / (1 + torch.exp(-x)))}
+    for act, want in spelled.items():
+        got = linear(a.cuda(), w.cuda(), True, None, act, None, 0, torch.float32).cpu()
+        # (1e-5: the gelu of -12 and -100, zero where it cancels and 1e-32 where it does not)
+        assert torch.allclose(got, want[:, None].expand(-1, n), rtol=1e-6, atol=1e-5, equal_nan=True), (act, got[:, 0], want)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows,cols", [(1100, 256), (6, 250), (6, 2048), (6, 9001), (6, 16384)])
+def test_layer_norm_in_place_and_with_values_that_are_not_finite(dtype, rows, cols):
+    gen = torch.Generator().manual_seed(rows)
+    x = torch.randn(rows, cols, generator=gen).to(dtype).cuda()
+    w, b = torch.randn(cols, generator=gen).to(dtype).cuda(), torch.randn(cols, generator=gen).to(dtype).cuda()
+
+    def norm(x, y):
+        rt.call("docc_rocm_layer_norm", 0, TYPE[dtype], rows, cols, 1e-5, ptr(x), ptr(w), ptr(b), ptr(y))
+        torch.cuda.synchronize()
+        return y
+
+    plain = norm(x, torch.empty_like(x))
+    same = x.clone()
+    assert torch.equal(norm(same, same), plain)
+    x[1, cols // 2], x[3, 0], x[4, cols - 1] = float("inf"), float("nan"), -float("inf")
+    got = norm(x, torch.empty_like(x))
+    spoilt = torch.zeros(rows, dtype=torch.bool, device="cuda")
+    spoilt[[1, 3, 4]] = True
+    assert bool(got[spoilt].isnan().all()) and torch.equal(got[~spoilt], plain[~spoilt])
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
