@@ -1,4 +1,4 @@
-"""Checks on the built kernel images that no run on a GPU makes visible.
+"""Checks on the built kernel images that no run on a GPU makes visible, or only as a time.
 
 The bf16 GEMM on the 16x16x32 MFMA (csrc/kernels/gemm_async16.h) writes its MFMAs as asm statements with the
 accumulator tied to its registers. The compiler therefore does not know their latency: an accumulator register read by
@@ -55,3 +55,26 @@ def test_no_accumulator_is_touched_between_the_mfmas_of_the_16x16x32_gemm(tmp_pa
         first_read = next(i for i, ln in enumerate(after) if ln.startswith("v_accvgpr"))
         assert sum(1 for ln in after[:first_read] if ln == "s_nop 15") >= 2, (m.group(1), after[:first_read][-6:])
     assert seen == 4, seen
+
+
+@pytest.mark.parametrize("image", ["gemm_bf16_async", "gemm_bf16_async_epilogue", "gemm_bf16_async_finish"])
+def test_the_k_loops_of_the_128_row_bf16_tiles_start_on_an_instruction_line(tmp_path, image):
+    path = ROOT / "docc_amd" / "lib" / f"docc_rocm_{image}.hsaco"
+    if not path.exists():
+        pytest.skip("kernel images are not built")
+    seen = 0
+    for body in re.split(r"\n(?=[0-9a-f]{16} <)", disassembly(path, tmp_path)):
+        m = re.match(r"[0-9a-f]{16} <(docc_bgemma_128x\w+)>:", body)
+        if not m:
+            continue
+        code = [(int(at, 16), text.strip()) for text, at in re.findall(r"\n(.*?)// ([0-9A-F]+):", body)]
+        loops = []      # (length, start) of the backward branches around at least one step's MFMAs
+        for at, text in code:
+            jump = re.match(r"s_c?branch\S* (\d+)$", text)
+            if jump and int(jump.group(1)) > 32767:
+                start = at + 4 + 4 * (int(jump.group(1)) - 65536)
+                if sum("v_mfma" in t for a, t in code if start <= a <= at) >= 8:
+                    loops.append((at - start, start))
+        assert loops and min(loops)[1] % 64 == 0, (m.group(1), min(loops))
+        seen += 1
+    assert seen >= 6, seen
