@@ -3,8 +3,9 @@
 #include "gemm_async.h"
 
 // Two tiles of 128 x 128: with stages of 64 k a work-group owns a CU (128 KB of LDS) and has 96 KB of copies in flight; with
-// stages of 32 k two work-groups share it. Where K gives the pipeline of the first time to fill it is the faster one whether the tiles
-// are one round over the CUs or several (2048^3 21.5 us against 23.0, 4096 x 2048 x 8192 139 against 165), below K = 1024 the second.
+// stages of 32 k two work-groups share it. The first is the faster one where each CU has one of them (2048^3 24.0 us against 25.4) and K
+// is long (4096 x 2048 x 8192 139 against 165), the second where there are a few more tiles than CUs (1509 x 2816 x 1032 28 against 22);
+// the estimate in csrc/rt/ops_gemm.cpp weighs them.
 DOCC_AGEMM_CONFIG(bgemm, uint16_t, float, 128, 128, 64, 2, 2, 4)
 DOCC_AGEMM_CONFIG(bgemm, uint16_t, float, 128, 128, 32, 2, 2, 4)
 // Between them and the 256 x 256 tile, for products whose 256 x 256 tiles would leave CUs without one: 144 KB of LDS.

@@ -30,18 +30,25 @@ size_t gemm_lds_bytes(const TileConfig& c, bool ta, bool tb, size_t elem) {
     return 2 * (a_elems + b_elems) * elem;
 }
 
-// Seconds a bf16 product of `count` matrices takes on tile `c`, fitted to 26 products from 64 x 2048 x 8192 to 8192 x 3072 x 768 and
-// 6144 x 4096 x 4096 (within 15 % on most): a launch, and for every round of tiles over the CUs the fp32 store of the tiles (all of
-// them at once: 11 us for 256 x 256) and their products at what the tile sustains. A last round that leaves CUs idle runs
-// faster (less traffic, higher clocks), but not in proportion, the smallest tile's, which waits for its copies, least of all.
-double bgemm_seconds(const TileConfig& c, int64_t m, int64_t n, int64_t k, bool tb, int64_t count, int cus) {
-    const int64_t tiles = ((m + c.bm - 1) / c.bm) * ((n + c.bn - 1) / c.bn) * count, last = tiles % cus;
+// Seconds a bf16 product of `count` matrices takes on tile `c`, fitted to 440 drawn products (64 to 8192 an extent, on and off whole lines,
+// a third with an epilogue) on all four tiles: a launch, and for every round of tiles over the CUs the fp32 store of the tiles (all of them at
+// once: 11 us for 256 x 256) and their products at what the tile sustains. A last round that leaves CUs idle runs faster (less traffic, higher
+// clocks), but not in proportion. The 128 x 128 tile with stages of 32 k sits two to a CU: 264 of them are little more than one round, where the
+// others need a second (1509 x 2816 x 1032: 22 us, the one with stages of 64 k 28, 128 x 256 26). `lines`: the operands' rows start on lines of
+// 128 bytes; a stage of 64 k that does not straddles two. On 660 other products the tile that this estimate takes is 0.8 % slower than the
+// fastest in the mean and more than 5 % on 33 of them; by the number of 256 x 256 tiles alone (from 192 on that tile, else 128 x 128 with
+// stages of 32 k) it is 5.0 % and 171.
+double bgemm_seconds(const TileConfig& c, int64_t m, int64_t n, int64_t k, bool tb, int64_t count, int cus, bool lines) {
+    const bool big = c.bm == 256, wide = c.bm < c.bn, two = !big && !wide && c.bk == 32, pairs = k % 64 == 0;   // pairs: K as the 16x16x32 MFMA takes it
+    const int64_t tiles = ((m + c.bm - 1) / c.bm) * ((n + c.bn - 1) / c.bn) * count, round = two ? 2 * cus : cus, last = tiles % round;
     const double part = (double) last / cus;
-    const double rounds = (double) (tiles / cus) + (!last ? 0.0 : tiles < cus && c.bn == 128 ? 0.7 + 0.2 * part : 0.5 + 0.4 * part);
-    // relative to the 256 x 256 tile on the 16x16x32 MFMA (which takes K in whole pairs of 32): the 128 x 256 one reads a k-major B from
-    // LDS at half the width (and has the deepest pipeline to fill); 128 x 128 tiles in several rounds read the operands from further away than L2
-    const double rel = c.bm == 256 ? (k % 64 == 0 ? 1.0 : 0.93) : c.bn == 256 ? (tb ? 0.88 : 0.80) : tiles > cus ? 0.75 : 0.86;
-    const double area = (double) c.bm * c.bn, fill = c.bm < c.bn ? (tb ? 1.5 : 3.0) : 0.0;
+    double rounds = (double) (tiles / round) * (two ? 1.44 : 1.0);
+    if (last) rounds += !two ? 0.66 + 0.37 * part : part <= 1.0 ? 0.41 + 0.33 * part : 0.68 + 0.38 * part;
+    if (!big && !wide && !two && tiles <= cus) rounds = 0.56 + 0.3 * (double) tiles / cus;
+    // relative to the 256 x 256 tile: the 128 x 256 one reads a k-major B from LDS at half the width; 128 x 128 tiles wait for their copies
+    double rel = big ? (pairs ? 1.0 : 0.88) : wide ? (tb ? 0.75 : 0.71) : two ? 0.44 : tiles > cus ? 0.68 : 0.61;
+    if (!lines) rel *= big ? (pairs ? 0.95 : 1.0) : wide ? 0.88 : 0.85;
+    const double area = (double) c.bm * c.bn, fill = big ? (pairs ? 1.0 : 2.0) : wide || two ? 0.0 : 0.4;   // us until a round's first products
     return 1e-6 * (4.0 + rounds * (fill + area * (11.0 / 65536) + area * (double) k * 3.6e-7 / rel));
 }
 
@@ -220,7 +227,7 @@ int gemv_launch(const char* prefix, hipStream_t s, bool ta, bool tb, int64_t m, 
 template <typename T, typename S = T>
 int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int trans_b, int64_t m, int64_t n,
                 int64_t k, S alpha, const T* A, int64_t lda, const T* B, int64_t ldb, S beta, S* C, int64_t ldc,
-                TileConfig (*pick)(int64_t m, int64_t n, int64_t k, bool tb, int64_t batch, bool aligned, int force, int cus), const S* bias = nullptr,
+                TileConfig (*pick)(int64_t m, int64_t n, int64_t k, bool tb, int64_t batch, int aligned, int force, int cus), const S* bias = nullptr,
                 int activation = -1, int64_t batch = 1, int64_t batch_a = 0, int64_t batch_b = 0, int64_t batch_c = 0,
                 const LinearFinish* fin = nullptr, int64_t k_total = 0) {
     if ((trans_a != DOCC_ROCM_NO_TRANS && trans_a != DOCC_ROCM_TRANS) ||
@@ -340,9 +347,11 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
     // the aligned kernels read whole 128-bit vectors: pointers, leading dimensions and the
     // contiguous extents of both operands must be multiples of the vector length
     const int64_t a_contig = ta ? m : k, b_contig = tb ? k : n;
-    const bool aligned = ((uintptr_t) A % 16 == 0) && ((uintptr_t) B % 16 == 0) && (lda % vec == 0) && (ldb % vec == 0) &&
+    const bool vectors = ((uintptr_t) A % 16 == 0) && ((uintptr_t) B % 16 == 0) && (lda % vec == 0) && (ldb % vec == 0) &&
                          (a_contig % (int64_t) vec == 0) && (b_contig % (int64_t) vec == 0) &&
                          (batch == 1 || (batch_a % (int64_t) vec == 0 && batch_b % (int64_t) vec == 0));
+    const bool lines = vectors && ((uintptr_t) A | (uintptr_t) B | (uintptr_t) (lda * (int64_t) sizeof(T)) | (uintptr_t) (ldb * (int64_t) sizeof(T))) % 128 == 0;
+    const int aligned = lines ? 2 : vectors ? 1 : 0;
     // A few rows against a wide fp32 matrix: B goes from global memory straight into the MFMA operands, 128 columns of one part
     // of K per work-group, the parts added in order by a second launch. With B stored [n][k] the lanes of a load walk different
     // rows, which pays up to 16 rows only. DOCC_ROCM_GEMM_SKINNY=0 switches it off, DOCC_ROCM_GEMM_SPLITK forces the number of
@@ -486,7 +495,7 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
     // the asynchronous kernels need aligned operands and address a tile with 32-bit byte offsets
     const int64_t max_edge = cfg.bm > cfg.bn ? (cfg.bm > cfg.bk ? cfg.bm : cfg.bk) : (cfg.bn > cfg.bk ? cfg.bn : cfg.bk);
     const bool offsets_fit = max_edge * (lda > ldb ? lda : ldb) * (int64_t) sizeof(T) < (int64_t(1) << 32);
-    if (cfg.stages > 0 && !(aligned && offsets_fit)) cfg = pick(m, n, k, tb, batch, false, 0, cus);
+    if (cfg.stages > 0 && !(aligned && offsets_fit)) cfg = pick(m, n, k, tb, batch, 0, 0, cus);
     const int64_t tiles = ((m + cfg.bm - 1) / cfg.bm) * ((n + cfg.bn - 1) / cfg.bn);
     if (tiles > 0x7fffffffLL) return fail(DOCC_ROCM_ERR_UNSUPPORTED, "%s: too many tiles", prefix);
     // Few output tiles and a long K extent (a handful of rows against a wide matrix: the product is bound by reading
@@ -509,9 +518,10 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
         // Estimated seconds of the product in `parts` parts on the tile the picker gives that many matrices: the work of
         // the padded tiles at what the tile sustains (relative to the 128 x 256 one) on the share of the CUs that get a
         // work-group, plus writing and reading the parts at 5 TB/s and a second launch.
+        const double behind = epilogue ? 4e-6 : 0.0;   // bias and activation are a launch of their own then (64 x 192 x 1093 bf16 whole 12 us, in parts 15)
         auto seconds = [&](const TileConfig& c, int64_t parts) {
             if (sizeof(T) == 2)
-                return bgemm_seconds(c, m, n, part_of(parts), tb, parts, cus) + (parts > 1 ? 2.0 * (double) parts * (double) m * (double) n * sizeof(S) / 5e12 + 2e-6 : 0.0);
+                return bgemm_seconds(c, m, n, part_of(parts), tb, parts, cus, lines) + (parts > 1 ? 2.0 * (double) parts * (double) m * (double) n * sizeof(S) / 5e12 + 2e-6 + behind : 0.0);
             const double tm = (double) ((m + c.bm - 1) / c.bm), tn = (double) ((n + c.bn - 1) / c.bn);
             const double area = (double) c.bm * c.bn;
             const double rel = area >= 65536 ? 1.03 : area >= 32768 ? 1.0 : area >= 16384 ? 0.97 : 0.75;
@@ -521,7 +531,7 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
             const double fill = per_cu < 1.0 ? per_cu : per_cu / (double) (int64_t) (per_cu + 0.999999);
             const double rate = sizeof(T) == 8 ? 68e12 : 141e12;
             double t = 2.0 * tm * c.bm * tn * c.bn * (double) k / (rate * rel * fill);
-            if (parts > 1) t += 2.0 * (double) parts * (double) m * (double) n * sizeof(S) / 5e12 + 3e-6;
+            if (parts > 1) t += 2.0 * (double) parts * (double) m * (double) n * sizeof(S) / 5e12 + 3e-6 + behind;
             return t;
         };
         int64_t splits = 1;
@@ -532,7 +542,7 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
             double best = seconds(cfg, 1);
             for (int64_t parts : {2, 3, 4, 5, 6, 8, 10, 12, 16, 20, 24, 32, 48, 64}) {
                 if (!allowed(parts)) continue;
-                const TileConfig c = pick(m, n, part_of(parts), tb, parts, true, 0, cus);
+                const TileConfig c = pick(m, n, part_of(parts), tb, parts, aligned, 0, cus);
                 if (c.stages == 0) break;
                 const double t = seconds(c, parts);
                 if (t < (splits > 1 ? 1.0 : sizeof(T) == 2 ? 0.95 : 0.9) * best) {   // cut for a clear gain only: the estimate is rough
@@ -611,7 +621,7 @@ template <typename T, typename S>
 static int gemm_batched(const char* prefix, docc_rocm_stream_t stream, int trans_a, int trans_b, int64_t m, int64_t n, int64_t k,
                         S alpha, const T* A, int64_t lda, int64_t stride_a, const T* B, int64_t ldb, int64_t stride_b, S beta, S* C,
                         int64_t ldc, int64_t stride_c, int64_t batch,
-                        TileConfig (*pick)(int64_t m, int64_t n, int64_t k, bool tb, int64_t batch, bool aligned, int force, int cus)) {
+                        TileConfig (*pick)(int64_t m, int64_t n, int64_t k, bool tb, int64_t batch, int aligned, int force, int cus)) {
     if (batch < 0) return fail(DOCC_ROCM_ERR_INVALID_ARGUMENT, "%s: negative batch", prefix);
     const int64_t kMaxGridY = 65535;
     for (int64_t b0 = 0; b0 < batch; b0 += kMaxGridY) {
@@ -626,12 +636,12 @@ static int gemm_batched(const char* prefix, docc_rocm_stream_t stream, int trans
 
 extern "C" {
 
-// Tile selection. `force`: +1 largest tile, -1 smallest tile, 0 by problem size. Asynchronous
-// (staged) configurations need aligned operands; the others handle everything.
+// Tile selection. `force`: +1 largest tile, -1 smallest tile, 0 by problem size. `aligned`: 1 on whole vectors, 2 on lines of 128 bytes too.
+// Asynchronous (staged) configurations need aligned operands; the others handle everything.
 // tiles of one matrix times the number of matrices: what there is to spread over the compute units
 static int64_t tiles_of(int64_t m, int64_t n, int bm, int bn, int64_t batch = 1) { return ((m + bm - 1) / bm) * ((n + bn - 1) / bn) * batch; }
 
-static TileConfig pick_sgemm(int64_t m, int64_t n, int64_t, bool, int64_t batch, bool aligned, int force, int cus) {
+static TileConfig pick_sgemm(int64_t m, int64_t n, int64_t, bool, int64_t batch, int aligned, int force, int cus) {
     const TileConfig huge{256, 256, 32, 4, 2}, wide{128, 256, 32, 4, 2}, big{128, 128, 32, 4, 3}, small{64, 64, 16, 4, 4};
     const TileConfig plain_big{128, 128, 16, 4, 0}, plain_small{64, 64, 16, 4, 0};
     if (!aligned) return force > 0 ? plain_big : force < 0 ? plain_small : (tiles_of(m, n, 128, 128, batch) >= 256 ? plain_big : plain_small);
@@ -652,7 +662,7 @@ static TileConfig pick_sgemm(int64_t m, int64_t n, int64_t, bool, int64_t batch,
     return sw >= sb && sw >= ss ? wide : sb >= ss ? big : small;
 }
 
-static TileConfig pick_dgemm(int64_t m, int64_t n, int64_t, bool, int64_t batch, bool aligned, int force, int) {
+static TileConfig pick_dgemm(int64_t m, int64_t n, int64_t, bool, int64_t batch, int aligned, int force, int) {
     const TileConfig big{128, 128, 16, 4, 3}, mid{64, 64, 16, 4, 4}, small{64, 32, 16, 4, 4};
     const TileConfig plain_big{128, 128, 16, 4, 0}, plain_small{64, 64, 16, 4, 0};
     if (!aligned) return force > 0 ? plain_big : plain_small;
@@ -661,16 +671,16 @@ static TileConfig pick_dgemm(int64_t m, int64_t n, int64_t, bool, int64_t batch,
     return t >= 2048 ? big : t > 512 ? mid : small;   // few tiles: halve them so that two work-groups share a CU
 }
 
-static TileConfig pick_bgemm(int64_t m, int64_t n, int64_t k, bool tb, int64_t batch, bool aligned, int force, int cus) {
+static TileConfig pick_bgemm(int64_t m, int64_t n, int64_t k, bool tb, int64_t batch, int aligned, int force, int cus) {
     // big: on the 16x16x32 MFMA where K allows it (see gemm_launch), else on the 32x32x16 one with the copies dealt out
     const TileConfig big{256, 256, 32, 4, 4, true, true}, wide{128, 256, 64, 4, 3}, deep{128, 128, 64, 4, 4}, small{128, 128, 32, 4, 4};
     const TileConfig plain_big{256, 256, 64, 4, 0}, plain_small{128, 128, 64, 4, 0};
     if (!aligned) return force > 0 ? plain_big : force < 0 ? plain_small : (tiles_of(m, n, 256, 256, batch) >= 256 ? plain_big : plain_small);
     if (force) return force > 0 ? big : small;
     const TileConfig* best = &big;
-    double least = bgemm_seconds(big, m, n, k, tb, batch, cus);
-    for (const TileConfig* c : {&wide, k >= 1024 ? &deep : &small}) {
-        const double t = bgemm_seconds(*c, m, n, k, tb, batch, cus);
+    double least = bgemm_seconds(big, m, n, k, tb, batch, cus, aligned == 2);
+    for (const TileConfig* c : {&wide, &deep, &small}) {
+        const double t = bgemm_seconds(*c, m, n, k, tb, batch, cus, aligned == 2);
         if (t < least) {
             least = t;
             best = c;

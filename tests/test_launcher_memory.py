@@ -193,3 +193,17 @@ rt.set_default_stream(b)
 rt.free_async(p)                                                      # the null stream stands for b here
 assert take() == ["record 1 on " + f"{b:#x}"]
 """)
+
+
+# bf16 products on which one tile was measured to be the fastest by a tenth or more, and one with an epilogue that parts of K do not pay for
+@pytest.mark.parametrize("m,n,k,ta,tb,epilogue,kernel", [(1509, 2816, 1032, 0, 0, 0, "128x128x32s4_nn"), (2944, 2912, 688, 0, 0, 1, "128x128x32s4_nn_e"),
+                                                         (3064, 1408, 3552, 0, 0, 0, "128x128x32s4_nn"), (4096, 4096, 4096, 0, 0, 0, "256x256x32q4_nn"),
+                                                         (4096, 2048, 8192, 0, 1, 0, "128x256x64s3_nt"), (2048, 2048, 2048, 0, 0, 0, "128x128x64s4_nn"),
+                                                         (5352, 3072, 96, 0, 0, 1, "128x128x32s4_nn_e"), (64, 192, 1093, 1, 0, 1, "128x128x32s4_tn_e")])
+def test_tiles_of_bf16_products(recorded, m, n, k, ta, tb, epilogue, kernel):
+    got = recorded(f"""
+rt.call("docc_rocm_bf16gemm_f32_epilogue", 0, {111 + ta}, {111 + tb}, {m}, {n}, {k}, 1.0, A, {m if ta else k}, B, {k if tb else n}, 0.0, C, {n}, D if {epilogue} else None,
+        2 if {epilogue} else -1)
+print("\\n".join(l for l in take() if l.startswith("launch")))
+""")
+    assert len(got) == 1 and got[0].split()[1] == "docc_bgemma_" + kernel, got
