@@ -26,10 +26,10 @@ AttentionRates attention_rates(int64_t D) {
 constexpr double kMemory = 6.0e6, kCombine = 2.5;   // bytes / us; us of the second launch
 
 // the split form with the best number of parts: its time, and the number in *best
-double attention_split_us(int64_t BH, int64_t SQ, int64_t SKV, int64_t D, int64_t* best) {
+double attention_split_us(int64_t BH, int64_t SQ, int64_t SKV, int64_t D, int64_t cus, int64_t* best) {
     const AttentionRates r = attention_rates(D);
     const int64_t tiles = (SQ + kSplitQueries - 1) / kSplitQueries, blocks = (SKV + kSplitBlock - 1) / kSplitBlock;
-    const int64_t cus = compute_units(), slots = cus * (D == 128 ? 1 : 2);   // what the rings' LDS lets a CU hold
+    const int64_t slots = cus * (D == 128 ? 1 : 2);   // what the rings' LDS lets a CU hold
     double best_us = 0;
     for (const int64_t parts : {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64}) {
         if (parts > 1 && (parts * kSplitWaves > blocks || BH > 65535)) break;
@@ -48,9 +48,9 @@ double attention_split_us(int64_t BH, int64_t SQ, int64_t SKV, int64_t D, int64_
 }
 
 // the form of 128 queries per work-group (the causal one takes a long and a short block of queries together)
-double attention_us(int64_t BH, int64_t SQ, int64_t SKV, int64_t D, bool causal) {
+double attention_us(int64_t BH, int64_t SQ, int64_t SKV, int64_t D, bool causal, int64_t cus) {
     const AttentionRates r = attention_rates(D);
-    const int64_t tiles = (SQ + 127) / 128, blocks = (SKV + 63) / 64, cus = compute_units();
+    const int64_t tiles = (SQ + 127) / 128, blocks = (SKV + 63) / 64;
     const int64_t groups = BH * (causal ? (tiles + 1) / 2 : tiles);
     const int64_t each = causal && 2 * tiles < blocks ? 2 * tiles + 2 : causal && tiles > 1 ? blocks + 2 : blocks;
     const double memory = (double) (BH * SKV * D * 4) / kMemory * 1.2, bound = (double) each * ((groups + cus - 1) / cus) * r.step;
@@ -112,20 +112,22 @@ int attention_fused(docc_rocm_stream_t stream, int64_t B, int64_t H, int64_t SQ,
     // MFMAs: fewer instructions per flop) once that still gives every CU its two resident work-groups, else 128
     // per work-group (more, smaller work-groups). DOCC_ROCM_ATTENTION_Q=32|128|256 forces one (tuning and tests).
     const int64_t BH = B * H, out_bytes = out_bf16 ? 2 : 4;
+    int64_t cus = compute_units();
+    if (cus <= 0) cus = 256;
     // ... and only where the larger groups do not add padded queries: a wavefront multiplies its 64 queries whether they
     // exist or not (SQ = 100 would run 256 queries in the large form and 128 in the small one)
     const bool no_extra_padding = (SQ + 255) / 256 * 256 <= (SQ + 127) / 128 * 128 || SQ >= 1024;
-    int per_group = ((SQ + 255) / 256) * BH >= 2 * compute_units() && no_extra_padding ? 256 : 128;
+    int per_group = ((SQ + 255) / 256) * BH >= 2 * cus && no_extra_padding ? 256 : 128;
     // head dim 128: the large form is eight wavefronts of 32 queries (one work-group per CU), the small one four
-    if (D == 128) per_group = ((SQ + 255) / 256) * BH >= compute_units() && no_extra_padding ? 256 : 128;
+    if (D == 128) per_group = ((SQ + 255) / 256) * BH >= cus && no_extra_padding ? 256 : 128;
     // Few queries, or few work-groups: the form that cuts the keys, where the estimates say so by more than they are off. Both forms,
     // measured (B, H, SQ, SKV, D, us of 128 queries a group / cut keys): 1,4,1,32768,128 609 / 17; 4,8,4,8192,64 104 / 16; 16,16,1,4096,128
     // 96-106 / 93; 32,32,1,1024,128 115 / 94; 1,4,2048,2048,64 28 / 15; 1,16,1024,1024,64 16 / 12; on the other side 2,16,1024,1024,64 17 / 23;
     // 4,16,256,256,128 10 / 14; 16,16,128,128,64 6 / 10
     int64_t parts = 1;
     if (per_group == 128) {
-        const double split = attention_split_us(BH, SQ, SKV, D, &parts);
-        if (split < 0.92 * attention_us(BH, SQ, SKV, D, causal)) per_group = kSplitQueries;
+        const double split = attention_split_us(BH, SQ, SKV, D, cus, &parts);
+        if (split < 0.92 * attention_us(BH, SQ, SKV, D, causal, cus)) per_group = kSplitQueries;
     }
     if (const char* force = std::getenv("DOCC_ROCM_ATTENTION_Q")) {
         const int v = std::atoi(force);

@@ -137,15 +137,18 @@ print("\\n".join(take()))
     assert len(got) == launches and all(l.startswith("launch docc_layernorm_f32") for l in got)
 
 
-def test_a_product_asks_for_the_device_a_few_times_however_many_forms_it_weighs(recorded):
-    # 512 x 512 x 4096 has fewer tiles than CUs: a dozen numbers of parts on three tiles each
-    got = recorded("""
+# a product with fewer tiles than CUs (a dozen numbers of parts on four tiles each), and attention: once for the entry point, once for the
+# planning, and once a launch, an allocation and a release
+@pytest.mark.parametrize("call,most", [("rt.bf16gemm_f32(512, 512, 4096, 1.0, A, 4096, B, 512, 0.0, C, 512)", 8),
+                                       ("rt.attention_bf16(4, 16, 64, 64, 64, 0.1, A, B, C, D)", 3)])
+def test_a_call_asks_for_the_device_a_few_times_however_many_forms_it_weighs(recorded, call, most):
+    got = recorded(f"""
 for _ in range(2):
     recorder.recorder_device_queries()
-    rt.bf16gemm_f32(512, 512, 4096, 1.0, A, 4096, B, 512, 0.0, C, 512)
+    {call}
 print(recorder.recorder_device_queries())
 """)
-    assert int(got[0]) <= 8
+    assert int(got[0]) <= most
 
 
 @pytest.mark.parametrize("form,channels,parts", [("t4-parts2", 32, 2), ("t2-parts2", 32, 2), ("t4m-parts3", 72, 3), ("t2m-parts4", 72, 4), ("t4-parts2", 24, 0)])
