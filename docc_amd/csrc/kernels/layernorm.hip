@@ -3,7 +3,8 @@
 // it). Bound by HBM: X is read once and Y written once, the row stays in registers between the two sums. As separate launches
 // (cast, mean, centre and square, mean, scale) the same work moved X seven times over: [4096, 2048] bf16 in 64 us, five
 // launches, against 12.8 us here. Rows of a few KB belong to a wavefront (four rows a work-group, no barrier); longer ones, and rows too few to fill the
-// device that way, to a work-group of 256; rows that do not fit its registers are read three times from L2.
+// device that way, to a work-group of 256; rows that do not fit its registers are read three times from L2, by one work-group a row or, from
+// 16384 columns on, in slices.
 #include "common.h"
 
 namespace docc_k {
@@ -132,6 +133,92 @@ __device__ __forceinline__ void layernorm_long(long cols, float eps, const void*
     }
 }
 
+// Long rows, cut into gridDim.x slices of `chunk` elements (at most 256, whole vectors): a launch for the sums, one for the squares of the
+// centred values, one for the result. A work-group of the latter two adds the row's parts itself, a thread a part. One
+// work-group a row and the slices, fp32: a row of 2^20 1241 / 11 us, 64 rows of 64 x 56 x 56 253 / 36.
+template <typename T, int V, typename F>
+__device__ __forceinline__ void layernorm_slice(const void* X, long cols, long chunk, F f) {
+    typedef LnElement<T> E;
+    typedef typename E::raw raw;
+    const raw* x = reinterpret_cast<const raw*>(X) + (long) blockIdx.y * cols;
+    const long first = blockIdx.x * chunk, end = first + chunk < cols ? first + chunk : cols;
+    for (long c = first + threadIdx.x * V; c < end; c += 256 * V) {
+        float v[V];
+        if constexpr (V == 1) {
+            v[0] = E::up(x[c]);
+        } else {
+            const typename E::vec h = *reinterpret_cast<const typename E::vec*>(x + c);
+#pragma unroll
+            for (int e = 0; e < V; e++) v[e] = E::up(h[e]);
+        }
+        f(c, v);
+    }
+}
+
+// the sum of this row's parts, in every thread
+__device__ __forceinline__ float ln_parts_sum(const float* parts, float* slot) {
+    return ln_row_sum<256>(threadIdx.x < gridDim.x ? parts[(long) blockIdx.y * gridDim.x + threadIdx.x] : 0.0f, slot);
+}
+
+template <typename T, int V>
+__device__ __forceinline__ void layernorm_slice_sum(long cols, long chunk, const void* X, float* sums) {
+    __shared__ float slots[4];
+    float sum = 0.0f;
+    layernorm_slice<T, V>(X, cols, chunk, [&](long, float (&v)[V]) {
+#pragma unroll
+        for (int e = 0; e < V; e++) sum += v[e];
+    });
+    sum = ln_row_sum<256>(sum, slots);
+    if (threadIdx.x == 0) sums[(long) blockIdx.y * gridDim.x + blockIdx.x] = sum;
+}
+
+template <typename T, int V>
+__device__ __forceinline__ void layernorm_slice_squares(long cols, long chunk, const void* X, const float* sums, float* squares) {
+    __shared__ float slots[2][4];
+    const float mean = ln_parts_sum(sums, slots[0]) / (float) cols;
+    float sq = 0.0f;
+    layernorm_slice<T, V>(X, cols, chunk, [&](long, float (&v)[V]) {
+#pragma unroll
+        for (int e = 0; e < V; e++) {
+            const float d = v[e] - mean;
+            sq += d * d;
+        }
+    });
+    sq = ln_row_sum<256>(sq, slots[1]);
+    if (threadIdx.x == 0) squares[(long) blockIdx.y * gridDim.x + blockIdx.x] = sq;
+}
+
+template <typename T, int V>
+__device__ __forceinline__ void layernorm_slice_apply(long cols, long chunk, float eps, const void* X, const float* sums, const float* squares, const void* W,
+                                                      const void* B, void* Y) {
+    typedef LnElement<T> E;
+    typedef typename E::raw raw;
+    __shared__ float slots[2][4];
+    const float mean = ln_parts_sum(sums, slots[0]) / (float) cols;
+    const float root = sqrtf(ln_parts_sum(squares, slots[1]) / (float) cols + eps);
+    raw* y = reinterpret_cast<raw*>(Y) + (long) blockIdx.y * cols;
+    const raw *w = reinterpret_cast<const raw*>(W), *b = reinterpret_cast<const raw*>(B);
+    layernorm_slice<T, V>(X, cols, chunk, [&](long c, float (&v)[V]) {
+        typename E::vec hw = {}, hb = {}, h;
+        if constexpr (V > 1) {
+            if (w) hw = *reinterpret_cast<const typename E::vec*>(w + c);
+            if (b) hb = *reinterpret_cast<const typename E::vec*>(b + c);
+        } else {
+            if (w) hw[0] = w[c];
+            if (b) hb[0] = b[c];
+        }
+#pragma unroll
+        for (int e = 0; e < V; e++) {
+            float r = (v[e] - mean) / root;
+            if (w) r *= E::up(hw[e]);
+            if (b) r += E::up(hb[e]);
+            h[e] = E::down(r);
+        }
+        if constexpr (V > 1) *reinterpret_cast<typename E::vec*>(y + c) = h;
+        else y[c] = h[0];
+    });
+}
+
 } // namespace docc_k
 
 #define DOCC_LN_ARGS long rows, long cols, float eps, const void *X, const void *W, const void *B, void *Y
@@ -140,7 +227,22 @@ __device__ __forceinline__ void layernorm_long(long cols, float eps, const void*
     extern "C" __global__ __launch_bounds__(256) void docc_layernorm_##TYPE##_##VTAG##_##RTAG##NV(DOCC_LN_ARGS) {             \
         docc_k::layernorm_row<T, V, NV, TPR>(rows, cols, eps, X, W, B, Y);                                                   \
     }
+// docc_layernorm_<type>_<v|s>_slice_<sum|squares|apply>
+#define DOCC_LN_SLICE(TYPE, T, VTAG, V)                                                                                       \
+    extern "C" __global__ __launch_bounds__(256) void docc_layernorm_##TYPE##_##VTAG##_slice_sum(long cols, long chunk, const void* X, float* sums) {   \
+        docc_k::layernorm_slice_sum<T, V>(cols, chunk, X, sums);                                                              \
+    }                                                                                                                         \
+    extern "C" __global__ __launch_bounds__(256) void docc_layernorm_##TYPE##_##VTAG##_slice_squares(long cols, long chunk, const void* X,              \
+                                                                                                     const float* sums, float* squares) {               \
+        docc_k::layernorm_slice_squares<T, V>(cols, chunk, X, sums, squares);                                                 \
+    }                                                                                                                         \
+    extern "C" __global__ __launch_bounds__(256) void docc_layernorm_##TYPE##_##VTAG##_slice_apply(                           \
+        long cols, long chunk, float eps, const void* X, const float* sums, const float* squares, const void* W, const void* B, void* Y) {              \
+        docc_k::layernorm_slice_apply<T, V>(cols, chunk, eps, X, sums, squares, W, B, Y);                                     \
+    }
 #define DOCC_LN_TYPE(TYPE, T, V)           \
+    DOCC_LN_SLICE(TYPE, T, v, V)             \
+    DOCC_LN_SLICE(TYPE, T, s, 1)             \
     DOCC_LN(TYPE, T, v, V, w, 64, 1)         \
     DOCC_LN(TYPE, T, v, V, w, 64, 2)         \
     DOCC_LN(TYPE, T, v, V, w, 64, 4)         \

@@ -1,5 +1,6 @@
 // Launcher of the layer normalisation kernels (see include/docc_rocm_ops.h, csrc/kernels/layernorm.hip).
 #include <cstdio>
+#include <cstdlib>
 
 #include "docc_rocm_ops.h"
 #include "rt_state.h"
@@ -32,6 +33,33 @@ extern "C" int docc_rocm_layer_norm(docc_rocm_stream_t stream, int type, int64_t
     const bool one = !wave && !b;   // a work-group of 1024 a row
     if (one) std::snprintf(name, sizeof(name), "docc_layernorm_%s_long", bf16 ? "bf16" : "f32");
     else std::snprintf(name, sizeof(name), "docc_layernorm_%s_%c_%c%d", bf16 ? "bf16" : "f32", vec ? 'v' : 's', wave ? 'w' : 'b', wave ? w : b);
+    if (one) {
+        // Rows in slices: three launches, from 16384 columns on faster than a work-group a row whatever their number (fp32, rows x columns, a
+        // work-group a row / slices: 4 x 12000 9.7 / 11.5 us, 4 x 20000 14.6 / 11.8, 1 x 2^20 1241 / 11, 1024 x 20000 65 / 53, 256 x
+        // 200704 320 / 146); without whole vectors up to a row a CU (256 x 33333 45 / 42, 512 x 33333 54 / 77).
+        // DOCC_ROCM_LAYERNORM=slices|rows takes one or the other (tests, tuning).
+        const char* force = std::getenv("DOCC_ROCM_LAYERNORM");
+        const bool pays = cols > 16384 && (vec || rows <= cus);
+        int64_t slices = rows < 4 * (int64_t) cus ? 4 * (int64_t) cus / rows : 1;
+        if (slices > 256) slices = 256;
+        if (slices > cols / 2048) slices = cols / 2048 > 1 ? cols / 2048 : 1;
+        const int64_t chunk = ((cols + slices - 1) / slices + lane - 1) / lane * lane;
+        slices = (cols + chunk - 1) / chunk;
+        hipStream_t s = (hipStream_t) stream;
+        PartialsLease lease;
+        if ((force ? force[0] == 's' : pays) && rows <= 65535 && 2 * rows * slices * (int64_t) sizeof(float) <= (int64_t) kPartialsBytes &&
+            (!foreign_capture(s) || partials_held(s)) && partials_for(s, &lease) == 0) {
+            float *sums = (float*) lease.ptr, *squares = sums + rows * slices;
+            auto step = [&](const char* what, auto... args) {
+                std::snprintf(name, sizeof(name), "docc_layernorm_%s_%c_slice_%s", bf16 ? "bf16" : "f32", vec ? 'v' : 's', what);
+                return launch(name, (uint32_t) slices, (uint32_t) rows, 1, 256, 0, s, (long) cols, (long) chunk, args...);
+            };
+            int rc = step("sum", X, sums);
+            if (!rc) rc = step("squares", X, (const float*) sums, squares);
+            if (!rc) rc = step("apply", eps, X, (const float*) sums, (const float*) squares, weight, bias, Y);
+            return rc;
+        }
+    }
     // a launch holds fewer than 2^32 threads: more rows than that takes go in several
     const int64_t threads = one ? 1024 : 256, per_group = wave ? 4 : 1, most = ((int64_t(1) << 32) / threads - 1) * per_group;
     const int64_t row_bytes = cols * (bf16 ? 2 : 4);

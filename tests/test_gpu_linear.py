@@ -144,7 +144,7 @@ def test_activations_of_values_that_are_not_finite(monkeypatch, n, splits):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("rows,cols", [(1100, 256), (6, 250), (6, 2048), (6, 9001), (6, 16384)])
+@pytest.mark.parametrize("rows,cols", [(1100, 256), (6, 250), (6, 2048), (6, 9001), (6, 16384), (6, 20000), (6, 33333)])
 def test_layer_norm_in_place_and_with_values_that_are_not_finite(dtype, rows, cols):
     gen = torch.Generator().manual_seed(rows)
     x = torch.randn(rows, cols, generator=gen).to(dtype).cuda()
@@ -183,7 +183,15 @@ def test_layer_norm_over_row_lengths(dtype, rows, cols):
         assert bool((err <= bound).all()), float((err / bound).max())
 
 
-@pytest.mark.parametrize("rows,cols", [(1100, 256), (3, 250), (5, 1024), (2, 4096), (3, 4097), (2, 16384)])
+# rows in slices: one and several of them, the last one short, more rows than would get more than one each; as many slices as there can be
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows,cols", [(1, 9000), (2, 9001), (700, 8200), (1, 300000), (3, 65537), (300, 16400)])
+def test_layer_norm_of_long_rows_in_slices(monkeypatch, dtype, rows, cols):
+    monkeypatch.setenv("DOCC_ROCM_LAYERNORM", "slices")
+    test_layer_norm_over_row_lengths(dtype, rows, cols)
+
+
+@pytest.mark.parametrize("rows,cols", [(1100, 256), (3, 250), (5, 1024), (2, 4096), (3, 4097), (2, 16384), (2, 20000), (3, 33333)])
 def test_layer_norm_divides_by_the_root(rows, cols):
     # small whole numbers whose mean is one too: both sums are exact in fp32 whatever their order, what is left is a division by cols, the
     # root and one division an element, each rounded once

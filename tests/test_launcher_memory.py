@@ -127,7 +127,7 @@ assert "im2col" in got and "sgemm" in got and "malloc" not in got, got
 """)
 
 
-@pytest.mark.parametrize("rows,cols,launches", [(2 ** 24 + 5, 2000, 2), (2 ** 26 + 1, 64, 2), (2 ** 22, 20000, 2), (2 ** 24 - 1, 2000, 1)])
+@pytest.mark.parametrize("rows,cols,launches", [(2 ** 24 + 5, 2000, 2), (2 ** 26 + 1, 64, 2), (2 ** 22, 16384, 2), (2 ** 24 - 1, 2000, 1)])
 def test_layer_norm_of_more_rows_than_a_launch_holds(recorded, rows, cols, launches):
     # 2^32 threads are one too many for a launch (the recorder refuses them as the device does)
     got = recorded(f"""
@@ -210,3 +210,27 @@ rt.call("docc_rocm_bf16gemm_f32_epilogue", 0, {111 + ta}, {111 + tb}, {m}, {n}, 
 print("\\n".join(l for l in take() if l.startswith("launch")))
 """)
     assert len(got) == 1 and got[0].split()[1] == "docc_bgemma_" + kernel, got
+
+
+# long rows go in slices, several work-groups a row where there are few of them; not in a capture on a stream that has no buffer for their sums
+@pytest.mark.parametrize("rows,cols,groups", [(1, 2 ** 20, "256,1,1"), (32, 200704, "32,32,1"), (2000, 20000, "1,2000,1"), (3, 33333, "16,3,1"), (2, 16384, None),
+                                              (300, 33333, None), (70000, 20000, None)])
+def test_layer_norm_of_long_rows(recorded, rows, cols, groups):
+    recorded(f"""
+s = rt.stream_create()
+def norm(): rt.call("docc_rocm_layer_norm", s, 2, {rows}, {cols}, 1e-5, A, None, None, B)
+def launches(): return [l for l in take() if l.startswith("launch")]
+recorder.recorder_capture(s)
+norm()
+assert all("_f32_long" in l for l in launches())
+recorder.recorder_capture(None)
+norm()
+got = launches()
+if {groups!r} is None:
+    assert all("_f32_long" in l for l in got), got
+else:
+    assert [l.split()[1].split("_slice_")[1] for l in got] == ["sum", "squares", "apply"] and all(" {groups} x 256 " in l for l in got), got
+    recorder.recorder_capture(s)
+    norm()
+    assert launches() == got
+""")
