@@ -2,7 +2,9 @@
 // bf16 rows, fp32 statistics in two steps (the variance from the centred values, as the chain of nodes it stands for computes
 // it). Bound by HBM: X is read once and Y written once, the row stays in registers between the two sums. As separate launches
 // (cast, mean, centre and square, mean, scale) the same work moved X seven times over: [4096, 2048] bf16 in 64 us, five
-// launches, against 12.8 us here. Rows of a few KB belong to a wavefront (four rows a work-group, no barrier); longer ones, and rows too few to fill the
+// launches, against 12.8 us here. Rows of at most 32 vectors belong to
+// that many lanes of a wavefront (a wavefront each took 226 us for 2^20 rows of 8 fp32, where the nodes took 62; 12.4),
+// rows of a few KB to a wavefront (four rows a work-group, no barrier); longer ones, and rows too few to fill the
 // device that way, to a work-group of 256; rows that do not fit its registers are read three times from L2, by one work-group a row or, from
 // 16384 columns on, in slices.
 #include "common.h"
@@ -25,9 +27,14 @@ template <> struct LnElement<uint16_t> {
     static __device__ __forceinline__ __bf16 down(float v) { return (__bf16) v; }
 };
 
-// sum over the TPR lanes that share a row; `slot`: TPR / 64 floats of LDS nobody else writes meanwhile
+// sum over the TPR lanes that share a row (a power of two of neighbours); `slot`: TPR / 64 floats of LDS nobody else writes meanwhile
 template <int TPR>
 __device__ __forceinline__ float ln_row_sum(float v, float* slot) {
+    if constexpr (TPR < 64) {
+#pragma unroll
+        for (int lanes = TPR / 2; lanes > 0; lanes /= 2) v += __shfl_xor(v, lanes);
+        return v;
+    }
     v = wave_sum(v);
     if (TPR == 64) return v;
     if ((threadIdx.x & 63) == 0) slot[threadIdx.x >> 6] = v;
@@ -43,9 +50,9 @@ template <typename T, int V, int NV, int TPR>
 __device__ __forceinline__ void layernorm_row(long rows, long cols, float eps, const void* X, const void* W, const void* B, void* Y) {
     typedef LnElement<T> E;
     typedef typename E::raw raw;
-    __shared__ float slots[2][TPR / 64];
+    __shared__ float slots[2][TPR > 64 ? TPR / 64 : 1];
     const int t = threadIdx.x % TPR;
-    const long row = TPR == 64 ? (long) blockIdx.x * 4 + (threadIdx.x >> 6) : (long) blockIdx.x;
+    const long row = (long) blockIdx.x * (256 / TPR) + threadIdx.x / TPR;
     if (row >= rows) return;
     const raw* x = reinterpret_cast<const raw*>(X) + row * cols;
     raw* y = reinterpret_cast<raw*>(Y) + row * cols;
@@ -222,7 +229,8 @@ __device__ __forceinline__ void layernorm_slice_apply(long cols, long chunk, flo
 } // namespace docc_k
 
 #define DOCC_LN_ARGS long rows, long cols, float eps, const void *X, const void *W, const void *B, void *Y
-// docc_layernorm_<type>_<v|s>_<w|b><NV>: vectors or single elements, a wavefront or a work-group a row
+// docc_layernorm_<type>_<v|s>_<w|b><NV>: vectors or single elements, a wavefront or a work-group a row; _p<lanes>: that many lanes a row, with one
+// vector or four elements each
 #define DOCC_LN(TYPE, T, VTAG, V, RTAG, TPR, NV)                                                                             \
     extern "C" __global__ __launch_bounds__(256) void docc_layernorm_##TYPE##_##VTAG##_##RTAG##NV(DOCC_LN_ARGS) {             \
         docc_k::layernorm_row<T, V, NV, TPR>(rows, cols, eps, X, W, B, Y);                                                   \
@@ -240,7 +248,20 @@ __device__ __forceinline__ void layernorm_slice_apply(long cols, long chunk, flo
         long cols, long chunk, float eps, const void* X, const float* sums, const float* squares, const void* W, const void* B, void* Y) {              \
         docc_k::layernorm_slice_apply<T, V>(cols, chunk, eps, X, sums, squares, W, B, Y);                                     \
     }
+#define DOCC_LN_SHORT(TYPE, T, VTAG, V, NV, TPR)                                                                             \
+    extern "C" __global__ __launch_bounds__(256) void docc_layernorm_##TYPE##_##VTAG##_p##TPR(DOCC_LN_ARGS) {                 \
+        docc_k::layernorm_row<T, V, NV, TPR>(rows, cols, eps, X, W, B, Y);                                                   \
+    }
+#define DOCC_LN_SHORTS(TYPE, T, VTAG, V, NV)  \
+    DOCC_LN_SHORT(TYPE, T, VTAG, V, NV, 1)    \
+    DOCC_LN_SHORT(TYPE, T, VTAG, V, NV, 2)    \
+    DOCC_LN_SHORT(TYPE, T, VTAG, V, NV, 4)    \
+    DOCC_LN_SHORT(TYPE, T, VTAG, V, NV, 8)    \
+    DOCC_LN_SHORT(TYPE, T, VTAG, V, NV, 16)   \
+    DOCC_LN_SHORT(TYPE, T, VTAG, V, NV, 32)
 #define DOCC_LN_TYPE(TYPE, T, V)           \
+    DOCC_LN_SHORTS(TYPE, T, v, V, 1)         \
+    DOCC_LN_SHORTS(TYPE, T, s, 1, 4)         \
     DOCC_LN_SLICE(TYPE, T, v, V)             \
     DOCC_LN_SLICE(TYPE, T, s, 1)             \
     DOCC_LN(TYPE, T, v, V, w, 64, 1)         \

@@ -29,9 +29,15 @@ extern "C" int docc_rocm_layer_norm(docc_rocm_stream_t stream, int type, int64_t
     // a wavefront a row where that gives every CU its four rows, or where a row is one access of 64 lanes
     const int w = held(64), b = held(256);
     const bool wave = w != 0 && (rows >= 4 * (int64_t) cus || cols <= 64 * lane);
+    // short rows: a power of two of lanes, at most 32, with a vector or four elements each
+    const int64_t wanted = (cols + (vec ? full : 4) - 1) / (vec ? full : 4);
+    int64_t sub = 1;
+    while (sub < wanted && sub < 64) sub *= 2;
+    const bool part = sub <= 32;
     char name[64];
-    const bool one = !wave && !b;   // a work-group of 1024 a row
-    if (one) std::snprintf(name, sizeof(name), "docc_layernorm_%s_long", bf16 ? "bf16" : "f32");
+    const bool one = !part && !wave && !b;   // a work-group of 1024 a row
+    if (part) std::snprintf(name, sizeof(name), "docc_layernorm_%s_%c_p%d", bf16 ? "bf16" : "f32", vec ? 'v' : 's', (int) sub);
+    else if (one) std::snprintf(name, sizeof(name), "docc_layernorm_%s_long", bf16 ? "bf16" : "f32");
     else std::snprintf(name, sizeof(name), "docc_layernorm_%s_%c_%c%d", bf16 ? "bf16" : "f32", vec ? 'v' : 's', wave ? 'w' : 'b', wave ? w : b);
     if (one) {
         // Rows in slices: three launches, from 16384 columns on faster than a work-group a row whatever their number (fp32, rows x columns, a
@@ -61,7 +67,7 @@ extern "C" int docc_rocm_layer_norm(docc_rocm_stream_t stream, int type, int64_t
         }
     }
     // a launch holds fewer than 2^32 threads: more rows than that takes go in several
-    const int64_t threads = one ? 1024 : 256, per_group = wave ? 4 : 1, most = ((int64_t(1) << 32) / threads - 1) * per_group;
+    const int64_t threads = one ? 1024 : 256, per_group = part ? 256 / sub : wave ? 4 : 1, most = ((int64_t(1) << 32) / threads - 1) * per_group;
     const int64_t row_bytes = cols * (bf16 ? 2 : 4);
     for (int64_t r0 = 0; r0 < rows; r0 += most) {
         const int64_t n = rows - r0 < most ? rows - r0 : most;

@@ -144,7 +144,7 @@ def test_activations_of_values_that_are_not_finite(monkeypatch, n, splits):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("rows,cols", [(1100, 256), (6, 250), (6, 2048), (6, 9001), (6, 16384), (6, 20000), (6, 33333)])
+@pytest.mark.parametrize("rows,cols", [(700, 3), (600, 8), (70, 64), (1100, 256), (6, 250), (6, 2048), (6, 9001), (6, 16384), (6, 20000), (6, 33333)])
 def test_layer_norm_in_place_and_with_values_that_are_not_finite(dtype, rows, cols):
     gen = torch.Generator().manual_seed(rows)
     x = torch.randn(rows, cols, generator=gen).to(dtype).cuda()
@@ -166,7 +166,8 @@ def test_layer_norm_in_place_and_with_values_that_are_not_finite(dtype, rows, co
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("rows,cols", [(1, 8), (3, 250), (5, 1000), (1025, 256), (2000, 1024), (8, 2048), (1030, 2048), (7, 4096), (5, 4097), (3, 8192),
+@pytest.mark.parametrize("rows,cols", [(1, 1), (700, 1), (1, 2), (513, 3), (1000, 4), (300, 5), (259, 8), (130, 16), (65, 17), (40, 32), (30, 40), (17, 64), (9, 100), (9, 128),
+                                       (9, 129), (5, 248), (5, 256), (1, 8), (3, 250), (5, 1000), (1025, 256), (2000, 1024), (8, 2048), (1030, 2048), (7, 4096), (5, 4097), (3, 8192),
                                        (2, 16384), (2, 9001)])
 def test_layer_norm_over_row_lengths(dtype, rows, cols):
     gen = torch.Generator().manual_seed(cols)
@@ -191,7 +192,7 @@ def test_layer_norm_of_long_rows_in_slices(monkeypatch, dtype, rows, cols):
     test_layer_norm_over_row_lengths(dtype, rows, cols)
 
 
-@pytest.mark.parametrize("rows,cols", [(1100, 256), (3, 250), (5, 1024), (2, 4096), (3, 4097), (2, 16384), (2, 20000), (3, 33333)])
+@pytest.mark.parametrize("rows,cols", [(700, 3), (700, 4), (300, 8), (200, 24), (90, 50), (60, 128), (1100, 256), (3, 250), (5, 1024), (2, 4096), (3, 4097), (2, 16384), (2, 20000), (3, 33333)])
 def test_layer_norm_divides_by_the_root(rows, cols):
     # small whole numbers whose mean is one too: both sums are exact in fp32 whatever their order, what is left is a division by cols, the
     # root and one division an element, each rounded once

@@ -127,7 +127,7 @@ assert "im2col" in got and "sgemm" in got and "malloc" not in got, got
 """)
 
 
-@pytest.mark.parametrize("rows,cols,launches", [(2 ** 24 + 5, 2000, 2), (2 ** 26 + 1, 64, 2), (2 ** 22, 16384, 2), (2 ** 24 - 1, 2000, 1)])
+@pytest.mark.parametrize("rows,cols,launches", [(2 ** 24 + 5, 2000, 2), (2 ** 26 + 1, 256, 2), (2 ** 32, 4, 2), (2 ** 22, 16384, 2), (2 ** 24 - 1, 2000, 1)])
 def test_layer_norm_of_more_rows_than_a_launch_holds(recorded, rows, cols, launches):
     # 2^32 threads are one too many for a launch (the recorder refuses them as the device does)
     got = recorded(f"""
@@ -234,3 +234,15 @@ else:
     norm()
     assert launches() == got
 """)
+
+
+@pytest.mark.parametrize("cols,form", [(4, "v_p1"), (8, "v_p2"), (24, "v_p8"), (128, "v_p32"), (132, "v_w1"), (3, "s_p1"), (5, "s_p2"), (30, "s_p8"), (127, "s_p32"), (129, "s_w4")])
+def test_layer_norm_of_short_rows(recorded, cols, form):
+    got = recorded(f"""
+rt.call("docc_rocm_layer_norm", 0, 2, 100000, {cols}, 1e-5, A, None, None, B)
+print(take()[0])
+""")
+    assert got[0].split()[1] == "docc_layernorm_f32_" + form
+    if "p" in form:
+        per_group = 256 // int(form.split("p")[1])
+        assert f" {-(-100000 // per_group)},1,1 x 256 " in got[0]
