@@ -45,6 +45,20 @@ __device__ __forceinline__ float ln_row_sum(float v, float* slot) {
     return s;
 }
 
+// a / root, rounded once, without the ten instructions of a division for every element (bf16 4096 x 2048 with them 10.7 us, with a plain product by
+// 1 / root, one rounding more, 8.3; so 8.8): q = a (1 / root) is off by a bit at most, its remainder is exact in a fused multiply-add, and what
+// that adds to q rounds to the quotient (Markstein, 1990). Where the root is far from 1 (an infinity, a NaN or an underflow on the way would not
+// be the quotient's) the caller divides beforehand (`direct`) and the value passes through.
+struct LnQuotient {
+    float root, inv;
+    bool direct;
+    __device__ __forceinline__ explicit LnQuotient(float r) : root(r), inv(1.0f / r), direct(!(r > 0x1p-60f && r < 0x1p60f)) {}
+    __device__ __forceinline__ float operator()(float a) const {
+        const float q = a * inv;
+        return direct ? a : __builtin_fmaf(__builtin_fmaf(-q, root, a), inv, q);
+    }
+};
+
 // NV vectors of V elements a lane, TPR lanes a row; cols <= TPR * NV * V and a multiple of V
 template <typename T, int V, int NV, int TPR>
 __device__ __forceinline__ void layernorm_row(long rows, long cols, float eps, const void* X, const void* W, const void* B, void* Y) {
@@ -89,6 +103,13 @@ __device__ __forceinline__ void layernorm_row(long rows, long cols, float eps, c
             }
         }
     const float root = sqrtf(ln_row_sum<TPR>(sq, slots[1]) / (float) cols + eps);
+    const LnQuotient quotient(root);
+    if (quotient.direct) {
+#pragma unroll
+        for (int i = 0; i < NV; i++)
+#pragma unroll
+            for (int e = 0; e < V; e++) v[i][e] /= root;
+    }
 #pragma unroll
     for (int i = 0; i < NV; i++) {
         const long c = (long) (i * TPR + t) * V;
@@ -98,7 +119,7 @@ __device__ __forceinline__ void layernorm_row(long rows, long cols, float eps, c
         if (B) load(reinterpret_cast<const raw*>(B), c, b);
 #pragma unroll
         for (int e = 0; e < V; e++) {
-            float r = v[i][e] / root;
+            float r = quotient(v[i][e]);
             if (W) r *= w[e];
             if (B) r += b[e];
             v[i][e] = r;
@@ -205,6 +226,7 @@ __device__ __forceinline__ void layernorm_slice_apply(long cols, long chunk, flo
     const float root = sqrtf(ln_parts_sum(squares, slots[1]) / (float) cols + eps);
     raw* y = reinterpret_cast<raw*>(Y) + (long) blockIdx.y * cols;
     const raw *w = reinterpret_cast<const raw*>(W), *b = reinterpret_cast<const raw*>(B);
+    const LnQuotient quotient(root);
     layernorm_slice<T, V>(X, cols, chunk, [&](long c, float (&v)[V]) {
         typename E::vec hw = {}, hb = {}, h;
         if constexpr (V > 1) {
@@ -216,7 +238,8 @@ __device__ __forceinline__ void layernorm_slice_apply(long cols, long chunk, flo
         }
 #pragma unroll
         for (int e = 0; e < V; e++) {
-            float r = (v[e] - mean) / root;
+            const float d = v[e] - mean;
+            float r = quotient.direct ? d / root : quotient(d);
             if (w) r *= E::up(hw[e]);
             if (b) r += E::up(hb[e]);
             h[e] = E::down(r);

@@ -143,6 +143,23 @@ def test_activations_of_values_that_are_not_finite(monkeypatch, n, splits):
         assert torch.allclose(got, want[:, None].expand(-1, n), rtol=1e-6, atol=1e-5, equal_nan=True), (act, got[:, 0], want)
 
 
+@pytest.mark.parametrize("rows,cols", [(700, 4), (1100, 256), (3, 250), (5, 1024), (3, 4097), (2, 20000)])
+def test_layer_norm_of_values_far_from_one(rows, cols):
+    # roots from 0 to infinity, some where the quotient is not formed from the reciprocal; whole numbers times a power of two keep the sums exact
+    gen = torch.Generator().manual_seed(cols)
+    half = torch.randint(1, 8, (rows, cols // 2), generator=gen).float().numpy()
+    x = np.concatenate([half, -half, np.zeros((rows, cols % 2), np.float32)], 1)
+    for scale in (2.0 ** -120, 2.0 ** -66, 2.0 ** -40, 2.0 ** 40, 2.0 ** 62, 2.0 ** 100):
+        d = x * np.float32(scale)
+        dx = torch.from_numpy(d).cuda()
+        y = torch.full_like(dx, 5.0)
+        rt.call("docc_rocm_layer_norm", 0, 2, rows, cols, 0.0, ptr(dx), None, None, ptr(y))
+        torch.cuda.synchronize()
+        with np.errstate(all="ignore"):
+            want = d / np.sqrt(np.square(d).sum(1, keepdims=True) / np.float32(cols))
+        assert np.array_equal(y.cpu().numpy(), want, equal_nan=True), scale
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("rows,cols", [(700, 3), (600, 8), (70, 64), (1100, 256), (6, 250), (6, 2048), (6, 9001), (6, 16384), (6, 20000), (6, 33333)])
 def test_layer_norm_in_place_and_with_values_that_are_not_finite(dtype, rows, cols):
