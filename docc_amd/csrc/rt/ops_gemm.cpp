@@ -518,10 +518,12 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
         // Estimated seconds of the product in `parts` parts on the tile the picker gives that many matrices: the work of
         // the padded tiles at what the tile sustains (relative to the 128 x 256 one) on the share of the CUs that get a
         // work-group, plus writing and reading the parts at 5 TB/s and a second launch.
+        // (the second launch of a bf16 product counts 3.5 us: with 2 us 25 of 274 drawn products were cut that gained a tenth at most or lost, and a
+        // feed-forward block of 3 tokens x 192, which is bound by its launches, took 23.7 us instead of 20.6)
         const double behind = epilogue ? 4e-6 : 0.0;   // bias and activation are a launch of their own then (64 x 192 x 1093 bf16 whole 12 us, in parts 15)
         auto seconds = [&](const TileConfig& c, int64_t parts) {
             if (sizeof(T) == 2)
-                return bgemm_seconds(c, m, n, part_of(parts), tb, parts, cus, lines) + (parts > 1 ? 2.0 * (double) parts * (double) m * (double) n * sizeof(S) / 5e12 + 2e-6 + behind : 0.0);
+                return bgemm_seconds(c, m, n, part_of(parts), tb, parts, cus, lines) + (parts > 1 ? 2.0 * (double) parts * (double) m * (double) n * sizeof(S) / 5e12 + 3.5e-6 + behind : 0.0);
             const double tm = (double) ((m + c.bm - 1) / c.bm), tn = (double) ((n + c.bn - 1) / c.bn);
             const double area = (double) c.bm * c.bn;
             const double rel = area >= 65536 ? 1.03 : area >= 32768 ? 1.0 : area >= 16384 ? 0.97 : 0.75;

@@ -202,7 +202,8 @@ assert take() == ["record 1 on " + f"{b:#x}"]
 @pytest.mark.parametrize("m,n,k,ta,tb,epilogue,kernel", [(1509, 2816, 1032, 0, 0, 0, "128x128x32s4_nn"), (2944, 2912, 688, 0, 0, 1, "128x128x32s4_nn_e"),
                                                          (3064, 1408, 3552, 0, 0, 0, "128x128x32s4_nn"), (4096, 4096, 4096, 0, 0, 0, "256x256x32q4_nn"),
                                                          (4096, 2048, 8192, 0, 1, 0, "128x256x64s3_nt"), (2048, 2048, 2048, 0, 0, 0, "128x128x64s4_nn"),
-                                                         (5352, 3072, 96, 0, 0, 1, "128x128x32s4_nn_e"), (64, 192, 1093, 1, 0, 1, "128x128x32s4_tn_e")])
+                                                         (5352, 3072, 96, 0, 0, 1, "128x128x32s4_nn_e"), (64, 192, 1093, 1, 0, 1, "128x128x32s4_tn_e"),
+                                                         (3, 192, 768, 0, 1, 0, "128x128x32s4_nt"), (512, 256, 2048, 0, 1, 1, "128x128x32s4_nt_e")])
 def test_tiles_of_bf16_products(recorded, m, n, k, ta, tb, epilogue, kernel):
     got = recorded(f"""
 rt.call("docc_rocm_bf16gemm_f32_epilogue", 0, {111 + ta}, {111 + tb}, {m}, {n}, {k}, 1.0, A, {m if ta else k}, B, {k if tb else n}, 0.0, C, {n}, D if {epilogue} else None,
