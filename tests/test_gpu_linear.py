@@ -143,6 +143,31 @@ def test_activations_of_values_that_are_not_finite(monkeypatch, n, splits):
         assert torch.allclose(got, want[:, None].expand(-1, n), rtol=1e-6, atol=1e-5, equal_nan=True), (act, got[:, 0], want)
 
 
+def test_a_captured_layer_norm_in_slices_replays():
+    # its sums are in the stream's buffer, which the program's own calls on that stream use between the replays
+    gen = torch.Generator().manual_seed(1)
+    x, other = (torch.randn(3, 40000, generator=gen).cuda() for _ in range(2))
+    y, z, want = torch.empty_like(x), torch.empty_like(x), torch.empty_like(x)
+    norm = lambda x, y, s: rt.call("docc_rocm_layer_norm", s, 2, 3, 40000, 1e-5, ptr(x), None, None, ptr(y))
+    norm(x, want, 0)
+    torch.cuda.synchronize()
+    s = rt.stream_create()
+    try:
+        norm(other, z, s)
+        with rt.Graph.capture(s) as graph:
+            norm(x, y, s)
+        for _ in range(3):
+            y.fill_(float("nan"))
+            torch.cuda.synchronize()
+            graph.launch()
+            norm(other, z, s)
+            rt.stream_sync(s)
+            assert torch.equal(y, want)
+        graph.destroy()
+    finally:
+        rt.stream_destroy(s)
+
+
 @pytest.mark.parametrize("rows,cols", [(700, 4), (1100, 256), (3, 250), (5, 1024), (3, 4097), (2, 20000)])
 def test_layer_norm_of_values_far_from_one(rows, cols):
     # roots from 0 to infinity, some where the quotient is not formed from the reciprocal; whole numbers times a power of two keep the sums exact
