@@ -52,6 +52,47 @@ double bgemm_seconds(const TileConfig& c, int64_t m, int64_t n, int64_t k, bool 
     return 1e-6 * (4.0 + rounds * (fill + area * (11.0 / 65536) + area * (double) k * 3.6e-7 / rel));
 }
 
+// The same for an fp32 or fp64 product (`k`: of all its `parts` together): the work of the padded tiles at what the tile sustains (relative to the
+// 128 x 256 one), on the share of the CUs' time that does work: below one work-group per CU the CUs that get one, above it the whole
+// rounds (344 work-groups on 256 CUs take as long as 512).
+double sdgemm_seconds(const TileConfig& c, int64_t m, int64_t n, int64_t k, int64_t parts, int cus, size_t elem) {
+    const double tm = (double) ((m + c.bm - 1) / c.bm), tn = (double) ((n + c.bn - 1) / c.bn);
+    const double area = (double) c.bm * c.bn, rel = area >= 65536 ? 1.03 : area >= 32768 ? 1.0 : area >= 16384 ? 0.97 : 0.75;
+    const double per_cu = tm * tn * (double) parts / cus, fill = per_cu < 1.0 ? per_cu : per_cu / (double) (int64_t) (per_cu + 0.999999);
+    return 2.0 * tm * c.bm * tn * c.bn * (double) k / ((elem == 8 ? 68e12 : 141e12) * rel * fill);
+}
+
+using Picker = TileConfig (*)(int64_t m, int64_t n, int64_t k, bool tb, int64_t batch, int aligned, int force, int cus);
+
+constexpr int64_t kMaxPartsBytes = int64_t(64) << 20;   // of the parts of a product whose K is cut
+constexpr int64_t kPartCounts[] = {2, 3, 4, 5, 6, 8, 10, 12, 16, 20, 24, 32, 48, 64};
+// k of a part: whole steps of 64 of every tile; the last part takes what is left
+int64_t part_length(int64_t k, int64_t parts) { return ((k + parts - 1) / parts + 63) / 64 * 64; }
+
+// ... and with K in the best number of parts, as gemm_launch cuts it (below)
+double sdgemm_best_seconds(Picker pick, int64_t m, int64_t n, int64_t k, bool tb, int cus, size_t elem) {
+    const TileConfig whole = pick(m, n, k, tb, 1, 2, 0, cus);
+    double best = sdgemm_seconds(whole, m, n, k, 1, cus, elem);
+    if (k < 512 || ((m + whole.bm - 1) / whole.bm) * ((n + whole.bn - 1) / whole.bn) >= cus) return best;
+    for (const int64_t parts : kPartCounts) {
+        const int64_t part = part_length(k, parts), bytes = parts * m * n * (int64_t) elem;
+        if ((k + part - 1) / part != parts || part < 256 || bytes > kMaxPartsBytes) continue;
+        const double t = sdgemm_seconds(pick(m, n, part, tb, parts, 2, 0, cus), m, n, k, parts, cus, elem) + 2.0 * (double) bytes / 5e12 + 3e-6;
+        if (t < best) best = t;
+    }
+    return best;
+}
+
+// Microseconds of an fp32 or fp64 product on the element-wise tiles (operands off the vectors): a round of tiles over the CUs takes so long per k.
+// `turned`: an operand is read along m or n.
+double plain_us(Picker pick, int64_t m, int64_t n, int64_t k, bool tb, bool turned, int cus, size_t elem) {
+    const TileConfig c = pick(m, n, k, tb, 1, 0, 0, cus);
+    const int64_t tiles = ((m + c.bm - 1) / c.bm) * ((n + c.bn - 1) / c.bn), rounds = (tiles + cus - 1) / cus;
+    const double first = elem == 8 ? (turned ? 0.006 : 0.008) : c.bm == 64 ? (turned ? 0.015 : 0.0045) : turned ? 0.0 : 0.01;
+    const double each = elem == 8 ? (turned ? 0.036 : 0.0345) : c.bm == 64 ? (turned ? 0.0172 : 0.0165) : turned ? 0.08 : 0.065;
+    return 5.0 + (double) k * (first + each * (double) rounds);
+}
+
 // the number of CUs, asked for once per call of an entry point: a product with fewer tiles than CUs weighs up to 60 forms by it
 int cu_count() {
     const int cus = compute_units();
@@ -227,7 +268,7 @@ int gemv_launch(const char* prefix, hipStream_t s, bool ta, bool tb, int64_t m, 
 template <typename T, typename S = T>
 int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int trans_b, int64_t m, int64_t n,
                 int64_t k, S alpha, const T* A, int64_t lda, const T* B, int64_t ldb, S beta, S* C, int64_t ldc,
-                TileConfig (*pick)(int64_t m, int64_t n, int64_t k, bool tb, int64_t batch, int aligned, int force, int cus), const S* bias = nullptr,
+                Picker pick, const S* bias = nullptr,
                 int activation = -1, int64_t batch = 1, int64_t batch_a = 0, int64_t batch_b = 0, int64_t batch_c = 0,
                 const LinearFinish* fin = nullptr, int64_t k_total = 0) {
     if ((trans_a != DOCC_ROCM_NO_TRANS && trans_a != DOCC_ROCM_TRANS) ||
@@ -432,9 +473,10 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
     // off, both of them where k itself is no whole number of vectors. That costs a launch of 4-5 us and reading and writing the operands
     // once; the element-wise tiles sustain a tenth (bf16 read along m or n) to nine tenths (fp64) of the others' rate, and wait for every
     // step of a long k. Measured, k one off the vector: bf16 4096^3 649-1195 us plain against 134-208 packed, 512^3 13-27 against 12;
-    // fp32 2048^3 190-310 against 148-272, 512^3 read along n 23.6 against 15.8, otherwise 15.3 against 15.2, 3000 x 500 x 300 16-19
-    // against 21 (few steps, enough tiles: plain); fp64 2048^3 read along n 365 against 329, otherwise 279 against 286 (plain), 512^3 25
-    // against 20, 128 x 2048 x 8192 362 against 135. DOCC_ROCM_GEMM_PACK=0 switches it off, =1 packs whatever the size (tests, tuning).
+    // fp32 2048^3 190-310 against 148-272, 2800 x 517 x 3565 194 against 139, but 5120 x 2304 x 1391 312 against 359 (360 tiles: two
+    // rounds); fp64 6537 x 5561 x 221 289 against 329, 915 x 1581 x 3707 272 against 204. fp32 and fp64 weigh both forms in rounds over the CUs: of 220
+    // drawn products 6 are more than 5 % slower than plain (33 by the rates alone), in the mean 0.8 % off the better form (2.7 %).
+    // DOCC_ROCM_GEMM_PACK=0 switches it off, =1 packs whatever the size (tests, tuning).
     const char* pack_env = tuning("DOCC_ROCM_GEMM_PACK");
     if (!aligned && batch == 1 && !(pack_env && pack_env[0] == '0')) {
         const int64_t v = (int64_t) vec;
@@ -445,15 +487,18 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
         const double work = (double) m * (double) n * (double) k;
         const int64_t kp = pack_a && pack_b ? (k + 63) / 64 * 64 : k;
         const int64_t bytes_a = pack_a ? m * kp * (int64_t) sizeof(T) : 0, bytes_b = pack_b ? n * kp * (int64_t) sizeof(T) : 0;
-        // the plain tiles: the chain of K-steps of one tile, or all of them at the rate they sustain; against the copies and the rate of the
-        // asynchronous ones (flop per us)
-        const double step_us = sizeof(T) == 2 ? (turned ? 2.3 : 0.95) : sizeof(T) == 4 ? (turned ? 0.58 : 0.31) : turned ? 0.7 : 0.63;
-        const double plain_rate = sizeof(T) == 2 ? (turned ? 1.2e8 : 4.2e8) : sizeof(T) == 4 ? 1.0e8 : turned ? 4.8e7 : 6.2e7;
-        const double packed_rate = sizeof(T) == 2 ? 1.1e9 : sizeof(T) == 4 ? 1.4e8 : 6.6e7;
-        const double chain_us = step_us * (double) k / (sizeof(T) == 2 ? 64 : 16), all_us = 2.0 * work / plain_rate;
-        // (below k = 192 both are bound by storing C)
-        bool pays = (chain_us > 14.0 || k >= 192) && 5.0 + (chain_us > all_us ? chain_us : all_us) >
-                                                         14.0 + 2e-6 / 4.0 * (double) (bytes_a + bytes_b) + 2.0 * work / packed_rate;
+        bool pays = false;
+        if (sizeof(T) == 2) {
+            // the plain tiles: the chain of K-steps of one tile, or all of them at the rate they sustain; against the copies and the rate of
+            // the asynchronous ones (flop per us)
+            const double chain_us = (turned ? 2.3 : 0.95) * (double) k / 64, all_us = 2.0 * work / (turned ? 1.2e8 : 4.2e8);
+            // (below k = 192 both are bound by storing C)
+            pays = (chain_us > 14.0 || k >= 192) &&
+                   5.0 + (chain_us > all_us ? chain_us : all_us) > 14.0 + 2e-6 / 4.0 * (double) (bytes_a + bytes_b) + 2.0 * work / 1.1e9;
+        } else {
+            pays = k >= 192 && plain_us(pick, m, n, k, tb, turned, cus, sizeof(T)) >
+                                   8.0 + 0.9e-7 * (double) (bytes_a + bytes_b) + 1e6 * sdgemm_best_seconds(pick, m, n, kp, pack_b || tb, cus, sizeof(T));
+        }
         if (pack_env && pack_env[0] == '1') pays = true;
         const int64_t tiles_k = (kp + 63) / 64;
         const int64_t groups_a = pack_a ? (m + 63) / 64 * tiles_k : 0, groups_b = pack_b ? (n + 63) / 64 * tiles_k : 0;
@@ -508,31 +553,21 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
         const char* env = tuning("DOCC_ROCM_GEMM_SPLITK");
         // the parts' products: in the stream's buffer of partial results where they fit, else in a block of the device
         // block cache (taken and returned in stream order), up to 64 MiB; in a capture that keeps no blocks only in a buffer that is there
-        const int64_t kMaxPartBytes = !foreign_capture(s) ? int64_t(64) << 20 : partials_held(s) ? (int64_t) kPartialsBytes : 0;
-        // k of a part: whole steps of 64 of every tile; the last part takes what is left
-        auto part_of = [&](int64_t parts) { return ((k + parts - 1) / parts + 63) / 64 * 64; };
+        const int64_t max_bytes = !foreign_capture(s) ? kMaxPartsBytes : partials_held(s) ? (int64_t) kPartialsBytes : 0;
+        auto part_of = [&](int64_t parts) { return part_length(k, parts); };
         auto allowed = [&](int64_t parts) {
             const int64_t part = part_of(parts);
-            return parts <= 64 && (k + part - 1) / part == parts && part >= 256 && parts * m * n * (int64_t) sizeof(S) <= kMaxPartBytes;
+            return parts <= 64 && (k + part - 1) / part == parts && part >= 256 && parts * m * n * (int64_t) sizeof(S) <= max_bytes;
         };
-        // Estimated seconds of the product in `parts` parts on the tile the picker gives that many matrices: the work of
-        // the padded tiles at what the tile sustains (relative to the 128 x 256 one) on the share of the CUs that get a
-        // work-group, plus writing and reading the parts at 5 TB/s and a second launch.
+        // Estimated seconds of the product in `parts` parts on the tile the picker gives that many matrices, plus writing and reading the
+        // parts at 5 TB/s and a second launch.
         // (the second launch of a bf16 product counts 3.5 us: with 2 us 25 of 274 drawn products were cut that gained a tenth at most or lost, and a
         // feed-forward block of 3 tokens x 192, which is bound by its launches, took 23.7 us instead of 20.6)
         const double behind = epilogue ? 4e-6 : 0.0;   // bias and activation are a launch of their own then (64 x 192 x 1093 bf16 whole 12 us, in parts 15)
         auto seconds = [&](const TileConfig& c, int64_t parts) {
             if (sizeof(T) == 2)
                 return bgemm_seconds(c, m, n, part_of(parts), tb, parts, cus, lines) + (parts > 1 ? 2.0 * (double) parts * (double) m * (double) n * sizeof(S) / 5e12 + 3.5e-6 + behind : 0.0);
-            const double tm = (double) ((m + c.bm - 1) / c.bm), tn = (double) ((n + c.bn - 1) / c.bn);
-            const double area = (double) c.bm * c.bn;
-            const double rel = area >= 65536 ? 1.03 : area >= 32768 ? 1.0 : area >= 16384 ? 0.97 : 0.75;
-            // the share of the CUs' time that does work: below one work-group per CU the CUs that get one, above it the
-            // whole rounds (344 work-groups on 256 CUs take as long as 512)
-            const double per_cu = tm * tn * (double) parts / cus;
-            const double fill = per_cu < 1.0 ? per_cu : per_cu / (double) (int64_t) (per_cu + 0.999999);
-            const double rate = sizeof(T) == 8 ? 68e12 : 141e12;
-            double t = 2.0 * tm * c.bm * tn * c.bn * (double) k / (rate * rel * fill);
+            double t = sdgemm_seconds(c, m, n, k, parts, cus, sizeof(T));
             if (parts > 1) t += 2.0 * (double) parts * (double) m * (double) n * sizeof(S) / 5e12 + 3e-6 + behind;
             return t;
         };
@@ -542,7 +577,7 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
             while (splits * 2 <= wanted && allowed(splits * 2)) splits *= 2;
         } else if (tiles < cus) {   // CUs without a work-group: the case parts are for
             double best = seconds(cfg, 1);
-            for (int64_t parts : {2, 3, 4, 5, 6, 8, 10, 12, 16, 20, 24, 32, 48, 64}) {
+            for (const int64_t parts : kPartCounts) {
                 if (!allowed(parts)) continue;
                 const TileConfig c = pick(m, n, part_of(parts), tb, parts, aligned, 0, cus);
                 if (c.stages == 0) break;
@@ -623,7 +658,7 @@ template <typename T, typename S>
 static int gemm_batched(const char* prefix, docc_rocm_stream_t stream, int trans_a, int trans_b, int64_t m, int64_t n, int64_t k,
                         S alpha, const T* A, int64_t lda, int64_t stride_a, const T* B, int64_t ldb, int64_t stride_b, S beta, S* C,
                         int64_t ldc, int64_t stride_c, int64_t batch,
-                        TileConfig (*pick)(int64_t m, int64_t n, int64_t k, bool tb, int64_t batch, int aligned, int force, int cus)) {
+                        Picker pick) {
     if (batch < 0) return fail(DOCC_ROCM_ERR_INVALID_ARGUMENT, "%s: negative batch", prefix);
     const int64_t kMaxGridY = 65535;
     for (int64_t b0 = 0; b0 < batch; b0 += kMaxGridY) {

@@ -247,3 +247,13 @@ print(take()[0])
     if "p" in form:
         per_group = 256 // int(form.split("p")[1])
         assert f" {-(-100000 // per_group)},1,1 x 256 " in got[0]
+
+
+# k off the vectors: packed where that was measured to be faster, plain where the packed product's tiles end in a nearly empty round
+@pytest.mark.parametrize("m,n,k,packed", [(2048, 2048, 2047, True), (300, 300, 8001, True), (5120, 2304, 1391, False), (3000, 500, 300, False)])
+def test_operands_off_the_vectors_are_packed_where_it_pays(recorded, m, n, k, packed):
+    got = recorded(f"""
+rt.sgemm({m}, {n}, {k}, 1.0, A, {k}, B, {k}, 0.0, C, {n}, trans_b=rt.TRANS)
+print("\\n".join(l for l in take() if l.startswith("launch")))
+""")
+    assert ("docc_gemm_pack_b4" in got[0]) == packed, got
