@@ -2,11 +2,10 @@
 // bf16 rows, fp32 statistics in two steps (the variance from the centred values, as the chain of nodes it stands for computes
 // it). Bound by HBM: X is read once and Y written once, the row stays in registers between the two sums. As separate launches
 // (cast, mean, centre and square, mean, scale) the same work moved X seven times over: [4096, 2048] bf16 in 64 us, five
-// launches, against 12.8 us here. Rows of at most 32 vectors belong to
-// that many lanes of a wavefront (a wavefront each took 226 us for 2^20 rows of 8 fp32, where the nodes took 62; 12.4),
-// rows of a few KB to a wavefront (four rows a work-group, no barrier); longer ones, and rows too few to fill the
-// device that way, to a work-group of 256; rows that do not fit its registers are read three times from L2, by one work-group a row or, from
-// 16384 columns on, in slices.
+// launches, against 10.9 us here. Rows of at most 32 vectors belong to that many lanes of a wavefront (a wavefront each took 226 us
+// for 2^20 rows of 8 fp32, where the nodes took 62; the lanes 12.4), rows of a few KB to a wavefront (four rows a work-group, no barrier);
+// longer ones, and rows too few to fill the device that way, to a work-group of 256; rows that do not fit its registers are read three times
+// from L2, by one work-group a row or, from 16384 columns on, in slices.
 #include "common.h"
 
 namespace docc_k {
