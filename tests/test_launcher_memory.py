@@ -257,3 +257,21 @@ rt.sgemm({m}, {n}, {k}, 1.0, A, {k}, B, {k}, 0.0, C, {n}, trans_b=rt.TRANS)
 print("\\n".join(l for l in take() if l.startswith("launch")))
 """)
     assert ("docc_gemm_pack_b4" in got[0]) == packed, got
+
+
+# the shapes of tests/test_gpu_gemm_pack.py whose K is to be cut into parts of different lengths are cut so
+@pytest.mark.parametrize("kind", ["dgemm", "sgemm", "bf16gemm_f32"])
+def test_k_is_cut_into_parts_of_different_lengths(recorded, kind):
+    from test_gpu_gemm_pack import test_parts_of_different_lengths as cases
+    shapes = next(m for m in cases.pytestmark if m.name == "parametrize" and "m,n,k" in m.args[0]).args[1]
+    for m, n, k in shapes:
+        got = recorded(f"""
+rt.{kind}({m}, {n}, {k}, 1.0, A, {k}, B, {k}, 0.0, C, {n}, trans_b=rt.TRANS)
+print("\\n".join(l for l in take() if l.startswith("launch")))
+""")
+        parts = int(got[0].split()[2].split(",")[1])
+        part = ((k + parts - 1) // parts + 63) // 64 * 64
+        if (kind, m) == ("bf16gemm_f32", 16):
+            assert len(got) == 1            # one tile of 128 x 128, which parts of 256 k do not pay for
+        else:
+            assert parts > 1 and "splitk_combine" in got[1] and k % part, (m, n, k, got)
