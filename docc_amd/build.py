@@ -54,6 +54,7 @@ KERNEL_FAMILIES = {
     "gemm_f32_big_finish": "gemm_f32_big_finish.hip",
     "layernorm": "layernorm.hip",
     "conv2d": "conv2d.hip",
+    "conv_winograd": "conv_winograd.hip",
     "attention": "attention.hip",
     "attention_split": "attention_split.hip",
     "elementwise": "elementwise.hip",
@@ -81,6 +82,7 @@ FAMILY_FLAGS = {
     "gemm_bf16_async_finish": ["-mllvm", "-amdgpu-mfma-vgpr-form=1", "-falign-loops=64"],
     "gemm_f32_finish": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "conv2d": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+    "conv_winograd": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "attention": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "attention_split": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "gemm_skinny": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],

@@ -16,24 +16,10 @@
 // for the next K-step is rebuilt in LDS by BK threads per step, so no thread
 // divides in the inner loop.
 #include "gemm_mfma.h"
+#include "conv_params.h"
 #include <type_traits>
 
 namespace docc_k {
-
-struct ConvParams {
-    const float* X;
-    const float* Wt;
-    const float* bias;
-    float* Y;
-    int N, C, H, W, OC, KH, KW, OH, OW;
-    int stride_h, stride_w, pad_h, pad_w, dil_h, dil_w;
-    // channels of the tensors X and Y lie in: C and OC, or more when the call is one group of a grouped convolution (the
-    // images are then XC and YC channels apart)
-    int XC, YC;
-    // grouped convolution in one launch (the entry points with the suffix _g): blockIdx.z is the group, whose operands lie
-    // these many elements further on. The kernels of a single convolution do not look at them (their registers are full).
-    long GX, GW, GB, GY;
-};
 
 __device__ __forceinline__ void conv_select_group(ConvParams& p) {
     const long g = blockIdx.z;

@@ -1,0 +1,21 @@
+// Operands and extents of a 2-d convolution; must match ConvParams in csrc/rt/ops_conv.cpp.
+#pragma once
+
+namespace docc_k {
+
+struct ConvParams {
+    const float* X;
+    const float* Wt;
+    const float* bias;
+    float* Y;
+    int N, C, H, W, OC, KH, KW, OH, OW;
+    int stride_h, stride_w, pad_h, pad_w, dil_h, dil_w;
+    // channels of the tensors X and Y lie in: C and OC, or more when the call is one group of a grouped convolution (the
+    // images are then XC and YC channels apart)
+    int XC, YC;
+    // grouped convolution in one launch (the entry points with the suffix _g): blockIdx.z is the group, whose operands lie
+    // these many elements further on. The kernels of a single convolution do not look at them (their registers are full).
+    long GX, GW, GB, GY;
+};
+
+} // namespace docc_k

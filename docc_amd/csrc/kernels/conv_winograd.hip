@@ -1,0 +1,362 @@
+// ml::Conv, 2-d NCHW fp32, 3x3 with strides and dilations of one, by Winograd's minimal filtering F(2x2, 3x3)
+// (S. Winograd, Arithmetic Complexity of Computations, 1980; A. Lavin and S. Gray, Fast Algorithms for Convolutional
+// Neural Networks, 2016): a 2x2 tile of outputs is A^T [ sum over channels of (G g G^T) .* (B^T d B) ] A of the 4x4 input pixels d
+// around it, 16 products a channel instead of 36.
+//
+// What bounds the direct form is the fp32 matrix pipe (one work-group of docc_conv2d_f32_halo_* keeps it at two thirds of its peak); the 16
+// sums over the channels are the same matrix product of 16 / 36 of the size, and everything else a tile needs fits beside
+// it: fp32 MFMAs are long (32 cycles the 16x16x4 form), 32 additions and 16 loads a lane are issued under 32 of them.
+//
+// Work-group: 64 * NW threads, 32 output channels x 16 * NW tiles. A wave takes 16 tiles and all 16 components: lane l holds
+// tile l % 16 and channel l / 16 of a step of four channels, which is the B operand of v_mfma_f32_16x16x4_f32, so the
+// transformed input never leaves the registers that it is computed in, and neither do the sums: component by component they
+// lie in the same lane and register, and the output transform is additions of registers. The filters go through LDS: per chunk of eight channels
+// every thread transforms 4 / NW of the 32 x 8 filters and writes their 16 components, quads of components apart, so that a lane reads the A
+// operands of four components with 128 bits; two buffers, one barrier per chunk.
+//
+// The input comes by buffer loads: a row above or below the image (or of a tile beyond the last one) has an offset beyond the buffer's end,
+// for which the load gives 0, and the channel is the scalar offset.
+//
+// What bounds it now is the issue of everything that is no MFMA: such an instruction takes some five cycles of the wave and is only partly hidden
+// by the other wave of the SIMD. Measured on 166 x 256 x 14 x 14 -> 256 (four work-groups a CU): 150 us = 257 TFLOP/s of the direct form's count; the MFMAs
+// alone 124 us, without the filters' way 141, without loading pixels 135. Interleaved one MFMA, two others it took 179 us, the others in one run amid
+// eight MFMAs 164, and with fewer of them (vector loads of a row instead of its pixels, no factors of one half, buffers by constant
+// offsets) the 150. Against the direct form: 32 x 64 x 56 x 56 -> 64 71 -> 48 us, 32 x 256 x 14 x 14 -> 256 92 -> 48.
+//
+// Rounding: the chain of additions has C terms instead of 9 C, which outweighs the transforms' own. Relative error (2-norm) against 64 bits on
+// N(0, 1) images: C = 16 1.5e-7 (direct 2.1e-7), 64 2.6e-7 (4.1e-7), 512 6.8e-7 (1.2e-6); on their positive part 1.3e-7 (1.4e-7), 2.3e-7
+// (2.8e-7), 5.8e-7 (8.1e-7). An output depends on the pixels of its own window alone, as in the direct form, but where
+// products cancel (or a sum of pixels overflows) an infinity can come out as a NaN: outputs that are not finite are computed again, directly.
+#include "elementwise_ops.h"
+#include "conv_params.h"
+#include <type_traits>
+
+namespace docc_k {
+
+typedef float wf4 __attribute__((ext_vector_type(4)));
+
+// Work-groups are dealt to the 8 XCDs in turn: number them so that an XCD gets consecutive ones (whose work shares input).
+__device__ __forceinline__ int xcd_contiguous(int id, int n) {
+    const int xcd = id & 7, q = n >> 3, r = n & 7;
+    return xcd * q + (xcd < r ? xcd : r) + (id >> 3);
+}
+
+// one output the direct way: channels [0, C) of X and Wt as given
+__device__ __forceinline__ float conv3x3_direct(const float* xn, const float* w, int C, int H, int W, int ih0, int iw0) {
+    float sum = 0.f;
+    for (int c = 0; c < C; c++)
+        for (int t = 0; t < 9; t++) {
+            const int ih = ih0 + t / 3, iw = iw0 + t % 3;
+            const bool in = ih >= 0 && ih < H && iw >= 0 && iw < W;
+            // (a tap in the padding multiplies a zero, as in the other forms: an infinite weight gives a NaN there)
+            sum = __builtin_fmaf(w[c * 9 + t], in ? xn[((long) c * H + ih) * W + iw] : 0.f, sum);
+        }
+    return sum;
+}
+
+// WIDE: a lane loads the four pixels of a row as one vector. Rows then end in whole tiles (OW == W even, pad_w 1), so that only the outer
+// columns can lie in the padding; the vector reads a neighbouring row's pixel there, which is dropped after the row transform. Work-groups
+// with a tile for which that pixel lies outside the tensor load pixel by pixel.
+template <int NW>
+struct ConvWinograd {
+    static constexpr int CI = 8;                   // channels per chunk
+    static constexpr int CS = 4 * 128 + 4;         // floats from one channel's components in LDS to the next's (eight lanes write a channel each: a vector further)
+    static constexpr int STAGE = CI * CS;
+    static constexpr int RAW = 32 * CI * 9;        // filters of a chunk as they lie in memory
+    static constexpr int UT = 4 / NW;                                // filters a thread transforms per chunk
+    static constexpr int WL = (RAW / 4 + 64 * NW - 1) / (64 * NW);   // vectors of them a thread moves
+    static constexpr int LDS_FLOATS = 2 * STAGE + 2 * RAW + 4;
+
+    // channels [c0, c0 + 8 * chunks) of X and Wt; the work-group's tiles from tile0 on, output channels from oc0 on
+    template <bool WIDE>
+    static __device__ __forceinline__ void run(const ConvParams& p, float* lds, int tile0, int oc0, int c0, int chunks) {
+        const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+        const int l16 = lane & 15, lk = lane >> 4;
+        const int TH = (p.OH + 1) >> 1, TW = (p.OW + 1) >> 1, per_image = TH * TW;
+        const int tiles = p.N * per_image;
+
+        // this lane's tile
+        const int tile = tile0 + wave * 16 + l16;
+        const bool tile_ok = tile < tiles;
+        const int n0 = tile0 / per_image;                                    // first image of the work-group
+        const int n = (tile_ok ? tile : tile0) / per_image, rest = (tile_ok ? tile : tile0) % per_image;
+        const int oh = 2 * (rest / TW), ow = 2 * (rest % TW);
+        const int ih0 = oh - p.pad_h, iw0 = ow - p.pad_w;
+        const int HW4 = p.H * p.W * 4;
+
+        // X from image n0 on and the filters from oc0 on, as buffers; the launcher has seen to it that what a work-group addresses takes less
+        // than 2^30 bytes. (X four pixels early: the column before an image's first one has an offset as well.)
+        constexpr int kEarly = 4;
+        const long left = ((long) (p.N - n0) * p.XC * p.H * p.W - (long) c0 * p.H * p.W + kEarly) * 4;
+        const auto xbuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.X) + (((long) n0 * p.XC + c0) * p.H * p.W - kEarly), 0,
+                                                            (int) (left < 0x7fffffffL ? left : 0x7fffffffL), 0x00020000);
+        const long wleft = ((long) (p.OC - oc0) * p.C - c0) * 36;
+        const auto wbuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.Wt) + ((long) oc0 * p.C + c0) * 9, 0,
+                                                            (int) (wleft < 0x7fffffffL ? wleft : 0x7fffffffL), 0x00020000);
+        constexpr int kNone = (int) 0x80000000;      // an offset beyond either
+        const bool first_col = ow == 0, last_col = ow + 2 >= p.OW;
+        int voff[4][WIDE ? 1 : 4];
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+#pragma unroll
+            for (int c = 0; c < (WIDE ? 1 : 4); c++) {
+                const int ih = ih0 + r, iw = iw0 + c;
+                const bool in = tile_ok && ih >= 0 && ih < p.H && (WIDE || (iw >= 0 && iw < p.W));
+                voff[r][c] = in ? ((n - n0) * p.XC * p.H * p.W + (lk * p.H + ih) * p.W + iw + kEarly) * 4 : kNone;
+            }
+        float d[2][4][4];
+        auto xload = [&](int step, int r, int to) {
+            if constexpr (WIDE) {
+                const wf4 x = __builtin_bit_cast(wf4, __builtin_amdgcn_raw_buffer_load_b128(xbuf, voff[r][0], step * 4 * HW4, 0));
+#pragma unroll
+                for (int c = 0; c < 4; c++) d[to][r][c] = x[c];
+            } else {
+#pragma unroll
+                for (int c = 0; c < 4; c++)
+                    d[to][r][c] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xbuf, voff[r][c], step * 4 * HW4, 0));
+            }
+        };
+
+        // The filters' way: vectors of a chunk as they lie in memory ([output channel][channel][tap], 288 bytes of a row) to registers and to
+        // LDS, from there nine values to the thread that transforms them, 16 components back to LDS.
+        float* const raw = lds + 2 * STAGE;
+        int woff[WL];
+        float* wdst[WL];
+#pragma unroll
+        for (int u = 0; u < WL; u++) {
+            const int v = tid + u * 64 * NW, row = v / (CI * 9 / 4);
+            const bool in = v < RAW / 4;
+            woff[u] = in && oc0 + row < p.OC ? (row * p.C * 9 + (v % (CI * 9 / 4)) * 4) * 4 : kNone;
+            wdst[u] = in ? raw + v * 4 : raw + 2 * RAW;        // (surplus threads of the last round: a spare vector)
+        }
+        wf4 wr[WL];
+        auto wload = [&](int chunk) {
+#pragma unroll
+            for (int u = 0; u < WL; u++) wr[u] = __builtin_bit_cast(wf4, __builtin_amdgcn_raw_buffer_load_b128(wbuf, woff[u], chunk * (CI * 36), 0));
+        };
+        auto wraw = [&](int buf, int u) {
+            const bool spare = (u + 1) * 64 * NW > RAW / 4;    // the round with surplus threads: their vector is not moved between the buffers
+            *reinterpret_cast<wf4*>(wdst[u] + (spare && buf && tid + u * 64 * NW >= RAW / 4 ? 0 : buf * RAW)) = wr[u];
+        };
+        const int uc = tid & 7, uo = tid >> 3;
+        float g[UT][9];
+        const float* const gsrc = raw + uo * (CI * 9) + uc * 9;
+        auto gread = [&](int buf) {
+#pragma unroll
+            for (int u = 0; u < UT; u++)
+#pragma unroll
+                for (int t = 0; t < 9; t++) g[u][t] = gsrc[buf * RAW + u * 8 * NW * (CI * 9) + t];
+        };
+        // The filters are left without the factors of one half that G has in its middle rows: the output transform applies them.
+        float* const udst = lds + uc * CS + uo * 4;
+        auto ustage = [&](int buf, int i) {      // row i of the components
+#pragma unroll
+            for (int u = 0; u < UT; u++) {
+                float h[3];
+#pragma unroll
+                for (int c = 0; c < 3; c++) {
+                    const float a = g[u][c], b = g[u][3 + c], e = g[u][6 + c];
+                    h[c] = i == 0 ? a : i == 3 ? e : i == 1 ? (a + e) + b : (a + e) - b;
+                }
+                const float s = h[0] + h[2];
+                *reinterpret_cast<wf4*>(udst + buf * STAGE + u * 32 * NW + i * 128) = wf4{h[0], s + h[1], s - h[1], h[2]};
+            }
+        };
+
+        wf4 acc[16][2];
+        const float* const ulane = lds + lk * CS + l16 * 4;
+        wf4 a[2][2];
+        auto aread = [&](int buf, int half, int i, int to) {
+#pragma unroll
+            for (int o = 0; o < 2; o++) a[to][o] = *reinterpret_cast<const wf4*>(ulane + buf * STAGE + half * (4 * CS) + i * 128 + o * 64);
+        };
+        // the transformed pixels of row i of the components
+        float v[2][4];
+        auto vrow = [&](float (&x)[4][4], int i) {
+            float t[4];
+#pragma unroll
+            for (int c = 0; c < 4; c++) t[c] = i == 0 ? x[0][c] - x[2][c] : i == 1 ? x[1][c] + x[2][c] : i == 2 ? x[2][c] - x[1][c] : x[1][c] - x[3][c];
+            if constexpr (WIDE) {
+                t[0] = first_col ? 0.f : t[0];
+                t[3] = last_col ? 0.f : t[3];
+            }
+            v[i & 1][0] = t[0] - t[2], v[i & 1][1] = t[1] + t[2], v[i & 1][2] = t[2] - t[1], v[i & 1][3] = t[1] - t[3];
+        };
+        auto mfmas = [&](int i) {
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+#pragma unroll
+                for (int o = 0; o < 2; o++) acc[4 * i + j][o] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i & 1][o][j], v[i & 1][j], acc[4 * i + j][o], 0, 0, 0);
+        };
+        // Each row of components is a scheduling region: its eight MFMAs, between them the operands of the next row (filters from LDS,
+        // pixels transformed), the loads that refill the pixel registers freed by the row before, and filters.
+        auto shape = [&]() {
+            __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);     // LDS reads
+            __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);     // MFMA
+            __builtin_amdgcn_sched_group_barrier(0x020, 16, 0);    // loads
+            __builtin_amdgcn_sched_group_barrier(0x002, 40, 0);    // VALU
+            __builtin_amdgcn_sched_group_barrier(0x200, 4, 0);     // LDS writes
+            __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+
+        // chunk 0's filters all the way, chunk 1's as far as the registers, chunk 2's on their way
+        const int last = chunks - 1;
+        wload(0);
+#pragma unroll
+        for (int r = 0; r < 4; r++) xload(0, r, 0);
+#pragma unroll
+        for (int r = 0; r < 4; r++) xload(1, r, 1);
+#pragma unroll
+        for (int u = 0; u < WL; u++) wraw(0, u);
+        wload(last < 1 ? last : 1);
+        __syncthreads();
+        gread(0);
+#pragma unroll
+        for (int u = 0; u < WL; u++) wraw(1, u);
+        wload(last < 2 ? last : 2);
+#pragma unroll
+        for (int i = 0; i < 4; i++) ustage(0, i);
+        vrow(d[0], 0);
+        __syncthreads();
+        gread(1);
+        aread(0, 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int q = 0; q < 16; q++)
+#pragma unroll
+            for (int o = 0; o < 2; o++) acc[q][o] = wf4{0.f, 0.f, 0.f, 0.f};
+        // In chunk ch the filters of ch + 1 are transformed into the other buffer, those of ch + 2 written to LDS as they are, those of ch + 3
+        // loaded. The barrier stands before the last row of a chunk, whose operands are in registers by then: the first ones of the next
+        // chunk are read under it. (The last chunks load and stage once more what nobody reads.)
+        auto chunk = [&](int ch, auto buf_c) {
+            constexpr int buf = decltype(buf_c)::value;
+            const int s2 = ch < last ? 2 * ch + 2 : 2 * ch, s3 = s2 + 1, w3 = ch + 3 < last ? ch + 3 : last;
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                aread(buf, (i + 1) >> 2, (i + 1) & 3, (i + 1) & 1);
+                ustage(buf ^ 1, i);
+                if (i < 3) vrow(d[0], i + 1);
+                else vrow(d[1], 0);
+                if (i == 0) xload(s2, 0, 0);
+                if (i == 2) xload(s2, 2, 0);
+                if (i == 3) xload(s2, 1, 0);
+                mfmas(i);
+                shape();
+            }
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                if (i == 3) {
+                    __syncthreads();
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                if (i < 3) aread(buf, 1, i + 1, (i + 1) & 1);
+                else aread(buf ^ 1, 0, 0, 0);
+                if (i < 3) vrow(d[1], i + 1);
+                else vrow(d[0], 0);
+                if (i == 0) {
+                    xload(s2, 3, 0);
+                    xload(s3, 0, 1);
+                }
+                if (i == 1) {
+#pragma unroll
+                    for (int u = 0; u < WL; u++) wraw(buf, u);
+                    wload(w3);
+                }
+                if (i == 2) xload(s3, 2, 1);
+                if (i == 3) {
+                    xload(s3, 1, 1);
+                    xload(s3, 3, 1);
+                    gread(buf);
+                }
+                mfmas(i);
+                shape();
+            }
+        };
+        int ch = 0;
+        for (; ch + 1 < chunks; ch += 2) {
+            chunk(ch, std::integral_constant<int, 0>{});
+            chunk(ch + 1, std::integral_constant<int, 1>{});
+        }
+        if (ch < chunks) chunk(ch, std::integral_constant<int, 0>{});
+
+        // outputs: rows of A^T = (1 1 1 0), (0 1 -1 -1) on both sides, the middle components halved
+        if (!tile_ok) return;
+        const long plane = (long) p.OH * p.OW;
+        const bool right = ow + 1 < p.OW, below = oh + 1 < p.OH;
+        const bool pairs = (p.OW & 1) == 0 && ((uintptr_t) p.Y & 7) == 0;
+        float* const ytile = p.Y + ((long) n * p.YC) * plane + (long) oh * p.OW + ow;
+        float bias[2][4];
+#pragma unroll
+        for (int o = 0; o < 2; o++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int oc = oc0 + o * 16 + 4 * lk + r;
+                bias[o][r] = p.bias ? p.bias[oc < p.OC ? oc : p.OC - 1] : -0.f;
+            }
+        unsigned again = 0;      // outputs that are not finite: bit 16 * o + 4 * r + 2 * row + column
+        auto outputs = [&](auto fast_c) {
+            constexpr bool FAST = decltype(fast_c)::value;
+#pragma unroll
+            for (int o = 0; o < 2; o++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const int oc = oc0 + o * 16 + 4 * lk + r;
+                    float s[2][4];
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        const float m1 = acc[4 + j][o][r], m2 = acc[8 + j][o][r];
+                        s[0][j] = __builtin_fmaf(0.5f, m1 + m2, acc[j][o][r]);
+                        s[1][j] = __builtin_fmaf(0.5f, m1 - m2, -acc[12 + j][o][r]);
+                    }
+                    float* y = ytile + oc * plane;
+#pragma unroll
+                    for (int i = 0; i < 2; i++) {
+                        const float y0 = __builtin_fmaf(0.5f, s[i][1] + s[i][2], s[i][0]) + bias[o][r], y1 = __builtin_fmaf(0.5f, s[i][1] - s[i][2], -s[i][3]) + bias[o][r];
+                        again |= (__builtin_fabsf(y0) < __builtin_inff() ? 0u : 1u) << (16 * o + 4 * r + 2 * i);
+                        again |= (__builtin_fabsf(y1) < __builtin_inff() ? 0u : 2u) << (16 * o + 4 * r + 2 * i);
+                        if constexpr (FAST) {
+                            typedef float f2 __attribute__((ext_vector_type(2)));
+                            *reinterpret_cast<f2*>(y + i * p.OW) = f2{y0, y1};
+                        } else if (oc < p.OC && (i == 0 || below)) {
+                            y[i * p.OW] = y0;
+                            if (right) y[i * p.OW + 1] = y1;
+                        }
+                    }
+                }
+        };
+        if (pairs && oc0 + 32 <= p.OC && (p.OH & 1) == 0) outputs(std::integral_constant<bool, true>{});
+        else outputs(std::integral_constant<bool, false>{});
+        while (again) {
+            const int bit = __builtin_ctz(again);
+            again &= again - 1;
+            const int oc = oc0 + (bit >> 4) * 16 + 4 * lk + ((bit >> 2) & 3), i = (bit >> 1) & 1, j = bit & 1;
+            if (oc >= p.OC || oh + i >= p.OH || ow + j >= p.OW) continue;
+            const float sum = conv3x3_direct(p.X + ((long) n * p.XC + c0) * p.H * p.W, p.Wt + ((long) oc * p.C + c0) * 9, chunks * CI, p.H, p.W, ih0 + i, iw0 + j);
+            ytile[oc * plane + (long) i * p.OW + j] = sum + (p.bias ? p.bias[oc] : 0.f);
+        }
+    }
+};
+
+} // namespace docc_k
+
+namespace docc_k {
+template <int NW, bool WIDE>
+__device__ __forceinline__ void conv_winograd(const ConvParams& p) {
+    typedef ConvWinograd<NW> K;
+    __shared__ __attribute__((aligned(16))) float lds[K::LDS_FLOATS];
+    const int ocb = (p.OC + 31) >> 5, id = xcd_contiguous(blockIdx.x, gridDim.x);
+    const int oc0 = (id % ocb) * 32, tile0 = (id / ocb) * (16 * NW);
+    // WIDE: the last tile that reads the column before the first row of the tensor (row 0 of image 0 is among its rows), and the first
+    // that reads the column behind its last row
+    const int TH = (p.OH + 1) >> 1, TW = (p.OW + 1) >> 1;
+    const int before = (p.pad_h >> 1) * TW, bottom = (p.H - 3 + p.pad_h) >> 1;
+    const long behind = (long) (p.N - 1) * TH * TW + (long) (bottom > 0 ? bottom : 0) * TW + TW - 1;
+    if (WIDE && tile0 > before && tile0 + 16 * NW <= behind) K::template run<true>(p, lds, tile0, oc0, 0, p.C / 8);
+    else K::template run<false>(p, lds, tile0, oc0, 0, p.C / 8);
+}
+} // namespace docc_k
+
+extern "C" __global__ __launch_bounds__(256, 2) void docc_conv2d_f32_winograd(docc_k::ConvParams p) { docc_k::conv_winograd<4, false>(p); }
+extern "C" __global__ __launch_bounds__(256, 2) void docc_conv2d_f32_winograd_wide(docc_k::ConvParams p) { docc_k::conv_winograd<4, true>(p); }

@@ -33,6 +33,11 @@ int64_t out_dim(int64_t d_in, int64_t pad_begin, int64_t pad_end, int64_t dil, i
 
 namespace {
 
+constexpr int64_t kWinogradTiles = 64;   // output tiles of 2 x 2 of a work-group of docc_conv2d_f32_winograd, by 32 output channels
+int64_t winograd_groups(int64_t N, int64_t OC, int64_t OH, int64_t OW) {
+    return (N * ((OH + 1) / 2) * ((OW + 1) / 2) + kWinogradTiles - 1) / kWinogradTiles * ((OC + 31) / 32);
+}
+
 constexpr int64_t kConvWorkspaceCap = int64_t(2) << 30;   // images are processed in chunks that fit this
 
 // How a layer runs on the LDS-halo kernel. A work-group takes 64 output channels x a strip of TH full output rows
@@ -198,7 +203,7 @@ double gemm_time_us(int64_t N, int64_t OC, int64_t P, int64_t K, bool needs_colu
 // bytes of columns + GEMM result per image
 int64_t conv_bytes_per_image(int64_t OC, int64_t K, int64_t P) { return (K * P * 4 + 255) / 256 * 256 + (OC * P * 4 + 255) / 256 * 256; }
 
-enum class ConvPath { Halo, Gather, Gemm1x1, GemmColumns };
+enum class ConvPath { Halo, Gather, Gemm1x1, GemmColumns, Winograd };
 
 // shapes the LDS-halo kernel is built for (the launcher also wants 16-byte aligned weights)
 bool halo_shape_ok(int64_t C, int64_t KH, int64_t KW, int64_t OW, int64_t stride_h, int64_t stride_w, int64_t dil_h, int64_t dil_w) {
@@ -206,13 +211,34 @@ bool halo_shape_ok(int64_t C, int64_t KH, int64_t KW, int64_t OW, int64_t stride
            C % 8 == 0 && C > 0 && OW <= 448 && (C * KH * KW) % 4 == 0 && halo_strip_fits(1, OW, KH, KW, stride_h, stride_w);
 }
 
+// Winograd's form (csrc/kernels/conv_winograd.hip): 3x3 filters one pixel apart, whole chunks of eight channels. A work-group addresses its
+// images and filters by 32-bit offsets.
+bool winograd_shape_ok(int64_t N, int64_t C, int64_t H, int64_t W, int64_t OC, int64_t KH, int64_t KW, int64_t OH, int64_t OW, int64_t stride_h, int64_t stride_w,
+                       int64_t pad_h, int64_t pad_w, int64_t dil_h, int64_t dil_w) {
+    if (KH != 3 || KW != 3 || stride_h != 1 || stride_w != 1 || dil_h != 1 || dil_w != 1 || C <= 0 || C % 8 != 0) return false;
+    const int64_t per_image = ((OH + 1) / 2) * ((OW + 1) / 2), images = (kWinogradTiles + per_image - 2) / per_image + 1;
+    return images * C * H * W < (int64_t(1) << 28) && 32 * C * 9 < (int64_t(1) << 28) && N * per_image < (int64_t(1) << 30) &&
+           N * OH * OW * OC < (int64_t(1) << 40) && winograd_groups(N, OC, OH, OW) < (int64_t(1) << 30) && pad_h < (int64_t(1) << 20) && pad_w < (int64_t(1) << 20);
+}
+
+// us: a chunk of eight channels takes a work-group 1.17 of a CU's time where another one fills its gaps and 1.43 alone; 4 us around them.
+// Measured against the other forms on 60 drawn layers (1-64 images, 8-512 channels, 7x7 to 64x64), "before -> now": 8 x 272 x 40 x 40 244 -> 86 us,
+// 32 x 64 x 56 x 56 71 -> 48, 34 x 80 x 24 x 24 53 -> 24, 3 x 32 x 19 x 19 13.1 -> 11.5; 1 x 368 x 9 x 9 is left to the direct form with its channels
+// in parts (18 us; 65 here: 12 work-groups), as is 12 x 416 x 11 x 11 (58; 77).
+double winograd_time_us(int64_t N, int64_t C, int64_t OC, int64_t OH, int64_t OW, int cus) {
+    const int64_t groups = winograd_groups(N, OC, OH, OW), rounds = groups / (2 * cus), rest = groups % (2 * cus);
+    const double chunks = (double) (C / 8), pair = 2 * 1.17 * chunks + 4.0;
+    return (double) rounds * pair + (rest == 0 ? 0.0 : rest <= cus ? 1.43 * chunks + 4.0 : pair);
+}
+
 ConvPath choose_path(int64_t N, int64_t C, int64_t OC, int64_t KH, int64_t KW, int64_t OH, int64_t OW, int64_t stride_h, int64_t stride_w,
-                     int64_t pad_h, int64_t pad_w, bool halo_ok, bool have_workspace, bool parts_ok) {
-    const char* force = std::getenv("DOCC_ROCM_CONV");   // halo | gather | gemm (tuning and tests)
+                     int64_t pad_h, int64_t pad_w, bool halo_ok, bool have_workspace, bool parts_ok, bool winograd_ok) {
+    const char* force = std::getenv("DOCC_ROCM_CONV");   // halo | gather | gemm | winograd (tuning and tests)
     const bool pointwise = KH == 1 && KW == 1 && stride_h == 1 && stride_w == 1 && pad_h == 0 && pad_w == 0;
     const ConvPath gemm = pointwise ? ConvPath::Gemm1x1 : ConvPath::GemmColumns;
     const bool gemm_ok = pointwise || have_workspace;
     if (force && force[0] == 'h' && halo_ok) return ConvPath::Halo;
+    if (force && force[0] == 'w' && winograd_ok) return ConvPath::Winograd;
     if (force && force[0] == 'g' && force[1] == 'a') return ConvPath::Gather;
     if (force && force[0] == 'g' && force[1] == 'e' && gemm_ok) return gemm;
     int cus = compute_units();
@@ -224,7 +250,9 @@ ConvPath choose_path(int64_t N, int64_t C, int64_t OC, int64_t KH, int64_t KW, i
     // wins from 128 input channels on (C 256 -> 64 on 56 x 56: 50 against 65 us; C 64 -> 256: 99 against 74)
     if (pointwise) return gemm_fast && C >= 128 ? gemm : halo_ok ? ConvPath::Halo : ConvPath::Gather;
     const double direct = halo_ok ? halo_time_us(N, parts_ok ? C : 0, OC, OH, OW, KH, KW, stride_h, stride_w, K, cus) : gather_time_us(N, OC, P, K, cus);
-    if (gemm_fast && gemm_time_us(N, OC, P, K, true) < 0.75 * direct) return gemm;
+    const double columns = gemm_fast ? gemm_time_us(N, OC, P, K, true) : 1e30;
+    if (winograd_ok && winograd_time_us(N, C, OC, OH, OW, cus) < 0.95 * ((columns < direct ? columns : direct) + 4.0)) return ConvPath::Winograd;
+    if (columns < 0.75 * direct) return gemm;
     return halo_ok ? ConvPath::Halo : ConvPath::Gather;
 }
 
@@ -242,9 +270,9 @@ extern "C" int64_t docc_rocm_conv2d_f32_pads_workspace_bytes(int64_t N, int64_t 
     pad_w = pad_w > pad_w_end ? pad_w : pad_w_end;
     if (KH == 1 && KW == 1 && stride_h == 1 && stride_w == 1 && pad_h == 0 && pad_w == 0) return 0;   // the input is the column matrix
     // nothing either when one of the direct kernels would be chosen anyway (operands assumed aligned, the channels in one
-    // piece: cutting them takes memory of its own, which the call may not get)
+    // piece: cutting them takes memory of its own, which the call may not get; Winograd's form aside, which a call may be forced off)
     const bool halo_ok = halo_shape_ok(C, KH, KW, OW, stride_h, stride_w, dil_h, dil_w);
-    if (choose_path(N, C, OC, KH, KW, OH, OW, stride_h, stride_w, pad_h, pad_w, halo_ok, true, false) != ConvPath::GemmColumns) return 0;
+    if (choose_path(N, C, OC, KH, KW, OH, OW, stride_h, stride_w, pad_h, pad_w, halo_ok, true, false, false) != ConvPath::GemmColumns) return 0;
     const int64_t per_image = conv_bytes_per_image(OC, C * KH * KW, OH * OW);
     int64_t images = kConvWorkspaceCap / per_image;
     if (images < 1) images = 1;
@@ -292,15 +320,24 @@ static int conv2d_run(docc_rocm_stream_t stream, int64_t N, int64_t C, int64_t H
     // Stride-1, dilation-1 3x3 and 1x1 convolutions take the LDS-halo kernel: 64 output channels x a
     // strip of TH full output rows (at most 448 pixels) per work-group, 8 input channels per chunk.
     const bool halo_shape = halo_shape_ok(C, KH, KW, OW, stride_h, stride_w, dil_h, dil_w) && ((uintptr_t) Wt % 16 == 0);
+    const bool winograd = !slice && winograd_shape_ok(N, C, H, W, OC, KH, KW, OH, OW, stride_h, stride_w, any_pad_h, any_pad_w, dil_h, dil_w);
     const int64_t need = !workspace ? 0 : docc_rocm_conv2d_f32_pads_workspace_bytes(N, C, H, W, OC, KH, KW, stride_h, stride_w, pad_h, pad_w, pad_h_end,
                                                                                     pad_w_end, dil_h, dil_w);
     const bool have_workspace = workspace && workspace_bytes >= need && need > 0 && ((uintptr_t) workspace % 256) == 0;
     const bool parts_ok = !slice && !foreign_capture((hipStream_t) stream);   // cutting the channels takes a block of the cache
     ConvPath path = C == 0 ? ConvPath::Gather
-                           : choose_path(N, C, OC, KH, KW, OH, OW, stride_h, stride_w, any_pad_h, any_pad_w, halo_shape, have_workspace, parts_ok);
+                           : choose_path(N, C, OC, KH, KW, OH, OW, stride_h, stride_w, any_pad_h, any_pad_w, halo_shape, have_workspace, parts_ok,
+                                         winograd);
     // one group of a grouped convolution: the direct kernels, which take the distance between the images as it is (the
     // GEMM paths write whole [N, OC, P] tensors)
     if (slice && (path == ConvPath::Gemm1x1 || path == ConvPath::GemmColumns)) path = halo_shape ? ConvPath::Halo : ConvPath::Gather;
+    if (path == ConvPath::Winograd) {
+        // rows of whole tiles between one column of padding on either side: four pixels a load
+        const char* force = std::getenv("DOCC_ROCM_CONV");
+        const bool wide = any_pad_w == 1 && OW == W && W % 2 == 0 && !(force && std::strstr(force, "-narrow"));
+        return launch(wide ? "docc_conv2d_f32_winograd_wide" : "docc_conv2d_f32_winograd", (uint32_t) winograd_groups(N, OC, OH, OW), 1, 1, 256, 0,
+                      (hipStream_t) stream, p);
+    }
     if (path == ConvPath::Gemm1x1) {
         // Y[n] (OC x P) = W (OC x C) X[n] (C x P): one batched GEMM on the tensors as they lie; the bias is
         // written first and accumulated onto

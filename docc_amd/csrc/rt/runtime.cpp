@@ -52,6 +52,7 @@ const char* const kKernelImages[] = {
     "docc_rocm_gemm_f32_big_finish.hsaco",
     "docc_rocm_layernorm.hsaco",
     "docc_rocm_conv2d.hsaco",
+    "docc_rocm_conv_winograd.hsaco",
     "docc_rocm_attention.hsaco",
     "docc_rocm_attention_split.hsaco",
     "docc_rocm_elementwise.hsaco",

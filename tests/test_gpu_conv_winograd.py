@@ -1,0 +1,87 @@
+"""3x3 convolutions in Winograd's form (csrc/kernels/conv_winograd.hip) against the oracle, forced through DOCC_ROCM_CONV: work-groups of 64 output
+tiles of 2x2 pixels by 32 output channels, chunks of eight input channels.
+
+Tolerance: 1e-5 of the largest value, as for the direct forms; a sum over C channels in fp32 is off by about sqrt(C) ulp (4e-6 at C = 512)."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from gpu_util import dev, host, rel_err_max
+
+pytestmark = pytest.mark.gpu
+
+CASES = [  # N, C, H, W, OC, pads (top, left, bottom, right)
+    (1, 8, 1, 1, 1, (1, 1, 1, 1)),        # one output, one chunk
+    (1, 8, 3, 3, 2, (0, 0, 0, 0)),        # one window, no padding
+    (2, 16, 5, 7, 31, (1, 1, 1, 1)),      # odd extents, a channel short of a block
+    (3, 24, 16, 16, 33, (1, 1, 1, 1)),    # 64 tiles an image: work-groups that begin with an image; three chunks
+    (9, 8, 8, 8, 40, (1, 1, 1, 1)),       # four images a work-group
+    (2, 32, 9, 200, 32, (1, 1, 1, 1)),    # rows of more tiles than a work-group has; odd height (the rows end in the next to last row of tiles)
+    (70, 8, 2, 2, 32, (1, 1, 1, 1)),      # an image a tile
+    (2, 16, 7, 12, 64, (2, 1, 0, 1)),     # padding of two above: the first row is read by two rows of tiles
+    (1, 16, 130, 4, 32, (3, 1, 2, 1)),    # rows of two tiles, three rows of padding
+    (2, 16, 10, 11, 32, (0, 2, 1, 3)),    # columns that are padding alone
+    (4, 64, 14, 14, 96, (1, 1, 1, 1)),
+]
+
+
+def run(rt, X, W, bias, pads):
+    N, C, H, Wd = X.shape
+    OC = W.shape[0]
+    OH, OW = H + pads[0] + pads[2] - 2, Wd + pads[1] + pads[3] - 2
+    y = torch.full((N, OC, OH, OW), float("nan"), device="cuda")
+    x, w = dev(X), dev(W)
+    b = dev(bias) if bias is not None else None
+    rt.conv2d_f32_pads(N, C, H, Wd, OC, 3, 3, (1, 1), pads, (1, 1), x.data_ptr(), w.data_ptr(), b.data_ptr() if b is not None else 0, y.data_ptr())
+    torch.cuda.synchronize()
+    return host(y)
+
+
+def padded_reference(X, W, bias, pads):
+    """The oracle takes the same padding on both sides: the rest is put around the image."""
+    Xp = np.pad(X, ((0, 0), (0, 0), (pads[0], pads[2]), (pads[1], pads[3])))
+    return oracle.conv2d(Xp, W, bias)
+
+
+@pytest.mark.parametrize("force", ["winograd", "winograd-narrow"])
+@pytest.mark.parametrize("case", CASES, ids=[f"n{c[0]}c{c[1]}_{c[2]}x{c[3]}_oc{c[4]}_p{''.join(map(str, c[5]))}" for c in CASES])
+def test_winograd_matches_oracle(rt, monkeypatch, force, case):
+    N, C, H, W, OC, pads = case
+    monkeypatch.setenv("DOCC_ROCM_CONV", force)
+    rng = np.random.default_rng(C + H + W)
+    X = rng.integers(-4, 5, (N, C, H, W)).astype(np.float32)
+    Wt = rng.integers(-4, 5, (OC, C, 3, 3)).astype(np.float32)
+    b = rng.integers(-4, 5, OC).astype(np.float32)
+    # whole numbers: the transforms give multiples of a quarter, nothing rounds
+    assert np.array_equal(run(rt, X, Wt, b, pads), padded_reference(X, Wt, b, pads))
+    X = rng.standard_normal(X.shape).astype(np.float32)
+    Wt = (rng.standard_normal(Wt.shape) * np.sqrt(2.0 / (9 * C))).astype(np.float32)
+    assert rel_err_max(run(rt, X, Wt, None, pads), padded_reference(X, Wt, None, pads)) <= 1e-5
+
+
+@pytest.mark.parametrize("force", ["winograd", "winograd-narrow"])
+def test_values_that_are_not_finite_stay_where_they_are(rt, monkeypatch, force):
+    """Infinities, NaNs and values near the largest (whose sums the input transform overflows) give the direct form's outputs in
+    their windows, and change no output elsewhere."""
+    monkeypatch.setenv("DOCC_ROCM_CONV", force)
+    rng = np.random.default_rng(5)
+    X = rng.standard_normal((6, 16, 10, 10)).astype(np.float32)
+    Wt = (rng.standard_normal((32, 16, 3, 3)) * 0.1).astype(np.float32)
+    clean = oracle.conv2d(X, Wt, None, pad=(1, 1))
+    X[0, 3, 4, 4] = np.inf
+    X[1, 2, 0, 0] = -np.inf
+    X[2, 1, 9, 9] = np.nan
+    X[3, 0, 5, 5], X[3, 0, 5, 6] = np.inf, -np.inf
+    X[4, 7, 4, 4], X[4, 7, 4, 6], X[4, 7, 6, 4] = 3e38, -3e38, 3e38
+    Wt[31, 15, 0, 0] = 0.0
+    with np.errstate(all="ignore"):
+        ref = oracle.conv2d(X, Wt, None, pad=(1, 1))
+    Y = run(rt, X, Wt, None, (1, 1, 1, 1))
+    assert np.array_equal(np.isnan(Y), np.isnan(ref)) and np.array_equal(np.isinf(Y), np.isinf(ref.astype(np.float32)))
+    assert np.array_equal(np.sign(Y[np.isinf(Y)]), np.sign(ref[np.isinf(ref)]))
+    ok = np.isfinite(ref)
+    large = np.abs(ref) > 1e30
+    assert np.abs(Y[large & ok] / ref[large & ok] - 1).max() <= 1e-4
+    small = ok & ~large
+    assert np.abs(Y[small] - ref[small]).max() <= 1e-5 * np.abs(clean).max()
