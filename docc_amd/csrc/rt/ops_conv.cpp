@@ -182,10 +182,6 @@ HaloPlan plan_halo(int64_t N, int64_t C, int64_t OC, int64_t OH, int64_t OW, int
 // tiles fill the CUs evenly. The GEMM on a column matrix runs at
 // about 75 TFLOP/s on these shapes; the columns are written and read once at about 5 TB/s, and the extra launches
 // (columns, bias, transpose) cost about 15 us.
-double halo_time_us(int64_t N, int64_t C, int64_t OC, int64_t OH, int64_t OW, int64_t KH, int64_t KW, int64_t stride_h, int64_t stride_w, int64_t K, int cus) {
-    return plan_halo(N, C, OC, OH, OW, KH, KW, stride_h, stride_w, cus).cost * halo_unit_us(K);
-}
-
 double gather_time_us(int64_t N, int64_t OC, int64_t P, int64_t K, int cus) {
     const int64_t tiles = ((OC + 63) / 64) * ((N * P + 127) / 128);
     const int64_t rounds = (tiles + cus - 1) / cus;
@@ -249,9 +245,13 @@ ConvPath choose_path(int64_t N, int64_t C, int64_t OC, int64_t KH, int64_t KW, i
     // 1x1 layers move more bytes than they compute, which the models above do not see: measured, the batched GEMM
     // wins from 128 input channels on (C 256 -> 64 on 56 x 56: 50 against 65 us; C 64 -> 256: 99 against 74)
     if (pointwise) return gemm_fast && C >= 128 ? gemm : halo_ok ? ConvPath::Halo : ConvPath::Gather;
-    const double direct = halo_ok ? halo_time_us(N, parts_ok ? C : 0, OC, OH, OW, KH, KW, stride_h, stride_w, K, cus) : gather_time_us(N, OC, P, K, cus);
+    const HaloPlan halo = halo_ok ? plan_halo(N, parts_ok ? C : 0, OC, OH, OW, KH, KW, stride_h, stride_w, cus) : HaloPlan{};
+    const double direct = halo_ok ? halo.cost * halo_unit_us(K) : gather_time_us(N, OC, P, K, cus);
     const double columns = gemm_fast ? gemm_time_us(N, OC, P, K, true) : 1e30;
-    if (winograd_ok && winograd_time_us(N, C, OC, OH, OW, cus) < 0.95 * ((columns < direct ? columns : direct) + 4.0)) return ConvPath::Winograd;
+    if (winograd_ok) {
+        const double around = columns < direct || halo.parts == 1 ? 4.0 : 0.0;   // what the other estimates leave out (that of the parts does not)
+        if (winograd_time_us(N, C, OC, OH, OW, cus) < 0.95 * ((columns < direct ? columns : direct) + around)) return ConvPath::Winograd;
+    }
     if (columns < 0.75 * direct) return gemm;
     return halo_ok ? ConvPath::Halo : ConvPath::Gather;
 }
