@@ -917,11 +917,13 @@ DOCC_CONV_PARTS(1, t2, 2, false)
 DOCC_CONV_PARTS(1, t4m, 4, true)
 DOCC_CONV_PARTS(1, t2m, 2, true)
 
-// Y = bias + the parts' sums, in the order of the parts; `total` values, a plane of them per channel. A thread takes four
+namespace docc_k {
+
+// Y = bias + the parts' sums, in the order of the parts, and what the layer has behind that; `total` values, a plane of them per channel. A thread takes four
 // consecutive ones where `total` is a multiple of four (VEC), which may lie in two planes.
 template <int VEC>
-__device__ __forceinline__ void conv_add_parts(const float* __restrict__ sums, const float* __restrict__ bias, float* __restrict__ Y, long total,
-                                               int plane, int OC, int parts) {
+__device__ __forceinline__ void conv_add_parts(const float* __restrict__ sums, const float* __restrict__ bias, float* Y, long total,
+                                               int plane, int OC, int parts, const ConvFinish& fin) {
     typedef float vec_t __attribute__((ext_vector_type(VEC)));
     for (long e = ((long) blockIdx.x * 256 + threadIdx.x) * VEC; e < total; e += (long) gridDim.x * 256 * VEC) {
         vec_t v = *reinterpret_cast<const vec_t*>(sums + e);
@@ -931,16 +933,25 @@ __device__ __forceinline__ void conv_add_parts(const float* __restrict__ sums, c
 #pragma unroll
             for (int i = 0; i < VEC; i++) v[i] += bias[(e + i) / plane % OC];
         }
+        vec_t r;
+#pragma unroll
+        for (int i = 0; i < VEC; i++) r[i] = -0.f;
+        if (fin.residual) r = *reinterpret_cast<const vec_t*>(fin.residual + e);
+#pragma unroll
+        for (int i = 0; i < VEC; i++) v[i] = conv_finished(fin, v[i], r[i]);
         *reinterpret_cast<vec_t*>(Y + e) = v;
     }
 }
+
+} // namespace docc_k
+
 extern "C" __global__ __launch_bounds__(256) void docc_conv2d_add_parts_f32_v4(const float* sums, const float* bias, float* Y, long total, int plane, int OC,
-                                                                              int parts) {
-    conv_add_parts<4>(sums, bias, Y, total, plane, OC, parts);
+                                                                              int parts, docc_k::ConvFinish fin) {
+    docc_k::conv_add_parts<4>(sums, bias, Y, total, plane, OC, parts, fin);
 }
 extern "C" __global__ __launch_bounds__(256) void docc_conv2d_add_parts_f32(const float* sums, const float* bias, float* Y, long total, int plane, int OC,
-                                                                           int parts) {
-    conv_add_parts<1>(sums, bias, Y, total, plane, OC, parts);
+                                                                           int parts, docc_k::ConvFinish fin) {
+    docc_k::conv_add_parts<1>(sums, bias, Y, total, plane, OC, parts, fin);
 }
 
 extern "C" __global__ __launch_bounds__(256) void docc_conv2d_f32_halo_3x3_split(docc_k::ConvParams p, int TH) {

@@ -1,4 +1,4 @@
-// Operands and extents of a 2-d convolution; must match ConvParams in csrc/rt/ops_conv.cpp.
+// Operands and extents of a 2-d convolution; must match ConvParams and ConvFinish in csrc/rt/ops_conv.cpp.
 #pragma once
 
 namespace docc_k {
@@ -17,5 +17,15 @@ struct ConvParams {
     // these many elements further on. The kernels of a single convolution do not look at them (their registers are full).
     long GX, GW, GB, GY;
 };
+
+// The rest of a layer behind a convolution, applied where it is stored: Y = act(convolution + bias + residual).
+struct ConvFinish {
+    const float* residual;   // dense like Y, or null
+    int relu;
+};
+__device__ __forceinline__ float conv_finished(const ConvFinish& f, float v, float residual) {
+    v += residual;           // -0.0 where there is none: no value changes
+    return f.relu ? fmaxf(v, 0.0f) : v;
+}
 
 } // namespace docc_k

@@ -69,7 +69,7 @@ struct ConvWinograd {
 
     // channels [c0, c0 + 8 * chunks) of X and Wt; the work-group's tiles from tile0 on, output channels from oc0 on
     template <bool WIDE>
-    static __device__ __forceinline__ void run(const ConvParams& p, float* lds, int tile0, int oc0, int c0, int chunks) {
+    static __device__ __forceinline__ void run(const ConvParams& p, const ConvFinish& fin, float* lds, int tile0, int oc0, int c0, int chunks) {
         const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
         const int l16 = lane & 15, lk = lane >> 4;
         const int TH = (p.OH + 1) >> 1, TW = (p.OW + 1) >> 1, per_image = TH * TW;
@@ -285,8 +285,10 @@ struct ConvWinograd {
         if (!tile_ok) return;
         const long plane = (long) p.OH * p.OW;
         const bool right = ow + 1 < p.OW, below = oh + 1 < p.OH;
-        const bool pairs = (p.OW & 1) == 0 && ((uintptr_t) p.Y & 7) == 0;
-        float* const ytile = p.Y + ((long) n * p.YC) * plane + (long) oh * p.OW + ow;
+        const bool pairs = (p.OW & 1) == 0 && (((uintptr_t) p.Y | (uintptr_t) fin.residual) & 7) == 0;
+        const long at = ((long) n * p.YC) * plane + (long) oh * p.OW + ow;
+        float* const ytile = p.Y + at;
+        const float* const rtile = fin.residual + at;
         float bias[2][4];
 #pragma unroll
         for (int o = 0; o < 2; o++)
@@ -296,8 +298,28 @@ struct ConvWinograd {
                 bias[o][r] = p.bias ? p.bias[oc < p.OC ? oc : p.OC - 1] : -0.f;
             }
         unsigned again = 0;      // outputs that are not finite: bit 16 * o + 4 * r + 2 * row + column
-        auto outputs = [&](auto fast_c) {
-            constexpr bool FAST = decltype(fast_c)::value;
+        typedef float f2 __attribute__((ext_vector_type(2)));
+        auto outputs = [&](auto fast_c, auto residual_c) {
+            constexpr bool FAST = decltype(fast_c)::value, RESIDUAL = decltype(residual_c)::value;
+            f2 res[2][4][2];         // all of them on their way before the first is needed
+#pragma unroll
+            for (int o = 0; o < 2; o++)
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+#pragma unroll
+                    for (int i = 0; i < 2; i++) {
+                        res[o][r][i] = f2{-0.f, -0.f};
+                        if constexpr (RESIDUAL) {
+                            const int oc = oc0 + o * 16 + 4 * lk + r;
+                            const float* from = rtile + oc * plane + i * p.OW;
+                            if constexpr (FAST) {
+                                res[o][r][i] = *reinterpret_cast<const f2*>(from);
+                            } else if (oc < p.OC && (i == 0 || below)) {
+                                res[o][r][i][0] = from[0];
+                                if (right) res[o][r][i][1] = from[1];
+                            }
+                        }
+                    }
 #pragma unroll
             for (int o = 0; o < 2; o++)
 #pragma unroll
@@ -313,11 +335,11 @@ struct ConvWinograd {
                     float* y = ytile + oc * plane;
 #pragma unroll
                     for (int i = 0; i < 2; i++) {
-                        const float y0 = __builtin_fmaf(0.5f, s[i][1] + s[i][2], s[i][0]) + bias[o][r], y1 = __builtin_fmaf(0.5f, s[i][1] - s[i][2], -s[i][3]) + bias[o][r];
+                        float y0 = __builtin_fmaf(0.5f, s[i][1] + s[i][2], s[i][0]) + bias[o][r], y1 = __builtin_fmaf(0.5f, s[i][1] - s[i][2], -s[i][3]) + bias[o][r];
                         again |= (__builtin_fabsf(y0) < __builtin_inff() ? 0u : 1u) << (16 * o + 4 * r + 2 * i);
                         again |= (__builtin_fabsf(y1) < __builtin_inff() ? 0u : 2u) << (16 * o + 4 * r + 2 * i);
+                        y0 = conv_finished(fin, y0, res[o][r][i][0]), y1 = conv_finished(fin, y1, res[o][r][i][1]);
                         if constexpr (FAST) {
-                            typedef float f2 __attribute__((ext_vector_type(2)));
                             *reinterpret_cast<f2*>(y + i * p.OW) = f2{y0, y1};
                         } else if (oc < p.OC && (i == 0 || below)) {
                             y[i * p.OW] = y0;
@@ -326,15 +348,19 @@ struct ConvWinograd {
                     }
                 }
         };
-        if (pairs && oc0 + 32 <= p.OC && (p.OH & 1) == 0) outputs(std::integral_constant<bool, true>{});
-        else outputs(std::integral_constant<bool, false>{});
+        typedef std::integral_constant<bool, true> yes;
+        typedef std::integral_constant<bool, false> no;
+        const bool fast = pairs && oc0 + 32 <= p.OC && (p.OH & 1) == 0;
+        if (fin.residual) fast ? outputs(yes{}, yes{}) : outputs(no{}, yes{});
+        else fast ? outputs(yes{}, no{}) : outputs(no{}, no{});
         while (again) {
             const int bit = __builtin_ctz(again);
             again &= again - 1;
             const int oc = oc0 + (bit >> 4) * 16 + 4 * lk + ((bit >> 2) & 3), i = (bit >> 1) & 1, j = bit & 1;
             if (oc >= p.OC || oh + i >= p.OH || ow + j >= p.OW) continue;
             const float sum = conv3x3_direct(p.X + ((long) n * p.XC + c0) * p.H * p.W, p.Wt + ((long) oc * p.C + c0) * 9, chunks * CI, p.H, p.W, ih0 + i, iw0 + j);
-            ytile[oc * plane + (long) i * p.OW + j] = sum + (p.bias ? p.bias[oc] : 0.f);
+            const long to = oc * plane + (long) i * p.OW + j;
+            ytile[to] = conv_finished(fin, sum + (p.bias ? p.bias[oc] : 0.f), fin.residual ? rtile[to] : -0.f);
         }
     }
 };
@@ -343,7 +369,7 @@ struct ConvWinograd {
 
 namespace docc_k {
 template <int NW, bool WIDE>
-__device__ __forceinline__ void conv_winograd(const ConvParams& p) {
+__device__ __forceinline__ void conv_winograd(const ConvParams& p, const ConvFinish& fin) {
     typedef ConvWinograd<NW> K;
     __shared__ __attribute__((aligned(16))) float lds[K::LDS_FLOATS];
     const int ocb = (p.OC + 31) >> 5, id = xcd_contiguous(blockIdx.x, gridDim.x);
@@ -353,10 +379,10 @@ __device__ __forceinline__ void conv_winograd(const ConvParams& p) {
     const int TH = (p.OH + 1) >> 1, TW = (p.OW + 1) >> 1;
     const int before = (p.pad_h >> 1) * TW, bottom = (p.H - 3 + p.pad_h) >> 1;
     const long behind = (long) (p.N - 1) * TH * TW + (long) (bottom > 0 ? bottom : 0) * TW + TW - 1;
-    if (WIDE && tile0 > before && tile0 + 16 * NW <= behind) K::template run<true>(p, lds, tile0, oc0, 0, p.C / 8);
-    else K::template run<false>(p, lds, tile0, oc0, 0, p.C / 8);
+    if (WIDE && tile0 > before && tile0 + 16 * NW <= behind) K::template run<true>(p, fin, lds, tile0, oc0, 0, p.C / 8);
+    else K::template run<false>(p, fin, lds, tile0, oc0, 0, p.C / 8);
 }
 } // namespace docc_k
 
-extern "C" __global__ __launch_bounds__(256, 2) void docc_conv2d_f32_winograd(docc_k::ConvParams p) { docc_k::conv_winograd<4, false>(p); }
-extern "C" __global__ __launch_bounds__(256, 2) void docc_conv2d_f32_winograd_wide(docc_k::ConvParams p) { docc_k::conv_winograd<4, true>(p); }
+extern "C" __global__ __launch_bounds__(256, 2) void docc_conv2d_f32_winograd(docc_k::ConvParams p, docc_k::ConvFinish f) { docc_k::conv_winograd<4, false>(p, f); }
+extern "C" __global__ __launch_bounds__(256, 2) void docc_conv2d_f32_winograd_wide(docc_k::ConvParams p, docc_k::ConvFinish f) { docc_k::conv_winograd<4, true>(p, f); }

@@ -11,7 +11,7 @@ using namespace docc::rt::rocm;
 
 namespace {
 
-// must match docc_k::ConvParams in csrc/kernels/conv2d.hip
+// must match docc_k::ConvParams and ConvFinish in csrc/kernels/conv_params.h
 struct ConvParams {
     const float* X;
     const float* Wt;
@@ -21,6 +21,11 @@ struct ConvParams {
     int stride_h, stride_w, pad_h, pad_w, dil_h, dil_w;
     int XC, YC;   // channels of the tensors X and Y lie in (C and OC, or more for the groups of a grouped convolution)
     long GX, GW, GB, GY;   // grouped convolution in one launch: elements from one group's operands to the next's (grid z = groups)
+};
+
+struct ConvFinish {
+    const float* residual;
+    int relu;
 };
 
 int64_t out_dim(int64_t d_in, int64_t pad_begin, int64_t pad_end, int64_t dil, int64_t kernel, int64_t stride) {
@@ -291,7 +296,8 @@ extern "C" int64_t docc_rocm_conv2d_f32_workspace_bytes(int64_t N, int64_t C, in
 static int conv2d_run(docc_rocm_stream_t stream, int64_t N, int64_t C, int64_t H, int64_t W, int64_t OC, int64_t KH, int64_t KW,
                       int64_t stride_h, int64_t stride_w, int64_t pad_h, int64_t pad_w, int64_t pad_h_end, int64_t pad_w_end, int64_t dil_h,
                       int64_t dil_w, const float* X, const float* Wt, const float* bias, float* Y, void* workspace, int64_t workspace_bytes,
-                      int64_t x_channels = -1, int64_t y_channels = -1, int64_t groups = 1) {
+                      int64_t x_channels = -1, int64_t y_channels = -1, int64_t groups = 1, ConvFinish fin = {nullptr, 0}, bool* finished = nullptr) {
+    // fin: what the layer has behind the convolution, where the form that runs stores it as well (*finished is set then)
     // x_channels, y_channels: the channels of the tensors X and Y point into, where this call is a grouped convolution (the
     // images are then that many channels apart); -1: C and OC. groups: that many convolutions of these extents in one launch
     // (grid z), group g on the channels g * C .. of X, g * OC .. of Y, filters and bias
@@ -335,8 +341,9 @@ static int conv2d_run(docc_rocm_stream_t stream, int64_t N, int64_t C, int64_t H
         // rows of whole tiles between one column of padding on either side: four pixels a load
         const char* force = std::getenv("DOCC_ROCM_CONV");
         const bool wide = any_pad_w == 1 && OW == W && W % 2 == 0 && !(force && std::strstr(force, "-narrow"));
+        if (finished) *finished = true;
         return launch(wide ? "docc_conv2d_f32_winograd_wide" : "docc_conv2d_f32_winograd", (uint32_t) winograd_groups(N, OC, OH, OW), 1, 1, 256, 0,
-                      (hipStream_t) stream, p);
+                      (hipStream_t) stream, p, fin);
     }
     if (path == ConvPath::Gemm1x1) {
         // Y[n] (OC x P) = W (OC x C) X[n] (C x P): one batched GEMM on the tensors as they lie; the bias is
@@ -401,11 +408,12 @@ static int conv2d_run(docc_rocm_stream_t stream, int64_t N, int64_t C, int64_t H
             const int64_t total = N * OC * OH * OW;
             rc = launch(name, (uint32_t) (plan.images > 1 ? (N + plan.images - 1) / plan.images : N * strips), (uint32_t) ((OC + 63) / 64),
                         (uint32_t) plan.parts, 256, (uint32_t) (3 * stage * 4), (hipStream_t) stream, p, (int) TH, (int) plan.images, sums);
-            const bool vectors = total % 4 == 0 && (uintptr_t) Y % 16 == 0;
+            const bool vectors = total % 4 == 0 && ((uintptr_t) Y | (uintptr_t) fin.residual) % 16 == 0;
+            if (finished) *finished = true;
             const int64_t items = vectors ? total / 4 : total, blocks = (items + 255) / 256;
             if (!rc)
                 rc = launch(vectors ? "docc_conv2d_add_parts_f32_v4" : "docc_conv2d_add_parts_f32", (uint32_t) (blocks < 2048 ? blocks : 2048), 1, 1, 256, 0,
-                            (hipStream_t) stream, (const float*) sums, bias, Y, (long) total, (int) (OH * OW), (int) OC, (int) plan.parts);
+                            (hipStream_t) stream, (const float*) sums, bias, Y, (long) total, (int) (OH * OW), (int) OC, (int) plan.parts, fin);
             const int freed = docc_rocm_free_async(sums, stream);
             return rc ? rc : freed;
         }
@@ -580,4 +588,29 @@ extern "C" int docc_rocm_conv2d_f32_grouped(docc_rocm_stream_t stream, int64_t N
         if (rc) return rc;
     }
     return 0;
+}
+
+// Y = act(convolution + bias + residual): in the store of the forms that have it, else an elementwise pass over Y behind the convolution.
+extern "C" int docc_rocm_conv2d_f32_chain(docc_rocm_stream_t stream, int64_t N, int64_t C, int64_t H, int64_t W, int64_t OC, int64_t KH, int64_t KW,
+                                          int64_t stride_h, int64_t stride_w, int64_t pad_h, int64_t pad_w, int64_t pad_h_end, int64_t pad_w_end,
+                                          int64_t dil_h, int64_t dil_w, int64_t group, const float* X, const float* Wt, const float* bias,
+                                          const float* residual, int activation, float* Y, void* workspace, int64_t workspace_bytes) {
+    if (activation < -1 || activation > DOCC_ROCM_UNARY_ERF) return fail(DOCC_ROCM_ERR_INVALID_ARGUMENT, "conv2d: unknown activation %d", activation);
+    bool finished = false;
+    int rc;
+    if (group == 1) {
+        const bool in_store = activation == -1 || activation == DOCC_ROCM_UNARY_RELU;
+        const ConvFinish fin{residual, activation == DOCC_ROCM_UNARY_RELU};
+        rc = conv2d_run(stream, N, C, H, W, OC, KH, KW, stride_h, stride_w, pad_h, pad_w, pad_h_end, pad_w_end, dil_h, dil_w, X, Wt, bias, Y, workspace,
+                        workspace_bytes, -1, -1, 1, in_store ? fin : ConvFinish{nullptr, 0}, in_store ? &finished : nullptr);
+    } else {
+        rc = docc_rocm_conv2d_f32_grouped(stream, N, C, H, W, OC, KH, KW, stride_h, stride_w, pad_h, pad_w, pad_h_end, pad_w_end, dil_h, dil_w, group, X, Wt, bias,
+                                          Y, workspace, workspace_bytes);
+    }
+    if (rc || finished || (!residual && activation < 0)) return rc;
+    const int64_t total = N * OC * out_dim(H, pad_h, pad_h_end, dil_h, KH, stride_h) * out_dim(W, pad_w, pad_w_end, dil_w, KW, stride_w);
+    if (total == 0) return 0;
+    if (!residual) return docc_rocm_elementwise_unary(stream, activation, 32, total, Y, Y);
+    const int64_t shape[1] = {total};
+    return docc_rocm_elementwise_fused(stream, 32, 1, shape, DOCC_ROCM_BINARY_ADD, shape, Y, 0.0, shape, residual, 0.0, activation >= 0 ? 1 : 0, &activation, Y);
 }

@@ -3,6 +3,7 @@
 // instrumented by) and only the generated calls change:
 //   * a GEMM and the elementwise block that alone reads its result - bias, activation, rounding to bf16, residual - become
 //     docc_rocm_linear, which has the chain in the product's store;
+//   * a convolution and the elementwise block that alone reads its result - residual, ReLU - become docc_rocm_conv2d_f32_chain;
 //   * Mean, centre and square, Mean, scale and shift (how a layer norm is spelled with tensor nodes), with the casts around
 //     them for bf16, become docc_rocm_layer_norm.
 // A transformer's feed-forward block of nine to eleven launches is three calls this way. The reference stops at fusing Maps
@@ -17,6 +18,7 @@
 namespace sdfg::rocm {
 
 namespace blas = math::blas;
+namespace tensor = math::tensor;
 using data_flow::LibraryNode;
 
 namespace {
@@ -45,6 +47,15 @@ public:
     P type = P::Float, bias_type = P::Float, residual_type = P::Float, y_type = P::Float;
     bool has_bias = false, has_residual = false;
     int activation = -1, rounding = 0;
+};
+
+class ConvChainLaunch : public LaunchNode {
+public:
+    ConvChainLaunch(std::vector<std::string> inputs) : LaunchNode(LibraryNodeType_ROCM_ConvChain, std::move(inputs)) {}
+    std::string extents;
+    Expression group;
+    bool has_bias = false, has_residual = false;
+    int activation = -1;
 };
 
 class LayerNormLaunch : public LaunchNode {
@@ -199,7 +210,7 @@ public:
         bool applied = false;
         for (bool changed = true; changed;) {
             changed = false;
-            for (size_t j = 0; j < blocks_.size() && !changed; j++) changed = layer_norm(j) || linear(j);
+            for (size_t j = 0; j < blocks_.size() && !changed; j++) changed = layer_norm(j) || linear(j) || conv_chain(j);
             applied = applied || changed;
         }
         restore_lifetimes(applied);
@@ -434,6 +445,60 @@ private:
         return true;
     }
 
+    // ---- a convolution and the block behind it ---------------------------------------------------------
+    bool conv_chain(size_t j) {
+        if (!ours(j)) return false;
+        std::optional<MapForm> f = convert_.form_of(blocks_[j]);
+        if (!f || f->results.size() != 1 || f->results[0].element != P::Float) return false;
+        const Values v(*f);
+        for (auto& s : f->statements)
+            if (s.type != P::Float) return false;
+        const std::vector<Expression> whole = dense_strides(f->bounds, 0, f->bounds.size());
+        if (!same_strides(f->results[0].strides, whole)) return false;
+        int act = -1;
+        const std::string inner = activation_of(v, f->results[0].value, &act);
+        if (act != -1 && act != 2) return false;
+        auto dense = [&](const std::string& name) -> const MapForm::Read* {
+            const MapForm::Read* r = v.read(name);
+            return r && r->element == P::Float && same_strides(r->strides, whole) ? r : nullptr;
+        };
+        // what the activation is of: the convolution's result, or its sum with a tensor of the same extents - either operand of which may be it
+        const Statement* sum = v.statement(inner, "fp_add");
+        if (!sum) return act != -1 && dense(inner) && conv_chain(j, *f, dense(inner), nullptr, act);
+        const MapForm::Read *a = dense(sum->args[0]), *b = dense(sum->args[1]);
+        return a && b && a->data != b->data && (conv_chain(j, *f, a, b, act) || conv_chain(j, *f, b, a, act));
+    }
+
+    bool conv_chain(size_t j, const MapForm& f, const MapForm::Read* link, const MapForm::Read* residual, int act) {
+        const long w = writer_of(link->data, j);
+        if (w < 0 || !ours((size_t) w)) return false;
+        const size_t i = (size_t) w;
+        const auto* c = dynamic_cast<const tensor::ConvNode*>(blocks_[i].node.get());
+        if (!c || c->element() != P::Float || c->shape().size() != 4) return false;
+        const Expression whole = symbolic::mul(symbolic::mul(c->shape()[0], c->output_channels()), symbolic::mul(c->output_dim(0), c->output_dim(1)));
+        if (!symbolic::equal(symbolic::product(f.bounds, 0, f.bounds.size()), whole) || !private_to(link->data, {i, j})) return false;
+        // what the convolution reads it now reads where block j stands; the result overlaps none of it, nor the residual
+        std::vector<std::string> connectors{"X", "W"};
+        if (c->has_bias()) connectors.push_back("B");
+        std::vector<ConnectorBinding> inputs;
+        for (auto& name : connectors) {
+            inputs.push_back(*blocks_[i].input(name));
+            if (inputs.back().is_constant || lost_between(inputs.back().data, i, j) || inputs.back().data == f.results[0].data) return false;
+        }
+        if (residual) {
+            if (residual->data == f.results[0].data) return false;
+            connectors.push_back("_residual"), inputs.push_back(bind("_residual", residual->data));
+        }
+        auto node = std::make_unique<ConvChainLaunch>(connectors);
+        node->extents = conv_launch_extents(*c);
+        node->group = c->group();
+        node->has_bias = c->has_bias();
+        node->has_residual = residual != nullptr;
+        node->activation = act;
+        install(j, std::move(node), std::move(inputs), f.results[0].data, {i}, {link->data});
+        return true;
+    }
+
     // ---- layer norm ------------------------------------------------------------------------------------
     // the Mean over the trailing loops from `trailing` on whose result a form of loops `bounds` loads once per row
     const tensor::ReduceNode* row_mean(const std::string& name, size_t before, size_t* at) const {
@@ -599,6 +664,19 @@ public:
               << (l->has_bias ? "_bias" : "nullptr") << ", " << type_code(l->bias_type) << ", " << l->activation << ", "
               << (l->has_residual ? "_residual" : "nullptr") << ", " << type_code(l->residual_type) << ", " << l->rounding << ", _y, " << type_code(l->y_type)
               << "));" << std::endl;
+        } else if (const auto* c = dynamic_cast<const ConvChainLaunch*>(&node_)) {
+            s << "{" << std::endl;
+            s.setIndent(s.indent() + 4);
+            int64_t group = 0;
+            const bool whole = symbolic::is_integer(c->group, &group) && group == 1;   // grouped convolutions take no workspace
+            s << "const int64_t __ws_bytes = " << (whole ? "docc_rocm_conv2d_f32_pads_workspace_bytes(" + c->extents + ")" : std::string("0")) << ";" << std::endl;
+            s << "void *__ws = nullptr;" << std::endl;
+            s << "if (__ws_bytes > 0) DOCC_ROCM_CHECK(docc_rocm_malloc_async(&__ws, (size_t) __ws_bytes, nullptr));" << std::endl;
+            s << "DOCC_ROCM_CHECK(docc_rocm_conv2d_f32_chain(nullptr, " << c->extents << ", (int64_t) (" << c->group << "), X, W, " << (c->has_bias ? "B" : "nullptr") << ", "
+              << (c->has_residual ? "_residual" : "nullptr") << ", " << c->activation << ", _y, __ws, __ws_bytes));" << std::endl;
+            s << "if (__ws) DOCC_ROCM_CHECK(docc_rocm_free_async(__ws, nullptr));" << std::endl;
+            s.setIndent(s.indent() - 4);
+            s << "}" << std::endl;
         } else if (const auto* n = dynamic_cast<const LayerNormLaunch*>(&node_)) {
             s << "DOCC_ROCM_CHECK(docc_rocm_layer_norm(nullptr, " << type_code(n->type) << ", " << n->rows << ", " << n->cols << ", (float) (" << n->eps
               << "), _x, " << (n->has_weight ? "_weight" : "nullptr") << ", " << (n->has_bias ? "_bias" : "nullptr") << ", _y));" << std::endl;
@@ -611,7 +689,7 @@ public:
 bool RocmLaunchFusionPass::run_pass(builder::StructuredSDFGBuilder& builder, analysis::AnalysisManager&) { return LaunchFusion(builder.subject()).run(); }
 
 void register_launch_dispatchers(codegen::LibraryNodeDispatcherRegistry& reg) {
-    for (auto& code : {LibraryNodeType_ROCM_Linear, LibraryNodeType_ROCM_LayerNorm})
+    for (auto& code : {LibraryNodeType_ROCM_Linear, LibraryNodeType_ROCM_ConvChain, LibraryNodeType_ROCM_LayerNorm})
         reg.register_library_node_dispatcher(code + "::" + ImplementationType_ROCMWithoutTransfers,
                                              [](codegen::LanguageExtension& le, const Function& f, const data_flow::DataFlowGraph& b, const LibraryNode& n) {
                                                  return std::make_unique<LaunchDispatcher>(le, f, b, n);

@@ -285,18 +285,13 @@ protected:
 
     void emit_launch(PrettyPrinter& s, const std::function<std::string(const std::string&)>& name_of) override {
         const auto& c = conv();
-        auto get = [](const std::vector<Expression>& v, size_t i, const char* dflt) { return v.empty() ? Expression(dflt) : v[i]; };
-        std::ostringstream dims;
-        dims << c.shape()[0] << ", " << c.shape()[1] << ", " << c.shape()[2] << ", " << c.shape()[3] << ", " << c.output_channels() << ", "
-             << c.kernel_shape()[0] << ", " << c.kernel_shape()[1] << ", " << get(c.strides(), 0, "1") << ", " << get(c.strides(), 1, "1")
-             << ", " << get(c.pads(), 0, "0") << ", " << get(c.pads(), 1, "0") << ", " << get(c.pads(), 2, "0") << ", " << get(c.pads(), 3, "0")
-             << ", " << get(c.dilations(), 0, "1") << ", " << get(c.dilations(), 1, "1");   // pads: begins, then ends
+        const std::string dims = conv_launch_extents(c);
         // layers that run as im2col + GEMM take their column matrix from a workspace that lives around the node;
         // for the others the size is 0 and nothing is allocated
         int64_t group = 1;
         if (!symbolic::is_integer(c.group(), &group) || group != 1) {
             // the node's group (weights [C_out][C_in / group][kh][kw]): the direct kernels, once per group
-            s << "DOCC_ROCM_CHECK(docc_rocm_conv2d_f32_grouped(nullptr, " << dims.str() << ", (int64_t) (" << c.group() << "), (const float *) "
+            s << "DOCC_ROCM_CHECK(docc_rocm_conv2d_f32_grouped(nullptr, " << dims << ", (int64_t) (" << c.group() << "), (const float *) "
               << name_of("X") << ", (const float *) " << name_of("W") << ", "
               << (c.has_bias() ? "(const float *) " + name_of("B") : std::string("nullptr")) << ", (float *) " << name_of("Y")
               << ", nullptr, 0));" << std::endl;
@@ -304,10 +299,10 @@ protected:
         }
         s << "{" << std::endl;
         s.setIndent(s.indent() + 4);
-        s << "const int64_t __ws_bytes = docc_rocm_conv2d_f32_pads_workspace_bytes(" << dims.str() << ");" << std::endl;
+        s << "const int64_t __ws_bytes = docc_rocm_conv2d_f32_pads_workspace_bytes(" << dims << ");" << std::endl;
         s << "void *__ws = nullptr;" << std::endl;
         s << "if (__ws_bytes > 0) DOCC_ROCM_CHECK(docc_rocm_malloc_async(&__ws, (size_t) __ws_bytes, nullptr));" << std::endl;
-        s << "DOCC_ROCM_CHECK(docc_rocm_conv2d_f32_pads(nullptr, " << dims.str() << ", (const float *) " << name_of("X")
+        s << "DOCC_ROCM_CHECK(docc_rocm_conv2d_f32_pads(nullptr, " << dims << ", (const float *) " << name_of("X")
           << ", (const float *) " << name_of("W") << ", "
           << (c.has_bias() ? "(const float *) " + name_of("B") : std::string("nullptr")) << ", (float *) " << name_of("Y")
           << ", __ws, __ws_bytes));" << std::endl;
@@ -900,6 +895,15 @@ std::unique_ptr<LibraryNode> deserialize_attention(const json::Value& j) { retur
 std::unique_ptr<LibraryNode> deserialize_offloading(const json::Value& j) { return ROCMDataOffloadingNode::from_json(j); }
 
 } // namespace
+
+std::string conv_launch_extents(const tensor::ConvNode& c) {
+    auto get = [](const std::vector<Expression>& v, size_t i, const char* dflt) { return v.empty() ? Expression(dflt) : v[i]; };
+    std::ostringstream s;
+    s << c.shape()[0] << ", " << c.shape()[1] << ", " << c.shape()[2] << ", " << c.shape()[3] << ", " << c.output_channels() << ", " << c.kernel_shape()[0] << ", "
+      << c.kernel_shape()[1] << ", " << get(c.strides(), 0, "1") << ", " << get(c.strides(), 1, "1") << ", " << get(c.pads(), 0, "0") << ", " << get(c.pads(), 1, "0")
+      << ", " << get(c.pads(), 2, "0") << ", " << get(c.pads(), 3, "0") << ", " << get(c.dilations(), 0, "1") << ", " << get(c.dilations(), 1, "1");
+    return s.str();
+}
 
 void register_plugin(plugins::Context& context) {
     auto& ser = context.library_node_serializer_registry;

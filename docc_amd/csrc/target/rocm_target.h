@@ -94,8 +94,8 @@ public:
     bool run_pass(builder::StructuredSDFGBuilder& builder, analysis::AnalysisManager& analysis_manager);
 };
 
-// Merges launches when host code is generated (launch_fusion.cpp): a GEMM with the elementwise block behind it, the blocks a layer
-// norm is spelled with. Runs on the copy of the SDFG that the generator works on, if the program was scheduled with fusion (which
+// Merges launches when host code is generated (launch_fusion.cpp): a GEMM or a convolution with the elementwise block behind it, the blocks a
+// layer norm is spelled with. Runs on the copy of the SDFG that the generator works on, if the program was scheduled with fusion (which
 // the scheduler notes in the metadata); not for an instrumented program, whose nodes are regions of their own.
 inline const std::string Metadata_FuseLaunches = "rocm_fuse_launches";
 class RocmLaunchFusionPass {
@@ -103,9 +103,12 @@ public:
     std::string name() { return "RocmLaunchFusion"; }
     bool run_pass(builder::StructuredSDFGBuilder& builder, analysis::AnalysisManager& analysis_manager);
 };
+inline const std::string LibraryNodeType_ROCM_ConvChain = "ROCMConvChain";
 inline const std::string LibraryNodeType_ROCM_Linear = "ROCMLinear";
 inline const std::string LibraryNodeType_ROCM_LayerNorm = "ROCMLayerNorm";
 void register_launch_dispatchers(codegen::LibraryNodeDispatcherRegistry& reg);
+// the extents of a 2-d convolution as the launchers take them: N, C, H, W, OC, KH, KW, strides, pads (begins, then ends), dilations
+std::string conv_launch_extents(const math::tensor::ConvNode& conv);
 
 // Preamble every rocm dispatcher puts into the globals stream (duplicates are folded by the generator).
 void emit_runtime_preamble(codegen::PrettyPrinter& globals, const Function& function);

@@ -244,6 +244,17 @@ int docc_rocm_conv2d_f32_grouped(docc_rocm_stream_t stream, int64_t N, int64_t C
                                  const float* bias, float* Y, void* workspace, int64_t workspace_bytes);
 
 /*
+ * A convolution and what a layer has behind it:  Y = act(convolution + bias + residual),  `residual` dense like Y or NULL (it must not overlap
+ * Y), `activation` one of DOCC_ROCM_UNARY_* or -1, every step rounded to float32 as the separate nodes would. The sum and a ReLU are applied where
+ * the product is stored by the forms that have it (csrc/kernels/conv_winograd.hip, the channels in parts); behind the others one
+ * elementwise pass over Y follows.
+ */
+int docc_rocm_conv2d_f32_chain(docc_rocm_stream_t stream, int64_t N, int64_t C, int64_t H, int64_t W, int64_t OC, int64_t KH, int64_t KW,
+                               int64_t stride_h, int64_t stride_w, int64_t pad_h, int64_t pad_w, int64_t pad_h_end, int64_t pad_w_end,
+                               int64_t dil_h, int64_t dil_w, int64_t group, const float* X, const float* Wt, const float* bias,
+                               const float* residual, int activation, float* Y, void* workspace, int64_t workspace_bytes);
+
+/*
  * ml::Attention (a node the rocm target adds; the reference has none):
  *   O[b,h,i,:] = sum_j softmax_j(scale * <Q[b,h,i,:], K[b,h,j,:]>) * V[b,h,j,:]
  * Q [B,H,SQ,D], K and V [B,H,SKV,D], all contiguous bf16 (raw bits); fp32

@@ -85,3 +85,35 @@ def test_values_that_are_not_finite_stay_where_they_are(rt, monkeypatch, force):
     assert np.abs(Y[large & ok] / ref[large & ok] - 1).max() <= 1e-4
     small = ok & ~large
     assert np.abs(Y[small] - ref[small]).max() <= 1e-5 * np.abs(clean).max()
+
+
+@pytest.mark.parametrize("force", ["", "winograd", "halo-t4-parts2", "halo", "gather", "gemm"])
+@pytest.mark.parametrize("case", [(2, 32, 14, 14, 64, 1, 3), (3, 40, 7, 9, 33, 1, 3), (2, 32, 14, 14, 64, 2, 3), (2, 64, 9, 9, 32, 2, 1), (2, 128, 8, 8, 32, 1, 1)])
+@pytest.mark.parametrize("residual,activation", [(False, 2), (True, 2), (True, -1), (True, 5)])
+def test_chain_is_the_convolution_and_the_pass_behind_it(rt, monkeypatch, force, case, residual, activation):
+    """docc_rocm_conv2d_f32_chain against the convolution, the sum and the activation (ReLU, tanh) as launches of their own: the same roundings."""
+    N, C, H, W, OC, stride, k = case
+    if force:
+        monkeypatch.setenv("DOCC_ROCM_CONV", force)
+    g = torch.Generator().manual_seed(C)
+    x, w, b = torch.randn(N, C, H, W, generator=g).cuda(), (torch.randn(OC, C, k, k, generator=g) * (2 / (C * k * k)) ** 0.5).cuda(), torch.randn(OC, generator=g).cuda()
+    p = k // 2
+    OH, OW = (H + 2 * p - k) // stride + 1, (W + 2 * p - k) // stride + 1
+    r = torch.randn(N, OC, OH, OW, generator=g).cuda()
+    x[0, 0, 1, 1] = float("inf")
+    sizes = (N, C, H, W, OC, k, k, stride, stride, p, p, p, p, 1, 1)
+    ws = torch.empty(max(1, rt.lib().docc_rocm_conv2d_f32_pads_workspace_bytes(*sizes)), dtype=torch.uint8, device="cuda")
+    args = (x.data_ptr(), w.data_ptr(), b.data_ptr())
+    got, ref = torch.full_like(r, float("nan")), torch.empty_like(r)
+    rt.call("docc_rocm_conv2d_f32_chain", 0, *sizes, 1, *args, r.data_ptr() if residual else None, activation, got.data_ptr(), ws.data_ptr(), ws.numel())
+    rt.call("docc_rocm_conv2d_f32_pads", 0, *sizes, *args, ref.data_ptr(), ws.data_ptr(), ws.numel())
+    torch.cuda.synchronize()
+    if residual:
+        ref = ref + r
+    if activation == 2:
+        ref = torch.where(ref > 0, ref, torch.zeros_like(ref))       # (a NaN is not larger: fmax(x, 0))
+        assert torch.equal(got, ref)
+    elif activation < 0:
+        assert torch.equal(got.nan_to_num(nan=7e33), ref.nan_to_num(nan=7e33))
+    else:
+        assert (got.nan_to_num() - torch.tanh(ref).nan_to_num()).abs().max() <= 1e-6

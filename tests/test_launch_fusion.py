@@ -174,3 +174,39 @@ def test_c_is_read_unless_beta_is_the_number_zero(tmp_path, beta, read):
     s = b.move()
     s.schedule("rocm")
     assert s.loop_report()["H2D"] == (3 if read else 2)
+
+
+class ConvBlock(torch.nn.Module):
+    def __init__(self, tail):
+        super().__init__()
+        self.tail = tail
+
+    def forward(self, x, r, w, b):
+        return self.tail(F.conv2d(x, w, b, padding=1), r)
+
+
+CONV = "2, 8, 6, 6, 16, 3, 3, 1, 1, 1, 1, 1, 1, 1, 1, (int64_t) (1), X, W, B"
+
+
+@pytest.mark.parametrize("tail,emitted", [
+    (lambda y, r: torch.relu(y), f"{CONV}, nullptr, 2, _y"),
+    (lambda y, r: torch.relu(y + r), f"{CONV}, _residual, 2, _y"),
+    (lambda y, r: torch.relu(r + y), f"{CONV}, _residual, 2, _y"),
+    (lambda y, r: y + r, f"{CONV}, _residual, -1, _y"),
+    (lambda y, r: torch.sigmoid(y), None),                     # no activation of the store
+    (lambda y, r: torch.relu(y) + y, None),                    # a second reader
+    (lambda y, r: torch.relu(y - r), None),
+    (lambda y, r: torch.relu(y + y), None),
+    (lambda y, r: torch.relu(y + r), "repeated"),
+])
+def test_a_convolution_with_the_block_behind_it(tmp_path, tail, emitted):
+    images = 1 if emitted == "repeated" else 2          # a residual of one image for both
+    emitted = emitted if images == 2 else None
+    s = docc_torch.compile_torch(ConvBlock(tail), None, target="rocm").to_sdfg(torch.randn(2, 8, 6, 6), torch.randn(images, 16, 6, 6), torch.randn(16, 8, 3, 3), torch.randn(16))
+    s.schedule("rocm", options={"offload": "none"})
+    assert [n["code"] for n in s.library_nodes()].count("ml::Conv") == 1      # the scheduled form keeps its nodes
+    text = re.sub(r"\s+", " ", open(s.generate(str(tmp_path))["source"]).read())
+    if emitted:
+        assert f"docc_rocm_conv2d_f32_chain(nullptr, {emitted}, __ws, __ws_bytes)" in text and "elementwise" not in text and text.count("docc_rocm_malloc_async(") == 1
+    else:
+        assert "docc_rocm_conv2d_f32_chain" not in text and "docc_rocm_conv2d_f32_pads(" in text
