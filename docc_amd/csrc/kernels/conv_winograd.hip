@@ -1,7 +1,11 @@
-// ml::Conv, 2-d NCHW fp32, 3x3 with strides and dilations of one, by Winograd's minimal filtering F(2x2, 3x3)
+// ml::Conv, 2-d NCHW fp32, 3x3 without dilation and with steps of one or two, by Winograd's minimal filtering F(2x2, 3x3)
 // (S. Winograd, Arithmetic Complexity of Computations, 1980; A. Lavin and S. Gray, Fast Algorithms for Convolutional
 // Neural Networks, 2016): a 2x2 tile of outputs is A^T [ sum over channels of (G g G^T) .* (B^T d B) ] A of the 4x4 input pixels d
 // around it, 16 products a channel instead of 36.
+//
+// Steps of two: a 2x2 tile of outputs reads 5x5 pixels. Along an axis taps 0 and 2 meet the pixels 0, 2 and 4, a two-tap filter with two outputs: (x0 - x2) w0,
+// x2 (w0 + w2), (x4 - x2) w2; tap 1 meets x1 and x3. Five products for six, 25 for 36 in two axes, and as the products that go to one output alone
+// share a sum with those of tap 1, nine sums. The filters have 16 components again, so that their way is the same.
 //
 // What bounds the direct form is the fp32 matrix pipe (one work-group of docc_conv2d_f32_halo_* keeps it at two thirds of its peak); the 16
 // sums over the channels are the same matrix product of 16 / 36 of the size, and everything else a tile needs fits beside
@@ -21,7 +25,9 @@
 // by the other wave of the SIMD. Measured on 166 x 256 x 14 x 14 -> 256 (four work-groups a CU): 150 us = 257 TFLOP/s of the direct form's count; the MFMAs
 // alone 124 us, without the filters' way 141, without loading pixels 135. Interleaved one MFMA, two others it took 179 us, the others in one run amid
 // eight MFMAs 164, and with fewer of them (vector loads of a row instead of its pixels, no factors of one half, buffers by constant
-// offsets) the 150. Against the direct form: 32 x 64 x 56 x 56 -> 64 71 -> 48 us, 32 x 256 x 14 x 14 -> 256 92 -> 48.
+// offsets) the 150. Against the direct form: 32 x 64 x 56 x 56 -> 64 71 -> 48 us, 32 x 256 x 14 x 14 -> 256 92 -> 48; steps of
+// two: 50 x 80 x 52 x 52 -> 160 153 -> 57, 3 x 448 x 51 x 51 -> 896 257 -> 106 (its MFMAs 1.52 us a chunk and work-group, measured 1.6). Pixel by pixel a row's loads touch
+// their cache lines once each, which bounds steps of two: 12 x 96 x 8 x 8 51 us for 25 with vectors or pairs.
 //
 // Rounding: the chain of additions has C terms instead of 9 C, which outweighs the transforms' own. Relative error (2-norm) against 64 bits on
 // N(0, 1) images: C = 16 1.5e-7 (direct 2.1e-7), 64 2.6e-7 (4.1e-7), 512 6.8e-7 (1.2e-6); on their positive part 1.3e-7 (1.4e-7), 2.3e-7
@@ -34,6 +40,7 @@
 namespace docc_k {
 
 typedef float wf4 __attribute__((ext_vector_type(4)));
+typedef float wf2 __attribute__((ext_vector_type(2)));
 
 // Work-groups are dealt to the 8 XCDs in turn: number them so that an XCD gets consecutive ones (whose work shares input).
 __device__ __forceinline__ int xcd_contiguous(int id, int n) {
@@ -54,21 +61,33 @@ __device__ __forceinline__ float conv3x3_direct(const float* xn, const float* w,
     return sum;
 }
 
-// WIDE: a lane loads the four pixels of a row as one vector. Rows then end in whole tiles (OW == W even, pad_w 1), so that only the outer
-// columns can lie in the padding; the vector reads a neighbouring row's pixel there, which is dropped after the row transform. Work-groups
-// with a tile for which that pixel lies outside the tensor load pixel by pixel.
-template <int NW>
+// How a lane loads the pixels of a row:
+//   kPixels   one by one, each with an offset of its own; any padding
+//   kVector   four as one vector, with steps of two the column before them apart. One column of padding: only the outer columns can lie in it. The
+//             vector reads a neighbouring row's pixels there, which are dropped after the row transform; work-groups with a tile for which they lie
+//             outside the tensor load pixel by pixel. With steps of two rows are whole vectors and nothing of the kind happens.
+//   kVectorOdd  (steps of one) the same for rows of odd length, whose last tile has two columns in the padding
+//   kPairs    (steps of two) the column before, then two pairs. Of a pair that begins with the row's last pixel the one before is loaded and shifted.
+enum WinogradLoads { kPixels, kVector, kVectorOdd, kPairs };
+
+template <int S>
 struct ConvWinograd {
+    static constexpr int NW = 4;                   // waves
     static constexpr int CI = 8;                   // channels per chunk
     static constexpr int CS = 4 * 128 + 4;         // floats from one channel's components in LDS to the next's (eight lanes write a channel each: a vector further)
     static constexpr int STAGE = CI * CS;
     static constexpr int RAW = 32 * CI * 9;        // filters of a chunk as they lie in memory
-    static constexpr int UT = 4 / NW;                                // filters a thread transforms per chunk
+    static constexpr int PX = S == 1 ? 4 : 5;      // pixels a tile reads along a row or column
+    static constexpr int RG = PX;                  // rows of products per channel
+    static constexpr int NA = S == 1 ? 4 : 3;      // rows of sums
+    // the row of filter components and the row of sums that row i of products goes with
+    static constexpr int filter_row(int i) { return i == 4 ? 3 : i; }
+    static constexpr int sum_row(int i) { return S == 1 ? i : i == 3 ? 0 : i == 4 ? 2 : i; }
     static constexpr int WL = (RAW / 4 + 64 * NW - 1) / (64 * NW);   // vectors of them a thread moves
     static constexpr int LDS_FLOATS = 2 * STAGE + 2 * RAW + 4;
 
     // channels [c0, c0 + 8 * chunks) of X and Wt; the work-group's tiles from tile0 on, output channels from oc0 on
-    template <bool WIDE>
+    template <int LOADS>
     static __device__ __forceinline__ void run(const ConvParams& p, const ConvFinish& fin, float* lds, int tile0, int oc0, int c0, int chunks) {
         const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
         const int l16 = lane & 15, lk = lane >> 4;
@@ -81,7 +100,7 @@ struct ConvWinograd {
         const int n0 = tile0 / per_image;                                    // first image of the work-group
         const int n = (tile_ok ? tile : tile0) / per_image, rest = (tile_ok ? tile : tile0) % per_image;
         const int oh = 2 * (rest / TW), ow = 2 * (rest % TW);
-        const int ih0 = oh - p.pad_h, iw0 = ow - p.pad_w;
+        const int ih0 = S * oh - p.pad_h, iw0 = S * ow - p.pad_w;
         const int HW4 = p.H * p.W * 4;
 
         // X from image n0 on and the filters from oc0 on, as buffers; the launcher has seen to it that what a work-group addresses takes less
@@ -94,26 +113,43 @@ struct ConvWinograd {
         const auto wbuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.Wt) + ((long) oc0 * p.C + c0) * 9, 0,
                                                             (int) (wleft < 0x7fffffffL ? wleft : 0x7fffffffL), 0x00020000);
         constexpr int kNone = (int) 0x80000000;      // an offset beyond either
-        const bool first_col = ow == 0, last_col = ow + 2 >= p.OW;
-        int voff[4][WIDE ? 1 : 4];
+        const bool first_col = ow == 0, odd_col = ow + 1 >= p.W, last_col = ow + 2 >= p.W;   // kVector, kVectorOdd: columns 0, 2 and 3 in the padding
+        constexpr int NOFF = LOADS == kPixels ? PX : LOADS == kPairs ? 3 : S;
+        int voff[PX][NOFF];
+        bool shifted[2] = {false, false};
 #pragma unroll
-        for (int r = 0; r < 4; r++)
+        for (int r = 0; r < PX; r++)
 #pragma unroll
-            for (int c = 0; c < (WIDE ? 1 : 4); c++) {
-                const int ih = ih0 + r, iw = iw0 + c;
-                const bool in = tile_ok && ih >= 0 && ih < p.H && (WIDE || (iw >= 0 && iw < p.W));
+            for (int c = 0; c < NOFF; c++) {
+                const int ih = ih0 + r;
+                int iw = iw0 + (LOADS == kPairs && c > 0 ? 2 * c - 1 : c);
+                bool in = tile_ok && ih >= 0 && ih < p.H && ((LOADS != kPixels && LOADS != kPairs && S == 1) || (iw >= 0 && iw < p.W));
+                if (LOADS == kPairs && c > 0) {
+                    // (the launcher takes no padding for which a pair begins with the column before the first)
+                    if (iw == p.W - 1) shifted[c - 1] = true, iw--;
+                    in = tile_ok && ih >= 0 && ih < p.H && iw >= 0 && iw + 1 < p.W;
+                }
                 voff[r][c] = in ? ((n - n0) * p.XC * p.H * p.W + (lk * p.H + ih) * p.W + iw + kEarly) * 4 : kNone;
             }
-        float d[2][4][4];
+        float d[2][PX][PX];
         auto xload = [&](int step, int r, int to) {
-            if constexpr (WIDE) {
-                const wf4 x = __builtin_bit_cast(wf4, __builtin_amdgcn_raw_buffer_load_b128(xbuf, voff[r][0], step * 4 * HW4, 0));
+            const int at = step * 4 * HW4;
+            auto one = [&](int c, int off) { d[to][r][c] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xbuf, voff[r][off], at, 0)); };
+            if constexpr (LOADS == kVector || LOADS == kVectorOdd) {
+                const wf4 x = __builtin_bit_cast(wf4, __builtin_amdgcn_raw_buffer_load_b128(xbuf, voff[r][S - 1], at, 0));
 #pragma unroll
-                for (int c = 0; c < 4; c++) d[to][r][c] = x[c];
+                for (int c = 0; c < 4; c++) d[to][r][S - 1 + c] = x[c];
+                if constexpr (S == 2) one(0, 0);
+            } else if constexpr (LOADS == kPairs) {
+                one(0, 0);
+#pragma unroll
+                for (int q = 0; q < 2; q++) {
+                    const wf2 x = __builtin_bit_cast(wf2, __builtin_amdgcn_raw_buffer_load_b64(xbuf, voff[r][1 + q], at, 0));
+                    d[to][r][1 + 2 * q] = x[0], d[to][r][2 + 2 * q] = x[1];
+                }
             } else {
 #pragma unroll
-                for (int c = 0; c < 4; c++)
-                    d[to][r][c] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xbuf, voff[r][c], step * 4 * HW4, 0));
+                for (int c = 0; c < PX; c++) one(c, c);
             }
         };
 
@@ -139,64 +175,81 @@ struct ConvWinograd {
             *reinterpret_cast<wf4*>(wdst[u] + (spare && buf && tid + u * 64 * NW >= RAW / 4 ? 0 : buf * RAW)) = wr[u];
         };
         const int uc = tid & 7, uo = tid >> 3;
-        float g[UT][9];
+        float g[9];
         const float* const gsrc = raw + uo * (CI * 9) + uc * 9;
         auto gread = [&](int buf) {
 #pragma unroll
-            for (int u = 0; u < UT; u++)
-#pragma unroll
-                for (int t = 0; t < 9; t++) g[u][t] = gsrc[buf * RAW + u * 8 * NW * (CI * 9) + t];
+            for (int t = 0; t < 9; t++) g[t] = gsrc[buf * RAW + t];
         };
-        // The filters are left without the factors of one half that G has in its middle rows: the output transform applies them.
         float* const udst = lds + uc * CS + uo * 4;
         auto ustage = [&](int buf, int i) {      // row i of the components
+            float h[3];
 #pragma unroll
-            for (int u = 0; u < UT; u++) {
-                float h[3];
-#pragma unroll
-                for (int c = 0; c < 3; c++) {
-                    const float a = g[u][c], b = g[u][3 + c], e = g[u][6 + c];
-                    h[c] = i == 0 ? a : i == 3 ? e : i == 1 ? (a + e) + b : (a + e) - b;
-                }
-                const float s = h[0] + h[2];
-                *reinterpret_cast<wf4*>(udst + buf * STAGE + u * 32 * NW + i * 128) = wf4{h[0], s + h[1], s - h[1], h[2]};
+            for (int c = 0; c < 3; c++) {
+                const float a = g[c], b = g[3 + c], e = g[6 + c];
+                if constexpr (S == 1) h[c] = i == 0 ? a : i == 3 ? e : i == 1 ? (a + e) + b : (a + e) - b;   // (without G's halves: the output transform has them)
+                else h[c] = i == 0 ? a : i == 1 ? a + e : i == 2 ? e : b;
             }
+            const float s = h[0] + h[2];
+            wf4 u;
+            if constexpr (S == 1) u = wf4{h[0], s + h[1], s - h[1], h[2]};
+            else u = wf4{h[0], s, h[2], h[1]};
+            *reinterpret_cast<wf4*>(udst + buf * STAGE + i * 128) = u;
         };
 
-        wf4 acc[16][2];
+        wf4 acc[NA * NA][2];
         const float* const ulane = lds + lk * CS + l16 * 4;
         wf4 a[2][2];
-        auto aread = [&](int buf, int half, int i, int to) {
+        auto aread = [&](int buf, int half, int f) {      // row f of the filter components
 #pragma unroll
-            for (int o = 0; o < 2; o++) a[to][o] = *reinterpret_cast<const wf4*>(ulane + buf * STAGE + half * (4 * CS) + i * 128 + o * 64);
+            for (int o = 0; o < 2; o++) a[f & 1][o] = *reinterpret_cast<const wf4*>(ulane + buf * STAGE + half * (4 * CS) + f * 128 + o * 64);
         };
-        // the transformed pixels of row i of the components
-        float v[2][4];
-        auto vrow = [&](float (&x)[4][4], int i) {
-            float t[4];
+        // the transformed pixels of row i of the products
+        float v[2][RG];
+        auto vrow = [&](float (&x)[PX][PX], int i, int to) {
+            float t[PX];
 #pragma unroll
-            for (int c = 0; c < 4; c++) t[c] = i == 0 ? x[0][c] - x[2][c] : i == 1 ? x[1][c] + x[2][c] : i == 2 ? x[2][c] - x[1][c] : x[1][c] - x[3][c];
-            if constexpr (WIDE) {
-                t[0] = first_col ? 0.f : t[0];
-                t[3] = last_col ? 0.f : t[3];
+            for (int c = 0; c < PX; c++) {
+                if constexpr (S == 1) t[c] = i == 0 ? x[0][c] - x[2][c] : i == 1 ? x[1][c] + x[2][c] : i == 2 ? x[2][c] - x[1][c] : x[1][c] - x[3][c];
+                else t[c] = i == 0 ? x[0][c] - x[2][c] : i == 1 ? x[2][c] : i == 2 ? x[4][c] - x[2][c] : i == 3 ? x[1][c] : x[3][c];
             }
-            v[i & 1][0] = t[0] - t[2], v[i & 1][1] = t[1] + t[2], v[i & 1][2] = t[2] - t[1], v[i & 1][3] = t[1] - t[3];
-        };
-        auto mfmas = [&](int i) {
+            if constexpr (S == 1) {
+                if constexpr (LOADS != kPixels) {
+                    t[0] = first_col ? 0.f : t[0];
+                    if constexpr (LOADS == kVectorOdd) t[2] = odd_col ? 0.f : t[2];
+                    t[3] = last_col ? 0.f : t[3];
+                }
+                v[to][0] = t[0] - t[2], v[to][1] = t[1] + t[2], v[to][2] = t[2] - t[1], v[to][3] = t[1] - t[3];
+            } else {
+                if constexpr (LOADS == kPairs) {
 #pragma unroll
-            for (int j = 0; j < 4; j++)
-#pragma unroll
-                for (int o = 0; o < 2; o++) acc[4 * i + j][o] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i & 1][o][j], v[i & 1][j], acc[4 * i + j][o], 0, 0, 0);
+                    for (int q = 0; q < 2; q++) {
+                        t[1 + 2 * q] = shifted[q] ? t[2 + 2 * q] : t[1 + 2 * q];
+                        t[2 + 2 * q] = shifted[q] ? 0.f : t[2 + 2 * q];
+                    }
+                }
+                v[to][0] = t[0] - t[2], v[to][1] = t[2], v[to][2] = t[4] - t[2], v[to][3] = t[1], v[to][4] = t[3];
+            }
         };
-        // Each row of components is a scheduling region: its eight MFMAs, between them the operands of the next row (filters from LDS,
-        // pixels transformed), the loads that refill the pixel registers freed by the row before, and filters.
+        auto mfmas = [&](int i, int from) {
+            const int f = filter_row(i);
+#pragma unroll
+            for (int j = 0; j < RG; j++)
+#pragma unroll
+                for (int o = 0; o < 2; o++) {
+                    wf4& sum = acc[NA * sum_row(i) + sum_row(j)][o];
+                    sum = __builtin_amdgcn_mfma_f32_16x16x4f32(a[f & 1][o][filter_row(j)], v[from][j], sum, 0, 0, 0);
+                }
+        };
+        // Each row of products is a scheduling region: its MFMAs, between them the operands of the next row (filters from LDS,
+        // pixels transformed), the loads that refill the pixel registers that are free, and filters.
         auto shape = [&]() {
             __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);     // LDS reads
-            __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);     // MFMA
+            __builtin_amdgcn_sched_group_barrier(0x008, RG, 0);    // MFMA
             __builtin_amdgcn_sched_group_barrier(0x020, 16, 0);    // loads
             __builtin_amdgcn_sched_group_barrier(0x002, 40, 0);    // VALU
             __builtin_amdgcn_sched_group_barrier(0x200, 4, 0);     // LDS writes
-            __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, RG, 0);
             __builtin_amdgcn_sched_barrier(0);
         };
 
@@ -204,9 +257,10 @@ struct ConvWinograd {
         const int last = chunks - 1;
         wload(0);
 #pragma unroll
-        for (int r = 0; r < 4; r++) xload(0, r, 0);
+        for (int r = 0; r < PX; r++) xload(0, r, 0);
 #pragma unroll
-        for (int r = 0; r < 4; r++) xload(1, r, 1);
+        for (int r = 0; r < PX; r++)
+            if (r != 3 || S == 1) xload(1, r, 1);
 #pragma unroll
         for (int u = 0; u < WL; u++) wraw(0, u);
         wload(last < 1 ? last : 1);
@@ -217,13 +271,13 @@ struct ConvWinograd {
         wload(last < 2 ? last : 2);
 #pragma unroll
         for (int i = 0; i < 4; i++) ustage(0, i);
-        vrow(d[0], 0);
+        vrow(d[0], 0, 0);
         __syncthreads();
         gread(1);
-        aread(0, 0, 0, 0);
+        aread(0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int q = 0; q < 16; q++)
+        for (int q = 0; q < NA * NA; q++)
 #pragma unroll
             for (int o = 0; o < 2; o++) acc[q][o] = wf4{0.f, 0.f, 0.f, 0.f};
         // In chunk ch the filters of ch + 1 are transformed into the other buffer, those of ch + 2 written to LDS as they are, those of ch + 3
@@ -234,45 +288,43 @@ struct ConvWinograd {
             const int s2 = ch < last ? 2 * ch + 2 : 2 * ch, s3 = s2 + 1, w3 = ch + 3 < last ? ch + 3 : last;
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                aread(buf, (i + 1) >> 2, (i + 1) & 3, (i + 1) & 1);
-                ustage(buf ^ 1, i);
-                if (i < 3) vrow(d[0], i + 1);
-                else vrow(d[1], 0);
-                if (i == 0) xload(s2, 0, 0);
-                if (i == 2) xload(s2, 2, 0);
-                if (i == 3) xload(s2, 1, 0);
-                mfmas(i);
-                shape();
-            }
+            for (int h = 0; h < 2; h++)
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                if (i == 3) {
-                    __syncthreads();
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-                if (i < 3) aread(buf, 1, i + 1, (i + 1) & 1);
-                else aread(buf ^ 1, 0, 0, 0);
-                if (i < 3) vrow(d[1], i + 1);
-                else vrow(d[0], 0);
-                if (i == 0) {
-                    xload(s2, 3, 0);
-                    xload(s3, 0, 1);
-                }
-                if (i == 1) {
+                for (int i = 0; i < RG; i++) {
+                    const bool ends = i + 1 == RG;
+                    if (h == 1 && ends) {
+                        __syncthreads();
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                    const int ni = ends ? 0 : i + 1, nh = ends ? h ^ 1 : h;
+                    if (ends || filter_row(ni) != filter_row(i)) aread(ends && h == 1 ? buf ^ 1 : buf, nh, filter_row(ni));
+                    vrow(d[nh], ni, (h * RG + i + 1) & 1);
+                    if (h == 0 && i < 4) ustage(buf ^ 1, i);
+                    if (h == 1 && i == 1) {
 #pragma unroll
-                    for (int u = 0; u < WL; u++) wraw(buf, u);
-                    wload(w3);
+                        for (int u = 0; u < WL; u++) wraw(buf, u);
+                        wload(w3);
+                    }
+                    if (h == 1 && ends) gread(buf);
+                    // the pixels of two steps on, each row once this step has transformed it for the last time
+                    if constexpr (S == 1) {
+                        const int s = h ? s3 : s2;
+                        if (i == 0) xload(s, 0, h);
+                        if (i == 2) xload(s, 2, h);
+                        if (i == 3) xload(s, 1, h);
+                        if (i == 3 && h == 1) xload(s, 3, h);
+                        if (i == 0 && h == 1) xload(s2, 3, 0);
+                    } else {
+                        const int s = h ? s3 : s2;
+                        if (i == 0) xload(s, 0, h);
+                        if (i == 2) xload(s, 2, h);
+                        if (i == 3) xload(s, 4, h);
+                        if (i == 4) xload(s, 1, h);
+                        if (i == 0) xload(h ? s2 : 2 * ch + 1, 3, h ^ 1);
+                    }
+                    mfmas(i, (h * RG + i) & 1);
+                    shape();
                 }
-                if (i == 2) xload(s3, 2, 1);
-                if (i == 3) {
-                    xload(s3, 1, 1);
-                    xload(s3, 3, 1);
-                    gread(buf);
-                }
-                mfmas(i);
-                shape();
-            }
         };
         int ch = 0;
         for (; ch + 1 < chunks; ch += 2) {
@@ -281,7 +333,7 @@ struct ConvWinograd {
         }
         if (ch < chunks) chunk(ch, std::integral_constant<int, 0>{});
 
-        // outputs: rows of A^T = (1 1 1 0), (0 1 -1 -1) on both sides, the middle components halved
+        // outputs: rows of A^T = (1 1 1 0), (0 1 -1 -1) on both sides, the middle components halved; strides of two (1 1 0), (0 1 1)
         if (!tile_ok) return;
         const long plane = (long) p.OH * p.OW;
         const bool right = ow + 1 < p.OW, below = oh + 1 < p.OH;
@@ -325,17 +377,30 @@ struct ConvWinograd {
 #pragma unroll
                 for (int r = 0; r < 4; r++) {
                     const int oc = oc0 + o * 16 + 4 * lk + r;
-                    float s[2][4];
+                    float s[2][NA];
 #pragma unroll
-                    for (int j = 0; j < 4; j++) {
-                        const float m1 = acc[4 + j][o][r], m2 = acc[8 + j][o][r];
-                        s[0][j] = __builtin_fmaf(0.5f, m1 + m2, acc[j][o][r]);
-                        s[1][j] = __builtin_fmaf(0.5f, m1 - m2, -acc[12 + j][o][r]);
+                    for (int j = 0; j < NA; j++) {
+                        const float m0 = acc[j][o][r], m1 = acc[NA + j][o][r], m2 = acc[2 * NA + j][o][r];
+                        if constexpr (S == 1) {
+                            s[0][j] = __builtin_fmaf(0.5f, m1 + m2, m0);
+                            s[1][j] = __builtin_fmaf(0.5f, m1 - m2, -acc[12 + j][o][r]);
+                        } else {
+                            s[0][j] = m0 + m1;
+                            s[1][j] = m1 + m2;
+                        }
                     }
                     float* y = ytile + oc * plane;
 #pragma unroll
                     for (int i = 0; i < 2; i++) {
-                        float y0 = __builtin_fmaf(0.5f, s[i][1] + s[i][2], s[i][0]) + bias[o][r], y1 = __builtin_fmaf(0.5f, s[i][1] - s[i][2], -s[i][3]) + bias[o][r];
+                        float y0, y1;
+                        if constexpr (S == 1) {
+                            y0 = __builtin_fmaf(0.5f, s[i][1] + s[i][2], s[i][0]);
+                            y1 = __builtin_fmaf(0.5f, s[i][1] - s[i][2], -s[i][3]);
+                        } else {
+                            y0 = s[i][0] + s[i][1];
+                            y1 = s[i][1] + s[i][2];
+                        }
+                        y0 += bias[o][r], y1 += bias[o][r];
                         again |= (__builtin_fabsf(y0) < __builtin_inff() ? 0u : 1u) << (16 * o + 4 * r + 2 * i);
                         again |= (__builtin_fabsf(y1) < __builtin_inff() ? 0u : 2u) << (16 * o + 4 * r + 2 * i);
                         y0 = conv_finished(fin, y0, res[o][r][i][0]), y1 = conv_finished(fin, y1, res[o][r][i][1]);
@@ -358,7 +423,7 @@ struct ConvWinograd {
             again &= again - 1;
             const int oc = oc0 + (bit >> 4) * 16 + 4 * lk + ((bit >> 2) & 3), i = (bit >> 1) & 1, j = bit & 1;
             if (oc >= p.OC || oh + i >= p.OH || ow + j >= p.OW) continue;
-            const float sum = conv3x3_direct(p.X + ((long) n * p.XC + c0) * p.H * p.W, p.Wt + ((long) oc * p.C + c0) * 9, chunks * CI, p.H, p.W, ih0 + i, iw0 + j);
+            const float sum = conv3x3_direct(p.X + ((long) n * p.XC + c0) * p.H * p.W, p.Wt + ((long) oc * p.C + c0) * 9, chunks * CI, p.H, p.W, ih0 + S * i, iw0 + S * j);
             const long to = oc * plane + (long) i * p.OW + j;
             ytile[to] = conv_finished(fin, sum + (p.bias ? p.bias[oc] : 0.f), fin.residual ? rtile[to] : -0.f);
         }
@@ -368,21 +433,42 @@ struct ConvWinograd {
 } // namespace docc_k
 
 namespace docc_k {
-template <int NW, bool WIDE>
-__device__ __forceinline__ void conv_winograd(const ConvParams& p, const ConvFinish& fin) {
-    typedef ConvWinograd<NW> K;
+// sums: null, or where the part blockIdx.y of the channels (of gridDim.y) leaves its sums as [part][N][OC][OH][OW]
+template <int S, int LOADS>
+__device__ __forceinline__ void conv_winograd(ConvParams p, ConvFinish fin, float* sums) {
+    typedef ConvWinograd<S> K;
+    constexpr int TILES = 16 * K::NW;
     __shared__ __attribute__((aligned(16))) float lds[K::LDS_FLOATS];
     const int ocb = (p.OC + 31) >> 5, id = xcd_contiguous(blockIdx.x, gridDim.x);
-    const int oc0 = (id % ocb) * 32, tile0 = (id / ocb) * (16 * NW);
-    // WIDE: the last tile that reads the column before the first row of the tensor (row 0 of image 0 is among its rows), and the first
-    // that reads the column behind its last row
-    const int TH = (p.OH + 1) >> 1, TW = (p.OW + 1) >> 1;
-    const int before = (p.pad_h >> 1) * TW, bottom = (p.H - 3 + p.pad_h) >> 1;
-    const long behind = (long) (p.N - 1) * TH * TW + (long) (bottom > 0 ? bottom : 0) * TW + TW - 1;
-    if (WIDE && tile0 > before && tile0 + 16 * NW <= behind) K::template run<true>(p, fin, lds, tile0, oc0, 0, p.C / 8);
-    else K::template run<false>(p, fin, lds, tile0, oc0, 0, p.C / 8);
+    const int oc0 = (id % ocb) * 32, tile0 = (id / ocb) * TILES;
+    int first = 0, chunks = p.C / K::CI;
+    if (sums) {
+        first = (int) ((long) chunks * blockIdx.y / gridDim.y);
+        chunks = (int) ((long) chunks * (blockIdx.y + 1) / gridDim.y) - first;
+        p.Y = sums + (long) blockIdx.y * p.N * p.OC * p.OH * p.OW;
+        p.bias = nullptr;
+        fin = ConvFinish{nullptr, 0};
+    }
+    if constexpr (S == 1 && LOADS != kPixels) {
+        // the last tile that reads the column before the first row of the tensor (row 0 of image 0 is among its rows), and the first
+        // that reads columns behind its last row
+        const int TH = (p.OH + 1) >> 1, TW = (p.OW + 1) >> 1;
+        const int before = (p.pad_h >> 1) * TW, bottom = (p.H - 3 + p.pad_h) >> 1;
+        const long behind = (long) (p.N - 1) * TH * TW + (long) (bottom > 0 ? bottom : 0) * TW + TW - 1;
+        if (tile0 > before && tile0 + TILES <= behind) K::template run<LOADS>(p, fin, lds, tile0, oc0, first * K::CI, chunks);
+        else K::template run<kPixels>(p, fin, lds, tile0, oc0, first * K::CI, chunks);
+    } else {
+        K::template run<LOADS>(p, fin, lds, tile0, oc0, first * K::CI, chunks);
+    }
 }
 } // namespace docc_k
 
-extern "C" __global__ __launch_bounds__(256, 2) void docc_conv2d_f32_winograd(docc_k::ConvParams p, docc_k::ConvFinish f) { docc_k::conv_winograd<4, false>(p, f); }
-extern "C" __global__ __launch_bounds__(256, 2) void docc_conv2d_f32_winograd_wide(docc_k::ConvParams p, docc_k::ConvFinish f) { docc_k::conv_winograd<4, true>(p, f); }
+#define DOCC_CONV_WINOGRAD(NAME, S, LOADS)                                                                                                \
+    extern "C" __global__ __launch_bounds__(256, 2) void NAME(docc_k::ConvParams p, docc_k::ConvFinish f, float* sums) {                  \
+        docc_k::conv_winograd<S, docc_k::LOADS>(p, f, sums);                                                                              \
+    }
+DOCC_CONV_WINOGRAD(docc_conv2d_f32_winograd_pixels, 1, kPixels)
+DOCC_CONV_WINOGRAD(docc_conv2d_f32_winograd_vector, 1, kVector)
+DOCC_CONV_WINOGRAD(docc_conv2d_f32_winograd_vector_odd, 1, kVectorOdd)
+DOCC_CONV_WINOGRAD(docc_conv2d_f32_winograd_s2_vector, 2, kVector)
+DOCC_CONV_WINOGRAD(docc_conv2d_f32_winograd_s2_pairs, 2, kPairs)

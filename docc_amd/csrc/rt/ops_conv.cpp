@@ -204,6 +204,14 @@ double gemm_time_us(int64_t N, int64_t OC, int64_t P, int64_t K, bool needs_colu
 // bytes of columns + GEMM result per image
 int64_t conv_bytes_per_image(int64_t OC, int64_t K, int64_t P) { return (K * P * 4 + 255) / 256 * 256 + (OC * P * 4 + 255) / 256 * 256; }
 
+// Y = act(bias + the sums of the channels' parts + residual)
+int add_parts(hipStream_t stream, const float* sums, const float* bias, float* Y, int64_t total, int64_t plane, int64_t OC, int64_t parts, const ConvFinish& fin) {
+    const bool vectors = total % 4 == 0 && ((uintptr_t) Y | (uintptr_t) fin.residual) % 16 == 0;
+    const int64_t items = vectors ? total / 4 : total, blocks = (items + 255) / 256;
+    return launch(vectors ? "docc_conv2d_add_parts_f32_v4" : "docc_conv2d_add_parts_f32", (uint32_t) (blocks < 2048 ? blocks : 2048), 1, 1, 256, 0, stream, sums, bias, Y,
+                  (long) total, (int) plane, (int) OC, (int) parts, fin);
+}
+
 enum class ConvPath { Halo, Gather, Gemm1x1, GemmColumns, Winograd };
 
 // shapes the LDS-halo kernel is built for (the launcher also wants 16-byte aligned weights)
@@ -212,24 +220,46 @@ bool halo_shape_ok(int64_t C, int64_t KH, int64_t KW, int64_t OW, int64_t stride
            C % 8 == 0 && C > 0 && OW <= 448 && (C * KH * KW) % 4 == 0 && halo_strip_fits(1, OW, KH, KW, stride_h, stride_w);
 }
 
-// Winograd's form (csrc/kernels/conv_winograd.hip): 3x3 filters one pixel apart, whole chunks of eight channels. A work-group addresses its
+// Winograd's form (csrc/kernels/conv_winograd.hip): 3x3 filters one or two pixels apart, whole chunks of eight channels. A work-group addresses its
 // images and filters by 32-bit offsets.
 bool winograd_shape_ok(int64_t N, int64_t C, int64_t H, int64_t W, int64_t OC, int64_t KH, int64_t KW, int64_t OH, int64_t OW, int64_t stride_h, int64_t stride_w,
                        int64_t pad_h, int64_t pad_w, int64_t dil_h, int64_t dil_w) {
-    if (KH != 3 || KW != 3 || stride_h != 1 || stride_w != 1 || dil_h != 1 || dil_w != 1 || C <= 0 || C % 8 != 0) return false;
+    if (stride_w == 2 && (W < 2 || (pad_w > 0 && pad_w % 2 == 0))) return false;   // (pairs of pixels, see the kernel)
+    if (KH != 3 || KW != 3 || stride_h != stride_w || stride_h < 1 || stride_h > 2 || dil_h != 1 || dil_w != 1 || C <= 0 || C % 8 != 0) return false;
     const int64_t per_image = ((OH + 1) / 2) * ((OW + 1) / 2), images = (kWinogradTiles + per_image - 2) / per_image + 1;
     return images * C * H * W < (int64_t(1) << 28) && 32 * C * 9 < (int64_t(1) << 28) && N * per_image < (int64_t(1) << 30) &&
            N * OH * OW * OC < (int64_t(1) << 40) && winograd_groups(N, OC, OH, OW) < (int64_t(1) << 30) && pad_h < (int64_t(1) << 20) && pad_w < (int64_t(1) << 20);
 }
 
-// us: a chunk of eight channels takes a work-group 1.17 of a CU's time where another one fills its gaps and 1.43 alone; 4 us around them.
+// How a layer runs in Winograd's form. us: a chunk of eight channels takes a work-group 1.17 of a CU's time where another one fills its gaps and
+// 1.43 alone (steps of two 1.62 and 1.9; they have 25 products a channel for 16), 4 us around them. Few work-groups with many chunks: the channels go
+// to several of them, whose sums a second launch adds (3 us, and the parts at 3 TB/s).
 // Measured against the other forms on 60 drawn layers (1-64 images, 8-512 channels, 7x7 to 64x64), "before -> now": 8 x 272 x 40 x 40 244 -> 86 us,
-// 32 x 64 x 56 x 56 71 -> 48, 34 x 80 x 24 x 24 53 -> 24, 3 x 32 x 19 x 19 13.1 -> 11.5; 1 x 368 x 9 x 9 is left to the direct form with its channels
-// in parts (18 us; 65 here: 12 work-groups), as is 12 x 416 x 11 x 11 (58; 77).
-double winograd_time_us(int64_t N, int64_t C, int64_t OC, int64_t OH, int64_t OW, int cus) {
-    const int64_t groups = winograd_groups(N, OC, OH, OW), rounds = groups / (2 * cus), rest = groups % (2 * cus);
-    const double chunks = (double) (C / 8), pair = 2 * 1.17 * chunks + 4.0;
-    return (double) rounds * pair + (rest == 0 ? 0.0 : rest <= cus ? 1.43 * chunks + 4.0 : pair);
+// 32 x 64 x 56 x 56 71 -> 48, 34 x 80 x 24 x 24 53 -> 24, 3 x 32 x 19 x 19 13.1 -> 11.5; steps of two: 23 x 240 x 36 x 36 240 -> 101.
+struct WinogradPlan {
+    int64_t parts = 1;
+    double us = 0;
+};
+WinogradPlan plan_winograd(int64_t N, int64_t C, int64_t OC, int64_t OH, int64_t OW, int64_t stride, bool parts_ok, int cus) {
+    const int64_t chunks = C / 8, total = N * OC * OH * OW;
+    auto us = [&](int64_t parts) {
+        const int64_t groups = winograd_groups(N, OC, OH, OW) * parts, rounds = groups / (2 * cus), rest = groups % (2 * cus);
+        const double each = (double) ((chunks + parts - 1) / parts), pair = 2 * (stride == 1 ? 1.17 : 1.62) * each + 4.0, alone = (stride == 1 ? 1.43 : 1.9) * each + 4.0;
+        return (double) rounds * pair + (rest == 0 ? 0.0 : rest <= cus ? alone : pair) + (parts > 1 ? 3.0 + (double) (parts + 1) * 4.0 * (double) total / 3e6 : 0.0);
+    };
+    WinogradPlan plan{1, us(1)};
+    if (!parts_ok || total > (int64_t(1) << 26)) return plan;
+    const char* force = std::getenv("DOCC_ROCM_CONV");
+    const char* cut = force && force[0] == 'w' ? std::strstr(force, "-parts") : nullptr;   // winograd-parts<n>: that many (tests, tuning)
+    if (cut && std::atoll(cut + 6) >= 1 && std::atoll(cut + 6) <= chunks) return WinogradPlan{std::atoll(cut + 6), us(std::atoll(cut + 6))};
+    if (cut) return plan;
+    double best = plan.us / 1.1;
+    for (const int64_t parts : {2, 3, 4, 6, 8, 12, 16, 24, 32}) {
+        if (parts * 2 > chunks || parts * total > (int64_t(1) << 26)) break;
+        const double t = us(parts);
+        if (t < best) best = t, plan = WinogradPlan{parts, t};
+    }
+    return plan;
 }
 
 ConvPath choose_path(int64_t N, int64_t C, int64_t OC, int64_t KH, int64_t KW, int64_t OH, int64_t OW, int64_t stride_h, int64_t stride_w,
@@ -254,8 +284,9 @@ ConvPath choose_path(int64_t N, int64_t C, int64_t OC, int64_t KH, int64_t KW, i
     const double direct = halo_ok ? halo.cost * halo_unit_us(K) : gather_time_us(N, OC, P, K, cus);
     const double columns = gemm_fast ? gemm_time_us(N, OC, P, K, true) : 1e30;
     if (winograd_ok) {
+        const WinogradPlan plan = plan_winograd(N, C, OC, OH, OW, stride_h, parts_ok, cus);
         const double around = columns < direct || halo.parts == 1 ? 4.0 : 0.0;   // what the other estimates leave out (that of the parts does not)
-        if (winograd_time_us(N, C, OC, OH, OW, cus) < 0.95 * ((columns < direct ? columns : direct) + around)) return ConvPath::Winograd;
+        if (plan.us < 0.95 * ((columns < direct ? columns : direct) + around)) return ConvPath::Winograd;
     }
     if (columns < 0.75 * direct) return gemm;
     return halo_ok ? ConvPath::Halo : ConvPath::Gather;
@@ -326,7 +357,7 @@ static int conv2d_run(docc_rocm_stream_t stream, int64_t N, int64_t C, int64_t H
     // Stride-1, dilation-1 3x3 and 1x1 convolutions take the LDS-halo kernel: 64 output channels x a
     // strip of TH full output rows (at most 448 pixels) per work-group, 8 input channels per chunk.
     const bool halo_shape = halo_shape_ok(C, KH, KW, OW, stride_h, stride_w, dil_h, dil_w) && ((uintptr_t) Wt % 16 == 0);
-    const bool winograd = !slice && winograd_shape_ok(N, C, H, W, OC, KH, KW, OH, OW, stride_h, stride_w, any_pad_h, any_pad_w, dil_h, dil_w);
+    const bool winograd = !slice && winograd_shape_ok(N, C, H, W, OC, KH, KW, OH, OW, stride_h, stride_w, pad_h, pad_w, dil_h, dil_w);
     const int64_t need = !workspace ? 0 : docc_rocm_conv2d_f32_pads_workspace_bytes(N, C, H, W, OC, KH, KW, stride_h, stride_w, pad_h, pad_w, pad_h_end,
                                                                                     pad_w_end, dil_h, dil_w);
     const bool have_workspace = workspace && workspace_bytes >= need && need > 0 && ((uintptr_t) workspace % 256) == 0;
@@ -338,12 +369,22 @@ static int conv2d_run(docc_rocm_stream_t stream, int64_t N, int64_t C, int64_t H
     // GEMM paths write whole [N, OC, P] tensors)
     if (slice && (path == ConvPath::Gemm1x1 || path == ConvPath::GemmColumns)) path = halo_shape ? ConvPath::Halo : ConvPath::Gather;
     if (path == ConvPath::Winograd) {
-        // rows of whole tiles between one column of padding on either side: four pixels a load
+        int cus = compute_units();
+        if (cus <= 0) cus = 256;
         const char* force = std::getenv("DOCC_ROCM_CONV");
-        const bool wide = any_pad_w == 1 && OW == W && W % 2 == 0 && !(force && std::strstr(force, "-narrow"));
+        const bool pixels = force && std::strstr(force, "-pixels");   // tests: without the wider loads
+        const char* name = stride_w == 2 ? (pad_w == 1 && OW * 2 == W && W % 4 == 0 && !pixels ? "docc_conv2d_f32_winograd_s2_vector" : "docc_conv2d_f32_winograd_s2_pairs")
+                           : any_pad_w == 1 && OW == W && !pixels ? (W % 2 == 0 ? "docc_conv2d_f32_winograd_vector" : "docc_conv2d_f32_winograd_vector_odd")
+                                                                  : "docc_conv2d_f32_winograd_pixels";
+        const int64_t parts = plan_winograd(N, C, OC, OH, OW, stride_h, parts_ok, cus).parts, total = N * OC * OH * OW;
+        float* sums = nullptr;
+        if (parts > 1 && docc_rocm_malloc_async((void**) &sums, (size_t) (parts * total * 4), stream) != 0) sums = nullptr;   // without memory for the sums the layer runs whole
         if (finished) *finished = true;
-        return launch(wide ? "docc_conv2d_f32_winograd_wide" : "docc_conv2d_f32_winograd", (uint32_t) winograd_groups(N, OC, OH, OW), 1, 1, 256, 0,
-                      (hipStream_t) stream, p, fin);
+        rc = launch(name, (uint32_t) winograd_groups(N, OC, OH, OW), sums ? (uint32_t) parts : 1, 1, 256, 0, (hipStream_t) stream, p, fin, sums);
+        if (!sums) return rc;
+        if (!rc) rc = add_parts((hipStream_t) stream, sums, bias, Y, total, OH * OW, OC, parts, fin);
+        const int freed = docc_rocm_free_async(sums, stream);
+        return rc ? rc : freed;
     }
     if (path == ConvPath::Gemm1x1) {
         // Y[n] (OC x P) = W (OC x C) X[n] (C x P): one batched GEMM on the tensors as they lie; the bias is
@@ -408,12 +449,8 @@ static int conv2d_run(docc_rocm_stream_t stream, int64_t N, int64_t C, int64_t H
             const int64_t total = N * OC * OH * OW;
             rc = launch(name, (uint32_t) (plan.images > 1 ? (N + plan.images - 1) / plan.images : N * strips), (uint32_t) ((OC + 63) / 64),
                         (uint32_t) plan.parts, 256, (uint32_t) (3 * stage * 4), (hipStream_t) stream, p, (int) TH, (int) plan.images, sums);
-            const bool vectors = total % 4 == 0 && ((uintptr_t) Y | (uintptr_t) fin.residual) % 16 == 0;
             if (finished) *finished = true;
-            const int64_t items = vectors ? total / 4 : total, blocks = (items + 255) / 256;
-            if (!rc)
-                rc = launch(vectors ? "docc_conv2d_add_parts_f32_v4" : "docc_conv2d_add_parts_f32", (uint32_t) (blocks < 2048 ? blocks : 2048), 1, 1, 256, 0,
-                            (hipStream_t) stream, (const float*) sums, bias, Y, (long) total, (int) (OH * OW), (int) OC, (int) plan.parts, fin);
+            if (!rc) rc = add_parts((hipStream_t) stream, sums, bias, Y, total, OH * OW, OC, plan.parts, fin);
             const int freed = docc_rocm_free_async(sums, stream);
             return rc ? rc : freed;
         }

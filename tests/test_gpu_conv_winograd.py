@@ -26,27 +26,36 @@ CASES = [  # N, C, H, W, OC, pads (top, left, bottom, right)
 ]
 
 
-def run(rt, X, W, bias, pads):
+# strides of two
+STRIDED = [
+    (1, 8, 1, 1, 1, (1, 1, 1, 1)), (1, 8, 3, 3, 2, (0, 0, 0, 0)), (2, 16, 9, 13, 31, (1, 1, 1, 1)), (3, 24, 32, 32, 33, (1, 1, 1, 1)),
+    (9, 8, 16, 16, 40, (1, 1, 0, 0)), (2, 32, 17, 400, 32, (1, 1, 1, 1)), (70, 8, 4, 4, 32, (1, 1, 1, 1)), (2, 16, 14, 12, 64, (2, 1, 0, 1)),
+    (1, 16, 131, 8, 32, (3, 1, 2, 0)), (2, 16, 10, 11, 32, (0, 2, 1, 3)), (4, 64, 28, 28, 96, (1, 1, 1, 1)),
+]
+
+
+def run(rt, X, W, bias, pads, stride=1):
     N, C, H, Wd = X.shape
     OC = W.shape[0]
-    OH, OW = H + pads[0] + pads[2] - 2, Wd + pads[1] + pads[3] - 2
+    OH, OW = (H + pads[0] + pads[2] - 3) // stride + 1, (Wd + pads[1] + pads[3] - 3) // stride + 1
     y = torch.full((N, OC, OH, OW), float("nan"), device="cuda")
     x, w = dev(X), dev(W)
     b = dev(bias) if bias is not None else None
-    rt.conv2d_f32_pads(N, C, H, Wd, OC, 3, 3, (1, 1), pads, (1, 1), x.data_ptr(), w.data_ptr(), b.data_ptr() if b is not None else 0, y.data_ptr())
+    rt.conv2d_f32_pads(N, C, H, Wd, OC, 3, 3, (stride, stride), pads, (1, 1), x.data_ptr(), w.data_ptr(), b.data_ptr() if b is not None else 0, y.data_ptr())
     torch.cuda.synchronize()
     return host(y)
 
 
-def padded_reference(X, W, bias, pads):
+def padded_reference(X, W, bias, pads, stride=1):
     """The oracle takes the same padding on both sides: the rest is put around the image."""
     Xp = np.pad(X, ((0, 0), (0, 0), (pads[0], pads[2]), (pads[1], pads[3])))
-    return oracle.conv2d(Xp, W, bias)
+    return oracle.conv2d(Xp, W, bias, (stride, stride))
 
 
-@pytest.mark.parametrize("force", ["winograd", "winograd-narrow"])
-@pytest.mark.parametrize("case", CASES, ids=[f"n{c[0]}c{c[1]}_{c[2]}x{c[3]}_oc{c[4]}_p{''.join(map(str, c[5]))}" for c in CASES])
-def test_winograd_matches_oracle(rt, monkeypatch, force, case):
+@pytest.mark.parametrize("force", ["winograd", "winograd-pixels", "winograd-parts2", "winograd-parts3"])
+@pytest.mark.parametrize("stride,case", [(1, c) for c in CASES] + [(2, c) for c in STRIDED],
+                         ids=[f"s{k}n{c[0]}c{c[1]}_{c[2]}x{c[3]}_oc{c[4]}_p{''.join(map(str, c[5]))}" for k, cs in ((1, CASES), (2, STRIDED)) for c in cs])
+def test_winograd_matches_oracle(rt, monkeypatch, force, stride, case):
     N, C, H, W, OC, pads = case
     monkeypatch.setenv("DOCC_ROCM_CONV", force)
     rng = np.random.default_rng(C + H + W)
@@ -54,21 +63,22 @@ def test_winograd_matches_oracle(rt, monkeypatch, force, case):
     Wt = rng.integers(-4, 5, (OC, C, 3, 3)).astype(np.float32)
     b = rng.integers(-4, 5, OC).astype(np.float32)
     # whole numbers: the transforms give multiples of a quarter, nothing rounds
-    assert np.array_equal(run(rt, X, Wt, b, pads), padded_reference(X, Wt, b, pads))
+    assert np.array_equal(run(rt, X, Wt, b, pads, stride), padded_reference(X, Wt, b, pads, stride))
     X = rng.standard_normal(X.shape).astype(np.float32)
     Wt = (rng.standard_normal(Wt.shape) * np.sqrt(2.0 / (9 * C))).astype(np.float32)
-    assert rel_err_max(run(rt, X, Wt, None, pads), padded_reference(X, Wt, None, pads)) <= 1e-5
+    assert rel_err_max(run(rt, X, Wt, None, pads, stride), padded_reference(X, Wt, None, pads, stride)) <= 1e-5
 
 
-@pytest.mark.parametrize("force", ["winograd", "winograd-narrow"])
-def test_values_that_are_not_finite_stay_where_they_are(rt, monkeypatch, force):
+@pytest.mark.parametrize("stride", [1, 2])
+@pytest.mark.parametrize("force", ["winograd", "winograd-pixels"])
+def test_values_that_are_not_finite_stay_where_they_are(rt, monkeypatch, force, stride):
     """Infinities, NaNs and values near the largest (whose sums the input transform overflows) give the direct form's outputs in
     their windows, and change no output elsewhere."""
     monkeypatch.setenv("DOCC_ROCM_CONV", force)
     rng = np.random.default_rng(5)
-    X = rng.standard_normal((6, 16, 10, 10)).astype(np.float32)
+    X = rng.standard_normal((6, 16, 12, 12)).astype(np.float32)
     Wt = (rng.standard_normal((32, 16, 3, 3)) * 0.1).astype(np.float32)
-    clean = oracle.conv2d(X, Wt, None, pad=(1, 1))
+    clean = oracle.conv2d(X, Wt, None, (stride, stride), (1, 1))
     X[0, 3, 4, 4] = np.inf
     X[1, 2, 0, 0] = -np.inf
     X[2, 1, 9, 9] = np.nan
@@ -76,8 +86,8 @@ def test_values_that_are_not_finite_stay_where_they_are(rt, monkeypatch, force):
     X[4, 7, 4, 4], X[4, 7, 4, 6], X[4, 7, 6, 4] = 3e38, -3e38, 3e38
     Wt[31, 15, 0, 0] = 0.0
     with np.errstate(all="ignore"):
-        ref = oracle.conv2d(X, Wt, None, pad=(1, 1))
-    Y = run(rt, X, Wt, None, (1, 1, 1, 1))
+        ref = oracle.conv2d(X, Wt, None, (stride, stride), (1, 1))
+    Y = run(rt, X, Wt, None, (1, 1, 1, 1), stride)
     assert np.array_equal(np.isnan(Y), np.isnan(ref)) and np.array_equal(np.isinf(Y), np.isinf(ref.astype(np.float32)))
     assert np.array_equal(np.sign(Y[np.isinf(Y)]), np.sign(ref[np.isinf(ref)]))
     ok = np.isfinite(ref)
