@@ -55,6 +55,7 @@ KERNEL_FAMILIES = {
     "layernorm": "layernorm.hip",
     "conv2d": "conv2d.hip",
     "conv_winograd": "conv_winograd.hip",
+    "conv_1x1": "conv_1x1.hip",
     "attention": "attention.hip",
     "attention_split": "attention_split.hip",
     "elementwise": "elementwise.hip",
@@ -83,6 +84,7 @@ FAMILY_FLAGS = {
     "gemm_f32_finish": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "conv2d": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "conv_winograd": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+    "conv_1x1": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "attention": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "attention_split": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "gemm_skinny": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],

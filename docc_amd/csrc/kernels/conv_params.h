@@ -28,4 +28,10 @@ __device__ __forceinline__ float conv_finished(const ConvFinish& f, float v, flo
     return f.relu ? fmaxf(v, 0.0f) : v;
 }
 
+// Work-groups are dealt to the 8 XCDs in turn: number them so that an XCD gets consecutive ones (whose work shares input).
+__device__ __forceinline__ int xcd_contiguous(int id, int n) {
+    const int xcd = id & 7, q = n >> 3, r = n & 7;
+    return xcd * q + (xcd < r ? xcd : r) + (id >> 3);
+}
+
 } // namespace docc_k

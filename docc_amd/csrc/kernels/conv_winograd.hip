@@ -42,12 +42,6 @@ namespace docc_k {
 typedef float wf4 __attribute__((ext_vector_type(4)));
 typedef float wf2 __attribute__((ext_vector_type(2)));
 
-// Work-groups are dealt to the 8 XCDs in turn: number them so that an XCD gets consecutive ones (whose work shares input).
-__device__ __forceinline__ int xcd_contiguous(int id, int n) {
-    const int xcd = id & 7, q = n >> 3, r = n & 7;
-    return xcd * q + (xcd < r ? xcd : r) + (id >> 3);
-}
-
 // one output the direct way: channels [0, C) of X and Wt as given
 __device__ __forceinline__ float conv3x3_direct(const float* xn, const float* w, int C, int H, int W, int ih0, int iw0) {
     float sum = 0.f;

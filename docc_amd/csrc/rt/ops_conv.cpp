@@ -212,7 +212,7 @@ int add_parts(hipStream_t stream, const float* sums, const float* bias, float* Y
                   (long) total, (int) plane, (int) OC, (int) parts, fin);
 }
 
-enum class ConvPath { Halo, Gather, Gemm1x1, GemmColumns, Winograd };
+enum class ConvPath { Halo, Gather, Gemm1x1, GemmColumns, Winograd, Direct1x1 };
 
 // shapes the LDS-halo kernel is built for (the launcher also wants 16-byte aligned weights)
 bool halo_shape_ok(int64_t C, int64_t KH, int64_t KW, int64_t OW, int64_t stride_h, int64_t stride_w, int64_t dil_h, int64_t dil_w) {
@@ -262,14 +262,34 @@ WinogradPlan plan_winograd(int64_t N, int64_t C, int64_t OC, int64_t OH, int64_t
     return plan;
 }
 
+// 1x1 filters on the kernel that takes X as it lies (csrc/kernels/conv_1x1.hip): vectors of four channels, 32-bit offsets within a work-group's images
+bool direct_1x1_shape_ok(int64_t N, int64_t C, int64_t H, int64_t W, int64_t OC, int64_t KH, int64_t KW, int64_t OH, int64_t OW, int64_t stride_h, int64_t stride_w,
+                         int64_t pad_h, int64_t pad_w) {
+    if (KH != 1 || KW != 1 || C <= 0 || C % 4 != 0) return false;
+    const int64_t images = (64 + OH * OW - 2) / (OH * OW) + 1, lim = int64_t(1) << 30;
+    return images * C * H * W < (int64_t(1) << 28) && 64 * C < (int64_t(1) << 28) && N * OH * OW < lim && (N * OH * OW + 63) / 64 * ((OC + 63) / 64) < lim &&
+           OH * stride_h < lim && OW * stride_w < lim && pad_h < lim && pad_w < lim;
+}
+
+// Where it pays, measured on 34 layers: with steps always (32 x 128 x 28 x 28 -> 256 19 -> 13 us, 13 x 256 x 57 x 57 -> 512 84 -> 46, 36 x 32 x 12 x 12 -> 64
+// 9 -> 7); without, 16 x 128 x 28 x 28 -> 512 52 -> 32 us, 64 x 2048 x 7 x 7 -> 512 189 -> 89, but not where few work-groups have many channels (1 x 512 x 28 x 28
+// -> 128: 17 us for the batched product's 13) nor where many have two chunks of them (32 x 64 x 56 x 56 -> 256: 70 us for the strips' 65).
+bool direct_1x1_pays(int64_t N, int64_t C, int64_t OC, int64_t OH, int64_t OW, int64_t stride_h, int64_t stride_w, int cus) {
+    if (stride_h > 1 || stride_w > 1) return true;
+    const int64_t groups = (N * OH * OW + 63) / 64 * ((OC + 63) / 64);
+    return C < 96 ? groups < 16 * (int64_t) cus : C <= 256 || groups >= cus / 2;
+}
+
 ConvPath choose_path(int64_t N, int64_t C, int64_t OC, int64_t KH, int64_t KW, int64_t OH, int64_t OW, int64_t stride_h, int64_t stride_w,
-                     int64_t pad_h, int64_t pad_w, bool halo_ok, bool have_workspace, bool parts_ok, bool winograd_ok) {
-    const char* force = std::getenv("DOCC_ROCM_CONV");   // halo | gather | gemm | winograd (tuning and tests)
+                     int64_t pad_h, int64_t pad_w, bool halo_ok, bool have_workspace, bool parts_ok, bool winograd_ok,
+                     bool direct_1x1_ok) {
+    const char* force = std::getenv("DOCC_ROCM_CONV");   // halo | gather | gemm | winograd | straight (tuning and tests)
     const bool pointwise = KH == 1 && KW == 1 && stride_h == 1 && stride_w == 1 && pad_h == 0 && pad_w == 0;
     const ConvPath gemm = pointwise ? ConvPath::Gemm1x1 : ConvPath::GemmColumns;
     const bool gemm_ok = pointwise || have_workspace;
     if (force && force[0] == 'h' && halo_ok) return ConvPath::Halo;
     if (force && force[0] == 'w' && winograd_ok) return ConvPath::Winograd;
+    if (force && force[0] == 's' && direct_1x1_ok) return ConvPath::Direct1x1;
     if (force && force[0] == 'g' && force[1] == 'a') return ConvPath::Gather;
     if (force && force[0] == 'g' && force[1] == 'e' && gemm_ok) return gemm;
     int cus = compute_units();
@@ -277,10 +297,14 @@ ConvPath choose_path(int64_t N, int64_t C, int64_t OC, int64_t KH, int64_t KW, i
     const int64_t K = C * KH * KW, P = OH * OW;
     // the aligned GEMM kernels want rows of the weight and column matrices that are multiples of 16 bytes
     const bool gemm_fast = gemm_ok && K % 4 == 0 && (pointwise ? P % 4 == 0 : true);
+    const HaloPlan halo = halo_ok ? plan_halo(N, parts_ok ? C : 0, OC, OH, OW, KH, KW, stride_h, stride_w, cus) : HaloPlan{};
+    if (direct_1x1_ok && direct_1x1_pays(N, C, OC, OH, OW, stride_h, stride_w, cus)) {
+        // (a chain of many chunks on few work-groups, 0.8 us each, is left to the strips with their channels in parts)
+        if (!(halo.parts > 1 && halo.cost * halo_unit_us(K) < 0.8 * (double) ((C + 31) / 32) + 4.0)) return ConvPath::Direct1x1;
+    }
     // 1x1 layers move more bytes than they compute, which the models above do not see: measured, the batched GEMM
     // wins from 128 input channels on (C 256 -> 64 on 56 x 56: 50 against 65 us; C 64 -> 256: 99 against 74)
     if (pointwise) return gemm_fast && C >= 128 ? gemm : halo_ok ? ConvPath::Halo : ConvPath::Gather;
-    const HaloPlan halo = halo_ok ? plan_halo(N, parts_ok ? C : 0, OC, OH, OW, KH, KW, stride_h, stride_w, cus) : HaloPlan{};
     const double direct = halo_ok ? halo.cost * halo_unit_us(K) : gather_time_us(N, OC, P, K, cus);
     const double columns = gemm_fast ? gemm_time_us(N, OC, P, K, true) : 1e30;
     if (winograd_ok) {
@@ -308,7 +332,7 @@ extern "C" int64_t docc_rocm_conv2d_f32_pads_workspace_bytes(int64_t N, int64_t 
     // nothing either when one of the direct kernels would be chosen anyway (operands assumed aligned, the channels in one
     // piece: cutting them takes memory of its own, which the call may not get; Winograd's form aside, which a call may be forced off)
     const bool halo_ok = halo_shape_ok(C, KH, KW, OW, stride_h, stride_w, dil_h, dil_w);
-    if (choose_path(N, C, OC, KH, KW, OH, OW, stride_h, stride_w, pad_h, pad_w, halo_ok, true, false, false) != ConvPath::GemmColumns) return 0;
+    if (choose_path(N, C, OC, KH, KW, OH, OW, stride_h, stride_w, pad_h, pad_w, halo_ok, true, false, false, false) != ConvPath::GemmColumns) return 0;
     const int64_t per_image = conv_bytes_per_image(OC, C * KH * KW, OH * OW);
     int64_t images = kConvWorkspaceCap / per_image;
     if (images < 1) images = 1;
@@ -364,7 +388,7 @@ static int conv2d_run(docc_rocm_stream_t stream, int64_t N, int64_t C, int64_t H
     const bool parts_ok = !slice && !foreign_capture((hipStream_t) stream);   // cutting the channels takes a block of the cache
     ConvPath path = C == 0 ? ConvPath::Gather
                            : choose_path(N, C, OC, KH, KW, OH, OW, stride_h, stride_w, any_pad_h, any_pad_w, halo_shape, have_workspace, parts_ok,
-                                         winograd);
+                                         winograd, !slice && direct_1x1_shape_ok(N, C, H, W, OC, KH, KW, OH, OW, stride_h, stride_w, any_pad_h, any_pad_w));
     // one group of a grouped convolution: the direct kernels, which take the distance between the images as it is (the
     // GEMM paths write whole [N, OC, P] tensors)
     if (slice && (path == ConvPath::Gemm1x1 || path == ConvPath::GemmColumns)) path = halo_shape ? ConvPath::Halo : ConvPath::Gather;
@@ -385,6 +409,10 @@ static int conv2d_run(docc_rocm_stream_t stream, int64_t N, int64_t C, int64_t H
         if (!rc) rc = add_parts((hipStream_t) stream, sums, bias, Y, total, OH * OW, OC, parts, fin);
         const int freed = docc_rocm_free_async(sums, stream);
         return rc ? rc : freed;
+    }
+    if (path == ConvPath::Direct1x1) {
+        if (finished) *finished = true;
+        return launch("docc_conv2d_f32_1x1", (uint32_t) ((N * OH * OW + 63) / 64 * ((OC + 63) / 64)), 1, 1, 256, 0, (hipStream_t) stream, p, fin);
     }
     if (path == ConvPath::Gemm1x1) {
         // Y[n] (OC x P) = W (OC x C) X[n] (C x P): one batched GEMM on the tensors as they lie; the bias is

@@ -53,6 +53,7 @@ const char* const kKernelImages[] = {
     "docc_rocm_layernorm.hsaco",
     "docc_rocm_conv2d.hsaco",
     "docc_rocm_conv_winograd.hsaco",
+    "docc_rocm_conv_1x1.hsaco",
     "docc_rocm_attention.hsaco",
     "docc_rocm_attention_split.hsaco",
     "docc_rocm_elementwise.hsaco",

@@ -97,7 +97,26 @@ def test_values_that_are_not_finite_stay_where_they_are(rt, monkeypatch, force, 
     assert np.abs(Y[small] - ref[small]).max() <= 1e-5 * np.abs(clean).max()
 
 
-@pytest.mark.parametrize("force", ["", "winograd", "halo-t4-parts2", "halo", "gather", "gemm"])
+# 1x1 filters on the kernel that takes X as it lies (csrc/kernels/conv_1x1.hip): work-groups of 64 pixels by 64 channels, chunks of 32 channels in
+@pytest.mark.parametrize("case", [  # N, C, H, W, OC, steps, pads (top, left, bottom, right)
+    (1, 4, 1, 1, 1, (1, 1), (0, 0, 0, 0)), (2, 32, 9, 7, 64, (1, 1), (0, 0, 0, 0)), (1, 36, 8, 8, 65, (2, 2), (0, 0, 0, 0)), (70, 12, 2, 3, 33, (2, 2), (0, 0, 0, 0)),
+    (3, 100, 15, 17, 70, (2, 1), (1, 0, 0, 1)), (2, 128, 28, 28, 256, (2, 2), (0, 0, 0, 0)), (2, 160, 5, 5, 48, (3, 2), (1, 2, 2, 1)),
+], ids=str)
+def test_1x1_matches_oracle(rt, monkeypatch, case):
+    N, C, H, W, OC, steps, pads = case
+    monkeypatch.setenv("DOCC_ROCM_CONV", "straight")
+    rng = np.random.default_rng(C + H)
+    for draw in (lambda *s: rng.integers(-4, 5, s), lambda *s: rng.standard_normal(s)):
+        X, Wt, b = (draw(*s).astype(np.float32) for s in ((N, C, H, W), (OC, C, 1, 1), (OC,)))
+        ref = oracle.conv2d(np.pad(X, ((0, 0), (0, 0), (pads[0], pads[2]), (pads[1], pads[3]))), Wt, b, steps)
+        y = torch.full(ref.shape, float("nan"), device="cuda")
+        x, w, bias = dev(X), dev(Wt), dev(b)
+        rt.conv2d_f32_pads(N, C, H, W, OC, 1, 1, steps, pads, (1, 1), x.data_ptr(), w.data_ptr(), bias.data_ptr(), y.data_ptr())
+        torch.cuda.synchronize()
+        assert rel_err_max(host(y), ref) <= 1e-6          # whole numbers: exact in the sums; chains of 32 + C / 32 roundings
+
+
+@pytest.mark.parametrize("force", ["", "winograd", "straight", "halo-t4-parts2", "halo", "gather", "gemm"])
 @pytest.mark.parametrize("case", [(2, 32, 14, 14, 64, 1, 3), (3, 40, 7, 9, 33, 1, 3), (2, 32, 14, 14, 64, 2, 3), (2, 64, 9, 9, 32, 2, 1), (2, 128, 8, 8, 32, 1, 1)])
 @pytest.mark.parametrize("residual,activation", [(False, 2), (True, 2), (True, -1), (True, 5)])
 def test_chain_is_the_convolution_and_the_pass_behind_it(rt, monkeypatch, force, case, residual, activation):
