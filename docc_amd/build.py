@@ -48,6 +48,7 @@ KERNEL_FAMILIES = {
     "gemm_f32_big_epilogue": "gemm_f32_big_epilogue.hip",
     "gemm_finish": "gemm_finish.hip",
     "gemm_pack": "gemm_pack.hip",
+    "gemm_rows": "gemm_rows.hip",
     "gemm_bf16_async_finish": "gemm_bf16_async_finish.hip",
     "gemm_bf16_async_big_finish": "gemm_bf16_async_big_finish.hip",
     "gemm_f32_finish": "gemm_f32_finish.hip",

@@ -330,6 +330,25 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
         return docc_rocm_elementwise_fused(stream, sizeof(S) == 8 ? 64 : 32, 2, shape, bias ? DOCC_ROCM_BINARY_ADD : -1, shape, C, 0.0,
                                            bias ? row : nullptr, bias, 0.0, activation >= 0 ? 1 : 0, post, C);
     }
+    // A layer on up to 32 rows, weights stored [n][k]: product and chain as one launch (csrc/kernels/gemm_rows.hip). Against the forms below (skinny
+    // kernels with K in parts, matrix-vector kernels, both with a pass behind them) in bf16: 8 x 2048 -> 8192 13.1 -> 9.2 us, 8 x 8192 -> 2048 15.0 -> 10.7,
+    // 3 x 1024 -> 4096 11.4 -> 5.5, fp32 21.1 -> 15.1, 25.0 -> 18.3 and 13.9 -> 6.5. Every block of columns reads A again: above 16 rows a large matrix is
+    // better read by the kernels that cut K (32 x 2048 -> 8192 22 us here for 15, fp32 32 x 1024 -> 4096 14 for 13, but 24 x 2048 -> 512 7.0 for 11), in fp32 above
+    // eight (16 x 2048 -> 8192 22.3 for 21.8, but 12 x 4096 -> 1024 12.8 for 15.6).
+    // DOCC_ROCM_GEMM_ROWS=0 switches it off, =1 and =2 give the blocks of eight columns a work-group takes (tests, tuning).
+    if constexpr (sizeof(T) <= 4) {
+        const char* rows_env = tuning("DOCC_ROCM_GEMM_ROWS");
+        const int64_t v = 16 / (int64_t) sizeof(T), lim = int64_t(1) << 23;
+        const int forced = rows_env ? rows_env[0] - '0' : -1;
+        const bool size_ok = forced > 0 || m <= 8 || n * k < (sizeof(T) == 2 ? (m <= 16 ? lim << 10 : int64_t(8) << 20) : m <= 16 ? int64_t(8) << 20 : int64_t(2) << 20);
+        if (fin && !ta && tb && batch == 1 && m <= 32 && size_ok && forced != 0 && n % 8 == 0 && k % v == 0 && lda % v == 0 && ldb % v == 0 && k < lim && lda < lim &&
+            ldb < lim && n < (int64_t(1) << 30) &&
+            ((uintptr_t) A | (uintptr_t) B | (uintptr_t) fin->bias | (uintptr_t) fin->residual | (uintptr_t) fin->out) % 16 == 0) {
+            const int mt = m <= 8 ? 1 : m <= 16 ? 2 : 4, nt = mt == 4 || forced == 1 ? 1 : forced == 2 || n >= 16 * (int64_t) cus ? 2 : 1;
+            std::snprintf(name, sizeof(name), "docc_%cgemm_rows_m%d_n%d_f", sizeof(T) == 2 ? 'b' : 's', mt, nt);
+            return launch(name, (uint32_t) ((n + 8 * nt - 1) / (8 * nt)), 1, 1, 512, 0, s, A, (long) lda, B, (long) ldb, (long) m, (long) n, (long) k, (float) alpha, *fin);
+        }
+    }
     const bool epilogue = bias || activation >= 0;
     // A tall matrix times a few columns held as numpy holds them (B [k][n], n small): rows of B are a few elements long, so
     // the kernels that read whole vectors along n do not apply (n = 2, 5, 9 ... went through the element-wise tiles at a

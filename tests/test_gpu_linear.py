@@ -70,6 +70,29 @@ def test_linear_over_the_launchers_forms(dtype, m, n, k):
         assert bool((err <= bound).all()), (act, float((err / bound).max()))
 
 
+# a few rows (csrc/kernels/gemm_rows.hip): blocks of eight rows and columns, K in lines of 128 bytes that eight wavefronts take in turn - less than a line, a
+# part of one behind many, more lines than are on their way at once - and rows of A and B that are longer than K
+@pytest.mark.parametrize("blocks", ["1", "2"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("m,n,k,ld", [(1, 8, 8, 8), (2, 24, 64, 64), (7, 40, 72, 80), (8, 16, 1032, 1032), (9, 520, 200, 208), (16, 72, 4168, 4168), (17, 8, 136, 136),
+                                      (32, 264, 2056, 2064)])
+def test_linear_on_a_few_rows(monkeypatch, blocks, dtype, m, n, k, ld):
+    monkeypatch.setenv("DOCC_ROCM_GEMM_ROWS", blocks)
+    gen = torch.Generator().manual_seed(m * 31 + n)
+    a, w = torch.randn(m, ld, generator=gen).to(dtype).cuda(), (torch.randn(n, ld, generator=gen) * k ** -0.5).to(dtype).cuda()
+    a[:, k:], w[:, k:] = float("nan"), float("inf")           # behind the rows: not read, or dropped
+    bias, res = torch.randn(n, generator=gen).to(dtype).cuda(), torch.randn(m, n, generator=gen).to(dtype).cuda()
+    for act, b, r in (("gelu", bias, None), (None, None, res), ("relu", bias, res)):
+        y = torch.full((m, n), float("nan"), device="cuda", dtype=dtype)
+        rt.call("docc_rocm_linear", 0, TYPE[dtype], rt.NO_TRANS, rt.TRANS, m, n, k, 0.5, ptr(a), ld, ptr(w), ld, ptr(b), TYPE[dtype], ACTS[act], ptr(r), TYPE[dtype], 0,
+                ptr(y), TYPE[dtype])
+        torch.cuda.synchronize()
+        ref = reference(a[:, :k] * 0.5, w[:, :k], True, b, act, r, 0)
+        bound = 2e-5 * (1 + ref.abs()) + (0 if dtype == torch.float32 else 2.0 ** -7 * ref.abs())      # as above, nothing rounded in between
+        err = (y.double().cpu() - ref).abs()
+        assert bool((err <= bound).all()), (act, float((err / bound).max()))
+
+
 # every tile with the chain in its store, ragged at both edges and along K where the tile allows it
 @pytest.mark.parametrize("cfg,dtype,k", [("128x128x32x4x4", torch.bfloat16, 104), ("128x128x64x4x4", torch.bfloat16, 328), ("128x256x64x4x3", torch.bfloat16, 328),
                                          ("256x256x32x4x4q", torch.bfloat16, 192), ("64x64x16x4x4", torch.float32, 84), ("128x128x32x4x3", torch.float32, 84),
