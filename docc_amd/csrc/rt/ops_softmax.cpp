@@ -214,6 +214,31 @@ int docc_rocm_softmax(docc_rocm_stream_t stream, int precision, int64_t outer, i
     return softmax_general((hipStream_t) stream, precision, outer, reduce, inner, X, Y, nullptr);
 }
 
+int docc_rocm_softmax_host(docc_rocm_stream_t stream, int precision, int64_t outer, int64_t reduce, int64_t inner, const void* X, void* Y) {
+    if (int rc = softmax_check(precision, outer, reduce, inner, X, Y)) return rc == 1 ? 0 : rc;
+    if (int rc = ensure_device()) return rc;
+    const size_t unit = (size_t) (reduce * inner) * (precision / 8), bytes = (size_t) outer * unit;
+    int rc = through_device((hipStream_t) stream, X, Y, outer, unit, [&](int64_t, int64_t count, const void* x, void* y) {
+        return docc_rocm_softmax(stream, precision, count, reduce, inner, x, y);
+    });
+    if (rc != 1) return rc;
+    void *x = nullptr, *y = nullptr;
+    if ((rc = docc_rocm_malloc_async(&x, bytes, stream))) return rc;
+    rc = docc_rocm_memcpy_h2d_async(x, X, bytes, stream);
+    if (!rc) rc = docc_rocm_malloc_async(&y, bytes, stream);
+    if (!rc) rc = docc_rocm_softmax(stream, precision, outer, reduce, inner, x, y);
+    if (!rc) rc = docc_rocm_memcpy_d2h_async(Y, y, bytes, stream);
+    const int ended = docc_rocm_stream_sync(stream);
+    if (!rc) rc = ended;
+    for (void* p : {x, y})
+        if (const int freed = p ? docc_rocm_free_async(p, stream) : 0; !rc) rc = freed;
+    return rc;
+}
+
+int docc_rocm_softmax_f32_host(docc_rocm_stream_t stream, int64_t rows, int64_t cols, const float* X, float* Y) {
+    return docc_rocm_softmax_host(stream, 32, rows, cols, 1, X, Y);
+}
+
 int64_t docc_rocm_softmax_workspace_bytes(int precision, int64_t outer, int64_t reduce, int64_t inner) {
     if ((precision != 32 && precision != 64) || outer <= 0 || reduce <= 0 || inner <= 0) return 0;
     if (inner != 1 && inner <= 32 && (inner & (inner - 1)) == 0) return 0;

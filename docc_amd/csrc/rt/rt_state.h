@@ -6,6 +6,7 @@
 
 #include <cstdarg>
 #include <cstdint>
+#include <functional>
 #include <mutex>
 #include <string>
 
@@ -50,6 +51,12 @@ bool capturing();
 // device memory its launches were given, and no block of the cache can be kept for it. A launcher that would take one runs in its
 // form without one, or refuses.
 bool foreign_capture(hipStream_t stream);
+
+// A host array of `units` pieces of `unit_bytes` through the device into another of that size: run(first, count, x, y) launches on `stream` what makes y of x
+// for `count` pieces on the device. Uploads, kernels and downloads of different pieces run beside each other; everything has ended on return. 1: nothing was
+// done, because the call is small, the results' array is not pinned, the arrays overlap, a capture is open or there is no memory: the caller copies, launches and copies.
+int through_device(hipStream_t stream, const void* src, void* dst, int64_t units, size_t unit_bytes,
+                   const std::function<int(int64_t first, int64_t count, const void* x, void* y)>& run);
 
 // The launchers' switches (tests, tuning) are environment variables read on every call: whether any DOCC_ROCM_GEM... variable is set at
 // all, in one walk over the environment instead of one per variable (seven for a GEMM, 0.2-0.3 us each).

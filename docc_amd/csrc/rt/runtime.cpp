@@ -484,8 +484,16 @@ private:
     size_t pending_ = 0;
 };
 
+// The streams and events of the copies that run beside each other (through_device()), one set per device
+struct CopyLanes {
+    hipStream_t up = nullptr, down = nullptr;
+    hipEvent_t begin = nullptr, arrived[2] = {}, computed[2] = {};
+    bool ready = false;
+};
+
 struct Stager {
     std::mutex mutex;              // one staged upload at a time
+    std::map<int, CopyLanes> lanes;
     bool tried = false, ready = false;
     int threads = 0;
     char* buffer[kStageBuffers] = {};
@@ -495,10 +503,8 @@ struct Stager {
 };
 Stager g_stager;
 
-// 0: done, 1: not staged (the caller falls back to the plain copy), other: error
-int staged_h2d(void* dst_dev, const void* src_host, size_t bytes, hipStream_t stream) {
-    Stager& st = g_stager;
-    std::lock_guard<std::mutex> lock(st.mutex);
+// with st.mutex held: whether there are pinned buffers and threads to fill them
+bool stager_ready(Stager& st) {
     if (!st.tried) {
         st.tried = true;
         int threads = 4;
@@ -518,7 +524,14 @@ int staged_h2d(void* dst_dev, const void* src_host, size_t bytes, hipStream_t st
             }
         }
     }
-    if (!st.ready) return 1;
+    return st.ready;
+}
+
+// 0: done, 1: not staged (the caller falls back to the plain copy), other: error
+int staged_h2d(void* dst_dev, const void* src_host, size_t bytes, hipStream_t stream) {
+    Stager& st = g_stager;
+    std::lock_guard<std::mutex> lock(st.mutex);
+    if (!stager_ready(st)) return 1;
     const char* src = (const char*) src_host;
     char* dst = (char*) dst_dev;
     int slot = 0;
@@ -539,7 +552,104 @@ int staged_h2d(void* dst_dev, const void* src_host, size_t bytes, hipStream_t st
     return 0;
 }
 
+int lanes_for_device(Stager& st, CopyLanes** lanes) {
+    int dev = 0;
+    if (int rc = check(hipGetDevice(&dev), "hipGetDevice")) return rc;
+    CopyLanes& l = st.lanes[dev];
+    if (!l.ready) {
+        bool ok = (l.up || hipStreamCreateWithFlags(&l.up, hipStreamNonBlocking) == hipSuccess) &&
+                  (l.down || hipStreamCreateWithFlags(&l.down, hipStreamNonBlocking) == hipSuccess);
+        for (hipEvent_t* e : {&l.begin, &l.arrived[0], &l.arrived[1], &l.computed[0], &l.computed[1]})
+            ok = ok && (*e || hipEventCreateWithFlags(e, hipEventDisableTiming) == hipSuccess);
+        if (!ok) {
+            (void) hipGetLastError();
+            return 1;
+        }
+        l.ready = true;
+    }
+    *lanes = &l;
+    return 0;
+}
+
 } // namespace
+
+namespace docc::rt::rocm {
+
+// PCIe carries both directions at once; a call that uploads, computes and downloads in turn uses one of them at a time. Uploads here go on a stream of
+// their own, the kernels on the caller's, downloads on a third, ordered by events. 64 MB in and out: 2.72 ms in turn, 1.87 ms this way (the upload alone is
+// 1.36; what does not overlap is the first chunk's staging and upload and the last one's download).
+int through_device(hipStream_t stream, const void* src, void* dst, int64_t units, size_t unit_bytes, const std::function<int(int64_t, int64_t, const void*, void*)>& run) {
+    hipStream_t s = resolve_stream(stream);
+    const size_t bytes = (size_t) units * unit_bytes;
+    const char *from = (const char*) src, *to = (const char*) dst;
+    if (bytes < kStageMin || capturing() || foreign_capture(stream) || !is_pinned(dst, bytes)) return 1;
+    if (from != to && from < to + bytes && to < from + bytes) return 1;      // a download would write what has not been read (in place it has)
+    // eight chunks where they have 4 to 8 MB (64 MB in and out: chunks of 2 MB 2.80 ms, 4 MB 2.03, 8 MB 1.87; 16 MB: 4 MB 0.67, 8 MB 0.77)
+    const size_t eighth = bytes / 8, chunk_bytes = eighth < kStageChunk / 2 ? kStageChunk / 2 : eighth > kStageChunk ? kStageChunk : eighth;
+    const int64_t per_chunk = unit_bytes >= chunk_bytes ? 1 : (int64_t) (chunk_bytes / unit_bytes);
+    if (unit_bytes > kStageChunk || per_chunk >= units) return 1;
+    const bool pinned = is_pinned(src, bytes);
+    Stager& st = g_stager;
+    std::unique_lock<std::mutex> lock(st.mutex);
+    CopyLanes* lanes = nullptr;
+    if (!pinned && !stager_ready(st)) return 1;
+    if (int rc = lanes_for_device(st, &lanes)) return rc;
+    void *x = nullptr, *y = nullptr;
+    if (docc_rocm_malloc_async(&x, bytes, stream)) return 1;
+    if (docc_rocm_malloc_async(&y, bytes, stream)) {
+        (void) docc_rocm_free_async(x, stream);
+        return 1;
+    }
+    // the blocks may still be in use by what their owner before has on the stream
+    int rc = check(hipEventRecord(lanes->begin, s), "hipEventRecord(copy lanes)");
+    if (!rc) rc = check(hipStreamWaitEvent(lanes->up, lanes->begin, 0), "hipStreamWaitEvent(copy lanes)");
+    int slot = 0, turn = 0;
+    for (int64_t first = 0; first < units && !rc; first += per_chunk, slot = (slot + 1) % kStageBuffers, turn ^= 1) {
+        const int64_t count = units - first < per_chunk ? units - first : per_chunk;
+        const size_t off = (size_t) first * unit_bytes, n = (size_t) count * unit_bytes;
+        const char* chunk = from + off;
+        if (!pinned) {
+            if (st.in_flight[slot]) {
+                if ((rc = check(hipEventSynchronize(st.sent[slot]), "hipEventSynchronize(H2D staging)"))) break;
+                st.in_flight[slot] = false;
+            }
+            st.pool->copy(st.buffer[slot], chunk, n, st.threads);
+            chunk = st.buffer[slot];
+        }
+        if ((rc = check(hipMemcpyAsync((char*) x + off, chunk, n, hipMemcpyHostToDevice, lanes->up), "hipMemcpyAsync(H2D, lanes)"))) break;
+        if (!pinned) {
+            if ((rc = check(hipEventRecord(st.sent[slot], lanes->up), "hipEventRecord(H2D staging)"))) break;
+            st.in_flight[slot] = true;
+        }
+        // (an event may be recorded again once the waits for its last record have been enqueued)
+        if ((rc = check(hipEventRecord(lanes->arrived[turn], lanes->up), "hipEventRecord(copy lanes)"))) break;
+        if ((rc = check(hipStreamWaitEvent(s, lanes->arrived[turn], 0), "hipStreamWaitEvent(copy lanes)"))) break;
+        if ((rc = run(first, count, (const char*) x + off, (char*) y + off))) break;
+        if ((rc = check(hipEventRecord(lanes->computed[turn], s), "hipEventRecord(copy lanes)"))) break;
+        if ((rc = check(hipStreamWaitEvent(lanes->down, lanes->computed[turn], 0), "hipStreamWaitEvent(copy lanes)"))) break;
+        rc = check(hipMemcpyAsync((char*) dst + off, (char*) y + off, n, hipMemcpyDeviceToHost, lanes->down), "hipMemcpyAsync(D2H, lanes)");
+    }
+    // The last download ends behind everything else of the call. It is waited for without the lock, so that another thread's uploads run beside it, by an
+    // event of the call's own (the others are recorded again by then). After a failure everything that may have been enqueued ends first.
+    hipEvent_t ended = nullptr;
+    if (!rc) rc = check(hipEventCreateWithFlags(&ended, hipEventDisableTiming), "hipEventCreate");
+    if (!rc) rc = check(hipEventRecord(ended, lanes->down), "hipEventRecord(copy lanes)");
+    if (rc) {
+        (void) hipStreamSynchronize(lanes->up);
+        (void) hipStreamSynchronize(s);
+        (void) hipStreamSynchronize(lanes->down);
+    }
+    lock.unlock();
+    if (!rc) rc = check(hipEventSynchronize(ended), "hipEventSynchronize(copy lanes)");
+    if (ended) (void) hipEventDestroy(ended);
+    for (void* p : {x, y}) {
+        const int freed = docc_rocm_free_async(p, stream);
+        if (!rc) rc = freed;
+    }
+    return rc;
+}
+
+} // namespace docc::rt::rocm
 
 extern "C" {
 

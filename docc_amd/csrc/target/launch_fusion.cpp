@@ -4,6 +4,7 @@
 //   * a GEMM and the elementwise block that alone reads its result - bias, activation, rounding to bf16, residual - become
 //     docc_rocm_linear, which has the chain in the product's store;
 //   * a convolution and the elementwise block that alone reads its result - residual, ReLU - become docc_rocm_conv2d_f32_chain;
+//   * an upload, a softmax and the download of its result become docc_rocm_softmax_host, which has the copies of different rows beside each other;
 //   * Mean, centre and square, Mean, scale and shift (how a layer norm is spelled with tensor nodes), with the casts around
 //     them for bf16, become docc_rocm_layer_norm.
 // A transformer's feed-forward block of nine to eleven launches is three calls this way. The reference stops at fusing Maps
@@ -56,6 +57,13 @@ public:
     Expression group;
     bool has_bias = false, has_residual = false;
     int activation = -1;
+};
+
+class SoftmaxHostLaunch : public LaunchNode {
+public:
+    SoftmaxHostLaunch() : LaunchNode(LibraryNodeType_ROCM_SoftmaxHost, {"_x"}) {}
+    Expression outer, extent, inner;
+    bool fp64 = false, rows = false;   // rows: over the last axis of floats
 };
 
 class LayerNormLaunch : public LaunchNode {
@@ -210,7 +218,7 @@ public:
         bool applied = false;
         for (bool changed = true; changed;) {
             changed = false;
-            for (size_t j = 0; j < blocks_.size() && !changed; j++) changed = layer_norm(j) || linear(j) || conv_chain(j);
+            for (size_t j = 0; j < blocks_.size() && !changed; j++) changed = layer_norm(j) || linear(j) || conv_chain(j) || softmax_host(j);
             applied = applied || changed;
         }
         restore_lifetimes(applied);
@@ -499,6 +507,37 @@ private:
         return true;
     }
 
+    // ---- a softmax between its operand's upload and its result's download ------------------------------
+    bool softmax_host(size_t j) {
+        const auto* n = dynamic_cast<const tensor::SoftmaxNode*>(blocks_[j].node.get());
+        if (!n || !ours(j)) return false;
+        const std::string x = blocks_[j].input("X")->data, y = blocks_[j].outputs[0].data;
+        const long w = writer_of(x, j);
+        if (w < 0 || !is_offloading(blocks_[(size_t) w])) return false;
+        const size_t i = (size_t) w;
+        const auto& up = static_cast<const ROCMDataOffloadingNode&>(*blocks_[i].node);
+        size_t l = j + 1;
+        while (l < blocks_.size() && !touches(blocks_[l], y)) l++;
+        if (l == blocks_.size() || !is_offloading(blocks_[l])) return false;
+        const auto& down = static_cast<const ROCMDataOffloadingNode&>(*blocks_[l].node);
+        if (!up.is_h2d() || !up.is_alloc() || !down.is_d2h() || !down.is_free() || !private_to(x, {i, j}) || !private_to(y, {j, l})) return false;
+        if (!symbolic::equal(up.size(), n->connector_bytes("X")) || !symbolic::equal(down.size(), n->connector_bytes("Y"))) return false;
+        int64_t bytes = 0;
+        if (symbolic::is_integer(up.size(), &bytes) && bytes < (int64_t(16) << 20)) return false;   // copied as a whole anyway
+        // the upload moves to where the download stands: nothing in between writes its source or touches the result
+        const std::string from = blocks_[i].inputs[0].data, to = blocks_[l].outputs[0].data;
+        if (lost_between(from, i, l)) return false;
+        for (size_t k = i + 1; k < l; k++)
+            if (k != j && touches(blocks_[k], to)) return false;
+        auto node = std::make_unique<SoftmaxHostLaunch>();
+        node->outer = n->outer(), node->extent = n->extent(), node->inner = n->inner();
+        node->fp64 = n->element() == P::Double;
+        node->rows = n->last_axis_only() && n->element() == P::Float;
+        if (node->rows) node->outer = n->rows(), node->extent = n->cols();
+        install(l, std::move(node), {bind("_x", from)}, to, {i, j}, {x, y});
+        return true;
+    }
+
     // ---- layer norm ------------------------------------------------------------------------------------
     // the Mean over the trailing loops from `trailing` on whose result a form of loops `bounds` loads once per row
     const tensor::ReduceNode* row_mean(const std::string& name, size_t before, size_t* at) const {
@@ -677,6 +716,10 @@ public:
             s << "if (__ws) DOCC_ROCM_CHECK(docc_rocm_free_async(__ws, nullptr));" << std::endl;
             s.setIndent(s.indent() - 4);
             s << "}" << std::endl;
+        } else if (const auto* h = dynamic_cast<const SoftmaxHostLaunch*>(&node_)) {
+            if (h->rows) s << "DOCC_ROCM_CHECK(docc_rocm_softmax_f32_host(nullptr, " << h->outer << ", " << h->extent << ", _x, _y));" << std::endl;
+            else s << "DOCC_ROCM_CHECK(docc_rocm_softmax_host(nullptr, " << (h->fp64 ? 64 : 32) << ", " << h->outer << ", " << h->extent << ", " << h->inner
+              << ", _x, _y));" << std::endl;
         } else if (const auto* n = dynamic_cast<const LayerNormLaunch*>(&node_)) {
             s << "DOCC_ROCM_CHECK(docc_rocm_layer_norm(nullptr, " << type_code(n->type) << ", " << n->rows << ", " << n->cols << ", (float) (" << n->eps
               << "), _x, " << (n->has_weight ? "_weight" : "nullptr") << ", " << (n->has_bias ? "_bias" : "nullptr") << ", _y));" << std::endl;
@@ -689,7 +732,7 @@ public:
 bool RocmLaunchFusionPass::run_pass(builder::StructuredSDFGBuilder& builder, analysis::AnalysisManager&) { return LaunchFusion(builder.subject()).run(); }
 
 void register_launch_dispatchers(codegen::LibraryNodeDispatcherRegistry& reg) {
-    for (auto& code : {LibraryNodeType_ROCM_Linear, LibraryNodeType_ROCM_ConvChain, LibraryNodeType_ROCM_LayerNorm})
+    for (auto& code : {LibraryNodeType_ROCM_Linear, LibraryNodeType_ROCM_ConvChain, LibraryNodeType_ROCM_SoftmaxHost, LibraryNodeType_ROCM_LayerNorm})
         reg.register_library_node_dispatcher(code + "::" + ImplementationType_ROCMWithoutTransfers,
                                              [](codegen::LanguageExtension& le, const Function& f, const data_flow::DataFlowGraph& b, const LibraryNode& n) {
                                                  return std::make_unique<LaunchDispatcher>(le, f, b, n);

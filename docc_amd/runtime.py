@@ -85,6 +85,8 @@ _SIGNATURES = {
     "docc_rocm_bf16gemm_f32_batched": [_vp, _int, _int, _i64, _i64, _i64, _f32, _vp, _i64, _i64, _vp, _i64, _i64, _f32, _vp, _i64, _i64, _i64],
     "docc_rocm_softmax_f32": [_vp, _i64, _i64, _vp, _vp],
     "docc_rocm_softmax": [_vp, _int, _i64, _i64, _i64, _vp, _vp],
+    "docc_rocm_softmax_f32_host": [_vp, _i64, _i64, _vp, _vp],
+    "docc_rocm_softmax_host": [_vp, _int, _i64, _i64, _i64, _vp, _vp],
     "docc_rocm_softmax_workspace_bytes": [_int, _i64, _i64, _i64],
     "docc_rocm_softmax_ws": [_vp, _int, _i64, _i64, _i64, _vp, _vp, _vp, _i64],
     "docc_rocm_softmax_noalloc": [_vp, _int, _i64, _i64, _i64, _vp, _vp],

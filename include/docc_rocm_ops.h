@@ -163,6 +163,13 @@ int docc_rocm_softmax(docc_rocm_stream_t stream, int precision, int64_t outer, i
                       const void* X, void* Y);
 
 /*
+ * docc_rocm_softmax on host arrays: X is uploaded, the result is in Y on return. Where Y is pinned (docc_rocm_host_malloc, or by the caller) and the arrays are large,
+ * uploads, kernels and downloads of different rows run beside each other. X and Y are one array or do not overlap. Refused under capture, as the copies are.
+ */
+int docc_rocm_softmax_host(docc_rocm_stream_t stream, int precision, int64_t outer, int64_t reduce, int64_t inner, const void* X, void* Y);
+int docc_rocm_softmax_f32_host(docc_rocm_stream_t stream, int64_t rows, int64_t cols, const float* X, float* Y);   /* rows of float32 */
+
+/*
  * The same with the partial results in memory of the caller: `workspace` is device memory, 256-byte
  * aligned, of at least docc_rocm_softmax_workspace_bytes(...) bytes (0 for the shapes that run as one
  * launch; at most 8 MiB); it may be reused as soon as the call's kernels have run. Same kernels and

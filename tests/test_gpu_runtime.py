@@ -270,6 +270,50 @@ def test_large_uploads_from_pageable_memory_are_staged_through_pinned_chunks(rt)
     rt.call("docc_rocm_stream_destroy", s)
 
 
+@pytest.mark.parametrize("dtype,shape", [(np.float32, (4111, 1031, 1)), (np.float32, (8192, 512, 1)), (np.float64, (300, 77, 100)), (np.float32, (3, 1 << 20, 1)),
+                                         (np.float32, (2, 3 << 20, 1)), (np.float32, (40, 100, 1))])
+@pytest.mark.parametrize("pinned_x,pinned_y", [(False, True), (True, True), (False, False)])
+def test_softmax_of_host_arrays(rt, dtype, shape, pinned_x, pinned_y):
+    """docc_rocm_softmax_host: rows in chunks whose copies run beside each other (large arrays into pinned memory; rows longer than a chunk and small or
+    pageable results go as a whole), in place, and from two threads at once, each with a stream of its own."""
+    import threading
+    rng = np.random.default_rng(1)
+    x = (rng.standard_normal(shape) * 8).astype(dtype)
+    ref = np.exp(x.astype(np.float64) - x.max(1, keepdims=True))
+    ref /= ref.sum(1, keepdims=True)
+    bits, tolerance = x.itemsize * 8, 2e-5 if dtype == np.float32 else 1e-13          # of a probability: the exponent's rounding at 8 standard deviations, a sum's
+
+    def array(pinned):
+        a = rt.result_array(shape, dtype) if pinned else np.empty(shape, dtype)
+        a[:] = x
+        return a
+
+    def check(stream=0):
+        for _ in range(2):
+            a, y = array(pinned_x), array(pinned_y)
+            rt.call("docc_rocm_softmax_host", stream, bits, *shape, a.ctypes.data, y.ctypes.data)
+            assert (np.abs(y - ref) <= tolerance * ref + 1e-30).all() and np.array_equal(a, x)
+            rt.call("docc_rocm_softmax_host", stream, bits, *shape, y.ctypes.data, y.ctypes.data)
+            again = np.exp(ref - ref.max(1, keepdims=True))
+            assert (np.abs(y * again.sum(1, keepdims=True) / again - 1) <= tolerance).all()
+
+    check()
+    failures, streams = [], [rt.stream_create() for _ in range(2)]
+
+    def work(s):
+        try:
+            check(s)
+        except BaseException as e:      # noqa: BLE001 - reported below
+            failures.append(e)
+
+    threads = [threading.Thread(target=work, args=(s,)) for s in streams]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failures, failures
+
+
 @pytest.mark.parametrize("precision", [64, 32, 16, 116])
 def test_mfma_probe_times_its_loop_and_nothing_else(rt, precision):
     """The ceiling probe's launch time must be its MFMA loop: twice the rounds take twice as long (operand

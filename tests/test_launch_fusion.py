@@ -210,3 +210,24 @@ def test_a_convolution_with_the_block_behind_it(tmp_path, tail, emitted):
         assert f"docc_rocm_conv2d_f32_chain(nullptr, {emitted}, __ws, __ws_bytes)" in text and "elementwise" not in text and text.count("docc_rocm_malloc_async(") == 1
     else:
         assert "docc_rocm_conv2d_f32_chain" not in text and "docc_rocm_conv2d_f32_pads(" in text
+
+
+@pytest.mark.parametrize("shape,merged", [(["n", "256"], "docc_rocm_softmax_f32_host(nullptr, n, 256, _x, _y)"), (["65536", "256"], "docc_rocm_softmax_f32_host(nullptr, 65536, 256, _x, _y)"),
+                                          (["64", "256"], None)])
+@pytest.mark.parametrize("reader", [False, True])
+def test_a_softmax_between_an_upload_and_a_download(tmp_path, shape, merged, reader):
+    """Large host arrays go through docc_rocm_softmax_host; not those that are known to be small, nor results that another node reads on the device."""
+    b = StructuredSDFGBuilder("rows")
+    b.add_container("n", Scalar(PrimitiveType.Int64), True)
+    for name in ("X", "Y", "Z"):
+        b.add_container(name, F32, True)
+    b.add_reduce_op("softmax", "X", "Y", shape, [1])
+    if reader:
+        b.add_elementwise_unary_op("relu", "Y", "Z", shape)
+    s = b.move()
+    s.schedule("rocm", options={"fuse_maps": False})
+    text = re.sub(r"\s+", " ", open(s.generate(str(tmp_path))["source"]).read())
+    if merged and not reader:
+        assert merged in text and "memcpy" not in text and "malloc" not in text
+    else:
+        assert "_host(" not in text and "docc_rocm_softmax_f32(nullptr, " in text and text.count("docc_rocm_memcpy_h2d_async(") == 1
