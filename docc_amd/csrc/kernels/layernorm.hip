@@ -6,7 +6,7 @@
 // for 2^20 rows of 8 fp32, where the nodes took 62; the lanes 12.4), rows of a few KB to a wavefront (four rows a work-group, no barrier);
 // longer ones, and rows too few to fill the device that way, to a work-group of 256; rows that do not fit its registers are read three times
 // from L2, by one work-group a row or, from 16384 columns on, in slices.
-#include "common.h"
+#include "layernorm.h"
 
 namespace docc_k {
 
@@ -43,20 +43,6 @@ __device__ __forceinline__ float ln_row_sum(float v, float* slot) {
     for (int w = 1; w < TPR / 64; w++) s += slot[w];
     return s;
 }
-
-// a / root, rounded once, without the ten instructions of a division for every element (bf16 4096 x 2048 with them 10.7 us, with a plain product by
-// 1 / root, one rounding more, 8.3; so 8.8): q = a (1 / root) is off by a bit at most, its remainder is exact in a fused multiply-add, and what
-// that adds to q rounds to the quotient (Markstein, 1990). Where the root is far from 1 (an infinity, a NaN or an underflow on the way would not
-// be the quotient's) the caller divides beforehand (`direct`) and the value passes through.
-struct LnQuotient {
-    float root, inv;
-    bool direct;
-    __device__ __forceinline__ explicit LnQuotient(float r) : root(r), inv(1.0f / r), direct(!(r > 0x1p-60f && r < 0x1p60f)) {}
-    __device__ __forceinline__ float operator()(float a) const {
-        const float q = a * inv;
-        return direct ? a : __builtin_fmaf(__builtin_fmaf(-q, root, a), inv, q);
-    }
-};
 
 // NV vectors of V elements a lane, TPR lanes a row; cols <= TPR * NV * V and a multiple of V
 template <typename T, int V, int NV, int TPR>

@@ -334,17 +334,21 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
     // kernels with K in parts, matrix-vector kernels, both with a pass behind them) in bf16: 8 x 2048 -> 8192 13.1 -> 9.2 us, 8 x 8192 -> 2048 15.0 -> 10.7,
     // 3 x 1024 -> 4096 11.4 -> 5.5, fp32 21.1 -> 15.1, 25.0 -> 18.3 and 13.9 -> 6.5. Every block of columns reads A again: above 16 rows a large matrix is
     // better read by the kernels that cut K (32 x 2048 -> 8192 22 us here for 15, fp32 32 x 1024 -> 4096 14 for 13, but 24 x 2048 -> 512 7.0 for 11), in fp32 above
-    // eight (16 x 2048 -> 8192 22.3 for 21.8, but 12 x 4096 -> 1024 12.8 for 15.6).
+    // eight (16 x 2048 -> 8192 22.3 for 21.8, but 12 x 4096 -> 1024 12.8 for 15.6); a single row by the matrix-vector kernel (fp32 1 x 3072 -> 12288 31 for 27;
+    // a block of 1 x 3072 in bf16 37.5 for 36.1, of 16 53.3 for 52.4).
+    // Two blocks of columns a work-group from three quarters of a work-group a CU on (8 x 8192 -> 2048 10.7 us with one, 14.3 with two; 12288 -> 3072 24.7 and 19.7).
     // DOCC_ROCM_GEMM_ROWS=0 switches it off, =1 and =2 give the blocks of eight columns a work-group takes (tests, tuning).
     if constexpr (sizeof(T) <= 4) {
         const char* rows_env = tuning("DOCC_ROCM_GEMM_ROWS");
         const int64_t v = 16 / (int64_t) sizeof(T), lim = int64_t(1) << 23;
         const int forced = rows_env ? rows_env[0] - '0' : -1;
-        const bool size_ok = forced > 0 || m <= 8 || n * k < (sizeof(T) == 2 ? (m <= 16 ? lim << 10 : int64_t(8) << 20) : m <= 16 ? int64_t(8) << 20 : int64_t(2) << 20);
+        const int64_t size = n * k, mi = int64_t(1) << 20;
+        const bool size_ok = forced > 0 || (sizeof(T) == 2 ? (m <= 1 || (m > 8 && m <= 16) ? size < 32 * mi : m <= 8 || size < 8 * mi)
+                                                           : m <= 1 ? size < 16 * mi : m <= 8 ? true : m <= 16 ? size < 8 * mi : size < 2 * mi);
         if (fin && !ta && tb && batch == 1 && m <= 32 && size_ok && forced != 0 && n % 8 == 0 && k % v == 0 && lda % v == 0 && ldb % v == 0 && k < lim && lda < lim &&
             ldb < lim && n < (int64_t(1) << 30) &&
             ((uintptr_t) A | (uintptr_t) B | (uintptr_t) fin->bias | (uintptr_t) fin->residual | (uintptr_t) fin->out) % 16 == 0) {
-            const int mt = m <= 8 ? 1 : m <= 16 ? 2 : 4, nt = mt == 4 || forced == 1 ? 1 : forced == 2 || n >= 16 * (int64_t) cus ? 2 : 1;
+            const int mt = m <= 8 ? 1 : m <= 16 ? 2 : 4, nt = mt == 4 || forced == 1 ? 1 : forced == 2 || n >= 12 * (int64_t) cus ? 2 : 1;
             std::snprintf(name, sizeof(name), "docc_%cgemm_rows_m%d_n%d_f", sizeof(T) == 2 ? 'b' : 's', mt, nt);
             return launch(name, (uint32_t) ((n + 8 * nt - 1) / (8 * nt)), 1, 1, 512, 0, s, A, (long) lda, B, (long) ldb, (long) m, (long) n, (long) k, (float) alpha, *fin);
         }
@@ -784,9 +788,9 @@ int docc_rocm_bf16gemm_f32_epilogue(docc_rocm_stream_t stream, int trans_a, int 
                                         pick_bgemm, bias, activation);
 }
 
-int docc_rocm_linear(docc_rocm_stream_t stream, int type, int trans_a, int trans_b, int64_t m, int64_t n, int64_t k, float alpha, const void* A,
-                     int64_t lda, const void* B, int64_t ldb, const void* bias, int bias_type, int activation, const void* residual,
-                     int residual_type, int rounding, void* Y, int y_type) {
+// the chain behind a product as the kernels take it, from the launchers' arguments
+static int linear_finish(int type, int64_t m, int64_t n, const void* bias, int bias_type, int activation, const void* residual, int residual_type, int rounding, void* Y,
+                         int y_type, LinearFinish* finish) {
     auto is = [](int t, int a, int b) { return t == a || t == b; };
     if (!is(type, DOCC_ROCM_TYPE_F32, DOCC_ROCM_TYPE_BF16) || !is(y_type, DOCC_ROCM_TYPE_F32, DOCC_ROCM_TYPE_BF16) ||
         (bias && !is(bias_type, DOCC_ROCM_TYPE_F32, DOCC_ROCM_TYPE_BF16)) || (residual && !is(residual_type, DOCC_ROCM_TYPE_F32, DOCC_ROCM_TYPE_BF16)))
@@ -796,17 +800,69 @@ int docc_rocm_linear(docc_rocm_stream_t stream, int type, int trans_a, int trans
         return fail(DOCC_ROCM_ERR_INVALID_ARGUMENT, "linear: unknown activation %d", activation);
     if (rounding & ~(DOCC_ROCM_ROUND_BEFORE_ACT | DOCC_ROCM_ROUND_AFTER_ACT)) return fail(DOCC_ROCM_ERR_INVALID_ARGUMENT, "linear: unknown rounding %d", rounding);
     if (m > 0 && n > 0 && !Y) return fail(DOCC_ROCM_ERR_INVALID_ARGUMENT, "linear: null pointer");
-    LinearFinish f{bias, residual, Y, 0, activation};
+    LinearFinish& f = *finish;
+    f = LinearFinish{bias, residual, Y, 0, activation};
     if (bias && bias_type == DOCC_ROCM_TYPE_BF16) f.flags |= kBiasBf16;
     if (residual && residual_type == DOCC_ROCM_TYPE_BF16) f.flags |= kResidualBf16;
     if (y_type == DOCC_ROCM_TYPE_BF16) f.flags |= kOutBf16;
     if (rounding & DOCC_ROCM_ROUND_BEFORE_ACT) f.flags |= kRoundBeforeAct;
     if (rounding & DOCC_ROCM_ROUND_AFTER_ACT) f.flags |= kRoundAfterAct;
+    return 0;
+}
+
+int docc_rocm_linear(docc_rocm_stream_t stream, int type, int trans_a, int trans_b, int64_t m, int64_t n, int64_t k, float alpha, const void* A,
+                     int64_t lda, const void* B, int64_t ldb, const void* bias, int bias_type, int activation, const void* residual,
+                     int residual_type, int rounding, void* Y, int y_type) {
+    LinearFinish f{};
+    if (int rc = linear_finish(type, m, n, bias, bias_type, activation, residual, residual_type, rounding, Y, y_type, &f)) return rc;
     if (type == DOCC_ROCM_TYPE_F32)
         return gemm_launch<float>("sgemm", stream, trans_a, trans_b, m, n, k, alpha, (const float*) A, lda, (const float*) B, ldb, 0.0f, (float*) nullptr, n,
                                   pick_sgemm, (const float*) nullptr, -1, 1, 0, 0, 0, &f);
     return gemm_launch<uint16_t, float>("bgemm", stream, trans_a, trans_b, m, n, k, alpha, (const uint16_t*) A, lda, (const uint16_t*) B, ldb, 0.0f,
                                         (float*) nullptr, n, pick_bgemm, (const float*) nullptr, -1, 1, 0, 0, 0, &f);
+}
+
+int docc_rocm_norm_linear(docc_rocm_stream_t stream, int type, int64_t m, int64_t n, int64_t k, float eps, const void* X, const void* weight, const void* norm_bias,
+                          float alpha, const void* B, int64_t ldb, const void* bias, int bias_type, int activation, const void* residual, int residual_type, int rounding,
+                          void* scratch, void* Y, int y_type) {
+    LinearFinish f{};
+    if (int rc = linear_finish(type, m, n, bias, bias_type, activation, residual, residual_type, rounding, Y, y_type, &f)) return rc;
+    if (m < 0 || n < 0 || k < 0 || ldb < (k > 1 ? k : 1)) return fail(DOCC_ROCM_ERR_INVALID_ARGUMENT, "norm_linear: bad shape");
+    if (m == 0 || n == 0) return 0;
+    // Rows that a wavefront holds, every work-group's in LDS (csrc/kernels/gemm_rows.hip): a launch of 3 to 4 us less. Every work-group normalises all rows again,
+    // 4 to 16 vectors a lane, while it waits for its first lines of B. DOCC_ROCM_GEMM_ROWS=0 or =3 keeps the layer norm a launch of its own (tests, tuning).
+    const char* rows_env = gemm_tuning_set() ? std::getenv("DOCC_ROCM_GEMM_ROWS") : nullptr;
+    const int forced = rows_env ? rows_env[0] - '0' : -1;
+    const bool bf16 = type == DOCC_ROCM_TYPE_BF16;
+    const int64_t v = bf16 ? 8 : 4, lim = int64_t(1) << 23;
+    const int mt = m <= 8 ? 1 : 2, vectors = k <= 256 * v ? 4 : 8;      // vectors a lane holds
+    const int64_t pitch = (k + v) * (bf16 ? 2 : 4);
+    if (m <= 16 && k >= 8 * v && k <= 512 * v && (mt == 1 || (vectors == 4 && (bf16 || n * k < int64_t(8) << 20))) && n % 8 == 0 && n < (int64_t(1) << 30) && k % v == 0 &&
+        ldb % v == 0 && ldb < lim && alpha != 0.0f && X && B && forced != 0 && forced != 3 &&
+        ((uintptr_t) X | (uintptr_t) weight | (uintptr_t) norm_bias | (uintptr_t) B | (uintptr_t) bias | (uintptr_t) residual | (uintptr_t) Y) % 16 == 0) {
+        if (int rc = ensure_device()) return rc;
+        const int cus = cu_count();
+        const int nt = (!bf16 && mt == 2) || forced == 1 ? 1 : forced == 2 || n >= 12 * (int64_t) cus ? 2 : 1;
+        const int64_t groups = (n + 8 * nt - 1) / (8 * nt), lds = 8192 * mt * nt + mt * 64 * (8 * nt + 4) + mt * 8 * pitch;
+        // all work-groups at once: the next ones would normalise the rows again with nothing to hide that behind (1 x 3072 -> 12288 27 us for 17). Up to
+        // two fit a CU by their registers, those with 8 vectors a lane or 16 rows of bf16 one.
+        const int64_t at_once = vectors == 4 && (mt == 1 || !bf16) && 2 * lds <= 160 * 1024 ? 2 : 1;
+        const bool fused = lds <= 160 * 1024 && (forced > 0 || groups <= at_once * cus);
+        if (fused) {
+            const struct {
+                const void *weight, *bias;
+                float eps;
+            } norm{weight, norm_bias, eps};
+            char name[64];
+            std::snprintf(name, sizeof(name), "docc_%cgemm_rows_m%d_n%d_norm%d_f", bf16 ? 'b' : 's', mt, nt, vectors);
+            return launch(name, (uint32_t) groups, 1, 1, 512, (uint32_t) (mt * 8 * pitch), (hipStream_t) stream, X, (long) k, B, (long) ldb, (long) m, (long) n, (long) k, alpha, f,
+                          norm);
+        }
+    }
+    if (!scratch && k > 0) return fail(DOCC_ROCM_ERR_INVALID_ARGUMENT, "norm_linear: null pointer");
+    if (int rc = docc_rocm_layer_norm(stream, type, m, k, eps, X, weight, norm_bias, scratch)) return rc;
+    return docc_rocm_linear(stream, type, DOCC_ROCM_NO_TRANS, DOCC_ROCM_TRANS, m, n, k, alpha, scratch, k > 1 ? k : 1, B, ldb, bias, bias_type, activation, residual,
+                            residual_type, rounding, Y, y_type);
 }
 
 int docc_rocm_sgemm_batched(docc_rocm_stream_t stream, int trans_a, int trans_b, int64_t m, int64_t n, int64_t k, float alpha,

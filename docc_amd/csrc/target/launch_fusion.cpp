@@ -6,7 +6,7 @@
 //   * a convolution and the elementwise block that alone reads its result - residual, ReLU - become docc_rocm_conv2d_f32_chain;
 //   * an upload, a softmax and the download of its result become docc_rocm_softmax_host, which has the copies of different rows beside each other;
 //   * Mean, centre and square, Mean, scale and shift (how a layer norm is spelled with tensor nodes), with the casts around
-//     them for bf16, become docc_rocm_layer_norm.
+//     them for bf16, become docc_rocm_layer_norm, and with a layer on a few rows behind it docc_rocm_norm_linear.
 // A transformer's feed-forward block of nine to eleven launches is three calls this way. The reference stops at fusing Maps
 // with Maps (python/bindings/py_structured_sdfg.cpp:258-260); its products and reductions stay apart.
 #include <algorithm>
@@ -47,6 +47,16 @@ public:
     Expression m, n, k, lda, ldb;
     P type = P::Float, bias_type = P::Float, residual_type = P::Float, y_type = P::Float;
     bool has_bias = false, has_residual = false;
+    int activation = -1, rounding = 0;
+};
+
+// both of them in one call; the result of the norm is its scratch
+class NormLinearLaunch : public LaunchNode {
+public:
+    NormLinearLaunch(std::vector<std::string> inputs) : LaunchNode(LibraryNodeType_ROCM_NormLinear, std::move(inputs)) {}
+    Expression m, n, k, ldb, eps;
+    P type = P::Float, bias_type = P::Float, residual_type = P::Float, y_type = P::Float;
+    bool has_weight = false, has_norm_bias = false, has_bias = false, has_residual = false;
     int activation = -1, rounding = 0;
 };
 
@@ -219,6 +229,12 @@ public:
         for (bool changed = true; changed;) {
             changed = false;
             for (size_t j = 0; j < blocks_.size() && !changed; j++) changed = layer_norm(j) || linear(j) || conv_chain(j) || softmax_host(j);
+            applied = applied || changed;
+        }
+        // (when nothing is left that becomes a layer norm or a linear layer)
+        for (bool changed = true; changed;) {
+            changed = false;
+            for (size_t j = 0; j < blocks_.size() && !changed; j++) changed = norm_linear(j);
             applied = applied || changed;
         }
         restore_lifetimes(applied);
@@ -507,6 +523,43 @@ private:
         return true;
     }
 
+    // ---- a layer norm and the layer on a few rows behind it ---------------------------------------------
+    bool norm_linear(size_t j) {
+        const auto* l = dynamic_cast<const LinearLaunch*>(blocks_[j].node.get());
+        if (!l || l->trans_a || !l->trans_b) return false;
+        const std::string link = blocks_[j].input("_a")->data;
+        const long w = writer_of(link, j);
+        const auto* norm = w < 0 ? nullptr : dynamic_cast<const LayerNormLaunch*>(blocks_[(size_t) w].node.get());
+        if (!norm || norm->type != l->type || !symbolic::equal(norm->rows, l->m) || !symbolic::equal(norm->cols, l->k) || !symbolic::equal(l->lda, l->k)) return false;
+        const size_t i = (size_t) w;
+        // up to 16 rows of a line of 128 bytes and more: what the launcher has a kernel for
+        int64_t m = 0, k = 0;
+        if (!symbolic::is_integer(l->m, &m) || !symbolic::is_integer(l->k, &k) || m > 16 || k * (l->type == P::BFloat ? 2 : 4) < 128) return false;
+        if (!private_to(link, {i, j})) return false;
+        std::vector<std::string> connectors{"_x"};
+        std::vector<ConnectorBinding> inputs{bind("_x", blocks_[i].input("_x")->data)};
+        for (const char* name : {"_weight", "_bias"}) {
+            if (!(name[1] == 'w' ? norm->has_weight : norm->has_bias)) continue;
+            connectors.push_back(name[1] == 'w' ? "_weight" : "_norm_bias");
+            inputs.push_back(bind(connectors.back(), blocks_[i].input(name)->data));
+        }
+        const std::string result = blocks_[j].outputs[0].data;
+        for (auto& in : inputs)      // read where block j stands, by every work-group
+            if (lost_between(in.data, i, j) || in.data == result) return false;
+        for (auto& in : blocks_[j].inputs) {
+            connectors.push_back(in.connector == "_a" ? "_scratch" : in.connector);
+            inputs.push_back(in);
+            inputs.back().connector = connectors.back();
+        }
+        auto node = std::make_unique<NormLinearLaunch>(connectors);
+        node->m = l->m, node->n = l->n, node->k = l->k, node->ldb = l->ldb, node->eps = norm->eps;
+        node->type = l->type, node->bias_type = l->bias_type, node->residual_type = l->residual_type, node->y_type = l->y_type;
+        node->has_weight = norm->has_weight, node->has_norm_bias = norm->has_bias, node->has_bias = l->has_bias, node->has_residual = l->has_residual;
+        node->activation = l->activation, node->rounding = l->rounding;
+        install(j, std::move(node), std::move(inputs), result, {i}, {});
+        return true;
+    }
+
     // ---- a softmax between its operand's upload and its result's download ------------------------------
     bool softmax_host(size_t j) {
         const auto* n = dynamic_cast<const tensor::SoftmaxNode*>(blocks_[j].node.get());
@@ -703,6 +756,12 @@ public:
               << (l->has_bias ? "_bias" : "nullptr") << ", " << type_code(l->bias_type) << ", " << l->activation << ", "
               << (l->has_residual ? "_residual" : "nullptr") << ", " << type_code(l->residual_type) << ", " << l->rounding << ", _y, " << type_code(l->y_type)
               << "));" << std::endl;
+        } else if (const auto* l = dynamic_cast<const NormLinearLaunch*>(&node_)) {
+            s << "if ((" << l->m << ") != 0 && (" << l->n << ") != 0) DOCC_ROCM_CHECK(docc_rocm_norm_linear(nullptr, " << type_code(l->type) << ", " << l->m << ", " << l->n << ", "
+              << l->k << ", (float) (" << l->eps << "), _x, " << (l->has_weight ? "_weight" : "nullptr") << ", " << (l->has_norm_bias ? "_norm_bias" : "nullptr")
+              << ", (float) __alpha, _b, " << l->ldb << ", " << (l->has_bias ? "_bias" : "nullptr") << ", " << type_code(l->bias_type) << ", " << l->activation << ", "
+              << (l->has_residual ? "_residual" : "nullptr") << ", " << type_code(l->residual_type) << ", " << l->rounding << ", _scratch, _y, " << type_code(l->y_type) << "));"
+              << std::endl;
         } else if (const auto* c = dynamic_cast<const ConvChainLaunch*>(&node_)) {
             s << "{" << std::endl;
             s.setIndent(s.indent() + 4);
@@ -732,7 +791,7 @@ public:
 bool RocmLaunchFusionPass::run_pass(builder::StructuredSDFGBuilder& builder, analysis::AnalysisManager&) { return LaunchFusion(builder.subject()).run(); }
 
 void register_launch_dispatchers(codegen::LibraryNodeDispatcherRegistry& reg) {
-    for (auto& code : {LibraryNodeType_ROCM_Linear, LibraryNodeType_ROCM_ConvChain, LibraryNodeType_ROCM_SoftmaxHost, LibraryNodeType_ROCM_LayerNorm})
+    for (auto& code : {LibraryNodeType_ROCM_Linear, LibraryNodeType_ROCM_NormLinear, LibraryNodeType_ROCM_ConvChain, LibraryNodeType_ROCM_SoftmaxHost, LibraryNodeType_ROCM_LayerNorm})
         reg.register_library_node_dispatcher(code + "::" + ImplementationType_ROCMWithoutTransfers,
                                              [](codegen::LanguageExtension& le, const Function& f, const data_flow::DataFlowGraph& b, const LibraryNode& n) {
                                                  return std::make_unique<LaunchDispatcher>(le, f, b, n);

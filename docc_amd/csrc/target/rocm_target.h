@@ -106,6 +106,7 @@ public:
 inline const std::string LibraryNodeType_ROCM_ConvChain = "ROCMConvChain";
 inline const std::string LibraryNodeType_ROCM_Linear = "ROCMLinear";
 inline const std::string LibraryNodeType_ROCM_SoftmaxHost = "ROCMSoftmaxHost";
+inline const std::string LibraryNodeType_ROCM_NormLinear = "ROCMNormLinear";
 inline const std::string LibraryNodeType_ROCM_LayerNorm = "ROCMLayerNorm";
 void register_launch_dispatchers(codegen::LibraryNodeDispatcherRegistry& reg);
 // the extents of a 2-d convolution as the launchers take them: N, C, H, W, OC, KH, KW, strides, pads (begins, then ends), dilations

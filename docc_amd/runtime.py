@@ -78,6 +78,7 @@ _SIGNATURES = {
     "docc_rocm_dgemm_epilogue": [_vp, _int, _int, _i64, _i64, _i64, _f64, _vp, _i64, _vp, _i64, _f64, _vp, _i64, _vp, _int],
     "docc_rocm_sgemm_epilogue": [_vp, _int, _int, _i64, _i64, _i64, _f32, _vp, _i64, _vp, _i64, _f32, _vp, _i64, _vp, _int],
     "docc_rocm_bf16gemm_f32_epilogue": [_vp, _int, _int, _i64, _i64, _i64, _f32, _vp, _i64, _vp, _i64, _f32, _vp, _i64, _vp, _int],
+    "docc_rocm_norm_linear": [_vp, _int, _i64, _i64, _i64, _f32, _vp, _vp, _vp, _f32, _vp, _i64, _vp, _int, _int, _vp, _int, _int, _vp, _vp, _int],
     "docc_rocm_linear": [_vp, _int, _int, _int, _i64, _i64, _i64, _f32, _vp, _i64, _vp, _i64, _vp, _int, _int, _vp, _int, _int, _vp, _int],
     "docc_rocm_layer_norm": [_vp, _int, _i64, _i64, _f32, _vp, _vp, _vp, _vp],
     "docc_rocm_dgemm_batched": [_vp, _int, _int, _i64, _i64, _i64, _f64, _vp, _i64, _i64, _vp, _i64, _i64, _f64, _vp, _i64, _i64, _i64],

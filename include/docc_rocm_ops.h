@@ -118,6 +118,14 @@ int docc_rocm_layer_norm(docc_rocm_stream_t stream, int type, int64_t rows, int6
                          const void* bias, void* Y);
 
 /*
+ * A layer norm of the rows of X [m, k] and the layer behind it: docc_rocm_layer_norm(X, weight, norm_bias) into `scratch` [m, k] of the same type, then
+ * docc_rocm_linear on that (A stored by rows, B [n, k]). A few rows are one launch, which leaves `scratch` as it is.
+ */
+int docc_rocm_norm_linear(docc_rocm_stream_t stream, int type, int64_t m, int64_t n, int64_t k, float eps, const void* X, const void* weight, const void* norm_bias,
+                          float alpha, const void* B, int64_t ldb, const void* bias, int bias_type, int activation, const void* residual, int residual_type, int rounding,
+                          void* scratch, void* Y, int y_type);
+
+/*
  * A batch of `batch` equally shaped products in one launch: entry z uses
  * A + z*stride_a, B + z*stride_b, C + z*stride_c (strides in elements; 0
  * shares an input across the batch, the C matrices must not overlap).

@@ -93,6 +93,31 @@ def test_linear_on_a_few_rows(monkeypatch, blocks, dtype, m, n, k, ld):
         assert bool((err <= bound).all()), (act, float((err / bound).max()))
 
 
+# the layer norm in front of it in the same launch: a line and a part of one, 4 and 8 vectors a lane and one short of that, and shapes that keep their two launches
+@pytest.mark.parametrize("blocks", ["1", "2", "3"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("m,n,k", [(1, 8, 64), (7, 40, 72), (8, 4096, 2048), (5, 24, 1016), (9, 72, 1024), (16, 520, 256), (16, 8, 2048), (8, 16, 4096), (3, 16, 4104), (17, 16, 128),
+                                   (4, 8, 16)])
+def test_layer_norm_and_linear_as_one(monkeypatch, blocks, dtype, m, n, k):
+    monkeypatch.setenv("DOCC_ROCM_GEMM_ROWS", blocks)
+    gen = torch.Generator().manual_seed(m * 31 + n)
+    x = (torch.randn(m, k, generator=gen) * 3 + 5).to(dtype).cuda()
+    gain, shift = (1 + torch.randn(k, generator=gen) * 0.1).to(dtype).cuda(), torch.randn(k, generator=gen).to(dtype).cuda()
+    w, bias = (torch.randn(n, k, generator=gen) * k ** -0.5).to(dtype).cuda(), torch.randn(n, generator=gen).to(dtype).cuda()
+    res = torch.randn(m, n, generator=gen).to(dtype).cuda()
+    for g, b, act, r in ((gain, shift, "gelu", None), (None, None, None, res), (gain, None, "relu", res)):
+        y, scratch = torch.full((m, n), float("nan"), device="cuda", dtype=dtype), torch.empty_like(x)
+        rt.call("docc_rocm_norm_linear", 0, TYPE[dtype], m, n, k, 1e-5, ptr(x), ptr(g), ptr(b), 1.0, ptr(w), k, ptr(bias), TYPE[dtype], ACTS[act], ptr(r), TYPE[dtype], 0,
+                ptr(scratch), ptr(y), TYPE[dtype])
+        torch.cuda.synchronize()
+        h = F.layer_norm(x.double().cpu(), (k,), g.double().cpu() if g is not None else None, b.double().cpu() if b is not None else None, 1e-5).to(dtype)
+        ref = reference(h, w, True, bias, act, r, 0)
+        # as above; the normalised rows of both sides may lie on different sides of a rounding to bf16 here and there: k terms of 2^-8 k^-1/2 at most a few times that
+        bound = 2e-5 * (1 + ref.abs()) + (0 if dtype == torch.float32 else 2.0 ** -7 * (1 + ref.abs()))
+        err = (y.double().cpu() - ref).abs()
+        assert bool((err <= bound).all()), (act, float((err / bound).max()))
+
+
 # every tile with the chain in its store, ragged at both edges and along K where the tile allows it
 @pytest.mark.parametrize("cfg,dtype,k", [("128x128x32x4x4", torch.bfloat16, 104), ("128x128x64x4x4", torch.bfloat16, 328), ("128x256x64x4x3", torch.bfloat16, 328),
                                          ("256x256x32x4x4q", torch.bfloat16, 192), ("64x64x16x4x4", torch.float32, 84), ("128x128x32x4x3", torch.float32, 84),

@@ -231,3 +231,21 @@ def test_a_softmax_between_an_upload_and_a_download(tmp_path, shape, merged, rea
         assert merged in text and "memcpy" not in text and "malloc" not in text
     else:
         assert "_host(" not in text and "docc_rocm_softmax_f32(nullptr, " in text and text.count("docc_rocm_memcpy_h2d_async(") == 1
+
+
+@pytest.mark.parametrize("rows,width,merged", [(8, 64, True), (1, 64, True), (16, 64, True), (17, 64, False), (8, 16, False)])
+def test_a_layer_norm_and_the_layer_behind_it(tmp_path, rows, width, merged):
+    class Layer(torch.nn.Module):
+        def forward(self, x, g, b, w, c):
+            return F.relu(F.linear(F.layer_norm(x, (width,), g, b), w, c))
+
+    t = lambda *s: torch.randn(*s).bfloat16()
+    s = docc_torch.compile_torch(Layer(), None, target="rocm").to_sdfg(t(rows, width), t(width), t(width), t(48, width), t(48))
+    s.schedule("rocm", options={"offload": "none"})
+    text = re.sub(r"\s+", " ", open(s.generate(str(tmp_path))["source"]).read())
+    if merged:
+        assert f"docc_rocm_norm_linear(nullptr, 1, {rows}, 48, {width}, (float) (1e-05), _x, _weight, _norm_bias, (float) __alpha, _b, {width}, _bias, 1, 2, nullptr, 2, 1, _scratch, _y, 1)" in text
+        assert "docc_rocm_layer_norm" not in text and "docc_rocm_linear" not in text
+        assert text.count("docc_rocm_malloc_async(") == text.count("docc_rocm_free_async(") == 1
+    else:
+        assert "docc_rocm_norm_linear" not in text and "docc_rocm_layer_norm(" in text and "docc_rocm_linear(" in text
