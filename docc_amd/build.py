@@ -48,7 +48,7 @@ KERNEL_FAMILIES = {
     "gemm_f32_big_epilogue": "gemm_f32_big_epilogue.hip",
     "gemm_finish": "gemm_finish.hip",
     "gemm_pack": "gemm_pack.hip",
-    "gemm_rows": "gemm_rows.hip",
+    "gemm_waves": "gemm_waves.hip",
     "gemm_bf16_async_finish": "gemm_bf16_async_finish.hip",
     "gemm_bf16_async_big_finish": "gemm_bf16_async_big_finish.hip",
     "gemm_f32_finish": "gemm_f32_finish.hip",
@@ -89,6 +89,7 @@ FAMILY_FLAGS = {
     "attention": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "attention_split": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "gemm_skinny": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+    "gemm_waves": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
 }
 
 # packed fp32 VALU ops are switched off for every device compile

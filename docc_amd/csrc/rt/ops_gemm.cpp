@@ -83,6 +83,46 @@ double sdgemm_best_seconds(Picker pick, int64_t m, int64_t n, int64_t k, bool tb
     return best;
 }
 
+// Seconds of a product A B^T of fp32 or bf16 operands that a chain follows, on the tiles, whole or in parts (the pass that adds them counted)
+double tiles_seconds(Picker pick, int64_t m, int64_t n, int64_t k, int cus, size_t elem, bool lines) {
+    if (elem == 4) return 4.0e-6 + sdgemm_best_seconds(pick, m, n, k, true, cus, elem);
+    const TileConfig whole = pick(m, n, k, true, 1, lines ? 2 : 1, 0, cus);
+    double best = bgemm_seconds(whole, m, n, k, true, 1, cus, lines);
+    if (k < 512 || ((m + whole.bm - 1) / whole.bm) * ((n + whole.bn - 1) / whole.bn) >= cus) return best;
+    for (const int64_t parts : kPartCounts) {
+        const int64_t part = part_length(k, parts), bytes = parts * m * n * 4;
+        if ((k + part - 1) / part != parts || part < 256 || bytes > kMaxPartsBytes) continue;
+        const double t = bgemm_seconds(pick(m, n, part, true, parts, lines ? 2 : 1, 0, cus), m, n, part, true, parts, cus, lines) + 2.0 * (double) bytes / 5e12 + 3.5e-6;
+        if (t < best) best = t;
+    }
+    return best;
+}
+
+// The tile of csrc/kernels/gemm_waves.hip and its estimate: a launch, and so long a tile on the compute unit that has most of them. Fitted to 58 products a type from
+// 33 x 64 x 256 to 4096 x 2048 x 512, of most of them less than 10 % off.
+struct WavesChoice {
+    int edge;
+    bool one;        // no compute unit has two
+    double seconds;
+};
+WavesChoice waves_choice(int64_t m, int64_t n, int64_t k, int cus, size_t elem, int forced) {
+    auto per_cu = [&](int64_t edge) { return (double) ((((m + edge - 1) / edge) * ((n + edge - 1) / edge) + cus - 1) / cus); };
+    const double n16 = per_cu(16), n32 = per_cu(32), n64 = per_cu(64), kd = (double) k;
+    const double t16 = elem == 2 ? 3.8 + n16 * (0.4 + 0.00065 * kd) : 4.0 + n16 * (0.5 + 0.00125 * kd);
+    const double t32 = elem == 2 ? 3.4 + n32 * (0.75 + 0.0010 * kd) : 3.7 + n32 * (0.75 + 0.0043 * kd);
+    const bool one = n64 <= 1.0 && (elem == 4 || k > 1024);
+    const double t64 = elem == 4 ? 3.7 + n64 * (1.2 + 0.0172 * kd) : one ? 4.75 + 0.0028 * kd : 1.9 + n64 * (2.1 + 0.0027 * kd);
+    if (forced > 0 ? forced == 16 : m <= 16 || (t16 < t32 && t16 < t64)) return {16, false, 1e-6 * t16};
+    if (forced > 0 ? forced == 32 : t32 <= t64) return {32, false, 1e-6 * t32};
+    return {64, forced > 0 ? forced == 1 : one, 1e-6 * t64};
+}
+// what the kernels read: whole vectors, a tile's rows within 32 bits of its first
+bool waves_shape_ok(int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb, size_t elem) {
+    const int64_t v = 16 / (int64_t) elem, lim = int64_t(1) << 23;
+    return n % 8 == 0 && k > 0 && k % v == 0 && lda % v == 0 && ldb % v == 0 && k < lim && lda < lim && ldb < lim && m < (int64_t(1) << 24) && n < (int64_t(1) << 24) &&
+           ((m + 15) / 16) * ((n + 15) / 16) < (int64_t(1) << 31);
+}
+
 // Microseconds of an fp32 or fp64 product on the element-wise tiles (operands off the vectors): a round of tiles over the CUs takes so long per k.
 // `turned`: an operand is read along m or n.
 double plain_us(Picker pick, int64_t m, int64_t n, int64_t k, bool tb, bool turned, int cus, size_t elem) {
@@ -330,27 +370,32 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
         return docc_rocm_elementwise_fused(stream, sizeof(S) == 8 ? 64 : 32, 2, shape, bias ? DOCC_ROCM_BINARY_ADD : -1, shape, C, 0.0,
                                            bias ? row : nullptr, bias, 0.0, activation >= 0 ? 1 : 0, post, C);
     }
-    // A layer on up to 32 rows, weights stored [n][k]: product and chain as one launch (csrc/kernels/gemm_rows.hip). Against the forms below (skinny
-    // kernels with K in parts, matrix-vector kernels, both with a pass behind them) in bf16: 8 x 2048 -> 8192 13.1 -> 9.2 us, 8 x 8192 -> 2048 15.0 -> 10.7,
-    // 3 x 1024 -> 4096 11.4 -> 5.5, fp32 21.1 -> 15.1, 25.0 -> 18.3 and 13.9 -> 6.5. Every block of columns reads A again: above 16 rows a large matrix is
-    // better read by the kernels that cut K (32 x 2048 -> 8192 22 us here for 15, fp32 32 x 1024 -> 4096 14 for 13, but 24 x 2048 -> 512 7.0 for 11), in fp32 above
-    // eight (16 x 2048 -> 8192 22.3 for 21.8, but 12 x 4096 -> 1024 12.8 for 15.6); a single row by the matrix-vector kernel (fp32 1 x 3072 -> 12288 31 for 27;
-    // a block of 1 x 3072 in bf16 37.5 for 36.1, of 16 53.3 for 52.4).
-    // Two blocks of columns a work-group from three quarters of a work-group a CU on (8 x 8192 -> 2048 10.7 us with one, 14.3 with two; 12288 -> 3072 24.7 and 19.7).
-    // DOCC_ROCM_GEMM_ROWS=0 switches it off, =1 and =2 give the blocks of eight columns a work-group takes (tests, tuning).
+    // A layer whose product has too few tiles for the kernels below to fill the compute units, weights stored [n][k]: K cut between the wavefronts of a work-group,
+    // the chain in the same launch (csrc/kernels/gemm_waves.hip). DOCC_ROCM_GEMM_WAVES=0 switches it off, =16, =32, =64 and =1 take the tile of that size, or that
+    // of a work-group a compute unit (tests, tuning).
     if constexpr (sizeof(T) <= 4) {
-        const char* rows_env = tuning("DOCC_ROCM_GEMM_ROWS");
-        const int64_t v = 16 / (int64_t) sizeof(T), lim = int64_t(1) << 23;
-        const int forced = rows_env ? rows_env[0] - '0' : -1;
-        const int64_t size = n * k, mi = int64_t(1) << 20;
-        const bool size_ok = forced > 0 || (sizeof(T) == 2 ? (m <= 1 || (m > 8 && m <= 16) ? size < 32 * mi : m <= 8 || size < 8 * mi)
-                                                           : m <= 1 ? size < 16 * mi : m <= 8 ? true : m <= 16 ? size < 8 * mi : size < 2 * mi);
-        if (fin && !ta && tb && batch == 1 && m <= 32 && size_ok && forced != 0 && n % 8 == 0 && k % v == 0 && lda % v == 0 && ldb % v == 0 && k < lim && lda < lim &&
-            ldb < lim && n < (int64_t(1) << 30) &&
+        const char* waves_env = tuning("DOCC_ROCM_GEMM_WAVES");
+        const int forced = waves_env ? std::atoi(waves_env) : -1;
+        if (fin && !ta && tb && batch == 1 && forced != 0 && waves_shape_ok(m, n, k, lda, ldb, sizeof(T)) &&
             ((uintptr_t) A | (uintptr_t) B | (uintptr_t) fin->bias | (uintptr_t) fin->residual | (uintptr_t) fin->out) % 16 == 0) {
-            const int mt = m <= 8 ? 1 : m <= 16 ? 2 : 4, nt = mt == 4 || forced == 1 ? 1 : forced == 2 || n >= 12 * (int64_t) cus ? 2 : 1;
-            std::snprintf(name, sizeof(name), "docc_%cgemm_rows_m%d_n%d_f", sizeof(T) == 2 ? 'b' : 's', mt, nt);
-            return launch(name, (uint32_t) ((n + 8 * nt - 1) / (8 * nt)), 1, 1, 512, 0, s, A, (long) lda, B, (long) ldb, (long) m, (long) n, (long) k, (float) alpha, *fin);
+            const bool on_lines = ((uintptr_t) A | (uintptr_t) B | (uintptr_t) (lda * (int64_t) sizeof(T)) | (uintptr_t) (ldb * (int64_t) sizeof(T))) % 128 == 0;
+            const WavesChoice w = waves_choice(m, n, k, cus, sizeof(T), forced);
+            // Up to 32 rows (against the kernels with K in parts and a pass behind them): bf16 1 x 2048 -> 8192 9.9 us and 7.8, 8 x 2048 -> 8192 12.7 and 7.8,
+            // 16 x 12288 -> 3072 21.3 and 14.2, 32 x 4096 -> 1024 14.6 and 5.6; fp32 21.2 and 12.7 (8 x 2048), 40.6 and 35.3, 16.2 and 9.1. But a single row of
+            // a large matrix is read by the matrix-vector kernel: fp32 1 x 4096 -> 14336 42.6 us here and 39.7, bf16 1 x 8192 -> 28672 78.8 and 73.4; a block of 1 x 3072
+            // whose weights come from HBM 66.6 us and 59.0, in bf16 38.0 and 36.2.
+            // Beyond by the estimates: bf16 1024 x 1024 x 256 9.9 -> 5.8 us, 1024 x 256 x 1024 13.8 -> 5.3, 1024 x 512 x 2048 14.2 -> 8.2, 512 x 4096 x 1024 15.0 ->
+            // 11.7, but 1024 x 4096 x 1024 17.3 and 20.7; fp32 1024 x 256 x 1024 13.1 -> 8.6, 256 x 2048 x 512 13.5 -> 8.6, 2048 x 3072 x 768 108 -> 86, but
+            // 2048 x 2048 x 512 41.5 and 43.6. (Both estimates are some 10 % off: for a clear gain only.)
+            const bool few = m <= 32 && (m > 1 || n * k * (int64_t) sizeof(T) < (int64_t(64) << 20));
+            if (forced > 0 || few || (m > 32 && w.seconds < 0.85 * tiles_seconds(pick, m, n, k, cus, sizeof(T), on_lines))) {
+                const int64_t tiles = ((m + w.edge - 1) / w.edge) * ((n + w.edge - 1) / w.edge);
+                std::snprintf(name, sizeof(name), "docc_%cgemm_waves_%dx%d%s_f", sizeof(T) == 2 ? 'b' : 's', w.edge, w.edge, w.one ? "_one" : "");
+                // a ring of two pieces of 16 bytes times `seg` of the tile's rows and columns a wavefront; the sums of all of them, or of half, take less
+                const int nw = w.edge == 16 || (w.one && sizeof(T) == 4) ? 8 : 4, seg = w.edge <= 32 || (w.one && sizeof(T) == 2) ? 8 : 4;
+                return launch(name, (uint32_t) tiles, 1, 1, 64 * nw, (uint32_t) (nw * 2 * 2 * w.edge * seg * 16), s, A, (long) lda, B, (long) ldb, (long) m, (long) n, (long) k,
+                              (float) alpha, *fin);
+            }
         }
     }
     const bool epilogue = bias || activation >= 0;
@@ -829,34 +874,30 @@ int docc_rocm_norm_linear(docc_rocm_stream_t stream, int type, int64_t m, int64_
     if (int rc = linear_finish(type, m, n, bias, bias_type, activation, residual, residual_type, rounding, Y, y_type, &f)) return rc;
     if (m < 0 || n < 0 || k < 0 || ldb < (k > 1 ? k : 1)) return fail(DOCC_ROCM_ERR_INVALID_ARGUMENT, "norm_linear: bad shape");
     if (m == 0 || n == 0) return 0;
-    // Rows that a wavefront holds, every work-group's in LDS (csrc/kernels/gemm_rows.hip): a launch of 3 to 4 us less. Every work-group normalises all rows again,
-    // 4 to 16 vectors a lane, while it waits for its first lines of B. DOCC_ROCM_GEMM_ROWS=0 or =3 keeps the layer norm a launch of its own (tests, tuning).
-    const char* rows_env = gemm_tuning_set() ? std::getenv("DOCC_ROCM_GEMM_ROWS") : nullptr;
-    const int forced = rows_env ? rows_env[0] - '0' : -1;
+    // Rows that a wavefront holds, every work-group's in LDS (csrc/kernels/gemm_waves.hip): a launch of 3 to 4 us less. Every work-group normalises all rows again,
+    // 4 to 16 vectors a lane, while it waits for its first pieces of B. DOCC_ROCM_GEMM_WAVES=0 or a tile other than 16 keeps the layer norm a launch of its own
+    // (tests, tuning).
+    const char* env = gemm_tuning_set() ? std::getenv("DOCC_ROCM_GEMM_WAVES") : nullptr;
+    const int forced = env ? std::atoi(env) : -1;
     const bool bf16 = type == DOCC_ROCM_TYPE_BF16;
-    const int64_t v = bf16 ? 8 : 4, lim = int64_t(1) << 23;
-    const int mt = m <= 8 ? 1 : 2, vectors = k <= 256 * v ? 4 : 8;      // vectors a lane holds
-    const int64_t pitch = (k + v) * (bf16 ? 2 : 4);
-    if (m <= 16 && k >= 8 * v && k <= 512 * v && (mt == 1 || (vectors == 4 && (bf16 || n * k < int64_t(8) << 20))) && n % 8 == 0 && n < (int64_t(1) << 30) && k % v == 0 &&
-        ldb % v == 0 && ldb < lim && alpha != 0.0f && X && B && forced != 0 && forced != 3 &&
+    const int64_t v = bf16 ? 8 : 4;
+    const int rows = m <= 8 ? 8 : 16, vectors = k <= 256 * v ? 4 : 8;      // vectors a lane holds
+    if (m <= 16 && k >= 8 * v && k <= 512 * v && (rows == 8 || vectors == 4) && waves_shape_ok(m, n, k, k, ldb, bf16 ? 2 : 4) && alpha != 0.0f && X && B &&
+        (forced < 0 || forced == 16) &&
         ((uintptr_t) X | (uintptr_t) weight | (uintptr_t) norm_bias | (uintptr_t) B | (uintptr_t) bias | (uintptr_t) residual | (uintptr_t) Y) % 16 == 0) {
         if (int rc = ensure_device()) return rc;
-        const int cus = cu_count();
-        const int nt = (!bf16 && mt == 2) || forced == 1 ? 1 : forced == 2 || n >= 12 * (int64_t) cus ? 2 : 1;
-        const int64_t groups = (n + 8 * nt - 1) / (8 * nt), lds = 8192 * mt * nt + mt * 64 * (8 * nt + 4) + mt * 8 * pitch;
-        // all work-groups at once: the next ones would normalise the rows again with nothing to hide that behind (1 x 3072 -> 12288 27 us for 17). Up to
-        // two fit a CU by their registers, those with 8 vectors a lane or 16 rows of bf16 one.
-        const int64_t at_once = vectors == 4 && (mt == 1 || !bf16) && 2 * lds <= 160 * 1024 ? 2 : 1;
-        const bool fused = lds <= 160 * 1024 && (forced > 0 || groups <= at_once * cus);
-        if (fused) {
+        // the rings, the rows, and a piece's length behind the last
+        const int64_t groups = (n + 15) / 16, lds = 8 * 2 * 16 * 128 + rows * (k + v) * (bf16 ? 2 : 4) + 128;
+        // all work-groups at once: the next ones would normalise the rows again with nothing to hide that behind
+        const int64_t at_once = (!bf16 || (vectors == 4 && rows == 8)) && 2 * lds <= 160 * 1024 ? 2 : 1;
+        if (lds <= 160 * 1024 && (forced > 0 || groups <= at_once * cu_count())) {
             const struct {
                 const void *weight, *bias;
                 float eps;
             } norm{weight, norm_bias, eps};
             char name[64];
-            std::snprintf(name, sizeof(name), "docc_%cgemm_rows_m%d_n%d_norm%d_f", bf16 ? 'b' : 's', mt, nt, vectors);
-            return launch(name, (uint32_t) groups, 1, 1, 512, (uint32_t) (mt * 8 * pitch), (hipStream_t) stream, X, (long) k, B, (long) ldb, (long) m, (long) n, (long) k, alpha, f,
-                          norm);
+            std::snprintf(name, sizeof(name), "docc_%cgemm_waves_norm%d_m%d_f", bf16 ? 'b' : 's', vectors, rows);
+            return launch(name, (uint32_t) groups, 1, 1, 512, (uint32_t) lds, (hipStream_t) stream, X, (long) k, B, (long) ldb, (long) m, (long) n, (long) k, alpha, f, norm);
         }
     }
     if (!scratch && k > 0) return fail(DOCC_ROCM_ERR_INVALID_ARGUMENT, "norm_linear: null pointer");

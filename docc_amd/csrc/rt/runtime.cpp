@@ -46,7 +46,7 @@ const char* const kKernelImages[] = {
     "docc_rocm_gemm_f32_big_epilogue.hsaco",
     "docc_rocm_gemm_finish.hsaco",
     "docc_rocm_gemm_pack.hsaco",
-    "docc_rocm_gemm_rows.hsaco",
+    "docc_rocm_gemm_waves.hsaco",
     "docc_rocm_gemm_bf16_async_finish.hsaco",
     "docc_rocm_gemm_bf16_async_big_finish.hsaco",
     "docc_rocm_gemm_f32_finish.hsaco",

@@ -70,14 +70,14 @@ def test_linear_over_the_launchers_forms(dtype, m, n, k):
         assert bool((err <= bound).all()), (act, float((err / bound).max()))
 
 
-# a few rows (csrc/kernels/gemm_rows.hip): blocks of eight rows and columns, K in lines of 128 bytes that eight wavefronts take in turn - less than a line, a
-# part of one behind many, more lines than are on their way at once - and rows of A and B that are longer than K
-@pytest.mark.parametrize("blocks", ["1", "2"])
+# K cut between the wavefronts of a work-group (csrc/kernels/gemm_waves.hip), in pieces of 64 or 128 bytes of a row that four or eight wavefronts take in turn: less
+# than a piece, a part of one behind many, more pieces than are on their way at once, ragged tiles - and rows of A and B that are longer than K
+@pytest.mark.parametrize("tile", ["16", "32", "64", "1"])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("m,n,k,ld", [(1, 8, 8, 8), (2, 24, 64, 64), (7, 40, 72, 80), (8, 16, 1032, 1032), (9, 520, 200, 208), (16, 72, 4168, 4168), (17, 8, 136, 136),
-                                      (32, 264, 2056, 2064)])
-def test_linear_on_a_few_rows(monkeypatch, blocks, dtype, m, n, k, ld):
-    monkeypatch.setenv("DOCC_ROCM_GEMM_ROWS", blocks)
+                                      (32, 264, 2056, 2064), (65, 136, 520, 520), (130, 72, 264, 272)])
+def test_linear_cut_between_wavefronts(monkeypatch, tile, dtype, m, n, k, ld):
+    monkeypatch.setenv("DOCC_ROCM_GEMM_WAVES", tile)
     gen = torch.Generator().manual_seed(m * 31 + n)
     a, w = torch.randn(m, ld, generator=gen).to(dtype).cuda(), (torch.randn(n, ld, generator=gen) * k ** -0.5).to(dtype).cuda()
     a[:, k:], w[:, k:] = float("nan"), float("inf")           # behind the rows: not read, or dropped
@@ -93,13 +93,13 @@ def test_linear_on_a_few_rows(monkeypatch, blocks, dtype, m, n, k, ld):
         assert bool((err <= bound).all()), (act, float((err / bound).max()))
 
 
-# the layer norm in front of it in the same launch: a line and a part of one, 4 and 8 vectors a lane and one short of that, and shapes that keep their two launches
-@pytest.mark.parametrize("blocks", ["1", "2", "3"])
+# the layer norm in front of it in the same launch: a piece and a part of one, 4 and 8 vectors a lane and one short of that, and shapes that keep their two launches
+@pytest.mark.parametrize("tile", ["16", "32"])      # 32: two launches
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("m,n,k", [(1, 8, 64), (7, 40, 72), (8, 4096, 2048), (5, 24, 1016), (9, 72, 1024), (16, 520, 256), (16, 8, 2048), (8, 16, 4096), (3, 16, 4104), (17, 16, 128),
                                    (4, 8, 16)])
-def test_layer_norm_and_linear_as_one(monkeypatch, blocks, dtype, m, n, k):
-    monkeypatch.setenv("DOCC_ROCM_GEMM_ROWS", blocks)
+def test_layer_norm_and_linear_as_one(monkeypatch, tile, dtype, m, n, k):
+    monkeypatch.setenv("DOCC_ROCM_GEMM_WAVES", tile)
     gen = torch.Generator().manual_seed(m * 31 + n)
     x = (torch.randn(m, k, generator=gen) * 3 + 5).to(dtype).cuda()
     gain, shift = (1 + torch.randn(k, generator=gen) * 0.1).to(dtype).cuda(), torch.randn(k, generator=gen).to(dtype).cuda()
