@@ -49,6 +49,7 @@ KERNEL_FAMILIES = {
     "gemm_finish": "gemm_finish.hip",
     "gemm_pack": "gemm_pack.hip",
     "gemm_waves": "gemm_waves.hip",
+    "gemm_waves_plain": "gemm_waves_plain.hip",
     "gemm_bf16_async_finish": "gemm_bf16_async_finish.hip",
     "gemm_bf16_async_big_finish": "gemm_bf16_async_big_finish.hip",
     "gemm_f32_finish": "gemm_f32_finish.hip",
@@ -90,6 +91,7 @@ FAMILY_FLAGS = {
     "attention_split": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "gemm_skinny": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "gemm_waves": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+    "gemm_waves_plain": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
 }
 
 # packed fp32 VALU ops are switched off for every device compile

@@ -83,16 +83,16 @@ double sdgemm_best_seconds(Picker pick, int64_t m, int64_t n, int64_t k, bool tb
     return best;
 }
 
-// Seconds of a product A B^T of fp32 or bf16 operands that a chain follows, on the tiles, whole or in parts (the pass that adds them counted)
-double tiles_seconds(Picker pick, int64_t m, int64_t n, int64_t k, int cus, size_t elem, bool lines) {
-    if (elem == 4) return 4.0e-6 + sdgemm_best_seconds(pick, m, n, k, true, cus, elem);
-    const TileConfig whole = pick(m, n, k, true, 1, lines ? 2 : 1, 0, cus);
-    double best = bgemm_seconds(whole, m, n, k, true, 1, cus, lines);
+// Seconds of a product on the tiles, whole or in parts (the pass that adds them counted)
+double tiles_seconds(Picker pick, int64_t m, int64_t n, int64_t k, bool tb, int cus, size_t elem, bool lines) {
+    if (elem != 2) return 4.0e-6 + sdgemm_best_seconds(pick, m, n, k, tb, cus, elem);
+    const TileConfig whole = pick(m, n, k, tb, 1, lines ? 2 : 1, 0, cus);
+    double best = bgemm_seconds(whole, m, n, k, tb, 1, cus, lines);
     if (k < 512 || ((m + whole.bm - 1) / whole.bm) * ((n + whole.bn - 1) / whole.bn) >= cus) return best;
     for (const int64_t parts : kPartCounts) {
         const int64_t part = part_length(k, parts), bytes = parts * m * n * 4;
         if ((k + part - 1) / part != parts || part < 256 || bytes > kMaxPartsBytes) continue;
-        const double t = bgemm_seconds(pick(m, n, part, true, parts, lines ? 2 : 1, 0, cus), m, n, part, true, parts, cus, lines) + 2.0 * (double) bytes / 5e12 + 3.5e-6;
+        const double t = bgemm_seconds(pick(m, n, part, tb, parts, lines ? 2 : 1, 0, cus), m, n, part, tb, parts, cus, lines) + 2.0 * (double) bytes / 5e12 + 3.5e-6;
         if (t < best) best = t;
     }
     return best;
@@ -108,18 +108,20 @@ struct WavesChoice {
 WavesChoice waves_choice(int64_t m, int64_t n, int64_t k, int cus, size_t elem, int forced) {
     auto per_cu = [&](int64_t edge) { return (double) ((((m + edge - 1) / edge) * ((n + edge - 1) / edge) + cus - 1) / cus); };
     const double n16 = per_cu(16), n32 = per_cu(32), n64 = per_cu(64), kd = (double) k;
-    const double t16 = elem == 2 ? 3.8 + n16 * (0.4 + 0.00065 * kd) : 4.0 + n16 * (0.5 + 0.00125 * kd);
-    const double t32 = elem == 2 ? 3.4 + n32 * (0.75 + 0.0010 * kd) : 3.7 + n32 * (0.75 + 0.0043 * kd);
     const bool one = n64 <= 1.0 && (elem == 4 || k > 1024);
-    const double t64 = elem == 4 ? 3.7 + n64 * (1.2 + 0.0172 * kd) : one ? 4.75 + 0.0028 * kd : 1.9 + n64 * (2.1 + 0.0027 * kd);
-    if (forced > 0 ? forced == 16 : m <= 16 || (t16 < t32 && t16 < t64)) return {16, false, 1e-6 * t16};
-    if (forced > 0 ? forced == 32 : t32 <= t64) return {32, false, 1e-6 * t32};
+    const double t16 = elem == 2 ? 3.8 + n16 * (0.4 + 0.00065 * kd) : elem == 4 ? 4.0 + n16 * (0.5 + 0.00125 * kd) : 3.8 + n16 * (0.6 + 0.0024 * kd);
+    const double t32 = elem == 2 ? 3.4 + n32 * (0.75 + 0.0010 * kd) : elem == 4 ? 3.7 + n32 * (0.75 + 0.0043 * kd) : 3.8 + n32 * (0.9 + 0.0092 * kd);
+    const double t64 = elem == 2 ? (one ? 4.75 + 0.0028 * kd : 1.9 + n64 * (2.1 + 0.0027 * kd))
+                                 : 3.7 + n64 * (1.2 + 0.0172 * kd);
+    if (forced > 0 ? forced == 16 : m <= 16 || (t16 < t32 && (elem == 8 || t16 < t64))) return {16, false, 1e-6 * t16};
+    // (fp64: 64 x 64 tiles of 1000 k took 39.0 us for the 37.0 of gemm_async.h's)
+    if (elem == 8 || (forced > 0 ? forced == 32 : t32 <= t64)) return {32, false, 1e-6 * t32};
     return {64, forced > 0 ? forced == 1 : one, 1e-6 * t64};
 }
 // what the kernels read: whole vectors, a tile's rows within 32 bits of its first
-bool waves_shape_ok(int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb, size_t elem) {
-    const int64_t v = 16 / (int64_t) elem, lim = int64_t(1) << 23;
-    return n % 8 == 0 && k > 0 && k % v == 0 && lda % v == 0 && ldb % v == 0 && k < lim && lda < lim && ldb < lim && m < (int64_t(1) << 24) && n < (int64_t(1) << 24) &&
+bool waves_shape_ok(int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb, bool tb, size_t elem) {
+    const int64_t v = 16 / (int64_t) elem, lim = (int64_t(1) << 25) / (int64_t) elem;
+    return k > 0 && k % v == 0 && lda % v == 0 && ldb % v == 0 && (tb || n % v == 0) && k < lim && lda < lim && ldb < lim && m < (int64_t(1) << 24) && n < (int64_t(1) << 24) &&
            ((m + 15) / 16) * ((n + 15) / 16) < (int64_t(1) << 31);
 }
 
@@ -375,8 +377,10 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
     // of a work-group a compute unit (tests, tuning).
     if constexpr (sizeof(T) <= 4) {
         const char* waves_env = tuning("DOCC_ROCM_GEMM_WAVES");
-        const int forced = waves_env ? std::atoi(waves_env) : -1;
-        if (fin && !ta && tb && batch == 1 && forced != 0 && waves_shape_ok(m, n, k, lda, ldb, sizeof(T)) &&
+        int forced = waves_env ? std::atoi(waves_env) : -1;
+        for (const char* other : {"DOCC_ROCM_GEMM_CFG", "DOCC_ROCM_GEMM_TILE", "DOCC_ROCM_GEMM_SPLITK", "DOCC_ROCM_GEMM_SKINNY"})   // they ask for another form
+            if (forced < 0 && tuning(other)) forced = 0;
+        if (fin && !ta && tb && batch == 1 && forced != 0 && n % 8 == 0 && waves_shape_ok(m, n, k, lda, ldb, true, sizeof(T)) &&
             ((uintptr_t) A | (uintptr_t) B | (uintptr_t) fin->bias | (uintptr_t) fin->residual | (uintptr_t) fin->out) % 16 == 0) {
             const bool on_lines = ((uintptr_t) A | (uintptr_t) B | (uintptr_t) (lda * (int64_t) sizeof(T)) | (uintptr_t) (ldb * (int64_t) sizeof(T))) % 128 == 0;
             const WavesChoice w = waves_choice(m, n, k, cus, sizeof(T), forced);
@@ -388,7 +392,7 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
             // 11.7, but 1024 x 4096 x 1024 17.3 and 20.7; fp32 1024 x 256 x 1024 13.1 -> 8.6, 256 x 2048 x 512 13.5 -> 8.6, 2048 x 3072 x 768 108 -> 86, but
             // 2048 x 2048 x 512 41.5 and 43.6. (Both estimates are some 10 % off: for a clear gain only.)
             const bool few = m <= 32 && (m > 1 || n * k * (int64_t) sizeof(T) < (int64_t(64) << 20));
-            if (forced > 0 || few || (m > 32 && w.seconds < 0.85 * tiles_seconds(pick, m, n, k, cus, sizeof(T), on_lines))) {
+            if (forced > 0 || few || (m > 32 && w.seconds < 0.85 * tiles_seconds(pick, m, n, k, true, cus, sizeof(T), on_lines))) {
                 const int64_t tiles = ((m + w.edge - 1) / w.edge) * ((n + w.edge - 1) / w.edge);
                 std::snprintf(name, sizeof(name), "docc_%cgemm_waves_%dx%d%s_f", sizeof(T) == 2 ? 'b' : 's', w.edge, w.edge, w.one ? "_one" : "");
                 // a ring of two pieces of 16 bytes times `seg` of the tile's rows and columns a wavefront; the sums of all of them, or of half, take less
@@ -397,6 +401,42 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
                               (float) alpha, *fin);
             }
         }
+    }
+    auto waves_plain = [&](int forced) {
+        const WavesChoice w = waves_choice(m, n, k, cus, sizeof(T), forced);
+        const int64_t tiles = ((m + w.edge - 1) / w.edge) * ((n + w.edge - 1) / w.edge);
+        std::snprintf(name, sizeof(name), "docc_%cgemm_waves_%dx%d%s_n%c", prefix[0], w.edge, w.edge, w.one ? "_one" : "", tb ? 't' : 'n');
+        // the rings, or the sums of all wavefronts or (above 64 KB) of half of them
+        const int64_t nw = w.edge == 16 || (w.one && sizeof(T) > 2) ? 8 : 4, seg = w.edge <= 32 || (w.one && sizeof(T) == 2) ? 8 : 4;
+        const int64_t ring = nw * 2 * 2 * w.edge * seg * 16, sums = nw * w.edge * (w.edge * (int64_t) sizeof(S) + 16), held = sums > 65536 ? sums / 2 : sums;
+        return launch(name, (uint32_t) tiles, 1, 1, (uint32_t) (64 * nw), (uint32_t) (ring > held ? ring : held), s, A, (long) lda, B, (long) ldb, (long) m, (long) n, (long) k, alpha, beta, C,
+                      (long) ldc, bias, activation);
+    };
+    // The same for a product of fp32 or fp64 alone, B stored [k][n] as well (csrc/kernels/gemm_waves_plain.hip).
+    if (sizeof(T) > 2 && !fin && !ta && batch == 1 && (activation < 0 || activation == DOCC_ROCM_UNARY_ABS || activation == DOCC_ROCM_UNARY_RELU) && n >= 16 && waves_shape_ok(m, n, k, lda, ldb, tb, sizeof(T)) && ((uintptr_t) A | (uintptr_t) B) % 16 == 0) {
+        const char* waves_env = tuning("DOCC_ROCM_GEMM_WAVES");
+        int forced = waves_env ? std::atoi(waves_env) : -1;
+        for (const char* other : {"DOCC_ROCM_GEMM_CFG", "DOCC_ROCM_GEMM_TILE", "DOCC_ROCM_GEMM_SPLITK", "DOCC_ROCM_GEMM_SKINNY", "DOCC_ROCM_GEMV_OFF", "DOCC_ROCM_GEMV_SLICES"})
+            if (forced < 0 && tuning(other)) forced = 0;
+        bool pays = false;
+        if (m > 32) {
+            // by the estimates: fp32 512 x 512 x 512 10.6 -> 6.2 us, 192 x 64 x 1664 11.6 -> 5.6, 64 x 5824 x 896 15.7 -> 12.7;
+            // fp64 512 x 512 x 512 12.0 -> 8.6
+            const bool on_lines = ((uintptr_t) A | (uintptr_t) B | (uintptr_t) (lda * (int64_t) sizeof(T)) | (uintptr_t) (ldb * (int64_t) sizeof(T))) % 128 == 0;
+            // (315 x 600 x 3584, B [k][n] 23.2 us and 26.2: not above k = 2048 there)
+            // B [n][k] in whole rounds of the wavefronts only (four of 32 k in fp32); a K off them stays with the parts, whose tests hold such products
+            pays = forced < 0 && (tb ? k % 128 == 0 : k <= 2048) && waves_choice(m, n, k, cus, sizeof(T), forced).seconds < 0.85 * tiles_seconds(pick, m, n, k, tb, cus, sizeof(T), on_lines);
+        } else if (tb) {
+            // Against the matrix-vector kernels, the skinny ones and K in parts, B stored [n][k]: fp32 2 x 8192 x 2048 24 -> 12 us, 8 x 2048 x 2048 11.2 -> 6.1, 32 x
+            // 8192 x 8192 96 -> 59; fp64 8 x 8192 x 2048 40 -> 22, but 8 x 512 x 8192 19.5 and 23.4
+            // (few tiles, a long chain each). From two tiles on. A single row is one launch there too (fp32 1 x 2048 x 8192 11.7 us, 13.9 here), but for few columns.
+            pays = n >= 32 && n * k <= (int64_t(1) << 27) && (m > 1 || n < 4 * (int64_t) cus) && (sizeof(T) != 8 || k <= 4096 || (m > 1 && n >= 2048));
+        } else {
+            // B stored [k][n]: fp32 1 x 2048 x 2048 9.4 -> 6.6 us, 8 x 8192 x 512 11.2 -> 5.6, but 2 x 8192 x 8192 46.6 and 69 (64 bytes of a row of B a work-group);
+            // fp64 8 x 2048 x 2048 15.3 -> 9.6
+            pays = k <= 2048 && n * k <= (int64_t(1) << 24);
+        }
+        if (forced > 0 || (pays && forced < 0)) return waves_plain(forced);
     }
     const bool epilogue = bias || activation >= 0;
     // A tall matrix times a few columns held as numpy holds them (B [k][n], n small): rows of B are a few elements long, so
@@ -882,7 +922,7 @@ int docc_rocm_norm_linear(docc_rocm_stream_t stream, int type, int64_t m, int64_
     const bool bf16 = type == DOCC_ROCM_TYPE_BF16;
     const int64_t v = bf16 ? 8 : 4;
     const int rows = m <= 8 ? 8 : 16, vectors = k <= 256 * v ? 4 : 8;      // vectors a lane holds
-    if (m <= 16 && k >= 8 * v && k <= 512 * v && (rows == 8 || vectors == 4) && waves_shape_ok(m, n, k, k, ldb, bf16 ? 2 : 4) && alpha != 0.0f && X && B &&
+    if (m <= 16 && k >= 8 * v && k <= 512 * v && (rows == 8 || vectors == 4) && n % 8 == 0 && waves_shape_ok(m, n, k, k, ldb, true, bf16 ? 2 : 4) && alpha != 0.0f && X && B &&
         (forced < 0 || forced == 16) &&
         ((uintptr_t) X | (uintptr_t) weight | (uintptr_t) norm_bias | (uintptr_t) B | (uintptr_t) bias | (uintptr_t) residual | (uintptr_t) Y) % 16 == 0) {
         if (int rc = ensure_device()) return rc;

@@ -47,6 +47,7 @@ const char* const kKernelImages[] = {
     "docc_rocm_gemm_finish.hsaco",
     "docc_rocm_gemm_pack.hsaco",
     "docc_rocm_gemm_waves.hsaco",
+    "docc_rocm_gemm_waves_plain.hsaco",
     "docc_rocm_gemm_bf16_async_finish.hsaco",
     "docc_rocm_gemm_bf16_async_big_finish.hsaco",
     "docc_rocm_gemm_f32_finish.hsaco",
