@@ -536,6 +536,8 @@ private:
         int64_t m = 0, k = 0;
         if (!symbolic::is_integer(l->m, &m) || !symbolic::is_integer(l->k, &k) || m > 16 || k * (l->type == P::BFloat ? 2 : 4) < 128) return false;
         if (!private_to(link, {i, j})) return false;
+        for (auto& in : blocks_[j].inputs)      // the rows as residual, weights or bias as well: the one launch does not store them
+            if (in.connector != "_a" && !in.is_constant && in.data == link) return false;
         std::vector<std::string> connectors{"_x"};
         std::vector<ConnectorBinding> inputs{bind("_x", blocks_[i].input("_x")->data)};
         for (const char* name : {"_weight", "_bias"}) {

@@ -321,3 +321,24 @@ def test_block_program(dtype, tokens, width, approximate):
     assert got.dtype == dtype and got.shape == ref.shape
     err = float((got.double().cpu() - ref).norm() / ref.norm())
     assert err <= (1e-5 if dtype == torch.float32 else 1e-2), err     # bf16: the three intermediate tensors are rounded to bf16
+
+
+class NormedResidual(torch.nn.Module):
+    def forward(self, x, g, b, w, c):
+        h = F.layer_norm(x, (x.shape[1],), g, b)
+        return h + F.linear(h, w, c)
+
+
+# the residual behind a layer is the layer norm in front of it
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("tokens", [1, 8, 17])
+def test_program_with_the_normalised_rows_as_residual(dtype, tokens):
+    import docc_amd.torch as docc_torch
+
+    gen = torch.Generator().manual_seed(tokens)
+    rand = lambda *s: torch.randn(*s, generator=gen).to(dtype).cuda()
+    args = (rand(tokens, 256), rand(256), rand(256), rand(256, 256) / 16, rand(256))
+    got = docc_torch.compile_torch(NormedResidual(), None, target="rocm")(*args)
+    ref = NormedResidual()(*[t.double().cpu() for t in args])
+    err = float((got.double().cpu() - ref).norm() / ref.norm())
+    assert err <= (1e-5 if dtype == torch.float32 else 1e-2), err     # as above, with two tensors in between

@@ -249,3 +249,20 @@ def test_a_layer_norm_and_the_layer_behind_it(tmp_path, rows, width, merged):
         assert text.count("docc_rocm_malloc_async(") == text.count("docc_rocm_free_async(") == 1
     else:
         assert "docc_rocm_norm_linear" not in text and "docc_rocm_layer_norm(" in text and "docc_rocm_linear(" in text
+
+
+# the one launch of both leaves the normalised rows nowhere: a layer that has them as its residual or as its weights too keeps them
+@pytest.mark.parametrize("again", ["residual", "weights"])
+def test_a_layer_norm_that_its_layer_reads_twice(tmp_path, again):
+    class Layer(torch.nn.Module):
+        def forward(self, x, g, b, w, c):
+            h = F.layer_norm(x, (64,), g, b)
+            if again == "residual":
+                return h + F.linear(h, w, c)
+            return F.relu(F.linear(h, h, c))
+
+    t = torch.randn
+    s = docc_torch.compile_torch(Layer(), None, target="rocm").to_sdfg(t(8, 64), t(64), t(64), t(64, 64), t(64 if again == "residual" else 8))
+    s.schedule("rocm", options={"offload": "none"})
+    text = re.sub(r"\s+", " ", open(s.generate(str(tmp_path))["source"]).read())
+    assert "docc_rocm_norm_linear" not in text and "docc_rocm_layer_norm(" in text
