@@ -325,7 +325,7 @@ def test_block_program(dtype, tokens, width, approximate):
 
 class NormedResidual(torch.nn.Module):
     def forward(self, x, g, b, w, c):
-        h = F.layer_norm(x, (x.shape[1],), g, b)
+        h = F.layer_norm(x, (256,), g, b)
         return h + F.linear(h, w, c)
 
 
