@@ -922,7 +922,16 @@ int docc_rocm_norm_linear(docc_rocm_stream_t stream, int type, int64_t m, int64_
     const bool bf16 = type == DOCC_ROCM_TYPE_BF16;
     const int64_t v = bf16 ? 8 : 4;
     const int rows = m <= 8 ? 8 : 16, vectors = k <= 256 * v ? 4 : 8;      // vectors a lane holds
-    if (m <= 16 && k >= 8 * v && k <= 512 * v && (rows == 8 || vectors == 4) && n % 8 == 0 && waves_shape_ok(m, n, k, k, ldb, true, bf16 ? 2 : 4) && alpha != 0.0f && X && B &&
+    // Two launches read X and the norm's operands before the first store to Y, and what lies in `scratch` behind the norm's store: one launch reads X while it
+    // stores Y, and stores no `scratch`.
+    auto meet = [](const void* p, int64_t p_bytes, const void* q, int64_t q_bytes) {
+        return p && q && (uintptr_t) p < (uintptr_t) q + (uintptr_t) q_bytes && (uintptr_t) q < (uintptr_t) p + (uintptr_t) p_bytes;
+    };
+    const int64_t e = bf16 ? 2 : 4, x_bytes = m * k * e, y_bytes = m * n * (f.flags & kOutBf16 ? 2 : 4);
+    const bool apart = !meet(X, x_bytes, Y, y_bytes) && !meet(weight, k * e, Y, y_bytes) && !meet(norm_bias, k * e, Y, y_bytes) &&
+                       !meet(scratch, x_bytes, residual, m * n * (f.flags & kResidualBf16 ? 2 : 4)) && !meet(scratch, x_bytes, B, ((n - 1) * ldb + k) * e) &&
+                       !meet(scratch, x_bytes, bias, n * (f.flags & kBiasBf16 ? 2 : 4));
+    if (apart && m <= 16 && k >= 8 * v && k <= 512 * v && (rows == 8 || vectors == 4) && n % 8 == 0 && waves_shape_ok(m, n, k, k, ldb, true, bf16 ? 2 : 4) && alpha != 0.0f && X && B &&
         (forced < 0 || forced == 16) &&
         ((uintptr_t) X | (uintptr_t) weight | (uintptr_t) norm_bias | (uintptr_t) B | (uintptr_t) bias | (uintptr_t) residual | (uintptr_t) Y) % 16 == 0) {
         if (int rc = ensure_device()) return rc;

@@ -119,7 +119,9 @@ int docc_rocm_layer_norm(docc_rocm_stream_t stream, int type, int64_t rows, int6
 
 /*
  * A layer norm of the rows of X [m, k] and the layer behind it: docc_rocm_layer_norm(X, weight, norm_bias) into `scratch` [m, k] of the same type, then
- * docc_rocm_linear on that (A stored by rows, B [n, k]). A few rows are one launch, which leaves `scratch` as it is.
+ * docc_rocm_linear on that (A stored by rows, B [n, k]). A few rows are one launch, which leaves `scratch` as it is, unless that
+ * shows: where Y overlaps X (in place, X == residual == Y), the norm's weight or bias, or `scratch` is read as the residual, the weights or the
+ * bias of the layer, there are two. `scratch` overlaps neither Y nor the norm's weight and bias.
  */
 int docc_rocm_norm_linear(docc_rocm_stream_t stream, int type, int64_t m, int64_t n, int64_t k, float eps, const void* X, const void* weight, const void* norm_bias,
                           float alpha, const void* B, int64_t ldb, const void* bias, int bias_type, int activation, const void* residual, int residual_type, int rounding,

@@ -118,6 +118,29 @@ def test_layer_norm_and_linear_as_one(monkeypatch, tile, dtype, m, n, k):
         assert bool((err <= bound).all()), (act, float((err / bound).max()))
 
 
+# the rows in place, and the normalised rows as residual or as weights: what two launches give
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("m,k", [(1, 64), (8, 2048), (16, 1024)])
+def test_layer_norm_and_linear_on_operands_that_overlap(dtype, m, k):
+    gen = torch.Generator().manual_seed(k)
+    x = (torch.randn(m, k, generator=gen) * 3 + 5).to(dtype).cuda()
+    w, bias = (torch.randn(k, k, generator=gen) * k ** -0.5).to(dtype).cuda(), torch.randn(k, generator=gen).to(dtype).cuda()
+    h = F.layer_norm(x.double().cpu(), (k,), None, None, 1e-5).to(dtype)
+    for case in ("in place", "normed residual", "normed weights"):
+        n = m if case == "normed weights" else k
+        scratch, y = torch.full_like(x, float("nan")), x.clone() if case == "in place" else torch.full((m, n), float("nan"), device="cuda", dtype=dtype)
+        X, W, r = (y, w, y) if case == "in place" else (x, w, scratch) if case == "normed residual" else (x, scratch, None)
+        rt.call("docc_rocm_norm_linear", 0, TYPE[dtype], m, n, k, 1e-5, ptr(X), None, None, 1.0, ptr(W), k, ptr(bias[:n]), TYPE[dtype], -1, ptr(r), TYPE[dtype], 0,
+                ptr(scratch), ptr(y), TYPE[dtype])
+        torch.cuda.synchronize()
+        ref = reference(h, h if case == "normed weights" else w, True, bias[:n], None, {"in place": x, "normed residual": h, "normed weights": None}[case], 0)
+        bound = 2e-5 * (1 + ref.abs()) + (0 if dtype == torch.float32 else 2.0 ** -7 * (1 + ref.abs()))      # as above
+        if case == "normed weights":      # k products of size 1, and their differences by the rows' roundings to bf16
+            bound = bound + (4e-6 if dtype == torch.float32 else 2.0 ** -7) * k ** 0.5 * 4
+        err = (y.double().cpu() - ref).abs()
+        assert bool((err <= bound).all()), (case, float((err / bound).max()))
+
+
 # every tile with the chain in its store, ragged at both edges and along K where the tile allows it
 @pytest.mark.parametrize("cfg,dtype,k", [("128x128x32x4x4", torch.bfloat16, 104), ("128x128x64x4x4", torch.bfloat16, 328), ("128x256x64x4x3", torch.bfloat16, 328),
                                          ("256x256x32x4x4q", torch.bfloat16, 192), ("64x64x16x4x4", torch.float32, 84), ("128x128x32x4x3", torch.float32, 84),

@@ -275,3 +275,24 @@ print("\\n".join(l for l in take() if l.startswith("launch")))
             assert len(got) == 1            # one tile of 128 x 128, which parts of 256 k do not pay for
         else:
             assert parts > 1 and "splitk_combine" in got[1] and k % part, (m, n, k, got)
+
+
+# a norm and a layer in one launch, but in two where that one would read what it stores, or what it does not store
+def test_a_norm_and_a_layer_on_operands_that_overlap(recorded):
+    recorded("""
+m, n, k = 8, 512, 256                                    # rows of X: 1024 bytes, of Y: 2048
+G, H, W, BIAS, S = (0x50000000 + i * 0x1000000 for i in range(5))
+def launches(X=A, weight=G, shift=H, w=W, bias=BIAS, residual=C, scratch=S, y=D, type=2, m=m, n=n):
+    rt.call("docc_rocm_norm_linear", 0, type, m, n, k, 1e-5, X, weight, shift, 1.0, w, k, bias, type, -1, residual, type, 0, scratch, y, type)
+    return len([l for l in take() if l.startswith("launch")])
+rows, out = m * k * 4, m * n * 4
+assert launches() == launches(type=1) == launches(residual=D) == launches(scratch=A) == 1
+assert launches(X=A, residual=A, y=A, n=k) == 2          # in place
+assert launches(X=A, residual=A, y=A, n=k, type=1) == 2
+assert launches(X=D + out) == launches(X=D - rows) == 1  # side by side
+assert launches(X=D + out - 16) == launches(X=D - rows + 16) == 2
+assert launches(weight=D) == launches(weight=D + out - 16) == launches(weight=D - k * 4 + 16) == launches(shift=D + 16) == 2
+assert launches(weight=D + out) == launches(shift=D - k * 4) == 1
+assert launches(residual=S) == launches(residual=S + rows - 16) == launches(residual=S - out + 16) == launches(w=S) == launches(bias=S + 16) == 2
+assert launches(residual=S + rows) == launches(w=S + rows) == launches(bias=S - n * 4) == 1
+""")
