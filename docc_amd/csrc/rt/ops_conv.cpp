@@ -397,8 +397,9 @@ static int conv2d_run(docc_rocm_stream_t stream, int64_t N, int64_t C, int64_t H
         if (cus <= 0) cus = 256;
         const char* force = std::getenv("DOCC_ROCM_CONV");
         const bool pixels = force && std::strstr(force, "-pixels");   // tests: without the wider loads
+        // (an image one pixel wide: four pixels from the one before a row's on reach two rows down, beyond what the kernel's bounds on its vectors count on)
         const char* name = stride_w == 2 ? (pad_w == 1 && OW * 2 == W && W % 4 == 0 && !pixels ? "docc_conv2d_f32_winograd_s2_vector" : "docc_conv2d_f32_winograd_s2_pairs")
-                           : any_pad_w == 1 && OW == W && !pixels ? (W % 2 == 0 ? "docc_conv2d_f32_winograd_vector" : "docc_conv2d_f32_winograd_vector_odd")
+                           : any_pad_w == 1 && OW == W && W > 1 && !pixels ? (W % 2 == 0 ? "docc_conv2d_f32_winograd_vector" : "docc_conv2d_f32_winograd_vector_odd")
                                                                   : "docc_conv2d_f32_winograd_pixels";
         const int64_t parts = plan_winograd(N, C, OC, OH, OW, stride_h, parts_ok, cus).parts, total = N * OC * OH * OW;
         float* sums = nullptr;

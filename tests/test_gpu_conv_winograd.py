@@ -23,6 +23,7 @@ CASES = [  # N, C, H, W, OC, pads (top, left, bottom, right)
     (1, 16, 130, 4, 32, (3, 1, 2, 1)),    # rows of two tiles, three rows of padding
     (2, 16, 10, 11, 32, (0, 2, 1, 3)),    # columns that are padding alone
     (4, 64, 14, 14, 96, (1, 1, 1, 1)),
+    (1, 16, 258, 1, 32, (1, 1, 1, 1)),    # a pixel a row: the last work-group's last tile ends a row above the last
 ]
 
 

@@ -296,3 +296,13 @@ assert launches(weight=D + out) == launches(shift=D - k * 4) == 1
 assert launches(residual=S) == launches(residual=S + rows - 16) == launches(residual=S - out + 16) == launches(w=S) == launches(bias=S + 16) == 2
 assert launches(residual=S + rows) == launches(w=S + rows) == launches(bias=S - n * 4) == 1
 """)
+
+
+# a vector of a row of odd length reaches into the next row, and that of an image one pixel wide a row further: it goes pixel by pixel
+@pytest.mark.parametrize("height,width,form", [(258, 1, "pixels"), (7, 1, "pixels"), (258, 3, "vector_odd"), (258, 2, "vector")])
+def test_loads_of_narrow_images_in_winograds_form(recorded, height, width, form):
+    got = recorded(f"""
+rt.conv2d_f32(1, 64, {height}, {width}, 64, 3, 3, (1, 1), (1, 1), (1, 1), A, B, C, D)
+print("\\n".join(l for l in take() if l.startswith("launch")))
+""", DOCC_ROCM_CONV="winograd")
+    assert got[0].split()[1] == "docc_conv2d_f32_winograd_" + form
