@@ -218,10 +218,11 @@ int docc_rocm_softmax_host(docc_rocm_stream_t stream, int precision, int64_t out
     if (int rc = softmax_check(precision, outer, reduce, inner, X, Y)) return rc == 1 ? 0 : rc;
     if (int rc = ensure_device()) return rc;
     const size_t unit = (size_t) (reduce * inner) * (precision / 8), bytes = (size_t) outer * unit;
+    bool taken = false;
     int rc = through_device((hipStream_t) stream, X, Y, outer, unit, [&](int64_t, int64_t count, const void* x, void* y) {
         return docc_rocm_softmax(stream, precision, count, reduce, inner, x, y);
-    });
-    if (rc != 1) return rc;
+    }, &taken);
+    if (taken || rc) return rc;
     void *x = nullptr, *y = nullptr;
     if ((rc = docc_rocm_malloc_async(&x, bytes, stream))) return rc;
     rc = docc_rocm_memcpy_h2d_async(x, X, bytes, stream);

@@ -53,10 +53,11 @@ bool capturing();
 bool foreign_capture(hipStream_t stream);
 
 // A host array of `units` pieces of `unit_bytes` through the device into another of that size: run(first, count, x, y) launches on `stream` what makes y of x
-// for `count` pieces on the device. Uploads, kernels and downloads of different pieces run beside each other; everything has ended on return. 1: nothing was
-// done, because the call is small, the results' array is not pinned, the arrays overlap, a capture is open or there is no memory: the caller copies, launches and copies.
+// for `count` pieces on the device. Uploads, kernels and downloads of different pieces run beside each other; everything has ended on return. *taken: false if
+// nothing was done, because the call is small, the results' array is not pinned, the arrays overlap, a capture is open or there is no memory, streams or events: the
+// caller copies, launches and copies. (Apart from the error, whose codes are HIP's: after one, rows may have been written.)
 int through_device(hipStream_t stream, const void* src, void* dst, int64_t units, size_t unit_bytes,
-                   const std::function<int(int64_t first, int64_t count, const void* x, void* y)>& run);
+                   const std::function<int(int64_t first, int64_t count, const void* x, void* y)>& run, bool* taken);
 
 // The launchers' switches (tests, tuning) are environment variables read on every call: whether any DOCC_ROCM_GEM... variable is set at
 // all, in one walk over the environment instead of one per variable (seven for a GEMM, 0.2-0.3 us each).

@@ -528,11 +528,12 @@ bool stager_ready(Stager& st) {
     return st.ready;
 }
 
-// 0: done, 1: not staged (the caller falls back to the plain copy), other: error
-int staged_h2d(void* dst_dev, const void* src_host, size_t bytes, hipStream_t stream) {
+// *taken: false if staging is switched off or could not be set up (the caller falls back to the plain copy)
+int staged_h2d(void* dst_dev, const void* src_host, size_t bytes, hipStream_t stream, bool* taken) {
     Stager& st = g_stager;
     std::lock_guard<std::mutex> lock(st.mutex);
-    if (!stager_ready(st)) return 1;
+    *taken = stager_ready(st);
+    if (!*taken) return 0;
     const char* src = (const char*) src_host;
     char* dst = (char*) dst_dev;
     int slot = 0;
@@ -553,23 +554,20 @@ int staged_h2d(void* dst_dev, const void* src_host, size_t bytes, hipStream_t st
     return 0;
 }
 
-int lanes_for_device(Stager& st, CopyLanes** lanes) {
+// with st.mutex held: the current device's, or null where they cannot be made
+CopyLanes* lanes_for_device(Stager& st) {
     int dev = 0;
-    if (int rc = check(hipGetDevice(&dev), "hipGetDevice")) return rc;
+    bool ok = hipGetDevice(&dev) == hipSuccess;
     CopyLanes& l = st.lanes[dev];
-    if (!l.ready) {
-        bool ok = (l.up || hipStreamCreateWithFlags(&l.up, hipStreamNonBlocking) == hipSuccess) &&
-                  (l.down || hipStreamCreateWithFlags(&l.down, hipStreamNonBlocking) == hipSuccess);
+    if (ok && !l.ready) {
+        ok = (l.up || hipStreamCreateWithFlags(&l.up, hipStreamNonBlocking) == hipSuccess) &&
+             (l.down || hipStreamCreateWithFlags(&l.down, hipStreamNonBlocking) == hipSuccess);
         for (hipEvent_t* e : {&l.begin, &l.arrived[0], &l.arrived[1], &l.computed[0], &l.computed[1]})
             ok = ok && (*e || hipEventCreateWithFlags(e, hipEventDisableTiming) == hipSuccess);
-        if (!ok) {
-            (void) hipGetLastError();
-            return 1;
-        }
-        l.ready = true;
+        l.ready = ok;
     }
-    *lanes = &l;
-    return 0;
+    if (!ok) (void) hipGetLastError();
+    return ok ? &l : nullptr;
 }
 
 } // namespace
@@ -579,28 +577,28 @@ namespace docc::rt::rocm {
 // PCIe carries both directions at once; a call that uploads, computes and downloads in turn uses one of them at a time. Uploads here go on a stream of
 // their own, the kernels on the caller's, downloads on a third, ordered by events. 64 MB in and out: 2.72 ms in turn, 1.87 ms this way (the upload alone is
 // 1.36; what does not overlap is the first chunk's staging and upload and the last one's download).
-int through_device(hipStream_t stream, const void* src, void* dst, int64_t units, size_t unit_bytes, const std::function<int(int64_t, int64_t, const void*, void*)>& run) {
+int through_device(hipStream_t stream, const void* src, void* dst, int64_t units, size_t unit_bytes, const std::function<int(int64_t, int64_t, const void*, void*)>& run,
+                   bool* taken) {
+    *taken = false;
     hipStream_t s = resolve_stream(stream);
     const size_t bytes = (size_t) units * unit_bytes;
     const char *from = (const char*) src, *to = (const char*) dst;
-    if (bytes < kStageMin || capturing() || foreign_capture(stream) || !is_pinned(dst, bytes)) return 1;
-    if (from != to && from < to + bytes && to < from + bytes) return 1;      // a download would write what has not been read (in place it has)
+    if (bytes < kStageMin || capturing() || foreign_capture(stream) || !is_pinned(dst, bytes)) return 0;
+    if (from != to && from < to + bytes && to < from + bytes) return 0;      // a download would write what has not been read (in place it has)
     // eight chunks where they have 4 to 8 MB (64 MB in and out: chunks of 2 MB 2.80 ms, 4 MB 2.03, 8 MB 1.87; 16 MB: 4 MB 0.67, 8 MB 0.77)
     const size_t eighth = bytes / 8, chunk_bytes = eighth < kStageChunk / 2 ? kStageChunk / 2 : eighth > kStageChunk ? kStageChunk : eighth;
     const int64_t per_chunk = unit_bytes >= chunk_bytes ? 1 : (int64_t) (chunk_bytes / unit_bytes);
-    if (unit_bytes > kStageChunk || per_chunk >= units) return 1;
+    if (unit_bytes > kStageChunk || per_chunk >= units) return 0;
     const bool pinned = is_pinned(src, bytes);
     Stager& st = g_stager;
     std::unique_lock<std::mutex> lock(st.mutex);
-    CopyLanes* lanes = nullptr;
-    if (!pinned && !stager_ready(st)) return 1;
-    if (int rc = lanes_for_device(st, &lanes)) return rc;
+    if (!pinned && !stager_ready(st)) return 0;
+    CopyLanes* const lanes = lanes_for_device(st);
+    if (!lanes) return 0;
     void *x = nullptr, *y = nullptr;
-    if (docc_rocm_malloc_async(&x, bytes, stream)) return 1;
-    if (docc_rocm_malloc_async(&y, bytes, stream)) {
-        (void) docc_rocm_free_async(x, stream);
-        return 1;
-    }
+    if (docc_rocm_malloc_async(&x, bytes, stream)) return 0;
+    if (docc_rocm_malloc_async(&y, bytes, stream)) return docc_rocm_free_async(x, stream);
+    *taken = true;
     // the blocks may still be in use by what their owner before has on the stream
     int rc = check(hipEventRecord(lanes->begin, s), "hipEventRecord(copy lanes)");
     if (!rc) rc = check(hipStreamWaitEvent(lanes->up, lanes->begin, 0), "hipStreamWaitEvent(copy lanes)");
@@ -937,8 +935,9 @@ int docc_rocm_host_free(void* host_ptr) {
 int docc_rocm_memcpy_h2d_async(void* dst_dev, const void* src_host, size_t bytes, docc_rocm_stream_t stream) {
     if (bytes == 0) return 0;
     if (bytes >= kStageMin && !capturing() && !is_pinned(src_host, bytes)) {
-        const int rc = staged_h2d(dst_dev, src_host, bytes, resolve_stream((hipStream_t) stream));
-        if (rc != 1) return rc;     // 1: staging is switched off or could not be set up
+        bool taken = false;
+        const int rc = staged_h2d(dst_dev, src_host, bytes, resolve_stream((hipStream_t) stream), &taken);
+        if (taken) return rc;
     }
     return check(hipMemcpyAsync(dst_dev, src_host, bytes, hipMemcpyHostToDevice, resolve_stream((hipStream_t) stream)), "hipMemcpyAsync(H2D)");
 }

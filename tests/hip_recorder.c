@@ -4,6 +4,7 @@
 #include <hip/hip_runtime_api.h>
 #include <stdarg.h>
 #include <stdio.h>
+#include <stdlib.h>
 #include <string.h>
 
 static char text[1 << 20];
@@ -22,6 +23,9 @@ static int device_queries;
 static hipError_t last;
 void recorder_capture(void* stream) { captured = (hipStream_t) stream; }
 void recorder_no_memory_from(size_t bytes) { no_memory_from = bytes; }
+/* the copy from now on that fails, as a HIP call does whose arguments are not valid; -1: none */
+static int failing_copy = -1;
+void recorder_fail_copy(int nth) { failing_copy = nth; }
 int recorder_device_queries(void) { int n = device_queries; device_queries = 0; return n; }
 const char* recorder_take(void) {
     static char taken[1 << 20];
@@ -95,4 +99,19 @@ hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned flags) {
     (void) flags;
     note("%p waits for %zu\n", (void*) s, (size_t) e);
     return hipSuccess;
+}
+/* host memory is the process's own; a pointer nobody has pinned makes the query of its kind fail */
+hipError_t hipHostMalloc(void** p, size_t bytes, unsigned flags) {
+    (void) flags;
+    *p = malloc(bytes);
+    return *p ? hipSuccess : hipErrorOutOfMemory;
+}
+hipError_t hipHostFree(void* p) { free(p); return hipSuccess; }
+hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void* p) { (void) a, (void) p; return last = hipErrorInvalidValue; }
+hipError_t hipMemcpyAsync(void* dst, const void* src, size_t bytes, hipMemcpyKind kind, hipStream_t s) {
+    (void) dst, (void) src;
+    const int fails = failing_copy == 0;
+    if (failing_copy >= 0) failing_copy--;
+    note("copy %zu %s on %p%s\n", bytes, kind == hipMemcpyHostToDevice ? "up" : kind == hipMemcpyDeviceToHost ? "down" : "across", (void*) s, fails ? " failed" : "");
+    return fails ? (last = hipErrorInvalidValue) : hipSuccess;
 }

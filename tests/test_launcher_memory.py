@@ -306,3 +306,48 @@ rt.conv2d_f32(1, 64, {height}, {width}, 64, 3, 3, (1, 1), (1, 1), (1, 1), A, B, 
 print("\\n".join(l for l in take() if l.startswith("launch")))
 """, DOCC_ROCM_CONV="winograd")
     assert got[0].split()[1] == "docc_conv2d_f32_winograd_" + form
+
+
+# an error's code is HIP's, and that of a copy with invalid arguments is 1: after it some rows have been written, so the call is not done again
+@pytest.mark.parametrize("failing", [0, 1, 4, 15])
+@pytest.mark.parametrize("pinned", [False, True])
+def test_a_copy_that_fails_among_chunks_fails_the_call(recorded, failing, pinned):
+    recorded(f"""
+import numpy as np
+shape = (4096, 2048)                                      # 32 MB, eight chunks
+y = rt.result_array(shape, np.float32)
+x = rt.result_array(shape, np.float32) if {pinned} else np.empty(shape, np.float32)
+def softmax(x): rt.call("docc_rocm_softmax_host", 0, 32, *shape, 1, x.ctypes.data, y.ctypes.data)
+softmax(x)
+whole = [l for l in take() if l.startswith("copy")]
+assert len(whole) == 16 and all(" 4194304 " in l for l in whole), whole
+for source in (x, y):                                     # y: in place
+    recorder.recorder_fail_copy({failing})
+    try:
+        softmax(source)
+        assert False
+    except rt.RocmRuntimeError as e:
+        assert "hipMemcpyAsync" in str(e), e
+    got = [l for l in take() if l.startswith("copy")]
+    assert len(got) == {failing} + 1 and got[-1].endswith("failed"), got
+# an upload through pinned buffers too
+if not {pinned}:
+    recorder.recorder_fail_copy(1)
+    try:
+        rt.call("docc_rocm_memcpy_h2d_async", A, x.ctypes.data, x.nbytes, 0)
+        assert False
+    except rt.RocmRuntimeError as e:
+        assert "hipMemcpyAsync" in str(e), e
+    assert len([l for l in take() if l.startswith("copy")]) == 2
+# where nothing can be set up the array goes as a whole
+recorder.recorder_fail_copy(-1)
+recorder.recorder_no_memory_from(1 << 20)
+rt.pool_trim()
+take()
+try:
+    softmax(x)
+    assert False
+except rt.RocmRuntimeError as e:
+    assert "emory" in str(e), e
+assert not [l for l in take() if l.startswith("copy")]
+""")
