@@ -5,7 +5,7 @@
 //
 // Steps of two: a 2x2 tile of outputs reads 5x5 pixels. Along an axis taps 0 and 2 meet the pixels 0, 2 and 4, a two-tap filter with two outputs: (x0 - x2) w0,
 // x2 (w0 + w2), (x4 - x2) w2; tap 1 meets x1 and x3. Five products for six, 25 for 36 in two axes, and as the products that go to one output alone
-// share a sum with those of tap 1, nine sums. The filters have 16 components again, so that their way is the same.
+// share a sum with those of tap 1, nine sums (and four, see below). The filters have 16 components again, so that their way is the same.
 //
 // What bounds the direct form is the fp32 matrix pipe (one work-group of docc_conv2d_f32_halo_* keeps it at two thirds of its peak); the 16
 // sums over the channels are the same matrix product of 16 / 36 of the size, and everything else a tile needs fits beside
@@ -29,9 +29,19 @@
 // two: 50 x 80 x 52 x 52 -> 160 153 -> 57, 3 x 448 x 51 x 51 -> 896 257 -> 106 (its MFMAs 1.52 us a chunk and work-group, measured 1.6). Pixel by pixel a row's loads touch
 // their cache lines once each, which bounds steps of two: 12 x 96 x 8 x 8 51 us for 25 with vectors or pairs.
 //
-// Rounding: the chain of additions has C terms instead of 9 C, which outweighs the transforms' own. Relative error (2-norm) against 64 bits on
-// N(0, 1) images: C = 16 1.5e-7 (direct 2.1e-7), 64 2.6e-7 (4.1e-7), 512 6.8e-7 (1.2e-6); on their positive part 1.3e-7 (1.4e-7), 2.3e-7
-// (2.8e-7), 5.8e-7 (8.1e-7). An output depends on the pixels of its own window alone, as in the direct form, but where
+// Rounding: the chain of additions has C terms instead of 9 C (steps of two: 3 C at most, with four sums more), the transforms add their own. An output's error is
+// bounded by the sum over the channels of the largest filter value times the largest pixel of its window, that of a direct sum by the products of its own taps: where
+// a few values are far larger than the others, or most are zero, the direct sum is the closer one. Relative error (2-norm) against 64 bits in units of the direct
+// form's with its channels in as many parts, 4 x C x 28 x 28, steps of one / two:
+//                                             C = 8        16          32          64 (both in parts)   512 (both in parts)
+//   N(0, 1)                                   0.91 / 0.95  0.77 / 0.87 0.68 / 0.82    0.78 / 0.89       0.70 / 0.89
+//   its positive part                         1.10 / 1.00  0.96 / 0.92 0.85 / 0.85    0.92 / 0.90       0.86 / 0.95
+//   that with half of the rest zero           1.48 / 1.24  1.25 / 1.12 1.10 / 1.02    1.20 / 1.08       1.07 / 1.07
+// Filters with one value that is not zero have exact direct sums; here 5e-8 of the result is lost with steps of one. Images with one value of a hundred 1e4 times as
+// large: 0.7 to 0.9 of the direct form's error as a whole, but the worst output, as a share of the sum of its taps' magnitudes, 40 times it at C = 32, 16 at 64, 1.5 at
+// 256. So the launcher takes this form from 32 channels on, and with no longer chains than keep the positive part's error at the direct form's (winograd_longest() in
+// csrc/rt/ops_conv.cpp): 90 drawn layers (1-64 images, 32-512 channels, 7 x 7 to 64 x 64) 0.68 / 0.80 of it on N(0, 1), 0.83 / 0.82 on the positive part
+// (geometric means; 1.05 and 1.02 at most). An output depends on the pixels of its own window alone, as in the direct form, but where
 // products cancel (or a sum of pixels overflows) an infinity can come out as a NaN: outputs that are not finite are computed again, directly.
 #include "elementwise_ops.h"
 #include "conv_params.h"
@@ -77,6 +87,13 @@ struct ConvWinograd {
     // the row of filter components and the row of sums that row i of products goes with
     static constexpr int filter_row(int i) { return i == 4 ? 3 : i; }
     static constexpr int sum_row(int i) { return S == 1 ? i : i == 3 ? 0 : i == 4 ? 2 : i; }
+    // Where four products would share a sum, the one that is a difference of pixels in both axes, the largest, has a sum of its own that is added at the end: with nine
+    // sums the error on N(0, 1) images was the direct form's (64 to 512 channels 1.00), with thirteen it is 0.89 of it, in the same time.
+    static constexpr int NS = S == 1 ? 16 : 13;
+    static constexpr int sum_of(int i, int j) {
+        const bool corner = S == 2 && (i == 0 || i == 2) && (j == 0 || j == 2);
+        return corner ? NA * NA + i + j / 2 : NA * sum_row(i) + sum_row(j);
+    }
     static constexpr int WL = (RAW / 4 + 64 * NW - 1) / (64 * NW);   // vectors of them a thread moves
     static constexpr int LDS_FLOATS = 2 * STAGE + 2 * RAW + 4;
 
@@ -191,7 +208,7 @@ struct ConvWinograd {
             *reinterpret_cast<wf4*>(udst + buf * STAGE + i * 128) = u;
         };
 
-        wf4 acc[NA * NA][2];
+        wf4 acc[NS][2];
         const float* const ulane = lds + lk * CS + l16 * 4;
         wf4 a[2][2];
         auto aread = [&](int buf, int half, int f) {      // row f of the filter components
@@ -231,7 +248,7 @@ struct ConvWinograd {
             for (int j = 0; j < RG; j++)
 #pragma unroll
                 for (int o = 0; o < 2; o++) {
-                    wf4& sum = acc[NA * sum_row(i) + sum_row(j)][o];
+                    wf4& sum = acc[sum_of(i, j)][o];
                     sum = __builtin_amdgcn_mfma_f32_16x16x4f32(a[f & 1][o][filter_row(j)], v[from][j], sum, 0, 0, 0);
                 }
         };
@@ -271,7 +288,7 @@ struct ConvWinograd {
         aread(0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int q = 0; q < NA * NA; q++)
+        for (int q = 0; q < NS; q++)
 #pragma unroll
             for (int o = 0; o < 2; o++) acc[q][o] = wf4{0.f, 0.f, 0.f, 0.f};
         // In chunk ch the filters of ch + 1 are transformed into the other buffer, those of ch + 2 written to LDS as they are, those of ch + 3
@@ -327,6 +344,12 @@ struct ConvWinograd {
         }
         if (ch < chunks) chunk(ch, std::integral_constant<int, 0>{});
 
+        if constexpr (S == 2) {
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+#pragma unroll
+                for (int o = 0; o < 2; o++) acc[q / 2 * 2 * NA + q % 2 * 2][o] += acc[NA * NA + q][o];
+        }
         // outputs: rows of A^T = (1 1 1 0), (0 1 -1 -1) on both sides, the middle components halved; strides of two (1 1 0), (0 1 1)
         if (!tile_ok) return;
         const long plane = (long) p.OH * p.OW;

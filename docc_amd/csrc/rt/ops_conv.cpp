@@ -236,18 +236,19 @@ bool winograd_shape_ok(int64_t N, int64_t C, int64_t H, int64_t W, int64_t OC, i
 // to several of them, whose sums a second launch adds (3 us, and the parts at 3 TB/s).
 // Measured against the other forms on 60 drawn layers (1-64 images, 8-512 channels, 7x7 to 64x64), "before -> now": 8 x 272 x 40 x 40 244 -> 86 us,
 // 32 x 64 x 56 x 56 71 -> 48, 34 x 80 x 24 x 24 53 -> 24, 3 x 32 x 19 x 19 13.1 -> 11.5; steps of two: 23 x 240 x 36 x 36 240 -> 101.
+// `longest`: no part has more chunks than that (forced parts are not held to it); us 1e30: no such plan.
 struct WinogradPlan {
     int64_t parts = 1;
     double us = 0;
 };
-WinogradPlan plan_winograd(int64_t N, int64_t C, int64_t OC, int64_t OH, int64_t OW, int64_t stride, bool parts_ok, int cus) {
+WinogradPlan plan_winograd(int64_t N, int64_t C, int64_t OC, int64_t OH, int64_t OW, int64_t stride, int64_t longest, bool parts_ok, int cus) {
     const int64_t chunks = C / 8, total = N * OC * OH * OW;
     auto us = [&](int64_t parts) {
         const int64_t groups = winograd_groups(N, OC, OH, OW) * parts, rounds = groups / (2 * cus), rest = groups % (2 * cus);
         const double each = (double) ((chunks + parts - 1) / parts), pair = 2 * (stride == 1 ? 1.17 : 1.62) * each + 4.0, alone = (stride == 1 ? 1.43 : 1.9) * each + 4.0;
         return (double) rounds * pair + (rest == 0 ? 0.0 : rest <= cus ? alone : pair) + (parts > 1 ? 3.0 + (double) (parts + 1) * 4.0 * (double) total / 3e6 : 0.0);
     };
-    WinogradPlan plan{1, us(1)};
+    WinogradPlan plan{1, chunks <= longest ? us(1) : 1e30};
     if (!parts_ok || total > (int64_t(1) << 26)) return plan;
     const char* force = std::getenv("DOCC_ROCM_CONV");
     const char* cut = force && force[0] == 'w' ? std::strstr(force, "-parts") : nullptr;   // winograd-parts<n>: that many (tests, tuning)
@@ -256,11 +257,22 @@ WinogradPlan plan_winograd(int64_t N, int64_t C, int64_t OC, int64_t OH, int64_t
     double best = plan.us / 1.1;
     for (const int64_t parts : {2, 3, 4, 6, 8, 12, 16, 24, 32}) {
         if (parts * 2 > chunks || parts * total > (int64_t(1) << 26)) break;
+        if ((chunks + parts - 1) / parts > longest) continue;
         const double t = us(parts);
         if (t < best) best = t, plan = WinogradPlan{parts, t};
     }
     return plan;
 }
+
+// The most chunks of eight channels that a part may have for its error, on images like those of a network's layers, to be no larger than that of the direct sum
+// in parts of `direct` chunks: in units of a direct sum's error over one chunk, squared, that of the direct sum grows as 1.15 a chunk and Winograd's as 0.9 + 0.55
+// a chunk, steps of two 0.6 + 0.67 (fitted to the positive part of N(0, 1) images, C from 8 to 512; on the images themselves it has more room). Without this a direct
+// sum in three parts gave way to the whole in Winograd's form: 12 x 48 x 27 x 27 1.3 times the error. Below four chunks the transforms' own roundings count: eight
+// channels 1.1 times, and filters or images with few values that are not zero 1.5 to 2 times.
+int64_t winograd_longest(int64_t direct, int64_t stride) {
+    return (int64_t) (stride == 1 ? (1.15 * (double) direct - 0.9) / 0.55 : (1.15 * (double) direct - 0.6) / 0.67);
+}
+constexpr int64_t kWinogradChunks = 4;   // that many at least, chosen without being asked for
 
 // 1x1 filters on the kernel that takes X as it lies (csrc/kernels/conv_1x1.hip): vectors of four channels, 32-bit offsets within a work-group's images
 bool direct_1x1_shape_ok(int64_t N, int64_t C, int64_t H, int64_t W, int64_t OC, int64_t KH, int64_t KW, int64_t OH, int64_t OW, int64_t stride_h, int64_t stride_w,
@@ -282,13 +294,18 @@ bool direct_1x1_pays(int64_t N, int64_t C, int64_t OC, int64_t OH, int64_t OW, i
 
 ConvPath choose_path(int64_t N, int64_t C, int64_t OC, int64_t KH, int64_t KW, int64_t OH, int64_t OW, int64_t stride_h, int64_t stride_w,
                      int64_t pad_h, int64_t pad_w, bool halo_ok, bool have_workspace, bool parts_ok, bool winograd_ok,
-                     bool direct_1x1_ok) {
-    const char* force = std::getenv("DOCC_ROCM_CONV");   // halo | gather | gemm | winograd | straight (tuning and tests)
+                     bool direct_1x1_ok, int64_t* winograd_parts) {
+    const char* force = std::getenv("DOCC_ROCM_CONV");   // halo | gather | gemm | winograd | straight (tuning and tests); direct: not Winograd's form
+    if (force && force[0] == 'd') winograd_ok = false;
     const bool pointwise = KH == 1 && KW == 1 && stride_h == 1 && stride_w == 1 && pad_h == 0 && pad_w == 0;
     const ConvPath gemm = pointwise ? ConvPath::Gemm1x1 : ConvPath::GemmColumns;
     const bool gemm_ok = pointwise || have_workspace;
     if (force && force[0] == 'h' && halo_ok) return ConvPath::Halo;
-    if (force && force[0] == 'w' && winograd_ok) return ConvPath::Winograd;
+    if (force && force[0] == 'w' && winograd_ok) {
+        const int have = compute_units();
+        *winograd_parts = plan_winograd(N, C, OC, OH, OW, stride_h, C, parts_ok, have > 0 ? have : 256).parts;
+        return ConvPath::Winograd;
+    }
     if (force && force[0] == 's' && direct_1x1_ok) return ConvPath::Direct1x1;
     if (force && force[0] == 'g' && force[1] == 'a') return ConvPath::Gather;
     if (force && force[0] == 'g' && force[1] == 'e' && gemm_ok) return gemm;
@@ -307,9 +324,11 @@ ConvPath choose_path(int64_t N, int64_t C, int64_t OC, int64_t KH, int64_t KW, i
     if (pointwise) return gemm_fast && C >= 128 ? gemm : halo_ok ? ConvPath::Halo : ConvPath::Gather;
     const double direct = halo_ok ? halo.cost * halo_unit_us(K) : gather_time_us(N, OC, P, K, cus);
     const double columns = gemm_fast ? gemm_time_us(N, OC, P, K, true) : 1e30;
-    if (winograd_ok) {
-        const WinogradPlan plan = plan_winograd(N, C, OC, OH, OW, stride_h, parts_ok, cus);
+    if (winograd_ok && C >= 8 * kWinogradChunks) {
+        const int64_t longest = winograd_longest((C / 8 + halo.parts - 1) / halo.parts, stride_h);
+        const WinogradPlan plan = plan_winograd(N, C, OC, OH, OW, stride_h, longest, parts_ok, cus);
         const double around = columns < direct || halo.parts == 1 ? 4.0 : 0.0;   // what the other estimates leave out (that of the parts does not)
+        *winograd_parts = plan.parts;
         if (plan.us < 0.95 * ((columns < direct ? columns : direct) + around)) return ConvPath::Winograd;
     }
     if (columns < 0.75 * direct) return gemm;
@@ -332,7 +351,8 @@ extern "C" int64_t docc_rocm_conv2d_f32_pads_workspace_bytes(int64_t N, int64_t 
     // nothing either when one of the direct kernels would be chosen anyway (operands assumed aligned, the channels in one
     // piece: cutting them takes memory of its own, which the call may not get; Winograd's form aside, which a call may be forced off)
     const bool halo_ok = halo_shape_ok(C, KH, KW, OW, stride_h, stride_w, dil_h, dil_w);
-    if (choose_path(N, C, OC, KH, KW, OH, OW, stride_h, stride_w, pad_h, pad_w, halo_ok, true, false, false, false) != ConvPath::GemmColumns) return 0;
+    int64_t winograd_parts = 1;
+    if (choose_path(N, C, OC, KH, KW, OH, OW, stride_h, stride_w, pad_h, pad_w, halo_ok, true, false, false, false, &winograd_parts) != ConvPath::GemmColumns) return 0;
     const int64_t per_image = conv_bytes_per_image(OC, C * KH * KW, OH * OW);
     int64_t images = kConvWorkspaceCap / per_image;
     if (images < 1) images = 1;
@@ -386,22 +406,21 @@ static int conv2d_run(docc_rocm_stream_t stream, int64_t N, int64_t C, int64_t H
                                                                                     pad_w_end, dil_h, dil_w);
     const bool have_workspace = workspace && workspace_bytes >= need && need > 0 && ((uintptr_t) workspace % 256) == 0;
     const bool parts_ok = !slice && !foreign_capture((hipStream_t) stream);   // cutting the channels takes a block of the cache
+    int64_t winograd_parts = 1;
     ConvPath path = C == 0 ? ConvPath::Gather
                            : choose_path(N, C, OC, KH, KW, OH, OW, stride_h, stride_w, any_pad_h, any_pad_w, halo_shape, have_workspace, parts_ok,
-                                         winograd, !slice && direct_1x1_shape_ok(N, C, H, W, OC, KH, KW, OH, OW, stride_h, stride_w, any_pad_h, any_pad_w));
+                                         winograd, !slice && direct_1x1_shape_ok(N, C, H, W, OC, KH, KW, OH, OW, stride_h, stride_w, any_pad_h, any_pad_w), &winograd_parts);
     // one group of a grouped convolution: the direct kernels, which take the distance between the images as it is (the
     // GEMM paths write whole [N, OC, P] tensors)
     if (slice && (path == ConvPath::Gemm1x1 || path == ConvPath::GemmColumns)) path = halo_shape ? ConvPath::Halo : ConvPath::Gather;
     if (path == ConvPath::Winograd) {
-        int cus = compute_units();
-        if (cus <= 0) cus = 256;
         const char* force = std::getenv("DOCC_ROCM_CONV");
         const bool pixels = force && std::strstr(force, "-pixels");   // tests: without the wider loads
         // (an image one pixel wide: four pixels from the one before a row's on reach two rows down, beyond what the kernel's bounds on its vectors count on)
         const char* name = stride_w == 2 ? (pad_w == 1 && OW * 2 == W && W % 4 == 0 && !pixels ? "docc_conv2d_f32_winograd_s2_vector" : "docc_conv2d_f32_winograd_s2_pairs")
                            : any_pad_w == 1 && OW == W && W > 1 && !pixels ? (W % 2 == 0 ? "docc_conv2d_f32_winograd_vector" : "docc_conv2d_f32_winograd_vector_odd")
                                                                   : "docc_conv2d_f32_winograd_pixels";
-        const int64_t parts = plan_winograd(N, C, OC, OH, OW, stride_h, parts_ok, cus).parts, total = N * OC * OH * OW;
+        const int64_t parts = winograd_parts, total = N * OC * OH * OW;
         float* sums = nullptr;
         if (parts > 1 && docc_rocm_malloc_async((void**) &sums, (size_t) (parts * total * 4), stream) != 0) sums = nullptr;   // without memory for the sums the layer runs whole
         if (finished) *finished = true;

@@ -351,3 +351,17 @@ except rt.RocmRuntimeError as e:
     assert "emory" in str(e), e
 assert not [l for l in take() if l.startswith("copy")]
 """)
+
+
+# Winograd's form from 32 channels on, and in parts where the direct sum would be in so many that the whole would be further off; not at all where the caller says so
+@pytest.mark.parametrize("N,C,size,stride,parts", [(4, 8, 28, 1, 0), (64, 8, 56, 1, 0), (32, 16, 56, 1, 0), (8, 24, 28, 2, 0), (64, 32, 56, 1, 1), (12, 48, 27, 1, 3), (15, 48, 21, 1, 3),
+                                                   (4, 32, 17, 2, 2), (32, 128, 28, 2, 1)])
+def test_chains_of_sums_in_winograds_form(recorded, N, C, size, stride, parts):
+    for choice in ("", "direct"):
+        got = recorded(f"""
+rt.conv2d_f32({N}, {C}, {size}, {size}, {C * stride}, 3, 3, ({stride}, {stride}), (1, 1), (1, 1), A, B, C, D)
+print("\\n".join(l for l in take() if l.startswith("launch")))
+""", **({"DOCC_ROCM_CONV": choice} if choice else {}))
+        assert ("winograd" in got[0]) == (parts > 0 and not choice), got
+        if "winograd" in got[0]:
+            assert f",{parts},1 x" in got[0], got
