@@ -42,7 +42,7 @@
 // 256. So the launcher takes this form from 32 channels on, and with no longer chains than keep the positive part's error at the direct form's (winograd_longest() in
 // csrc/rt/ops_conv.cpp): 90 drawn layers (1-64 images, 32-512 channels, 7 x 7 to 64 x 64) 0.68 / 0.80 of it on N(0, 1), 0.83 / 0.82 on the positive part
 // (geometric means; 1.05 and 1.02 at most). An output depends on the pixels of its own window alone, as in the direct form, but where
-// products cancel (or a sum of pixels overflows) an infinity can come out as a NaN: outputs that are not finite are computed again, directly.
+// products cancel (or a sum of pixels overflows) an infinity can come out as a NaN: a wavefront with outputs that are not finite sums its own again, directly.
 #include "elementwise_ops.h"
 #include "conv_params.h"
 #include <type_traits>
@@ -51,19 +51,6 @@ namespace docc_k {
 
 typedef float wf4 __attribute__((ext_vector_type(4)));
 typedef float wf2 __attribute__((ext_vector_type(2)));
-
-// one output the direct way: channels [0, C) of X and Wt as given
-__device__ __forceinline__ float conv3x3_direct(const float* xn, const float* w, int C, int H, int W, int ih0, int iw0) {
-    float sum = 0.f;
-    for (int c = 0; c < C; c++)
-        for (int t = 0; t < 9; t++) {
-            const int ih = ih0 + t / 3, iw = iw0 + t % 3;
-            const bool in = ih >= 0 && ih < H && iw >= 0 && iw < W;
-            // (a tap in the padding multiplies a zero, as in the other forms: an infinite weight gives a NaN there)
-            sum = __builtin_fmaf(w[c * 9 + t], in ? xn[((long) c * H + ih) * W + iw] : 0.f, sum);
-        }
-    return sum;
-}
 
 // How a lane loads the pixels of a row:
 //   kPixels   one by one, each with an offset of its own; any padding
@@ -97,33 +84,44 @@ struct ConvWinograd {
     static constexpr int WL = (RAW / 4 + 64 * NW - 1) / (64 * NW);   // vectors of them a thread moves
     static constexpr int LDS_FLOATS = 2 * STAGE + 2 * RAW + 4;
 
+    // where a lane's tile lies, and the work-group's operands as buffers: X from its first image n0 on and the filters from oc0 on; the launcher has seen to it that
+    // what a work-group addresses takes less than 2^30 bytes. (X four pixels early: the column before an image's first one has an offset as well.)
+    static constexpr int kEarly = 4;
+    static constexpr int kNone = (int) 0x80000000;      // an offset beyond either: the load gives 0
+    typedef decltype(__builtin_amdgcn_make_buffer_rsrc((void*) nullptr, 0, 0, 0)) buffer_t;
+    struct Place {
+        bool ok;
+        int n0, n, oh, ow, ih0, iw0;
+        buffer_t xbuf, wbuf;
+        __device__ __forceinline__ Place(const ConvParams& p, int tid, int tile0, int oc0, int c0) {
+            const int TW = (p.OW + 1) >> 1, per_image = ((p.OH + 1) >> 1) * TW;
+            const int tile = tile0 + (tid >> 6) * 16 + (tid & 15);
+            ok = tile < p.N * per_image;
+            n0 = tile0 / per_image;
+            const int rest = (ok ? tile : tile0) % per_image;
+            n = (ok ? tile : tile0) / per_image;
+            oh = 2 * (rest / TW), ow = 2 * (rest % TW);
+            ih0 = S * oh - p.pad_h, iw0 = S * ow - p.pad_w;
+            const long left = ((long) (p.N - n0) * p.XC * p.H * p.W - (long) c0 * p.H * p.W + kEarly) * 4;
+            xbuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.X) + (((long) n0 * p.XC + c0) * p.H * p.W - kEarly), 0,
+                                                     (int) (left < 0x7fffffffL ? left : 0x7fffffffL), 0x00020000);
+            const long wleft = ((long) (p.OC - oc0) * p.C - c0) * 36;
+            wbuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.Wt) + ((long) oc0 * p.C + c0) * 9, 0,
+                                                     (int) (wleft < 0x7fffffffL ? wleft : 0x7fffffffL), 0x00020000);
+        }
+    };
+
     // channels [c0, c0 + 8 * chunks) of X and Wt; the work-group's tiles from tile0 on, output channels from oc0 on
     template <int LOADS>
     static __device__ __forceinline__ void run(const ConvParams& p, const ConvFinish& fin, float* lds, int tile0, int oc0, int c0, int chunks) {
         const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
         const int l16 = lane & 15, lk = lane >> 4;
-        const int TH = (p.OH + 1) >> 1, TW = (p.OW + 1) >> 1, per_image = TH * TW;
-        const int tiles = p.N * per_image;
-
-        // this lane's tile
-        const int tile = tile0 + wave * 16 + l16;
-        const bool tile_ok = tile < tiles;
-        const int n0 = tile0 / per_image;                                    // first image of the work-group
-        const int n = (tile_ok ? tile : tile0) / per_image, rest = (tile_ok ? tile : tile0) % per_image;
-        const int oh = 2 * (rest / TW), ow = 2 * (rest % TW);
-        const int ih0 = S * oh - p.pad_h, iw0 = S * ow - p.pad_w;
+        const Place place(p, tid, tile0, oc0, c0);
+        const bool tile_ok = place.ok;
+        const int n0 = place.n0, n = place.n, ow = place.ow, ih0 = place.ih0, iw0 = place.iw0;
+        const buffer_t xbuf = place.xbuf, wbuf = place.wbuf;
         const int HW4 = p.H * p.W * 4;
 
-        // X from image n0 on and the filters from oc0 on, as buffers; the launcher has seen to it that what a work-group addresses takes less
-        // than 2^30 bytes. (X four pixels early: the column before an image's first one has an offset as well.)
-        constexpr int kEarly = 4;
-        const long left = ((long) (p.N - n0) * p.XC * p.H * p.W - (long) c0 * p.H * p.W + kEarly) * 4;
-        const auto xbuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.X) + (((long) n0 * p.XC + c0) * p.H * p.W - kEarly), 0,
-                                                            (int) (left < 0x7fffffffL ? left : 0x7fffffffL), 0x00020000);
-        const long wleft = ((long) (p.OC - oc0) * p.C - c0) * 36;
-        const auto wbuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.Wt) + ((long) oc0 * p.C + c0) * 9, 0,
-                                                            (int) (wleft < 0x7fffffffL ? wleft : 0x7fffffffL), 0x00020000);
-        constexpr int kNone = (int) 0x80000000;      // an offset beyond either
         const bool first_col = ow == 0, odd_col = ow + 1 >= p.W, last_col = ow + 2 >= p.W;   // kVector, kVectorOdd: columns 0, 2 and 3 in the padding
         constexpr int NOFF = LOADS == kPixels ? PX : LOADS == kPairs ? 3 : S;
         int voff[PX][NOFF];
@@ -344,6 +342,17 @@ struct ConvWinograd {
         }
         if (ch < chunks) chunk(ch, std::integral_constant<int, 0>{});
 
+        // (worked out again, where the tile lies: what is kept for this would take registers from the chunks)
+        int tid_again = tid;
+        asm volatile("" : "+v"(tid_again));
+        finish(p, fin, acc, tid_again, tile0, oc0, c0, chunks);
+    }
+
+    static __device__ __forceinline__ void finish(const ConvParams& p, const ConvFinish& fin, wf4 (&acc)[NS][2], int tid, int tile0, int oc0, int c0, int chunks) {
+        const int l16 = tid & 15, lk = (tid >> 4) & 3;
+        const Place place(p, tid, tile0, oc0, c0);
+        const bool tile_ok = place.ok;
+        const int n = place.n, oh = place.oh, ow = place.ow;
         if constexpr (S == 2) {
 #pragma unroll
             for (int q = 0; q < 4; q++)
@@ -351,7 +360,6 @@ struct ConvWinograd {
                 for (int o = 0; o < 2; o++) acc[q / 2 * 2 * NA + q % 2 * 2][o] += acc[NA * NA + q][o];
         }
         // outputs: rows of A^T = (1 1 1 0), (0 1 -1 -1) on both sides, the middle components halved; strides of two (1 1 0), (0 1 1)
-        if (!tile_ok) return;
         const long plane = (long) p.OH * p.OW;
         const bool right = ow + 1 < p.OW, below = oh + 1 < p.OH;
         const bool pairs = (p.OW & 1) == 0 && (((uintptr_t) p.Y | (uintptr_t) fin.residual) & 7) == 0;
@@ -433,17 +441,59 @@ struct ConvWinograd {
         typedef std::integral_constant<bool, true> yes;
         typedef std::integral_constant<bool, false> no;
         const bool fast = pairs && oc0 + 32 <= p.OC && (p.OH & 1) == 0;
-        if (fin.residual) fast ? outputs(yes{}, yes{}) : outputs(no{}, yes{});
-        else fast ? outputs(yes{}, no{}) : outputs(no{}, no{});
-        while (again) {
-            const int bit = __builtin_ctz(again);
-            again &= again - 1;
-            const int oc = oc0 + (bit >> 4) * 16 + 4 * lk + ((bit >> 2) & 3), i = (bit >> 1) & 1, j = bit & 1;
-            if (oc >= p.OC || oh + i >= p.OH || ow + j >= p.OW) continue;
-            const float sum = conv3x3_direct(p.X + ((long) n * p.XC + c0) * p.H * p.W, p.Wt + ((long) oc * p.C + c0) * 9, chunks * CI, p.H, p.W, ih0 + S * i, iw0 + S * j);
-            const long to = oc * plane + (long) i * p.OW + j;
-            ytile[to] = conv_finished(fin, sum + (p.bias ? p.bias[oc] : 0.f), fin.residual ? rtile[to] : -0.f);
+        if (tile_ok) {
+            if (fin.residual) fast ? outputs(yes{}, yes{}) : outputs(no{}, yes{});
+            else fast ? outputs(yes{}, no{}) : outputs(no{}, no{});
         }
+        if (__ballot(again != 0) == 0) return;
+
+        // The wavefront's outputs once more as direct sums, nine products for an output and channel on the same MFMA with pixels and filters as they lie (a tap in the
+        // padding multiplies a zero, as in the other forms: an infinite weight gives a NaN there). Those that were not finite take them. With every
+        // image a NaN 32 x 64 x 56 x 56 takes 227 us, 32 x 256 x 14 x 14 246 (direct 67 and 91; a lane and output at a time 3300 and 3000).
+        int poff[PX][PX], foff[2];
+#pragma unroll
+        for (int r = 0; r < PX; r++)
+#pragma unroll
+            for (int c = 0; c < PX; c++) {
+                const int ih = place.ih0 + r, iw = place.iw0 + c;
+                const bool in = tile_ok && ih >= 0 && ih < p.H && iw >= 0 && iw < p.W;
+                poff[r][c] = in ? ((n - place.n0) * p.XC * p.H * p.W + (lk * p.H + ih) * p.W + iw + kEarly) * 4 : kNone;
+            }
+#pragma unroll
+        for (int o = 0; o < 2; o++) foff[o] = oc0 + o * 16 + l16 < p.OC ? ((o * 16 + l16) * p.C + lk) * 36 : kNone;
+        wf4 sums[2][2][2];       // [row][column][block of channels]
+#pragma unroll
+        for (int q = 0; q < 8; q++) sums[q >> 2][(q >> 1) & 1][q & 1] = wf4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+        for (int step = 0; step < 2 * chunks; step++) {
+            float x[PX][PX], w[2][9];
+#pragma unroll
+            for (int t = 0; t < 9; t++)
+#pragma unroll
+                for (int o = 0; o < 2; o++) w[o][t] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(place.wbuf, foff[o], step * 144 + t * 4, 0));
+#pragma unroll
+            for (int r = 0; r < PX; r++)
+#pragma unroll
+                for (int c = 0; c < PX; c++) x[r][c] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(place.xbuf, poff[r][c], step * 16 * p.H * p.W, 0));
+#pragma unroll
+            for (int t = 0; t < 9; t++)
+#pragma unroll
+                for (int q = 0; q < 8; q++) {
+                    const int i = q >> 2, j = (q >> 1) & 1, o = q & 1;
+                    sums[i][j][o] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[o][t], x[S * i + t / 3][S * j + t % 3], sums[i][j][o], 0, 0, 0);
+                }
+        }
+#pragma unroll
+        for (int o = 0; o < 2; o++)
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    const int oc = oc0 + o * 16 + 4 * lk + r, i = q >> 1, j = q & 1;
+                    if (!((again >> (16 * o + 4 * r + q)) & 1) || oc >= p.OC || oh + i >= p.OH || ow + j >= p.OW) continue;
+                    const long to = oc * plane + (long) i * p.OW + j;
+                    ytile[to] = conv_finished(fin, sums[i][j][o][r] + bias[o][r], fin.residual ? rtile[to] : -0.f);
+                }
     }
 };
 
