@@ -23,6 +23,10 @@ CASES = [  # N, C, H, W, OC, pads (top, left, bottom, right)
     (1, 16, 130, 4, 32, (3, 1, 2, 1)),    # rows of two tiles, three rows of padding
     (2, 16, 10, 11, 32, (0, 2, 1, 3)),    # columns that are padding alone
     (4, 64, 14, 14, 96, (1, 1, 1, 1)),
+    (1, 16, 41, 41, 33, (1, 1, 1, 1)),    # odd rows as vectors: work-groups that begin and end amid the tensor, here 21 x 21 tiles
+    (5, 16, 15, 15, 32, (1, 1, 1, 1)),    # an image a work-group
+    (20, 8, 7, 7, 32, (1, 1, 1, 1)),      # four images a work-group
+    (70, 16, 3, 3, 40, (1, 1, 1, 1)),     # sixteen, two tiles a row
     (1, 16, 258, 1, 32, (1, 1, 1, 1)),    # a pixel a row: the last work-group's last tile ends a row above the last
 ]
 
