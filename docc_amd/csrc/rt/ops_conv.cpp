@@ -345,19 +345,36 @@ extern "C" int64_t docc_rocm_conv2d_f32_pads_workspace_bytes(int64_t N, int64_t 
     const int64_t OH = out_dim(H, pad_h, pad_h_end, dil_h, KH, stride_h), OW = out_dim(W, pad_w, pad_w_end, dil_w, KW, stride_w);
     if (OH <= 0 || OW <= 0) return 0;
     // what decides between the paths is whether there is padding at all: the larger of begin and end stands for both
+    const int64_t begin_h = pad_h, begin_w = pad_w;
     pad_h = pad_h > pad_h_end ? pad_h : pad_h_end;
     pad_w = pad_w > pad_w_end ? pad_w : pad_w_end;
     if (KH == 1 && KW == 1 && stride_h == 1 && stride_w == 1 && pad_h == 0 && pad_w == 0) return 0;   // the input is the column matrix
-    // nothing either when one of the direct kernels would be chosen anyway (operands assumed aligned, the channels in one
-    // piece: cutting them takes memory of its own, which the call may not get; Winograd's form aside, which a call may be forced off)
+    // nothing either when one of the other forms would be chosen anyway (operands assumed aligned, the channels in one
+    // piece: cutting them takes memory of its own, which the call may not get)
     const bool halo_ok = halo_shape_ok(C, KH, KW, OW, stride_h, stride_w, dil_h, dil_w);
     int64_t winograd_parts = 1;
-    if (choose_path(N, C, OC, KH, KW, OH, OW, stride_h, stride_w, pad_h, pad_w, halo_ok, true, false, false, false, &winograd_parts) != ConvPath::GemmColumns) return 0;
+    if (choose_path(N, C, OC, KH, KW, OH, OW, stride_h, stride_w, pad_h, pad_w, halo_ok, true, false,
+                    winograd_shape_ok(N, C, H, W, OC, KH, KW, OH, OW, stride_h, stride_w, begin_h, begin_w, dil_h, dil_w),
+                    direct_1x1_shape_ok(N, C, H, W, OC, KH, KW, OH, OW, stride_h, stride_w, pad_h, pad_w), &winograd_parts) != ConvPath::GemmColumns)
+        return 0;
     const int64_t per_image = conv_bytes_per_image(OC, C * KH * KW, OH * OW);
     int64_t images = kConvWorkspaceCap / per_image;
     if (images < 1) images = 1;
     if (images > N) images = N;
     return images * per_image;
+}
+
+extern "C" int docc_rocm_conv2d_f32_reads_workspace(docc_rocm_stream_t stream, int64_t N, int64_t C, int64_t H, int64_t W, int64_t OC, int64_t KH, int64_t KW,
+                                                    int64_t stride_h, int64_t stride_w, int64_t pad_h, int64_t pad_w, int64_t pad_h_end, int64_t pad_w_end,
+                                                    int64_t dil_h, int64_t dil_w, const float* Wt) {
+    if (docc_rocm_conv2d_f32_pads_workspace_bytes(N, C, H, W, OC, KH, KW, stride_h, stride_w, pad_h, pad_w, pad_h_end, pad_w_end, dil_h, dil_w) == 0) return 0;
+    const int64_t OH = out_dim(H, pad_h, pad_h_end, dil_h, KH, stride_h), OW = out_dim(W, pad_w, pad_w_end, dil_w, KW, stride_w);
+    const int64_t any_pad_h = pad_h > pad_h_end ? pad_h : pad_h_end, any_pad_w = pad_w > pad_w_end ? pad_w : pad_w_end;
+    int64_t winograd_parts = 1;
+    return choose_path(N, C, OC, KH, KW, OH, OW, stride_h, stride_w, any_pad_h, any_pad_w,
+                       halo_shape_ok(C, KH, KW, OW, stride_h, stride_w, dil_h, dil_w) && (uintptr_t) Wt % 16 == 0, true, !foreign_capture((hipStream_t) stream),
+                       winograd_shape_ok(N, C, H, W, OC, KH, KW, OH, OW, stride_h, stride_w, pad_h, pad_w, dil_h, dil_w),
+                       direct_1x1_shape_ok(N, C, H, W, OC, KH, KW, OH, OW, stride_h, stride_w, any_pad_h, any_pad_w), &winograd_parts) == ConvPath::GemmColumns;
 }
 
 extern "C" int64_t docc_rocm_conv2d_f32_workspace_bytes(int64_t N, int64_t C, int64_t H, int64_t W, int64_t OC, int64_t KH, int64_t KW,

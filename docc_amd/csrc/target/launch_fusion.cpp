@@ -769,7 +769,7 @@ public:
             s.setIndent(s.indent() + 4);
             int64_t group = 0;
             const bool whole = symbolic::is_integer(c->group, &group) && group == 1;   // grouped convolutions take no workspace
-            s << "const int64_t __ws_bytes = " << (whole ? "docc_rocm_conv2d_f32_pads_workspace_bytes(" + c->extents + ")" : std::string("0")) << ";" << std::endl;
+            s << "const int64_t __ws_bytes = " << (whole ? conv_launch_workspace(c->extents, "W") : std::string("0")) << ";" << std::endl;
             s << "void *__ws = nullptr;" << std::endl;
             s << "if (__ws_bytes > 0) DOCC_ROCM_CHECK(docc_rocm_malloc_async(&__ws, (size_t) __ws_bytes, nullptr));" << std::endl;
             s << "DOCC_ROCM_CHECK(docc_rocm_conv2d_f32_chain(nullptr, " << c->extents << ", (int64_t) (" << c->group << "), X, W, " << (c->has_bias ? "B" : "nullptr") << ", "

@@ -299,7 +299,7 @@ protected:
         }
         s << "{" << std::endl;
         s.setIndent(s.indent() + 4);
-        s << "const int64_t __ws_bytes = docc_rocm_conv2d_f32_pads_workspace_bytes(" << dims << ");" << std::endl;
+        s << "const int64_t __ws_bytes = " << conv_launch_workspace(dims, "(const float *) " + name_of("W")) << ";" << std::endl;
         s << "void *__ws = nullptr;" << std::endl;
         s << "if (__ws_bytes > 0) DOCC_ROCM_CHECK(docc_rocm_malloc_async(&__ws, (size_t) __ws_bytes, nullptr));" << std::endl;
         s << "DOCC_ROCM_CHECK(docc_rocm_conv2d_f32_pads(nullptr, " << dims << ", (const float *) " << name_of("X")
@@ -903,6 +903,10 @@ std::string conv_launch_extents(const tensor::ConvNode& c) {
       << c.kernel_shape()[1] << ", " << get(c.strides(), 0, "1") << ", " << get(c.strides(), 1, "1") << ", " << get(c.pads(), 0, "0") << ", " << get(c.pads(), 1, "0")
       << ", " << get(c.pads(), 2, "0") << ", " << get(c.pads(), 3, "0") << ", " << get(c.dilations(), 0, "1") << ", " << get(c.dilations(), 1, "1");
     return s.str();
+}
+
+std::string conv_launch_workspace(const std::string& extents, const std::string& weights) {
+    return "docc_rocm_conv2d_f32_reads_workspace(nullptr, " + extents + ", " + weights + ") ? docc_rocm_conv2d_f32_pads_workspace_bytes(" + extents + ") : 0";
 }
 
 void register_plugin(plugins::Context& context) {

@@ -111,6 +111,8 @@ inline const std::string LibraryNodeType_ROCM_LayerNorm = "ROCMLayerNorm";
 void register_launch_dispatchers(codegen::LibraryNodeDispatcherRegistry& reg);
 // the extents of a 2-d convolution as the launchers take them: N, C, H, W, OC, KH, KW, strides, pads (begins, then ends), dilations
 std::string conv_launch_extents(const math::tensor::ConvNode& conv);
+// the bytes of the column matrix that a launch with these extents and weights on the default stream reads, 0 for most layers
+std::string conv_launch_workspace(const std::string& extents, const std::string& weights);
 
 // Preamble every rocm dispatcher puts into the globals stream (duplicates are folded by the generator).
 void emit_runtime_preamble(codegen::PrettyPrinter& globals, const Function& function);

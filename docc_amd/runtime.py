@@ -93,6 +93,7 @@ _SIGNATURES = {
     "docc_rocm_softmax_noalloc": [_vp, _int, _i64, _i64, _i64, _vp, _vp],
     "docc_rocm_conv2d_f32": [_vp] + [_i64] * 13 + [_vp, _vp, _vp, _vp],
     "docc_rocm_conv2d_f32_pads_workspace_bytes": [_i64] * 15,
+    "docc_rocm_conv2d_f32_reads_workspace": [_vp] + [_i64] * 15 + [_vp],
     "docc_rocm_conv2d_f32_pads": [_vp] + [_i64] * 15 + [_vp, _vp, _vp, _vp, _vp, _i64],
     "docc_rocm_conv2d_f32_grouped": [_vp] + [_i64] * 16 + [_vp, _vp, _vp, _vp, _vp, _i64],
     "docc_rocm_conv2d_f32_chain": [_vp] + [_i64] * 16 + [_vp, _vp, _vp, _vp, _int, _vp, _vp, _i64],

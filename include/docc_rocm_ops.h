@@ -243,6 +243,11 @@ int docc_rocm_conv2d_f32_ws(docc_rocm_stream_t stream, int64_t N, int64_t C, int
 int64_t docc_rocm_conv2d_f32_pads_workspace_bytes(int64_t N, int64_t C, int64_t H, int64_t W, int64_t OC, int64_t KH, int64_t KW,
                                                   int64_t stride_h, int64_t stride_w, int64_t pad_h, int64_t pad_w,
                                                   int64_t pad_h_end, int64_t pad_w_end, int64_t dil_h, int64_t dil_w);
+/* Whether a call on `stream` with such a workspace would read it: _workspace_bytes answers for any call, also one that cannot have memory of its own to cut
+ * the channels with, which most layers that ask for a column matrix are faster with. What generated code allocates by. */
+int docc_rocm_conv2d_f32_reads_workspace(docc_rocm_stream_t stream, int64_t N, int64_t C, int64_t H, int64_t W, int64_t OC, int64_t KH, int64_t KW,
+                                         int64_t stride_h, int64_t stride_w, int64_t pad_h, int64_t pad_w, int64_t pad_h_end, int64_t pad_w_end,
+                                         int64_t dil_h, int64_t dil_w, const float* Wt);
 int docc_rocm_conv2d_f32_pads(docc_rocm_stream_t stream, int64_t N, int64_t C, int64_t H, int64_t W, int64_t OC,
                               int64_t KH, int64_t KW, int64_t stride_h, int64_t stride_w, int64_t pad_h, int64_t pad_w,
                               int64_t pad_h_end, int64_t pad_w_end, int64_t dil_h, int64_t dil_w, const float* X,

@@ -365,3 +365,43 @@ print("\\n".join(l for l in take() if l.startswith("launch")))
         assert ("winograd" in got[0]) == (parts > 0 and not choice), got
         if "winograd" in got[0]:
             assert f",{parts},1 x" in got[0], got
+
+
+# generated code asks for a column matrix where the call reads it, and a call that does not read one is the same without
+@pytest.mark.parametrize("size", [(8, 256, 14, 14, 256, 1), (64, 256, 7, 7, 256, 2), (25, 416, 12, 12, 416, 1), (1, 256, 14, 14, 256, 1), (16, 40, 30, 30, 40, 1), (2, 64, 5, 500, 64, 1),
+                                  (3, 20, 20, 20, 50, 1), (8, 100, 14, 14, 256, 1)])
+def test_a_workspace_is_asked_for_where_it_is_read(recorded, size):
+    recorded(f"""
+N, C, H, W, OC, stride = {size}
+size = (N, C, H, W, OC, 3, 3, stride, stride, 1, 1, 1, 1, 1, 1)
+need = rt.lib().docc_rocm_conv2d_f32_pads_workspace_bytes(*size)
+def names(workspace):
+    rt.call("docc_rocm_conv2d_f32_pads", s, *size, A, B, C_, D, workspace, need if workspace else 0)
+    return [l.split()[1] for l in take() if l.startswith("launch")]
+C_, s = 0x60000000, 0
+reads = rt.lib().docc_rocm_conv2d_f32_reads_workspace(s, *size, B)
+assert need > 0 or not reads
+assert reads == (need > 0 and "docc_conv2d_im2col_f32" in names(0x50000000))
+if not reads: assert names(0x50000000 if need else None) == names(None)
+# in another library's capture, where the channels cannot be cut
+s = rt.stream_create()
+recorder.recorder_capture(s)
+reads = rt.lib().docc_rocm_conv2d_f32_reads_workspace(s, *size, B)
+assert reads == (need > 0 and "docc_conv2d_im2col_f32" in names(0x50000000))
+""")
+
+
+def test_a_layer_in_winograds_form_asks_for_no_column_matrix(recorded):
+    got = recorded("""
+import random, math
+rng = random.Random(1)
+asked = 0
+for _ in range(300):
+    N, C, size, stride = round(math.exp(rng.uniform(0, 4.1))), 16 * round(math.exp(rng.uniform(0.7, 3.4))), rng.randint(7, 64), rng.choice([1, 1, 2])
+    shape = (N, C, size, size, C * stride, 3, 3, stride, stride, 1, 1, 1, 1, 1, 1)
+    rt.call("docc_rocm_conv2d_f32_pads", 0, *shape, A, B, None, D, None, 0)
+    if "winograd" in next(l for l in take() if l.startswith("launch")):
+        asked += rt.lib().docc_rocm_conv2d_f32_reads_workspace(0, *shape, B)
+print(asked)
+""")
+    assert int(got[0]) == 0
