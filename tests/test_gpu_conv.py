@@ -176,7 +176,7 @@ def test_conv_every_path_integer_exact(rt, monkeypatch, force, case):
     assert np.array_equal(Y, oracle.conv2d(X, Wt, b, stride, pad, dil))
 
 
-GEMM_LAYERS = [  # small images with many channels: the shapes the choice sends to im2col + GEMM, and a 1x1 layer with C >= 128
+GEMM_LAYERS = [  # small images with many channels: the shapes that go to im2col + GEMM where the channels cannot be cut, and a 1x1 layer with C >= 128
     (8, 256, 14, 14, 256, 3, 3, (1, 1), (1, 1), (1, 1), True), (8, 512, 7, 7, 512, 3, 3, (1, 1), (1, 1), (1, 1), True),
     (1, 256, 14, 14, 256, 3, 3, (1, 1), (1, 1), (1, 1), False), (4, 256, 28, 28, 64, 1, 1, (1, 1), (0, 0), (1, 1), True),
     (3, 128, 9, 9, 96, 3, 3, (2, 2), (1, 1), (1, 1), True),
@@ -184,7 +184,7 @@ GEMM_LAYERS = [  # small images with many channels: the shapes the choice sends 
 
 
 @pytest.mark.parametrize("case", GEMM_LAYERS, ids=[f"n{c[0]}c{c[1]}_{c[2]}x{c[3]}_oc{c[4]}k{c[5]}s{c[7][0]}" for c in GEMM_LAYERS])
-def test_conv_gemm_layers_match_oracle(rt, case):
+def test_conv_gemm_layers_match_oracle(rt, monkeypatch, case):
     N, C, H, W, OC, KH, KW, stride, pad, dil, use_bias = case
     rng = np.random.default_rng(C + H)
     X = rng.standard_normal((N, C, H, W)).astype(np.float32)
@@ -195,9 +195,13 @@ def test_conv_gemm_layers_match_oracle(rt, case):
     assert (need == 0) == pointwise            # the 1x1 layer multiplies the tensors as they lie
     ref = oracle.conv2d(X[:2], Wt, b, stride, pad, dil)
     assert rel_err_max(Y[:2], ref) <= 1e-5
-    # without the workspace the same call takes a direct kernel and agrees
+    # without the workspace the same call agrees
     Y0, _ = run_conv_ws(rt, X, Wt, b, stride, pad, dil, workspace_bytes=0)
     assert rel_err_max(Y0, Y) <= 1e-5
+    # the choice has other forms for most of these (tests/test_launcher_memory.py): columns and GEMM, and each direct kernel, by name
+    for force in ("gemm", "gather", "halo-t2"):
+        monkeypatch.setenv("DOCC_ROCM_CONV", force)
+        assert rel_err_max(run_conv_ws(rt, X, Wt, b, stride, pad, dil)[0][:2], ref) <= 1e-5, force
 
 
 def test_conv_workspace_chunks_over_images(rt, monkeypatch):

@@ -3,6 +3,8 @@ work-group, parts of different lengths, channels out and planes of no whole tile
 
 fp32 sums of n terms, in parts and then added: the error of a result is below n eps sum|x w|, and near sqrt(n) eps of the
 result's size for random operands; 1e-5 of the largest result holds a factor of ten for n = 9 x 512."""
+import os
+
 import pytest
 import torch
 import torch.nn.functional as F
@@ -19,14 +21,16 @@ pytestmark = pytest.mark.gpu
     (1, 512, 96, 9, 9, 1, 2, 0, True),         # 1x1 with steps of two
     (1, 320, 48, 40, 40, 3, 1, 1, False),
 ])
-def test_channels_in_parts(rt, N, C, OC, H, W, k, stride, pad, bias):
+def test_channels_in_parts(rt, monkeypatch, N, C, OC, H, W, k, stride, pad, bias):
     g = torch.Generator().manual_seed(C + OC)
     x, w = torch.randn(N, C, H, W, generator=g), torch.randn(OC, C, k, k, generator=g) * (C * k * k) ** -0.5
     b = torch.randn(OC, generator=g) if bias else None
     ref = F.conv2d(x.double(), w.double(), b.double() if bias else None, stride=stride, padding=pad)
     dx, dw, db = x.cuda(), w.cuda(), b.cuda() if bias else None
     y = torch.full(ref.shape, float("nan"), device="cuda")
-    for _ in range(2):
+    for choice in (None, None, "direct"):       # the last: the strips where the choice is Winograd's form
+        if choice and not os.environ.get("DOCC_ROCM_CONV"):
+            monkeypatch.setenv("DOCC_ROCM_CONV", choice)
         rt.conv2d_f32(N, C, H, W, OC, k, k, (stride, stride), (pad, pad), (1, 1), dx.data_ptr(), dw.data_ptr(), db.data_ptr() if bias else 0, y.data_ptr())
         torch.cuda.synchronize()
         assert (y.cpu().double() - ref).abs().max() <= 1e-5 * ref.abs().max()
@@ -39,4 +43,4 @@ def test_channels_in_parts(rt, N, C, OC, H, W, k, stride, pad, bias):
 def test_forms_in_parts(rt, monkeypatch, form, k, stride, pad):
     monkeypatch.setenv("DOCC_ROCM_CONV", "halo-" + form)
     for C, N in ((32 if "2" in form[-1] else 72, 3), (72, 5)):
-        test_channels_in_parts(rt, N, C, 70, 9, 7, k, stride, pad, True)
+        test_channels_in_parts(rt, monkeypatch, N, C, 70, 9, 7, k, stride, pad, True)

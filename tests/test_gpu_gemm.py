@@ -263,7 +263,7 @@ def test_gemm_alpha_zero_does_not_reference_a_and_b(rt, kind):
     assert np.array_equal(want, (c0 * -1.5).cpu().numpy())
 
 
-GEMV_CASES = [  # m, n, k, ta, tb: one output column or row, each operand layout; sizes that take the matrix-vector kernels
+GEMV_CASES = [  # m, n, k, ta, tb: one output column or row, each operand layout; sizes that take the matrix-vector kernels, some of them only without those that cut K between wavefronts
     (3000, 1, 700, N, N), (3000, 1, 701, N, T), (2048, 1, 1024, T, N), (1500, 1, 333, T, T),
     (1, 3000, 700, N, N), (1, 2048, 1024, N, T), (1, 1501, 333, T, N), (1, 4096, 96, T, T),
     (5000, 1, 8, N, N), (1, 300, 5000, N, N),
@@ -274,12 +274,15 @@ GEMV_CASES = [  # m, n, k, ta, tb: one output column or row, each operand layout
 ]
 
 
+@pytest.mark.parametrize("waves", ["", "0"])
 @pytest.mark.parametrize("dt", [np.float32, np.float64])
 @pytest.mark.parametrize("case", GEMV_CASES, ids=[f"{c[0]}x{c[1]}x{c[2]}" + "nt"[c[3] == T] + "nt"[c[4] == T] for c in GEMV_CASES])
-def test_gemm_with_one_column_or_one_row(rt, monkeypatch, dt, case):
+def test_gemm_with_one_column_or_one_row(rt, monkeypatch, dt, case, waves):
     """The matrix-vector kernels behind the GEMM entry points: integer-valued operands give the oracle's integers
     (any summation order), random ones stay within the GEMM bars; the tiled kernels (DOCC_ROCM_GEMV_OFF) agree."""
     m, n, k, ta, tb = case
+    if waves:
+        monkeypatch.setenv("DOCC_ROCM_GEMM_WAVES", waves)
     rng = np.random.default_rng(m + 3 * n + 7 * k)
     A = int_matrix(rng, (k, m) if ta == T else (m, k), dt, lim=4)
     B = int_matrix(rng, (n, k) if tb == T else (k, n), dt, lim=4)

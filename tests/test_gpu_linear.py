@@ -47,10 +47,13 @@ def reference(a, w, trans_b, bias, act, residual, rounding):
 
 
 # rows: matrix-vector, few-row kernels, tiles of 64 / 128 / 256 with ragged edges, K in parts; columns off a vector of eight too
+@pytest.mark.parametrize("waves", ["", "0"])       # 0: without the kernels that cut K between wavefronts, which take most of the few rows
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("m,n,k", [(1, 512, 512), (2, 1024, 2048), (8, 4096, 2048), (17, 8192, 1024), (64, 256, 1024), (100, 72, 96), (129, 200, 64),
                                    (130, 77, 33), (384, 1032, 512), (1000, 136, 4096), (2050, 1160, 128), (4100, 4104, 128)])
-def test_linear_over_the_launchers_forms(dtype, m, n, k):
+def test_linear_over_the_launchers_forms(monkeypatch, dtype, m, n, k, waves):
+    if waves:
+        monkeypatch.setenv("DOCC_ROCM_GEMM_WAVES", waves)
     gen = torch.Generator().manual_seed(m * 31 + n)
     a = torch.randn(m, k, generator=gen).to(dtype).cuda()
     w = (torch.randn(n, k, generator=gen) * k ** -0.5).to(dtype).cuda()

@@ -162,7 +162,7 @@ print("\\n".join(l for l in take() if l.startswith("launch")))
         assert f"_{form.split('-')[0]}_parts " in got[0] and f",2,{parts} " in got[0] and "add_parts" in got[1]
 
 
-# what the planner takes by itself: the shapes of tests/test_gpu_conv_parts.py are products of the cut form
+# what the planner takes by itself: the shapes of tests/test_gpu_conv_parts.py are products of the cut form, in the form that is chosen and among the direct ones
 def test_few_images_of_many_channels_are_cut(recorded):
     from test_gpu_conv_parts import test_channels_in_parts as cases
     rows = next(m for m in cases.pytestmark if m.name == "parametrize").args[1]
@@ -172,6 +172,38 @@ rt.conv2d_f32({N}, {C}, {H}, {W}, {OC}, {k}, {k}, ({stride}, {stride}), ({pad}, 
 print("\\n".join(l for l in take() if l.startswith("launch")))
 """)
         assert ("_parts" in " ".join(got)) == (C > 16), (N, C, got)
+        got = recorded(f"""
+rt.conv2d_f32({N}, {C}, {H}, {W}, {OC}, {k}, {k}, ({stride}, {stride}), ({pad}, {pad}), (1, 1), A, B, C, D)
+print("\\n".join(l for l in take() if l.startswith("launch")))
+""", DOCC_ROCM_CONV="direct")
+        first = got[0].split()
+        assert first[1].startswith("docc_conv2d_f32_halo_") and first[1].endswith("_parts") == (C > 16) and (int(first[2].split(",")[2]) > 1) == (C > 16), (N, C, got)
+
+
+# ... and the layers of tests/test_gpu_conv.py that are named for their columns and GEMM take them when asked to, with a workspace
+def test_layers_as_columns_and_gemm(recorded):
+    from test_gpu_conv import GEMM_LAYERS
+    for N, C, H, W, OC, KH, KW, stride, pad, dil, _ in GEMM_LAYERS:
+        for force, first in (("gemm", "docc_conv2d_im2col_f32" if KH == 3 else "gemm"), ("gather", "docc_conv2d_f32"), ("halo-t2", "docc_conv2d_f32_halo_")):
+            got = recorded(f"""
+size = ({N}, {C}, {H}, {W}, {OC}, {KH}, {KW}, {stride}, {pad}, {dil})
+need = rt.conv2d_f32_workspace_bytes(*size)
+rt.conv2d_f32_ws(*size, A, B, C, D, 0x50000000 if need else 0, need)
+print("\\n".join(l for l in take() if l.startswith("launch")))
+""", DOCC_ROCM_CONV=force)
+            assert first in " ".join(got) and "winograd" not in " ".join(got), (N, C, force, got)
+
+
+# the products of tests/test_gpu_gemm.py with one to eight rows or columns on the matrix-vector kernels, with the switch that its second run sets
+def test_few_rows_or_columns_without_the_kernels_that_cut_k_between_wavefronts(recorded):
+    from test_gpu_gemm import GEMV_CASES
+    for m, n, k, ta, tb in GEMV_CASES:
+        got = recorded(f"""
+rt.sgemm({m}, {n}, {k}, 1.0, A, {m if ta == 112 else k}, B, {k if tb == 112 else n}, 0.0, C, {n}, trans_a={ta}, trans_b={tb})
+print("\\n".join(l for l in take() if l.startswith("launch")))
+""", DOCC_ROCM_GEMM_WAVES="0")
+        tiles = (m, n, ta, tb) in ((8, 4200, 111, 111), (4100, 8, 112, 111))       # (eight vectors along the other operand's rows: there the tiles' margins are tried)
+        assert "waves" not in " ".join(got) and any("gemv" in l for l in got) != tiles, (m, n, k, got)
 
 
 def test_the_release_of_a_block_of_the_null_stream_is_recorded_when_somebody_else_takes_it(recorded):
