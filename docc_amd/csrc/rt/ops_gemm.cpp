@@ -105,11 +105,16 @@ struct WavesChoice {
     bool one;        // no compute unit has two
     double seconds;
 };
-WavesChoice waves_choice(int64_t m, int64_t n, int64_t k, int cus, size_t elem, int forced) {
+// `lines`: rows of both operands are whole lines of 128 bytes. Off them a piece of a row takes two lines, which for fp32 and fp64 on 16 x 16 tiles (the least work a byte)
+// are no longer in the caches when the next piece wants them: fp64 581 x 194 x 2322 1.35 times the estimate, 266 x 1411 x 3730 1.55, 968 x 183 x 5886 1.62, with a tile a
+// compute unit from 4300 k on; fp32 1130 x 262 x 5032 1.35, 1880 x 137 x 6228 1.49. Other tiles and bf16 no different.
+WavesChoice waves_choice(int64_t m, int64_t n, int64_t k, int cus, size_t elem, bool lines, int forced) {
     auto per_cu = [&](int64_t edge) { return (double) ((((m + edge - 1) / edge) * ((n + edge - 1) / edge) + cus - 1) / cus); };
     const double n16 = per_cu(16), n32 = per_cu(32), n64 = per_cu(64), kd = (double) k;
     const bool one = n64 <= 1.0 && (elem == 4 || k > 1024);
-    const double t16 = elem == 2 ? 3.8 + n16 * (0.4 + 0.00065 * kd) : elem == 4 ? 4.0 + n16 * (0.5 + 0.00125 * kd) : 3.8 + n16 * (0.6 + 0.0024 * kd);
+    const double straddle = lines || elem == 2 ? 1.0 : elem == 4 ? (n16 <= 1.0 ? 1.0 : k < 7800 ? 1.0 + kd / 13000.0 : 1.6)
+                            : n16 > 1.0 ? (k < 5400 ? 1.0 + kd / 9000.0 : 1.6) : k < 4300 ? 1.0 : 1.4;
+    const double t16 = elem == 2 ? 3.8 + n16 * (0.4 + 0.00065 * kd) : elem == 4 ? 4.0 + n16 * (0.5 + 0.00125 * straddle * kd) : 3.8 + n16 * (0.6 + 0.0024 * straddle * kd);
     const double t32 = elem == 2 ? 3.4 + n32 * (0.75 + 0.0010 * kd) : elem == 4 ? 3.7 + n32 * (0.75 + 0.0043 * kd) : 3.8 + n32 * (0.9 + 0.0092 * kd);
     const double t64 = elem == 2 ? (one ? 4.75 + 0.0028 * kd : 1.9 + n64 * (2.1 + 0.0027 * kd))
                                  : 3.7 + n64 * (1.2 + 0.0172 * kd);
@@ -383,7 +388,7 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
         if (fin && !ta && tb && batch == 1 && forced != 0 && n % 8 == 0 && waves_shape_ok(m, n, k, lda, ldb, true, sizeof(T)) &&
             ((uintptr_t) A | (uintptr_t) B | (uintptr_t) fin->bias | (uintptr_t) fin->residual | (uintptr_t) fin->out) % 16 == 0) {
             const bool on_lines = ((uintptr_t) A | (uintptr_t) B | (uintptr_t) (lda * (int64_t) sizeof(T)) | (uintptr_t) (ldb * (int64_t) sizeof(T))) % 128 == 0;
-            const WavesChoice w = waves_choice(m, n, k, cus, sizeof(T), forced);
+            const WavesChoice w = waves_choice(m, n, k, cus, sizeof(T), on_lines, forced);
             // Up to 32 rows (against the kernels with K in parts and a pass behind them): bf16 1 x 2048 -> 8192 9.9 us and 7.8, 8 x 2048 -> 8192 12.7 and 7.8,
             // 16 x 12288 -> 3072 21.3 and 14.2, 32 x 4096 -> 1024 14.6 and 5.6; fp32 21.2 and 12.7 (8 x 2048), 40.6 and 35.3, 16.2 and 9.1. But a single row of
             // a large matrix is read by the matrix-vector kernel: fp32 1 x 4096 -> 14336 42.6 us here and 39.7, bf16 1 x 8192 -> 28672 78.8 and 73.4; a block of 1 x 3072
@@ -402,8 +407,7 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
             }
         }
     }
-    auto waves_plain = [&](int forced) {
-        const WavesChoice w = waves_choice(m, n, k, cus, sizeof(T), forced);
+    auto waves_plain = [&](const WavesChoice& w) {
         const int64_t tiles = ((m + w.edge - 1) / w.edge) * ((n + w.edge - 1) / w.edge);
         std::snprintf(name, sizeof(name), "docc_%cgemm_waves_%dx%d%s_n%c", prefix[0], w.edge, w.edge, w.one ? "_one" : "", tb ? 't' : 'n');
         // the rings, or the sums of all wavefronts or (above 64 KB) of half of them
@@ -419,13 +423,16 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
         for (const char* other : {"DOCC_ROCM_GEMM_CFG", "DOCC_ROCM_GEMM_TILE", "DOCC_ROCM_GEMM_SPLITK", "DOCC_ROCM_GEMM_SKINNY", "DOCC_ROCM_GEMV_OFF", "DOCC_ROCM_GEMV_SLICES"})
             if (forced < 0 && tuning(other)) forced = 0;
         bool pays = false;
+        const bool on_lines = ((uintptr_t) A | (uintptr_t) B | (uintptr_t) (lda * (int64_t) sizeof(T)) | (uintptr_t) (ldb * (int64_t) sizeof(T))) % 128 == 0;
+        const WavesChoice w = waves_choice(m, n, k, cus, sizeof(T), on_lines || !tb, forced);
         if (m > 32) {
             // by the estimates: fp32 512 x 512 x 512 10.6 -> 6.2 us, 192 x 64 x 1664 11.6 -> 5.6, 64 x 5824 x 896 15.7 -> 12.7;
             // fp64 512 x 512 x 512 12.0 -> 8.6
-            const bool on_lines = ((uintptr_t) A | (uintptr_t) B | (uintptr_t) (lda * (int64_t) sizeof(T)) | (uintptr_t) (ldb * (int64_t) sizeof(T))) % 128 == 0;
-            // (315 x 600 x 3584, B [k][n] 23.2 us and 26.2: not above k = 2048 there)
-            // B [n][k] in whole rounds of the wavefronts only (four of 32 k in fp32); a K off them stays with the parts, whose tests hold such products
-            pays = forced < 0 && (tb ? k % 128 == 0 : k <= 2048) && waves_choice(m, n, k, cus, sizeof(T), forced).seconds < 0.85 * tiles_seconds(pick, m, n, k, tb, cus, sizeof(T), on_lines);
+            // (315 x 600 x 3584, B [k][n] 23.2 us and 26.2: not above k = 2048 there). Of 700 drawn products with B [n][k], k a multiple of 128 or not, 412 changed, fp32 1.47
+            // times as fast and fp64 1.34 (geometric means; 7 % slower at most); below 64 and 128 k a launch of either takes 5 us (52 x 1512 x 32 in fp64 4.5 and 6.0). From 40 us on the other estimate is
+            // too high by a quarter in fp64: 1242 x 251 x 3584 59 us for 47, on tiles of 16 x 16 here 51 (those of 32 x 32 still win there: 216 x 906 x 3844 44.3 -> 39.7).
+            const double margin = sizeof(T) == 8 && w.edge == 16 && w.seconds > 40e-6 ? 0.7 : 0.85;
+            pays = forced < 0 && (tb ? k >= (sizeof(T) == 4 ? 64 : 128) : k <= 2048) && w.seconds < margin * tiles_seconds(pick, m, n, k, tb, cus, sizeof(T), on_lines);
         } else if (tb) {
             // Against the matrix-vector kernels, the skinny ones and K in parts, B stored [n][k]: fp32 2 x 8192 x 2048 24 -> 12 us, 8 x 2048 x 2048 11.2 -> 6.1, 32 x
             // 8192 x 8192 96 -> 59; fp64 8 x 8192 x 2048 40 -> 22, but 8 x 512 x 8192 19.5 and 23.4
@@ -436,7 +443,7 @@ int gemm_launch(const char* prefix, docc_rocm_stream_t stream, int trans_a, int 
             // fp64 8 x 2048 x 2048 15.3 -> 9.6
             pays = k <= 2048 && n * k <= (int64_t(1) << 24);
         }
-        if (forced > 0 || (pays && forced < 0)) return waves_plain(forced);
+        if (forced > 0 || (pays && forced < 0)) return waves_plain(w);
     }
     const bool epilogue = bias || activation >= 0;
     // A tall matrix times a few columns held as numpy holds them (B [k][n], n small): rows of B are a few elements long, so

@@ -45,10 +45,13 @@ def test_packed_products_by_size_alone(kind):
 
 @pytest.mark.parametrize("kind", list(KINDS))
 @pytest.mark.parametrize("m,n,k", [(100, 104, 1000), (64, 128, 4264), (152, 200, 8016), (40, 320, 2056), (16, 16, 704)])
-def test_parts_of_different_lengths(kind, m, n, k):
-    for tb in (False, True):
-        check(kind, m, n, k, False, tb)
-    check(kind, m, n, k, True, False, alpha=0.5, beta=1.0)
+def test_parts_of_different_lengths(monkeypatch, kind, m, n, k):
+    for waves in (None, "0"):       # 0: not between the wavefronts of a work-group, which most of these are chosen for
+        if waves:
+            monkeypatch.setenv("DOCC_ROCM_GEMM_WAVES", waves)
+        for tb in (False, True):
+            check(kind, m, n, k, False, tb)
+        check(kind, m, n, k, True, False, alpha=0.5, beta=1.0)
 
 
 @pytest.mark.parametrize("kind", list(KINDS))

@@ -291,7 +291,7 @@ print("\\n".join(l for l in take() if l.startswith("launch")))
     assert ("docc_gemm_pack_b4" in got[0]) == packed, got
 
 
-# the shapes of tests/test_gpu_gemm_pack.py whose K is to be cut into parts of different lengths are cut so
+# the shapes of tests/test_gpu_gemm_pack.py whose K is to be cut into parts of different lengths are cut so, with the switch that its second run sets
 @pytest.mark.parametrize("kind", ["dgemm", "sgemm", "bf16gemm_f32"])
 def test_k_is_cut_into_parts_of_different_lengths(recorded, kind):
     from test_gpu_gemm_pack import test_parts_of_different_lengths as cases
@@ -300,7 +300,7 @@ def test_k_is_cut_into_parts_of_different_lengths(recorded, kind):
         got = recorded(f"""
 rt.{kind}({m}, {n}, {k}, 1.0, A, {k}, B, {k}, 0.0, C, {n}, trans_b=rt.TRANS)
 print("\\n".join(l for l in take() if l.startswith("launch")))
-""")
+""", DOCC_ROCM_GEMM_WAVES="0")
         parts = int(got[0].split()[2].split(",")[1])
         part = ((k + parts - 1) // parts + 63) // 64 * 64
         if (kind, m) == ("bf16gemm_f32", 16):
@@ -437,3 +437,15 @@ for _ in range(300):
 print(asked)
 """)
     assert int(got[0]) == 0
+
+
+# K between the wavefronts of a work-group whether it is a multiple of their rounds or not; in fp64 not where rows off the lines of 128 bytes are read over and over
+@pytest.mark.parametrize("kind,m,n,k,waves", [("s", 512, 512, 512, True), ("s", 512, 512, 576, True), ("s", 512, 512, 580, True), ("s", 204, 172, 100, True), ("s", 1402, 409, 32, False),
+                                              ("d", 512, 512, 512, True), ("d", 512, 512, 514, True), ("d", 97, 744, 286, True), ("d", 285, 205, 56, False),
+                                              ("d", 968, 183, 5886, False), ("d", 266, 1411, 3730, False), ("d", 1242, 251, 3584, False), ("d", 216, 906, 3844, True)])
+def test_k_off_the_rounds_of_the_wavefronts(recorded, kind, m, n, k, waves):
+    got = recorded(f"""
+rt.{kind}gemm({m}, {n}, {k}, 1.0, A, {k}, B, {k}, 0.0, C, {n}, trans_b=rt.TRANS)
+print("\\n".join(l for l in take() if l.startswith("launch")))
+""")
+    assert ("_waves_" in got[0]) == waves, got
