@@ -243,6 +243,22 @@ def main():
             entry.update(extra)
         kernels[name] = entry
 
+    def conv_matrix_pipe(flops, ms, stride, fn, iters):
+        """3x3 layers run in Winograd's form, with 16 (steps of two 25) products for the direct sum's 36, where that is the faster one: `flop` and `frac` stay the
+        direct sum's, a speed and no use of the pipe. What the pipe is used is the products that run; beside it the time as a direct sum."""
+        if os.environ.get("DOCC_ROCM_CONV"):
+            return {}
+        os.environ["DOCC_ROCM_CONV"] = "direct"
+        try:
+            direct_ms = time_kernel(fn, iters, 8)
+        finally:
+            del os.environ["DOCC_ROCM_CONV"]
+        if direct_ms < 1.05 * ms:       # the direct sum is what runs
+            return {"direct_sum_us": round(direct_ms * 1e3, 2)}
+        share = (16 if stride == 1 else 25) / 36
+        return {"direct_sum_us": round(direct_ms * 1e3, 2), "products_run_of_direct_sum": round(share, 4),
+                "products_run_TFLOPs": round(flops * share / ms / 1e9, 1), "frac_of_products_run": round(flops * share / ms / 1e9 / PEAK_TFLOPS["f32"], 4)}
+
     # ---- config 1: fp64 GEMM 1000^3 ---------------------------------------------------
     if want("dgemm"):
         n = 1000
@@ -372,7 +388,7 @@ def main():
             t = cpu_time(lambda: oracle.conv2d(x, w, bb, pad=(1, 1), lib=oracle_lib), reps=1)
             cpu = {"value": round(flops / t / 1e12, 4), "unit": "TFLOP/s", "cores": cores, "kind": "port",
                    "sample": "full problem, the reference's loop nest with a zero-padding guard (omp over n)"}
-        add_kernel("conv2d_n32c64hw56k3", "f32", flops, ms, cpu, fn=run)
+        add_kernel("conv2d_n32c64hw56k3", "f32", flops, ms, cpu, extra=conv_matrix_pipe(flops, ms, 1, run, 100), fn=run)
 
     # ---- elementwise tensor nodes on the softmax tensor's shape (HBM-bound) --------------------
     if want("elementwise"):
@@ -531,8 +547,9 @@ def main():
             b = (torch.randn(OC) * 0.1).cuda()
             OH = (H + 2 - 3) // st + 1
             Y = torch.empty(32, OC, OH, OH, device="cuda")
-            mfma(name, "f32", 2 * 32 * OC * OH * OH * C * 9,
-                 lambda i: rt.conv2d_f32(32, C, H, H, OC, 3, 3, (st, st), (1, 1), (1, 1), X.data_ptr(), W.data_ptr(), b.data_ptr(), Y.data_ptr(), stream=stream))
+            run = lambda i: rt.conv2d_f32(32, C, H, H, OC, 3, 3, (st, st), (1, 1), (1, 1), X.data_ptr(), W.data_ptr(), b.data_ptr(), Y.data_ptr(), stream=stream)
+            mfma(name, "f32", 2 * 32 * OC * OH * OH * C * 9, run)
+            other[name].update(conv_matrix_pipe(other[name]["flop"], other[name]["kernel_us"] / 1e3, st, run, 48))
             del X, W, b, Y
         # a depthwise layer (group == C): nine multiply-adds per element against eight bytes moved, bound by HBM; four
         # input tensors of 103 MB in turn
