@@ -285,16 +285,22 @@ bool direct_1x1_shape_ok(int64_t N, int64_t C, int64_t H, int64_t W, int64_t OC,
 
 // Where it pays, measured on 34 layers: with steps always (32 x 128 x 28 x 28 -> 256 19 -> 13 us, 13 x 256 x 57 x 57 -> 512 84 -> 46, 36 x 32 x 12 x 12 -> 64
 // 9 -> 7); without, 16 x 128 x 28 x 28 -> 512 52 -> 32 us, 64 x 2048 x 7 x 7 -> 512 189 -> 89, but not where few work-groups have many channels (1 x 512 x 28 x 28
-// -> 128: 17 us for the batched product's 13) nor where many have two chunks of them (32 x 64 x 56 x 56 -> 256: 70 us for the strips' 65).
-bool direct_1x1_pays(int64_t N, int64_t C, int64_t OC, int64_t OH, int64_t OW, int64_t stride_h, int64_t stride_w, int cus) {
-    if (stride_h > 1 || stride_w > 1) return true;
+// -> 128: 17 us for the batched product's 13) nor where many have two chunks of them (32 x 64 x 56 x 56 -> 256: 70 us for the strips' 65). Of a chunk of 32
+// channels with less than 16 the rest is padding, which counts where many work-groups have it (49 x 8 x 32 x 32 -> 133 21.6 us for 13.2, 56 x 8 x 55 x 55 -> 56 26.8 and 21.9).
+// `product`: the batched product applies. It needs a pass before and one behind its own for a bias, and one for what a chain has behind the convolution (`behind`); with
+// neither it is the faster one on 60 of 67 drawn layers from 128 channels on (56 x 208 x 64 x 19 -> 192 55 us for 76, 3 x 232 x 16 x 16 -> 514 7.5 and 10.4), but not where
+// many work-groups share many output channels (3 x 176 x 34 x 34 -> 1400 36 and 29, 15 x 352 x 40 x 40 -> 416 100 and 86).
+bool direct_1x1_pays(int64_t N, int64_t C, int64_t OC, int64_t OH, int64_t OW, int64_t stride_h, int64_t stride_w, bool product, bool behind, int cus) {
     const int64_t groups = (N * OH * OW + 63) / 64 * ((OC + 63) / 64);
+    if (C < 16 && groups >= 3 * (int64_t) cus) return false;
+    if (stride_h > 1 || stride_w > 1) return true;
+    if (product && !behind) return groups >= 4 * (int64_t) cus && OC > 192;
     return C < 96 ? groups < 16 * (int64_t) cus : C <= 256 || groups >= cus / 2;
 }
 
 ConvPath choose_path(int64_t N, int64_t C, int64_t OC, int64_t KH, int64_t KW, int64_t OH, int64_t OW, int64_t stride_h, int64_t stride_w,
                      int64_t pad_h, int64_t pad_w, bool halo_ok, bool have_workspace, bool parts_ok, bool winograd_ok,
-                     bool direct_1x1_ok, int64_t* winograd_parts) {
+                     bool direct_1x1_ok, bool behind, int64_t* winograd_parts) {
     const char* force = std::getenv("DOCC_ROCM_CONV");   // halo | gather | gemm | winograd | straight (tuning and tests); direct: not Winograd's form
     if (force && force[0] == 'd') winograd_ok = false;
     const bool pointwise = KH == 1 && KW == 1 && stride_h == 1 && stride_w == 1 && pad_h == 0 && pad_w == 0;
@@ -315,7 +321,7 @@ ConvPath choose_path(int64_t N, int64_t C, int64_t OC, int64_t KH, int64_t KW, i
     // the aligned GEMM kernels want rows of the weight and column matrices that are multiples of 16 bytes
     const bool gemm_fast = gemm_ok && K % 4 == 0 && (pointwise ? P % 4 == 0 : true);
     const HaloPlan halo = halo_ok ? plan_halo(N, parts_ok ? C : 0, OC, OH, OW, KH, KW, stride_h, stride_w, cus) : HaloPlan{};
-    if (direct_1x1_ok && direct_1x1_pays(N, C, OC, OH, OW, stride_h, stride_w, cus)) {
+    if (direct_1x1_ok && direct_1x1_pays(N, C, OC, OH, OW, stride_h, stride_w, pointwise && gemm_fast && C >= 128, behind, cus)) {
         // (a chain of many chunks on few work-groups, 0.8 us each, is left to the strips with their channels in parts)
         if (!(halo.parts > 1 && halo.cost * halo_unit_us(K) < 0.8 * (double) ((C + 31) / 32) + 4.0)) return ConvPath::Direct1x1;
     }
@@ -355,7 +361,7 @@ extern "C" int64_t docc_rocm_conv2d_f32_pads_workspace_bytes(int64_t N, int64_t 
     int64_t winograd_parts = 1;
     if (choose_path(N, C, OC, KH, KW, OH, OW, stride_h, stride_w, pad_h, pad_w, halo_ok, true, false,
                     winograd_shape_ok(N, C, H, W, OC, KH, KW, OH, OW, stride_h, stride_w, begin_h, begin_w, dil_h, dil_w),
-                    direct_1x1_shape_ok(N, C, H, W, OC, KH, KW, OH, OW, stride_h, stride_w, pad_h, pad_w), &winograd_parts) != ConvPath::GemmColumns)
+                    direct_1x1_shape_ok(N, C, H, W, OC, KH, KW, OH, OW, stride_h, stride_w, pad_h, pad_w), true, &winograd_parts) != ConvPath::GemmColumns)
         return 0;
     const int64_t per_image = conv_bytes_per_image(OC, C * KH * KW, OH * OW);
     int64_t images = kConvWorkspaceCap / per_image;
@@ -374,7 +380,7 @@ extern "C" int docc_rocm_conv2d_f32_reads_workspace(docc_rocm_stream_t stream, i
     return choose_path(N, C, OC, KH, KW, OH, OW, stride_h, stride_w, any_pad_h, any_pad_w,
                        halo_shape_ok(C, KH, KW, OW, stride_h, stride_w, dil_h, dil_w) && (uintptr_t) Wt % 16 == 0, true, !foreign_capture((hipStream_t) stream),
                        winograd_shape_ok(N, C, H, W, OC, KH, KW, OH, OW, stride_h, stride_w, pad_h, pad_w, dil_h, dil_w),
-                       direct_1x1_shape_ok(N, C, H, W, OC, KH, KW, OH, OW, stride_h, stride_w, any_pad_h, any_pad_w), &winograd_parts) == ConvPath::GemmColumns;
+                       direct_1x1_shape_ok(N, C, H, W, OC, KH, KW, OH, OW, stride_h, stride_w, any_pad_h, any_pad_w), true, &winograd_parts) == ConvPath::GemmColumns;
 }
 
 extern "C" int64_t docc_rocm_conv2d_f32_workspace_bytes(int64_t N, int64_t C, int64_t H, int64_t W, int64_t OC, int64_t KH, int64_t KW,
@@ -426,7 +432,8 @@ static int conv2d_run(docc_rocm_stream_t stream, int64_t N, int64_t C, int64_t H
     int64_t winograd_parts = 1;
     ConvPath path = C == 0 ? ConvPath::Gather
                            : choose_path(N, C, OC, KH, KW, OH, OW, stride_h, stride_w, any_pad_h, any_pad_w, halo_shape, have_workspace, parts_ok,
-                                         winograd, !slice && direct_1x1_shape_ok(N, C, H, W, OC, KH, KW, OH, OW, stride_h, stride_w, any_pad_h, any_pad_w), &winograd_parts);
+                                         winograd, !slice && direct_1x1_shape_ok(N, C, H, W, OC, KH, KW, OH, OW, stride_h, stride_w, any_pad_h, any_pad_w),
+                                         bias || fin.residual || fin.relu, &winograd_parts);
     // one group of a grouped convolution: the direct kernels, which take the distance between the images as it is (the
     // GEMM paths write whole [N, OC, P] tensors)
     if (slice && (path == ConvPath::Gemm1x1 || path == ConvPath::GemmColumns)) path = halo_shape ? ConvPath::Halo : ConvPath::Gather;

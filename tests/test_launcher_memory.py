@@ -449,3 +449,23 @@ rt.{kind}gemm({m}, {n}, {k}, 1.0, A, {k}, B, {k}, 0.0, C, {n}, trans_b=rt.TRANS)
 print("\\n".join(l for l in take() if l.startswith("launch")))
 """)
     assert ("_waves_" in got[0]) == waves, got
+
+
+# 1x1 layers: on the kernel that takes the pixels as they lie, but few channels on many work-groups on the strips, and without anything behind the product on the batched
+# product, unless many work-groups share many output channels
+@pytest.mark.parametrize("N,C,H,W,OC,stride,bias,kernel", [(32, 128, 28, 28, 256, 2, True, "f32_1x1"), (16, 128, 28, 28, 512, 1, True, "f32_1x1"), (49, 8, 32, 32, 133, 1, True, "halo"),
+                                                           (59, 8, 60, 62, 24, 1, False, "halo"), (34, 12, 61, 52, 10, 1, True, "gather"), (5, 8, 34, 34, 296, 1, True, "f32_1x1"),
+                                                           (56, 208, 64, 19, 192, 1, True, "f32_1x1"), (56, 208, 64, 19, 192, 1, False, "gemm"), (3, 232, 16, 16, 514, 1, False, "gemm"),
+                                                           (3, 176, 34, 34, 1400, 1, False, "f32_1x1"), (3, 160, 21, 33, 83, 1, False, "f32_1x1")])
+def test_kernels_of_1x1_layers(recorded, N, C, H, W, OC, stride, bias, kernel):
+    got = recorded(f"""
+rt.conv2d_f32({N}, {C}, {H}, {W}, {OC}, 1, 1, ({stride}, {stride}), (0, 0), (1, 1), A, B, C if {bias} else 0, D)
+print("\\n".join(l for l in take() if l.startswith("launch")))
+""")
+    assert kernel in " ".join(got) and len(got) == 1, got
+    if not bias:        # the sum with a tensor is a pass of its own behind the batched product too
+        got = recorded(f"""
+rt.call("docc_rocm_conv2d_f32_chain", 0, {N}, {C}, {H}, {W}, {OC}, 1, 1, {stride}, {stride}, 0, 0, 0, 0, 1, 1, 1, A, B, None, C, -1, D, None, 0)
+print("\\n".join(l for l in take() if l.startswith("launch")))
+""")
+        assert ("f32_1x1" in got[0]) == (kernel != "halo") and len(got) == (2 if kernel == "halo" else 1), got
