@@ -107,7 +107,9 @@ struct WavesChoice {
 };
 // `lines`: rows of both operands are whole lines of 128 bytes. Off them a piece of a row takes two lines, which for fp32 and fp64 on 16 x 16 tiles (the least work a byte)
 // are no longer in the caches when the next piece wants them: fp64 581 x 194 x 2322 1.35 times the estimate, 266 x 1411 x 3730 1.55, 968 x 183 x 5886 1.62, with a tile a
-// compute unit from 4300 k on; fp32 1130 x 262 x 5032 1.35, 1880 x 137 x 6228 1.49. Other tiles and bf16 no different.
+// compute unit from 4300 k on; fp32 1130 x 262 x 5032 1.35, 1880 x 137 x 6228 1.49. bf16 on its larger tiles once they read more than so many bytes in all: of 32 x 32 175
+// MB (581 x 752 x 4184 1.5, 499 x 728 x 7064 1.52; with 164, 162 x 2208 x 3096, 1.0), of 64 x 64 120 MB (1664 x 560 x 2536 1.59, 596 x 2664 x 3880 1.8; with 101, 98 x 6776 x
+// 1864, 1.0), on the lines 400 MB in rows of more than 3000 k (644 x 5696 x 4416 1.28, 262 x 6016 x 3904 1.24). fp32 and fp64 on those no different.
 WavesChoice waves_choice(int64_t m, int64_t n, int64_t k, int cus, size_t elem, bool lines, int forced) {
     auto per_cu = [&](int64_t edge) { return (double) ((((m + edge - 1) / edge) * ((n + edge - 1) / edge) + cus - 1) / cus); };
     const double n16 = per_cu(16), n32 = per_cu(32), n64 = per_cu(64), kd = (double) k;
@@ -115,8 +117,10 @@ WavesChoice waves_choice(int64_t m, int64_t n, int64_t k, int cus, size_t elem, 
     const double straddle = lines || elem == 2 ? 1.0 : elem == 4 ? (n16 <= 1.0 ? 1.0 : k < 7800 ? 1.0 + kd / 13000.0 : 1.6)
                             : n16 > 1.0 ? (k < 5400 ? 1.0 + kd / 9000.0 : 1.6) : k < 4300 ? 1.0 : 1.4;
     const double t16 = elem == 2 ? 3.8 + n16 * (0.4 + 0.00065 * kd) : elem == 4 ? 4.0 + n16 * (0.5 + 0.00125 * straddle * kd) : 3.8 + n16 * (0.6 + 0.0024 * straddle * kd);
-    const double t32 = elem == 2 ? 3.4 + n32 * (0.75 + 0.0010 * kd) : elem == 4 ? 3.7 + n32 * (0.75 + 0.0043 * kd) : 3.8 + n32 * (0.9 + 0.0092 * kd);
-    const double t64 = elem == 2 ? (one ? 4.75 + 0.0028 * kd : 1.9 + n64 * (2.1 + 0.0027 * kd))
+    auto reads_mb = [&](int64_t edge) { return 1e-6 * (double) (((m + edge - 1) / edge) * ((n + edge - 1) / edge)) * 4.0 * (double) edge * kd; };
+    const double far32 = !lines && reads_mb(32) > 175.0 ? 1.5 : 1.0, far64 = lines ? (k > 3000 && reads_mb(64) > 400.0 ? 1.25 : 1.0) : reads_mb(64) > 120.0 ? 1.5 : 1.0;
+    const double t32 = elem == 2 ? 3.4 + n32 * (0.75 + 0.0010 * far32 * kd) : elem == 4 ? 3.7 + n32 * (0.75 + 0.0043 * kd) : 3.8 + n32 * (0.9 + 0.0092 * kd);
+    const double t64 = elem == 2 ? (one ? 4.75 + 0.0028 * far64 * kd : 1.9 + n64 * (2.1 + 0.0027 * far64 * kd))
                                  : 3.7 + n64 * (1.2 + 0.0172 * kd);
     if (forced > 0 ? forced == 16 : m <= 16 || (t16 < t32 && (elem == 8 || t16 < t64))) return {16, false, 1e-6 * t16};
     // (fp64: 64 x 64 tiles of 1000 k took 39.0 us for the 37.0 of gemm_async.h's)

@@ -469,3 +469,14 @@ rt.call("docc_rocm_conv2d_f32_chain", 0, {N}, {C}, {H}, {W}, {OC}, 1, 1, {stride
 print("\\n".join(l for l in take() if l.startswith("launch")))
 """)
         assert ("f32_1x1" in got[0]) == (kernel != "halo") and len(got) == (2 if kernel == "halo" else 1), got
+
+
+# layers in bf16: K between the wavefronts, but not where the rows of many tiles are read from beyond the caches, off the lines of 128 bytes above all
+@pytest.mark.parametrize("m,n,k,waves", [(1024, 1024, 256, True), (162, 2208, 3096, True), (98, 6776, 1864, True), (596, 2664, 3880, False), (720, 2464, 4696, False), (146, 1952, 6488, False),
+                                         (489, 3408, 4680, False), (124, 1936, 3848, True), (644, 5696, 4416, False), (302, 2704, 5504, True)])
+def test_layers_with_long_rows(recorded, m, n, k, waves):
+    got = recorded(f"""
+rt.call("docc_rocm_linear", 0, 1, 111, 112, {m}, {n}, {k}, 1.0, A, {k}, B, {k}, C, 1, 2, None, 1, 0, D, 1)
+print("\\n".join(l for l in take() if l.startswith("launch")))
+""")
+    assert ("_waves_" in got[0]) == waves, got
